@@ -509,7 +509,8 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     const bool ring = in.ldo <= 2048 && (long long)in.xrows * in.ldo * es < (1LL << 31);
     items[hfjk::kPhSyrk] = ring ? 0 : (long long)in.npairs * in.nsplit;
     items[hfjk::kPhSyrkRing] = ring ? (long long)in.npairs * in.nsplit : 0;
-    items[hfjk::kPhSyrkReduce] = (nn + hfjk::kThreads - 1) / hfjk::kThreads;
+    // Strips of 512 elements of every lower tile.
+    items[hfjk::kPhSyrkReduce] = (long long)in.npairs * (in.st * in.st / (2 * hfjk::kThreads));
     items[hfjk::kPhCharges] = in.naux;
     for (int ph = 0; ph < hfjk::kPhCount; ++ph) {
       const size_t base = (size_t)ph * (ninst + 1);

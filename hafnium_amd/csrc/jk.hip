@@ -145,13 +145,27 @@ __global__ __launch_bounds__(kThreads) void gamma_kernel(const void* __restrict_
   }
 }
 
-__global__ __launch_bounds__(kThreads) void gamma_reduce_kernel(const double* __restrict__ partial, int ntiles,
-                                                                 int naux, double* __restrict__ gamma) {
-  const int q = blockIdx.x * kThreads + threadIdx.x;
-  if (q >= naux) return;
+// gamma[q] = sum over the tiles: 16 thread groups share the tiles of 64 aux
+// functions, combined in LDS in a fixed order (one thread per aux function
+// walking every tile took 57 us for 136 tiles).
+constexpr int kRedGroups = 16;
+
+__global__ __launch_bounds__(64 * kRedGroups) void gamma_reduce_kernel(const double* __restrict__ partial, int ntiles,
+                                                                       int naux, double* __restrict__ gamma) {
+  __shared__ double red[kRedGroups][64];
+  const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
+  const int q = blockIdx.x * 64 + lane;
   double s = 0.0;
-  for (int t = 0; t < ntiles; ++t) s += partial[(long long)t * naux + q];
-  gamma[q] = s;
+  if (q < naux) {
+#pragma unroll 4
+    for (int t = group; t < ntiles; t += kRedGroups) s += partial[(long long)t * naux + q];
+  }
+  red[group][lane] = s;
+  __syncthreads();
+  if (group == 0 && q < naux) {
+    for (int g = 1; g < kRedGroups; ++g) s += red[g][lane];
+    gamma[q] = s;
+  }
 }
 
 // partial[s][e] = sum over the s-th aux slice of gamma[q] B[q][e], one
@@ -182,24 +196,50 @@ __global__ __launch_bounds__(kThreads) void coulomb_accumulate_kernel(const void
   }
 }
 
-__global__ __launch_bounds__(kThreads) void coulomb_unpack_kernel(const double* __restrict__ partial, int nsplit,
-                                                                   long long p, int nao,
-                                                                   double* __restrict__ out) {
-  const long long total = (long long)nao * nao;
-  for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < total;
-       idx += (long long)gridDim.x * kThreads) {
-    const int row = (int)(idx / nao);
-    const int col = (int)(idx % nao);
-    const int r = row / kTile, c = col / kTile;
-    long long src;
-    if (r >= c) {
-      src = tile_index(r, c) * kTileElems + (row % kTile) * kTile + col % kTile;
-    } else {
-      src = tile_index(c, r) * kTileElems + (col % kTile) * kTile + row % kTile;
-    }
-    double s = 0.0;
-    for (int k = 0; k < nsplit; ++k) s += partial[(long long)k * p + src];
-    out[idx] = s;
+// J [nao][nao] from the packed partials: one workgroup per packed tile, PARTS
+// thread groups sharing the slices (combined in a fixed order), the tile and,
+// through LDS, its mirror written by rows. (One thread per element of J over
+// a serial chain of 75 slices, half of it reading by columns, took 26 us at
+// nao 100; four groups take 5.)
+template <int PARTS>
+__global__ __launch_bounds__(kThreads* PARTS) void coulomb_unpack_kernel(const double* __restrict__ partial,
+                                                                          int nsplit, long long p, int nao,
+                                                                          double* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) double sums[PARTS][kTileElems];
+  int r, c;
+  tile_rc(blockIdx.x, r, c);
+  const int part = threadIdx.x / kThreads;
+  const int e = (threadIdx.x % kThreads) * 4;
+  const double* src = partial + (long long)blockIdx.x * kTileElems + e;
+  double2 a = make_double2(0.0, 0.0), b = a;
+#pragma unroll 4
+  for (int k = part; k < nsplit; k += PARTS) {
+    const double2* v = (const double2*)(src + (long long)k * p);
+    const double2 v0 = v[0], v1 = v[1];
+    a.x += v0.x;
+    a.y += v0.y;
+    b.x += v1.x;
+    b.y += v1.y;
+  }
+  *(double2*)&sums[part][e] = a;
+  *(double2*)&sums[part][e + 2] = b;
+  __syncthreads();
+#pragma unroll
+  for (int local = threadIdx.x; local < kTileElems; local += kThreads * PARTS) {
+    double s = sums[0][local];
+#pragma unroll
+    for (int k = 1; k < PARTS; ++k) s += sums[k][local];
+    if (PARTS > 1) sums[0][local] = s;
+    const int row = r * kTile + local / kTile, col = c * kTile + local % kTile;
+    if (row < nao && col < nao) out[(long long)row * nao + col] = s;
+  }
+  if (r == c) return;
+  __syncthreads();
+#pragma unroll
+  for (int local = threadIdx.x; local < kTileElems; local += kThreads * PARTS) {
+    const int i = local / kTile, j = local % kTile;
+    const int row = c * kTile + i, col = r * kTile + j;
+    if (row < nao && col < nao) out[(long long)row * nao + col] = sums[0][j * kTile + i];
   }
 }
 
@@ -436,8 +476,8 @@ hipError_t launch_gamma(const void* b, int precision, long long p, int naux, int
 }
 
 hipError_t launch_gamma_reduce(const double* partial, int ntiles, int naux, double* gamma, hipStream_t s) {
-  hipLaunchKernelGGL(gamma_reduce_kernel, dim3((unsigned)((naux + kThreads - 1) / kThreads)), dim3(kThreads), 0, s,
-                     partial, ntiles, naux, gamma);
+  hipLaunchKernelGGL(gamma_reduce_kernel, dim3((unsigned)((naux + 63) / 64)), dim3(64 * kRedGroups), 0, s, partial,
+                     ntiles, naux, gamma);
   return hipGetLastError();
 }
 
@@ -460,9 +500,13 @@ hipError_t launch_coulomb_accumulate(const void* b, int precision, long long p, 
 
 hipError_t launch_coulomb_unpack(const double* partial, int nsplit, long long p, int nao, double* out,
                                  hipStream_t s) {
-  const long long n = (long long)nao * nao;
-  hipLaunchKernelGGL(coulomb_unpack_kernel, dim3(grid_for(n)), dim3(kThreads), 0, s,
-                     partial, nsplit, p, nao, out);
+  // Few slices (large nao): small workgroups, which find room beside a SYRK that holds most of
+  // every CU (1024-thread ones waited for its end: 0.4 ms at nao 1500).
+  const dim3 grid((unsigned)(p / kTileElems));
+  if (nsplit <= 8)
+    hipLaunchKernelGGL(coulomb_unpack_kernel<1>, grid, dim3(kThreads), 0, s, partial, nsplit, p, nao, out);
+  else
+    hipLaunchKernelGGL(coulomb_unpack_kernel<4>, grid, dim3(kThreads * 4), 0, s, partial, nsplit, p, nao, out);
   return hipGetLastError();
 }
 

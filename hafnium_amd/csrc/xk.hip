@@ -2347,90 +2347,95 @@ __global__ __launch_bounds__(kThreads) void expand_full16_kernel(const double* _
   }
 }
 
-// K from the partial tiles: one workgroup per (lower tile pair, 8-row strip
-// of the tile); each thread sums 4 elements of the strip over the slots in
-// a fixed order (reads coalesced along the tile's rows), writes them to
-// K[bm rows][bn columns], and for an off-diagonal pair the mirror
-// K[bn rows][bm columns] through an LDS transpose (writes coalesced too).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void syrk_reduce_kernel(const T* __restrict__ partial, int nslot,
-                                                                int npairs, int nao, double* __restrict__ out) {
-  constexpr int kStrip = 8;
-  __shared__ double mirror[kStrip][kSyrkTile + 1];
-  const int pair = blockIdx.x / (kSyrkTile / kStrip);
-  const int strip = blockIdx.x % (kSyrkTile / kStrip);
-  int bm, bn;
-  tile_of(pair, bm, bn);
-  const int t = threadIdx.x;
-  const int col = t & (kSyrkTile - 1);  // 0..127
-  const int r0 = t >> 7;                 // 0..1
+// Sum over the partial slots k = part, part + PARTS, ... of two neighbouring
+// elements, eight loads in flight.
+template <typename T, int PARTS>
+__device__ __forceinline__ double2 slot_sum(const T* __restrict__ src, int part, int nslot, long long stride) {
+  typedef T pair_t __attribute__((ext_vector_type(2)));
+  double2 sum = make_double2(0.0, 0.0);
+  int k = part;
+  for (; k + 7 * PARTS < nslot; k += 8 * PARTS) {
+    pair_t v[8];
 #pragma unroll
-  for (int rr = 0; rr < kStrip / 2; ++rr) {
-    const int lr = r0 + 2 * rr;              // row within the strip
-    const int trow = strip * kStrip + lr;    // row within the tile
-    const T* src = partial + (long long)pair * (kSyrkTile * kSyrkTile) + trow * kSyrkTile + col;
-    double sum = 0.0;
-    for (int k = 0; k < nslot; ++k) sum += (double)src[(long long)k * npairs * (kSyrkTile * kSyrkTile)];
-    const int row = bm * kSyrkTile + trow, c = bn * kSyrkTile + col;
-    if (row < nao && c < nao) out[(long long)row * nao + c] = sum;
-    mirror[lr][col] = sum;
+    for (int u = 0; u < 8; ++u) v[u] = *(const pair_t*)(src + (long long)(k + u * PARTS) * stride);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum.x += (double)v[u].x;
+      sum.y += (double)v[u].y;
+    }
   }
-  if (bm == bn) return;
-  __syncthreads();
-  // Mirror: K[bn * 128 + col][bm * 128 + strip rows] = strip[row][col].
-  for (int e = t; e < kStrip * kSyrkTile; e += kThreads) {
-    const int mc = e / kStrip;   // column of the tile -> row of the mirror
-    const int mr = e % kStrip;   // row of the strip -> column of the mirror
-    const int row = bn * kSyrkTile + mc, c = bm * kSyrkTile + strip * kStrip + mr;
-    if (row < nao && c < nao) out[(long long)row * nao + c] = mirror[mr][mc];
+  for (; k < nslot; k += PARTS) {
+    const pair_t v = *(const pair_t*)(src + (long long)k * stride);
+    sum.x += (double)v.x;
+    sum.y += (double)v.y;
   }
+  return sum;
 }
 
-// The symmetric-plus-antisymmetric reduce of the non-symmetric exchange:
-// per 8-row strip of a lower tile pair, S = sum of `sym`'s slots and A = sum
-// of `anti`'s; K[m][n] (+)= S + A on the tile, K[n][m] (+)= S - A on its
-// mirror (skipped for diagonal tiles, which hold both triangles).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void syrk_reduce2_kernel(const T* __restrict__ sym, const T* __restrict__ anti,
-                                                                 int nslot, int npairs, int nao, int accumulate,
-                                                                 double* __restrict__ out) {
-  constexpr int kStrip = 8;
-  __shared__ double mirror[kStrip][kSyrkTile + 1];
-  const int pair = blockIdx.x / (kSyrkTile / kStrip);
-  const int strip = blockIdx.x % (kSyrkTile / kStrip);
+// K from the partial tiles: one workgroup per (lower tile pair, STRIP rows of
+// the tile). 64 threads hold a row (two elements each, coalesced) and PARTS
+// thread groups share the slots, combined in LDS in a fixed order, so the
+// result does not depend on the run. The lower triangle is written to
+// K[bm rows][bn columns] and, through the LDS copy, to its mirror
+// K[bn rows][bm columns]; elements above the diagonal of a diagonal tile are
+// not read (the masked kernels leave them unwritten).
+// With ANTI (the non-symmetric exchange), S = sum of `partial`'s slots and
+// A = sum of `anti`'s: K[m][n] (+)= S + A, K[n][m] (+)= S - A.
+//
+// Bound by the latency of the slot chain when the tiles are few and the slots
+// many (one tile, 304 slots: 16 workgroups walking 304 dependent loads took
+// 311 us of a 362 us build at nao 100; 8 groups of 8 loads in flight take the
+// chain to a few), by HBM otherwise.
+constexpr int kRedThreads = 512;
+
+template <typename T, int STRIP, bool ANTI>
+__global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __restrict__ partial,
+                                                                  const T* __restrict__ anti, int nslot, int npairs,
+                                                                  int nao, int accumulate, double* __restrict__ out) {
+  constexpr int PARTS = kRedThreads / (STRIP * (kSyrkTile / 2));
+  constexpr int NS = ANTI ? 2 : 1;
+  constexpr int LD = kSyrkTile + 2;
+  __shared__ __attribute__((aligned(16))) double part_sum[NS][PARTS][STRIP][LD];
+  const int pair = blockIdx.x / (kSyrkTile / STRIP);
+  const int strip = blockIdx.x % (kSyrkTile / STRIP);
   int bm, bn;
   tile_of(pair, bm, bn);
+  const int row0 = bm * kSyrkTile + strip * STRIP;
+  if (row0 >= nao) return;
   const int t = threadIdx.x;
-  const int col = t & (kSyrkTile - 1);
-  const int r0 = t >> 7;
-#pragma unroll
-  for (int rr = 0; rr < kStrip / 2; ++rr) {
-    const int lr = r0 + 2 * rr;
-    const int trow = strip * kStrip + lr;
-    const long long base = (long long)pair * (kSyrkTile * kSyrkTile) + trow * kSyrkTile + col;
-    double ss = 0.0, aa = 0.0;
-    for (int k = 0; k < nslot; ++k) {
-      const long long o = base + (long long)k * npairs * (kSyrkTile * kSyrkTile);
-      ss += (double)sym[o];
-      aa += (double)anti[o];
-    }
-    const int row = bm * kSyrkTile + trow, c = bn * kSyrkTile + col;
-    if (row < nao && c < nao) {
-      const long long o = (long long)row * nao + c;
-      out[o] = (accumulate ? out[o] : 0.0) + ss + aa;
-    }
-    mirror[lr][col] = ss - aa;
+  const int col = (t & (kSyrkTile / 2 - 1)) * 2;
+  const int lr = (t / (kSyrkTile / 2)) % STRIP;
+  const int part = t / (STRIP * (kSyrkTile / 2));
+  const int row = row0 + lr, gcol = bn * kSyrkTile + col;
+  const long long stride = (long long)npairs * (kSyrkTile * kSyrkTile);
+  if (row < nao && gcol < nao && gcol <= row) {
+    const long long at = (long long)pair * (kSyrkTile * kSyrkTile) + (strip * STRIP + lr) * kSyrkTile + col;
+    *(double2*)&part_sum[0][part][lr][col] = slot_sum<T, PARTS>(partial + at, part, nslot, stride);
+    if constexpr (ANTI)
+      *(double2*)&part_sum[1][part][lr][col] = slot_sum<T, PARTS>(anti + at, part, nslot, stride);
   }
-  if (bm == bn) return;
   __syncthreads();
-  for (int e = t; e < kStrip * kSyrkTile; e += kThreads) {
-    const int mc = e / kStrip;
-    const int mr = e % kStrip;
-    const int row = bn * kSyrkTile + mc, c = bm * kSyrkTile + strip * kStrip + mr;
-    if (row < nao && c < nao) {
-      const long long o = (long long)row * nao + c;
-      out[o] = (accumulate ? out[o] : 0.0) + mirror[mr][mc];
+  for (int e = t; e < STRIP * kSyrkTile; e += kRedThreads) {
+    const int r = e / kSyrkTile, c = e % kSyrkTile;
+    const int gr = row0 + r, gc = bn * kSyrkTile + c;
+    if (gr >= nao || gc > gr) continue;
+    double ss = 0.0, aa = 0.0;
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) {
+      ss += part_sum[0][q][r][c];
+      if constexpr (ANTI) aa += part_sum[1][q][r][c];
     }
+    const long long o = (long long)gr * nao + gc;
+    out[o] = (ANTI && accumulate ? out[o] : 0.0) + ss + aa;
+    part_sum[0][0][r][c] = ss - aa;
+  }
+  __syncthreads();
+  for (int e = t; e < STRIP * kSyrkTile; e += kRedThreads) {
+    const int c = e / STRIP, r = e % STRIP;
+    const int gr = row0 + r, gc = bn * kSyrkTile + c;
+    if (gr >= nao || gc >= gr) continue;
+    const long long o = (long long)gc * nao + gr;
+    out[o] = (ANTI && accumulate ? out[o] : 0.0) + part_sum[0][0][r][c];
   }
 }
 
@@ -2751,30 +2756,38 @@ hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo,
   return hipGetLastError();
 }
 
-hipError_t launch_syrk_reduce2(const void* sym, const void* anti, int precision, int nslot, int nao,
-                               bool accumulate, double* out, hipStream_t s) {
+// Strip height: 8 rows (64-byte runs in the mirror) where that fills the
+// device four times over, else 2 and 1 rows, whose workgroups split the slots
+// over 4 and 8 thread groups (nao 100: 100 workgroups instead of 13).
+template <typename T, bool ANTI>
+static hipError_t launch_reduce_t(const T* partial, const T* anti, int nslot, int nao, bool accumulate, double* out,
+                                  hipStream_t s) {
   const int npairs = syrk_pairs(nao);
-  const unsigned grid = (unsigned)(npairs * (kSyrkTile / 8));
-  if (precision == HFJK_FP64)
-    hipLaunchKernelGGL(syrk_reduce2_kernel<double>, dim3(grid), dim3(kThreads), 0, s, (const double*)sym,
-                       (const double*)anti, nslot, npairs, nao, accumulate ? 1 : 0, out);
+  const int acc = accumulate ? 1 : 0;
+  const dim3 blk(kRedThreads);
+  if (npairs * (kSyrkTile / 8) >= 1024)
+    hipLaunchKernelGGL((syrk_reduce_kernel<T, 8, ANTI>), dim3((unsigned)(npairs * (kSyrkTile / 8))), blk, 0, s,
+                       partial, anti, nslot, npairs, nao, acc, out);
+  else if (npairs * (kSyrkTile / 2) >= 512)
+    hipLaunchKernelGGL((syrk_reduce_kernel<T, 2, ANTI>), dim3((unsigned)(npairs * (kSyrkTile / 2))), blk, 0, s,
+                       partial, anti, nslot, npairs, nao, acc, out);
   else
-    hipLaunchKernelGGL(syrk_reduce2_kernel<float>, dim3(grid), dim3(kThreads), 0, s, (const float*)sym,
-                       (const float*)anti, nslot, npairs, nao, accumulate ? 1 : 0, out);
+    hipLaunchKernelGGL((syrk_reduce_kernel<T, 1, ANTI>), dim3((unsigned)(npairs * kSyrkTile)), blk, 0, s, partial,
+                       anti, nslot, npairs, nao, acc, out);
   return hipGetLastError();
 }
 
-hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, double* out, hipStream_t s) {
-  const int npairs = syrk_pairs(nao);
-  // One workgroup per 8-row strip of every lower tile pair.
-  const unsigned grid = (unsigned)(npairs * (kSyrkTile / 8));
+hipError_t launch_syrk_reduce2(const void* sym, const void* anti, int precision, int nslot, int nao,
+                               bool accumulate, double* out, hipStream_t s) {
   if (precision == HFJK_FP64)
-    hipLaunchKernelGGL(syrk_reduce_kernel<double>, dim3(grid), dim3(kThreads), 0, s, (const double*)partial, nslot,
-                       npairs, nao, out);
-  else
-    hipLaunchKernelGGL(syrk_reduce_kernel<float>, dim3(grid), dim3(kThreads), 0, s, (const float*)partial, nslot,
-                       npairs, nao, out);
-  return hipGetLastError();
+    return launch_reduce_t<double, true>((const double*)sym, (const double*)anti, nslot, nao, accumulate, out, s);
+  return launch_reduce_t<float, true>((const float*)sym, (const float*)anti, nslot, nao, accumulate, out, s);
+}
+
+hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, double* out, hipStream_t s) {
+  if (precision == HFJK_FP64)
+    return launch_reduce_t<double, false>((const double*)partial, nullptr, nslot, nao, false, out, s);
+  return launch_reduce_t<float, false>((const float*)partial, nullptr, nslot, nao, false, out, s);
 }
 
 // ------------------------------------------------------------------ batched (persistent)
@@ -3016,9 +3029,15 @@ __global__ __launch_bounds__(kThreads, 1) void batch_syrk16_ring_kernel(BatchVie
   }
 }
 
+// K of every instance from its partial tiles: one item per (lower tile pair,
+// strip of 512 elements of the tile), two neighbouring elements per thread
+// and eight slots in flight (one element per thread over a serial slot chain,
+// the upper triangle reading the tiles by columns: 122 us for 12 water
+// clusters). The lower triangle is stored and, through LDS, its mirror.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v, const T* __restrict__ kbase,
                                                                       double* __restrict__ kout) {
+  __shared__ __attribute__((aligned(16))) double sum[2 * kThreads];
   const long long* pre = v.prefix + (long long)kPhSyrkReduce * (v.ninst + 1);
   for (;;) {
     long long end;
@@ -3026,27 +3045,31 @@ __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v
     if (item >= end) break;
     const int i = batch_find(pre, v.ninst, item);
     const BatchInst in = v.insts[i];
-    const long long idx = (item - pre[i]) * kThreads + threadIdx.x;
-    if (idx < (long long)in.nao * in.nao) {
-      const int row = (int)(idx / in.nao);
-      const int col = (int)(idx % in.nao);
-      const int st = in.st;
-      const int bm = row / st, bn = col / st;
-      long long pair;
-      int local;
-      if (bm >= bn) {
-        pair = tidx(bm, bn);
-        local = (row % st) * st + col % st;
-      } else {
-        pair = tidx(bn, bm);
-        local = (col % st) * st + row % st;
-      }
-      const T* part = kbase + in.kp_off;
-      double sum = 0.0;
-      for (int s = 0; s < in.nsplit; ++s)
-        sum += (double)part[((long long)s * in.npairs + pair) * ((long long)st * st) + local];
-      kout[in.d_off + idx] = sum;
+    const int st = in.st;
+    const int rows = 2 * kThreads / st;        // tile rows of a strip
+    const int strips = st / rows;              // strips of a tile
+    const long long local = item - pre[i];
+    const int pair = (int)(local / strips), strip = (int)(local % strips);
+    int bm, bn;
+    tile_of(pair, bm, bn);
+    const int row0 = bm * st + strip * rows;
+    if (row0 >= in.nao) continue;
+    const int e = 2 * threadIdx.x;
+    const int row = row0 + e / st, col = bn * st + e % st;
+    if (row < in.nao && col <= row)
+      *(double2*)&sum[e] = slot_sum<T, 1>(kbase + in.kp_off + (long long)pair * st * st + (long long)strip * 2 * kThreads + e,
+                                          0, in.nsplit, (long long)in.npairs * st * st);
+    __syncthreads();
+    double* k = kout + in.d_off;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int f = threadIdx.x + u * kThreads;
+      const int r = row0 + f / st, c = bn * st + f % st;
+      if (r < in.nao && c <= r) k[(long long)r * in.nao + c] = sum[f];
+      const int mr = row0 + f % rows, mc = bn * st + f / rows;
+      if (mr < in.nao && mc < mr) k[(long long)mc * in.nao + mr] = sum[(f % rows) * st + f / rows];
     }
+    // batch_next's barriers keep the next item's sums behind these reads.
   }
 }
 

@@ -1,0 +1,87 @@
+"""J and K at the sizes where the sums over partial tiles change their shape, on an MI355X.
+
+The reductions pick their strip height from the number of output tiles and
+split the partial slots over thread groups, so the sizes cover one tile with
+many slots, tile edges and remainders, and every strip height.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from hafnium_amd import synthetic
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1), (2, 700, 1), (100, 1200, 20), (127, 40, 5), (128, 9, 64), (129, 300, 33), (257, 97, 64),
+          (385, 33, 7), (640, 24, 10), (1290, 3, 2)]
+
+
+def _bound(terms, magnitude):
+    """Rounding bound of sums of ``terms`` products whose absolute values sum to ``magnitude``."""
+    return (terms + 16) * 2.0 ** -53 * magnitude
+
+
+@pytest.mark.parametrize("nao,naux,nocc", SHAPES)
+def test_occupied_build_within_the_rounding_bound(nao, naux, nocc):
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+
+    b = synthetic.tensor_full(3, naux, nao)
+    c = synthetic.occupied_orbitals(3, nao, nocc)
+    jk = MI355XCoulombExchange(b)
+    j, k = jk.jk_occupied(c)
+    x = np.einsum("qmn,ni->qmi", b, c)
+    xa = np.einsum("qmn,ni->qmi", np.abs(b), np.abs(c))
+    gamma, gamma_a = np.einsum("qmi,mi->q", x, c), np.einsum("qmi,mi->q", xa, np.abs(c))
+    j_abs = np.einsum("q,qmn->mn", gamma_a, np.abs(b))
+    k_abs = np.einsum("qmi,qni->mn", xa, xa)
+    # The reference sums round too: twice the bound.
+    assert np.all(np.abs(j - np.einsum("q,qmn->mn", gamma, b)) <= 2 * _bound(naux + nao * (nocc + 1), j_abs))
+    assert np.all(np.abs(k - np.einsum("qmi,qni->mn", x, x)) <= 2 * _bound(naux * nocc + 2 * nao, k_abs))
+    np.testing.assert_array_equal(k, k.T)
+    np.testing.assert_array_equal(j, j.T)
+    j2, k2 = jk.jk_occupied(c)
+    np.testing.assert_array_equal(j, j2)
+    np.testing.assert_array_equal(k, k2)
+    np.testing.assert_allclose(jk.coulomb(c @ c.T), j, rtol=0, atol=4 * np.max(_bound(naux + nao * (nocc + 1), j_abs)))
+
+
+@pytest.mark.parametrize("nao,naux", [(1, 3), (33, 40), (129, 12), (300, 5)])
+def test_non_symmetric_density(nao, naux):
+    """The symmetric-plus-antisymmetric reduction, diagonal tiles included."""
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+
+    b = synthetic.tensor_full(5, naux, nao)
+    d = synthetic.tensor_full(6, 2, nao)[0] + np.triu(synthetic.tensor_full(7, 1, nao)[0], 1)
+    k = MI355XCoulombExchange(b).exchange(d)
+    expect = np.einsum("qmn,nl,qls->ms", b, d, b, optimize=True)
+    # Products of the eigenvectors of D: its norm and the eigensolver's rounding (n eps) scale the error.
+    top = np.einsum("qmn->", np.abs(b).max(axis=(1, 2), keepdims=True) ** 2) * nao * np.linalg.norm(d, 2)
+    assert np.max(np.abs(k - expect)) <= 64 * nao * 2.0 ** -53 * top
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+def test_batch_equals_single_builds(precision):
+    import torch
+
+    from hafnium_amd.batch import BatchedCoulombExchange
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+    from tests.tolerances import BF16X3_REL_TOL, FP32_REL_TOL
+
+    shapes = [(1, 2, 1), (31, 300, 31), (64, 7, 3), (127, 50, 40), (129, 50, 33), (260, 11, 70)]
+    batch = BatchedCoulombExchange(shapes)
+    tensors = [synthetic.tensor_full(i, q, n) for i, (n, q, _) in enumerate(shapes)]
+    orbitals = [synthetic.occupied_orbitals(i, n, o) for i, (n, _, o) in enumerate(shapes)]
+    batch.set_tensors(tensors)
+    packed = batch.pack_orbitals(orbitals)
+    j1, k1 = batch.run(packed, precision=precision)
+    j2, k2 = batch.run(packed, batch.pack_matrices([c @ c.T for c in orbitals]), precision=precision)
+    torch.cuda.synchronize()
+    tol = {"fp64": 1e-12, "fp32": FP32_REL_TOL, "bf16x3": BF16X3_REL_TOL}[precision]  # fp64: 2e4 products, 2e4 2^-53
+    for i, (b, c) in enumerate(zip(tensors, orbitals)):
+        j, k = MI355XCoulombExchange(b).jk_occupied(c)
+        for got, want in ((j1, j), (j2, j), (k1, k), (k2, k)):
+            m = batch.matrix(got, i).cpu().numpy()
+            assert np.max(np.abs(m - want)) <= tol * np.max(np.abs(want)), (precision, i)
+            np.testing.assert_array_equal(m, m.T)
