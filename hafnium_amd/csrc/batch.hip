@@ -7,6 +7,7 @@
 // kernel and one persistent kernel per phase), so a run can be captured in a
 // hipGraph and replayed.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -420,6 +421,16 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
   bt->tile = tile != 0 ? tile : (max_ldo <= 32 ? 32 : max_ldo <= 64 ? 64 : 128);
   const int es = precision == HFJK_FP64 ? 8 : precision == HFJK_FP32 ? 4 : 2;  // bf16: per plane
   long long w64 = 0, cp = 0, xx = 0, kp = 0, qq = 0;
+  hipDeviceProp_t prop;
+  if (hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) prop.multiProcessorCount = 256;
+  const int cus = std::max(8, prop.multiProcessorCount);
+  double batch_us = 0.0;
+  for (int i = 0; i < ninst; ++i) {
+    double whole_us;
+    if (instances[i].nao > 0 && instances[i].nao <= 46000)
+      batch_us += hfjk::syrk_instance_us(precision, instances[i].naux, instances[i].nao, instances[i].nocc, true, whole_us);
+  }
+  const double item_us = std::min(1700.0, std::max(40.0, batch_us / (2.0 * cus) / 4.0));
   for (int i = 0; i < ninst; ++i) {
     const hfjk_batch_instance& src = instances[i];
     if (src.nao < 1 || src.naux < 1 || src.nocc < 1 || src.nocc > src.nao || src.nao > 46000 ||
@@ -446,6 +457,7 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
       in.st = fits_ring || precision == HFJK_BF16X3 ? hfjk::syrk_tile() : 64;
       const long long nb = (in.xrows + in.st - 1) / in.st;
       in.npairs = (int)(nb * (nb + 1) / 2);
+      in.se = fits_ring && precision != HFJK_BF16X3 ? hfjk::syrk_row_block(src.nao) : in.st;
     }
     // Half-transform column tile: the smallest of 32 / 64 / 128 that covers the instance's
     // columns, at most the batch's tile (whose multiples then cover them); a batch tile of 256
@@ -456,7 +468,15 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
       in.bn = in.ldo <= 32 ? 32 : in.ldo <= 64 ? 64 : 128;
       in.bn = std::min(in.bn, bt->tile);
     }
-    in.nsplit = (int)std::max(1LL, std::min(64LL, ((long long)src.naux * in.ldo + 8191) / 8192));
+    // Splits: about 8192 k per item, and where the batch is small enough that the longest such
+    // item would outlast the others, as many as bring an instance's slowest tile down to a quarter
+    // of the batch's mean load per workgroup slot (12 water clusters: 4 rounds of items instead of
+    // a first round that holds 1.7 ms items, 2.07 -> 0.8 ms).
+    double whole_us;
+    hfjk::syrk_instance_us(precision, src.naux, src.nao, src.nocc, in.se != 64, whole_us);
+    const long long by_k = std::min(64LL, ((long long)src.naux * in.ldo + 8191) / 8192);
+    const long long by_load = std::min<long long>(src.naux, (long long)std::ceil(whole_us / item_us));
+    in.nsplit = (int)std::max(1LL, std::max(by_k, by_load));
     in.bm = bt->tile == 256 ? hfjk::batch_tile_rows(precision, 0, 256) : hfjk::batch_tile_rows(precision, in.xrows, in.bn);
     // Items cover enough aux functions for about 32 pipelined k tiles (small instances have
     // few k tiles per aux function).
@@ -535,9 +555,6 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
   bt->off_kp = off;
   off = al256(off + (size_t)(precision == HFJK_FP64 ? 8 : 4) * kp);
   bt->bytes = off;
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) prop.multiProcessorCount = 256;
-  const int cus = std::max(8, prop.multiProcessorCount);
   bt->grid_mfma = ((2 * cus + 7) / 8) * 8;
   bt->grid_elem = ((4 * cus + 7) / 8) * 8;
   *out = bt;

@@ -144,7 +144,7 @@ Layout make_layout(const hfjk_ctx* ctx, int nocc, int precision, int nsplit_k = 
   L.nsplit_j = coulomb_splits(L.ntiles, naux);
   L.nsplit_k = nsplit_k > 0 ? nsplit_k
                : ctx->syrk_splits > 0 ? ((ctx->syrk_splits + 7) / 8) * 8
-                                       : syrk_splits(L.npairs, naux);
+                                       : hfjk::syrk_split_count(precision, naux, n, L.ldo, ctx->cus);
   L.nslot_k = hfjk::syrk_slots(precision, naux, L.ldo, L.nsplit_k);
   size_t off = 0;
   const size_t nn = (size_t)n * n;
@@ -316,7 +316,7 @@ void exchange_front(hfjk_ctx* ctx, const double* orbitals, int nocc, const doubl
 }
 
 // K = sum_P X_P S X_P^T from the X that exchange_front left in the workspace.
-void exchange_back(hfjk_ctx* ctx, bool is_signed, double* out, int precision, void* ws, const Layout& L,
+void exchange_back(hfjk_ctx* ctx, int nocc, bool is_signed, double* out, int precision, void* ws, const Layout& L,
                    hipStream_t s) {
   double* sg = at<double>(ws, L.xs);
   void* x = at<void>(ws, L.xx);
@@ -324,20 +324,21 @@ void exchange_back(hfjk_ctx* ctx, bool is_signed, double* out, int precision, vo
   {
     Stage st(ctx, s, "exchange_syrk");
     check_hip(hfjk::launch_syrk(x, precision, ctx->naux, ctx->nao, L.ldo, sg, is_signed, L.nsplit_k, part,
-                                ctx->syrk_kind, s, nullptr, 0, x16_interleaved(ctx, precision, is_signed, L.ldo)),
+                                ctx->syrk_kind, s, nullptr, 0, x16_interleaved(ctx, precision, is_signed, L.ldo), nocc),
               "syrk launch");
   }
   {
     Stage st(ctx, s, "exchange_reduce");
     const int rprec = precision == HFJK_FP64 ? HFJK_FP64 : HFJK_FP32;  // BF16X3 partials are FP32
-    check_hip(hfjk::launch_syrk_reduce(part, rprec, L.nslot_k, ctx->nao, out, s), "syrk reduce launch");
+    const int edge = hfjk::syrk_edge(precision, ctx->nao, L.ldo, is_signed, ctx->syrk_kind);
+    check_hip(hfjk::launch_syrk_reduce(part, rprec, L.nslot_k, ctx->nao, edge, out, s), "syrk reduce launch");
   }
 }
 
 void run_exchange(hfjk_ctx* ctx, const double* orbitals, int nocc, const double* signs, double* out, int precision,
                   void* ws, const Layout& L, hipStream_t s) {
   exchange_front(ctx, orbitals, nocc, signs, precision, ws, L, s);
-  exchange_back(ctx, signs != nullptr, out, precision, ws, L, s);
+  exchange_back(ctx, nocc, signs != nullptr, out, precision, ws, L, s);
 }
 
 // Grid cap of the Coulomb kernels that hfjk_jk_occ runs beside the SYRK. In
@@ -896,7 +897,7 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
     // coulomb_serial on s after the SYRK. Its buffers (charges, J partials)
     // lie outside the regions the SYRK uses.
     if (serial) {
-      exchange_back(ctx, false, exchange, precision, workspace, L, s);
+      exchange_back(ctx, nocc, false, exchange, precision, workspace, L, s);
     } else {
       check_hip(hipEventRecord(ctx->fork, s), "hipEventRecord");
       check_hip(hipStreamWaitEvent(side, ctx->fork, 0), "hipStreamWaitEvent");
@@ -928,7 +929,7 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
     }
     if (!serial) {
       check_hip(hipEventRecord(ctx->join, side), "hipEventRecord");
-      exchange_back(ctx, false, exchange, precision, workspace, L, s);
+      exchange_back(ctx, nocc, false, exchange, precision, workspace, L, s);
       check_hip(hipStreamWaitEvent(s, ctx->join, 0), "hipStreamWaitEvent");
     }
   });
@@ -1384,7 +1385,7 @@ int hfjk_kpoint_exchange(hfjk_ctx* ctx, int nk, int naux, int nao, const void* t
           Stage st(ctx, s, "kpoint_syrk");
           check_hip(hfjk::launch_syrk(x, HFJK_FP64, naux, 2 * n, ldo, sg, true, L.nsplit, part, 0, s, sig),
                     "k-point syrk launch");
-          check_hip(hfjk::launch_syrk_reduce(part, HFJK_FP64, L.nsplit, 2 * n, kh, s), "k-point reduce launch");
+          check_hip(hfjk::launch_syrk_reduce(part, HFJK_FP64, L.nsplit, 2 * n, hfjk::syrk_tile(), kh, s), "k-point reduce launch");
           check_hip(hfjk::launch_kp_fold(kh, n, true, (char*)exchange + 16 * k1 * nn, s), "k-point fold launch");
         }
       }

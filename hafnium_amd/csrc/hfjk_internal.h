@@ -202,7 +202,8 @@ hipError_t launch_half_transform(const void* b, int precision, long long p, int 
 // one workgroup per CU.
 // is_signed = false promises signs[i] = 1 for every occupied column, which
 // lets the direct-LDS kernel skip them.
-// Partials: FP64 keeps one 128 x 128 tile per split and lower tile pair;
+// Partials: FP64 keeps one 128 x 128 tile per split and lower tile pair
+// (blocks above the diagonal or past nao may be left unwritten);
 // the FP32-accumulating modes (FP32, BF16x3) one per run of
 // syrk_run_aux(precision, ldo) aux functions (at most kSyrkRunProducts
 // products per FP32 accumulator, whatever the split count).
@@ -211,6 +212,8 @@ hipError_t launch_half_transform(const void* b, int precision, long long p, int 
 constexpr int kSyrkRunProducts = 4096;
 int syrk_run_aux(int precision, int ldo);
 int syrk_slots(int precision, int naux, int ldo, int nsplit);
+// Default split count of the unsigned SYRK (a multiple of 8) on a device of `cus` compute units.
+int syrk_split_count(int precision, int naux, int nao, int ldo, int cus);
 // auxsign (optional, [naux]): one more factor per aux function on the signed
 // FP64/FP32 direct-LDS kernels; shift (a multiple of 32 below ldo): the
 // second operand's columns rotated, sum_k X[m][k] S_k X[n][(k + shift) mod
@@ -218,16 +221,25 @@ int syrk_slots(int precision, int naux, int ldo, int nsplit);
 // (hipErrorInvalidValue for a launch that would not run them).
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
                        bool is_signed, int nsplit, void* partial, int kind, hipStream_t s,
-                       const double* auxsign = nullptr, int shift = 0, bool x_ilv = false);
+                       const double* auxsign = nullptr, int shift = 0, bool x_ilv = false, int nocc = 0);
+// nocc (0 = ldo): X's columns past it are zero and may be skipped.
+// syrk_edge: rows and columns of K that one of launch_syrk's tiles holds for
+// these arguments (tile (r, c) starts at row r edge, column c edge);
+// syrk_row_block: the direct-LDS kernels' equal split of the rows.
+int syrk_row_block(int nao);
+int syrk_edge(int precision, int nao, int ldo, bool is_signed, int kind);
+// Modelled time of an instance's SYRK on one workgroup slot, over all its
+// tiles, and of its slowest tile alone (the batch's split counts).
+double syrk_instance_us(int precision, int naux, int nao, int nocc, bool ring, double& whole_us);
 // Whether launch_syrk runs the BF16X3 256 x 256-tile SYRK for these
 // arguments (only that kernel reads X interleaved: x_ilv).
 bool syrk16_tiles256(int nao, int ldo, bool is_signed, int kind, int shift);
 // K (+)= the symmetric tiles sym plus the antisymmetric tiles anti: lower
 // tiles give K[m][n] = sym + anti, their mirror K[n][m] = sym - anti
-// (diagonal tiles computed whole). accumulate adds to K instead of writing.
+// (diagonal tiles: from their lower triangle). accumulate adds to K instead of writing.
 hipError_t launch_syrk_reduce2(const void* sym, const void* anti, int precision, int nslot, int nao,
                                bool accumulate, double* out, hipStream_t s);
-hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, double* out,
+hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, int edge, double* out,
                               hipStream_t s);
 hipError_t launch_occ_signs(const double* signs_in, int nocc, int ldo, double* signs_out, hipStream_t s);
 
@@ -313,7 +325,8 @@ struct BatchInst {
   int nt, xrows, npairs, nsplit;
   int nbm, nbn;       // half-transform row / column blocks of the instance's tile
   int bm, qg;         // half-transform tile rows (64 or 128; BF16x3: 128); aux functions per item (FP64 / FP32)
-  int st, bn;         // SYRK tile edge (64 or 128); half-transform column tile (32, 64, 128 or 256)
+  int st, bn;         // SYRK tile storage (64 or 128); half-transform column tile (32, 64, 128 or 256)
+  int se;             // rows and columns of K per SYRK tile (at most st)
   long long p;        // packed elements per aux function
   long long b_off;    // batch tensor (element units of the bound copy)
   long long c_off;    // orbitals [nao][nocc] (float64)

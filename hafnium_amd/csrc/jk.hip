@@ -49,7 +49,6 @@ __device__ __forceinline__ void tile_rc(int tile, int& r, int& c) {
   c = tile - rr * (rr + 1) / 2;
 }
 
-__device__ __forceinline__ long long tile_index(int r, int c) { return (long long)r * (r + 1) / 2 + c; }
 
 __device__ __forceinline__ float bf16f(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 

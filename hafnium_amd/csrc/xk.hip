@@ -24,7 +24,9 @@
 // tiles stored transposed are transposed in registers (4 x 4 blocks) on their
 // way into a [row][k] LDS tile.
 #include <algorithm>
+#include <functional>
 #include <type_traits>
+#include <vector>
 
 #include "hfjk_internal.h"
 
@@ -1236,14 +1238,21 @@ __device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" :::
 // 128 rows of each operand read at step k from src(k, operand) plus this
 // lane's byte offsets off[] (operand A = chunks of waves 0-1, B = waves 2-3).
 // With SIGNED, the B operand's k values are scaled by sgn[sign_at(k) + k']
-// times scale_at(k) (one factor per step). With MASKED, the MFMAs of this
-// wave's 16 x 16 block (mi, ni) run only where bit mi of rbits and bit ni of
-// cbits are set (wave-uniform masks; the skipped accumulators stay as they
-// were).
-template <typename T, bool SIGNED, int CH, bool MASKED = false, typename Src, typename SignAt, typename ScaleAt>
+// times scale_at(k) (one factor per step).
+//
+// Wave (wm, wn) computes the 16 x 16 blocks (wm + 2 mi, wn + 2 ni) of the
+// tile, and the MFMAs of block (mi, ni) run only where bit 4 mi + ni of its
+// wave-uniform mask is set (the skipped accumulators stay as they were): tiles
+// at the edge of the matrix skip their padding, diagonal SYRK tiles their
+// upper triangle. Interleaving the blocks over the waves rather than giving
+// each a 64 x 64 quadrant spreads what is left over the four SIMDs: a
+// diagonal tile takes 10 of 16 blocks' time and one with 2 of 8 row blocks 4
+// of 16, where quadrants took 16 and 8. An FP64 MFMA holds its SIMD for 64
+// cycles, an FP32 one for 32, so the branches around them are free.
+template <typename T, bool SIGNED, int CH, typename Src, typename SignAt, typename ScaleAt>
 __device__ __forceinline__ void dma_ring(const Src& src, const int (&off)[4 * CH], int steps,
                                          const T* __restrict__ sgn, const SignAt& sign_at, const ScaleAt& scale_at,
-                                         typename Op<T>::acc_t (&acc)[4][4], int rbits = 15, int cbits = 15) {
+                                         typename Op<T>::acc_t (&acc)[4][4], unsigned mask) {
   typedef SyrkDma<T, CH> D;
   typedef typename D::unit unit;
   constexpr int E = D::E;
@@ -1270,10 +1279,10 @@ __device__ __forceinline__ void dma_ring(const Src& src, const int (&off)[4 * CH
   // the column signs applied to the B side.
   auto read_chunk = [&](const T* stage, int step, int c, unit (&a)[4], unit (&b)[4]) {
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) a[mi] = *(const unit*)(stage + ((((wm * 4 + mi) * CH + c) * 64 + lane) * E));
+    for (int mi = 0; mi < 4; ++mi) a[mi] = *(const unit*)(stage + ((((wm + 2 * mi) * CH + c) * 64 + lane) * E));
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni)
-      b[ni] = *(const unit*)(stage + D::STAGE / 2 + ((((wn * 4 + ni) * CH + c) * 64 + lane) * E));
+      b[ni] = *(const unit*)(stage + D::STAGE / 2 + ((((wn + 2 * ni) * CH + c) * 64 + lane) * E));
     if constexpr (SIGNED) {
       const unit sg = *(const unit*)(sgn + sign_at(step) + c * D::KC + (lane >> 4) * E) * scale_at(step);
 #pragma unroll
@@ -1287,9 +1296,7 @@ __device__ __forceinline__ void dma_ring(const Src& src, const int (&off)[4 * CH
       for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
         for (int ni = 0; ni < 4; ++ni) {
-          if constexpr (MASKED) {
-            if (!((rbits >> mi) & (cbits >> ni) & 1)) continue;
-          }
+          if (!((mask >> (4 * mi + ni)) & 1u)) continue;
           acc[mi][ni] = Op<T>::mma(a[mi][e], b[ni][e], acc[mi][ni]);
         }
   };
@@ -1352,11 +1359,43 @@ __device__ __forceinline__ void dma_ring(const Src& src, const int (&off)[4 * CH
   }
 }
 
+// Mask of dma_ring for wave (wm, wn): blocks below row block nrb and column
+// block ncb of the tile and, with `lower`, on or below its diagonal.
+__device__ __forceinline__ unsigned block_mask(int wm, int wn, int nrb, int ncb, bool lower) {
+  unsigned m = 0;
+#pragma unroll
+  for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni) {
+      const int r = wm + 2 * mi, c = wn + 2 * ni;
+      m |= (unsigned)(r < nrb && c < ncb && (!lower || c <= r)) << (4 * mi + ni);
+    }
+  return m;
+}
+
+// The masked blocks of a wave's accumulators into a row-major 128 x 128 tile.
+template <typename T>
+__device__ __forceinline__ void store_tile(T* __restrict__ dst, const typename Op<T>::acc_t (&acc)[4][4], int wm,
+                                           int wn, int lane, unsigned mask) {
+#pragma unroll
+  for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni) {
+      if (!((mask >> (4 * mi + ni)) & 1u)) continue;
+      const int col = (wn + 2 * ni) * 16 + (lane & 15);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        dst[((wm + 2 * mi) * 16 + Op<T>::row(lane, r)) * kSyrkTile + col] = acc[mi][ni][r];
+    }
+}
+
 // SIGNED = false: every sign is +1 on the occupied columns (the padded
 // columns of X are zero), so the sign table is neither built nor applied.
+// Only the blocks of the lower triangle that hold rows of K are computed and
+// written.
 template <typename T, bool SIGNED, int CH>
-__global__ __launch_bounds__(kThreads, CH == 1 ? 2 : 1) void syrk_dma_kernel(
-    const T* __restrict__ x, int naux, int xrows, int ldo, const double* __restrict__ signs,
+__global__ __launch_bounds__(kThreads, 1) void syrk_dma_kernel(
+    const T* __restrict__ x, int naux, int nao, int xrows, int ldo, const double* __restrict__ signs,
     const double* __restrict__ auxsign, int shift, int nsplit, int npairs, int run, T* __restrict__ partial) {
   typedef SyrkDma<T, CH> D;
   constexpr int E = D::E;
@@ -1396,6 +1435,8 @@ __global__ __launch_bounds__(kThreads, CH == 1 ? 2 : 1) void syrk_dma_kernel(
   }
   const int nch = ldo / D::KS;
   auto sign_at = [&](int step) { return (step % nch) * D::KS; };
+  const int nblk = (nao + 15) / 16;
+  const unsigned mask = block_mask(wm, wn, nblk - 8 * mb, nblk - 8 * nb, mb == nb);
 
   for (int c = cb; c < ce; ++c) {
     int qb, qe;
@@ -1424,32 +1465,23 @@ __global__ __launch_bounds__(kThreads, CH == 1 ? 2 : 1) void syrk_dma_kernel(
     // slot's ring have returned (each ring ends waiting for them), so the
     // stage buffers may take this slot's loads.
     __syncthreads();
-    dma_ring<T, SIGNED, CH>(src, off, steps, sgn, sign_at, scale_at, acc);
+    dma_ring<T, SIGNED, CH>(src, off, steps, sgn, sign_at, scale_at, acc, mask);
 
     T* dst = partial + ((long long)c * npairs + pair) * (kSyrkTile * kSyrkTile);
-#pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-        const int col = wn * 64 + ni * 16 + (lane & 15);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = wm * 64 + mi * 16 + Op<T>::row(lane, r);
-          dst[row * kSyrkTile + col] = acc[mi][ni][r];
-        }
-      }
+    store_tile<T>(dst, acc, wm, wn, lane, mask);
   }
 }
 
-// One 128 x 128 tile (mb, nb) of sum_{q in [qb, qe)} X_q X_q^T on the ring
-// (all column signs +1: X's padded columns are zero), stored row-major into
-// dst; the MFMAs of 16-row blocks at or past nrow (X's rows past nao) are
-// skipped, and those rows and columns of dst hold zeros. The whole
+// One tile (mb, nb) of sum_{q in [qb, qe)} X_q X_q^T on the ring: rows from
+// mb edge, columns from nb edge (edge a multiple of 16 up to 128), the first
+// kcols columns of X (all signs +1, the others are zero), stored row-major
+// with 128 columns into dst; 16-row blocks at or past nrow (X's rows past nao) and blocks above the
+// diagonal of a diagonal tile are neither computed nor written. The whole
 // workgroup calls it; its LDS reads of an earlier call must have returned (a
 // workgroup barrier between calls).
 template <typename T, int CH>
-__device__ __forceinline__ void syrk_ring_tile(const T* __restrict__ x, int xrows, int ldo, int mb, int nb, int qb,
-                                               int qe, T* __restrict__ dst, int nrow) {
+__device__ __forceinline__ void syrk_ring_tile(const T* __restrict__ x, int xrows, int ldo, int kcols, int mb, int nb,
+                                               int edge, int qb, int qe, T* __restrict__ dst, int nrow) {
   typedef SyrkDma<T, CH> D;
   constexpr int E = D::E;
   constexpr int LOADS = D::LOADS;
@@ -1464,11 +1496,11 @@ __device__ __forceinline__ void syrk_ring_tile(const T* __restrict__ x, int xrow
   for (int v = 0; v < LOADS; ++v) {
     const int ch = wave * LOADS + v;
     const int blk = ch >= 8 * CH ? nb : mb;
-    int row = blk * kSyrkTile + ((ch / CH) % 8) * 16 + (lane & 15);
+    int row = blk * edge + ((ch / CH) % 8) * 16 + (lane & 15);
     row = row < xrows ? row : 0;
     off[v] = (row * ldo + (ch % CH) * D::KC + (lane >> 4) * E) * (int)sizeof(T);
   }
-  const int nch = ldo / D::KS;
+  const int nch = (kcols + D::KS - 1) / D::KS;  // ldo is a multiple of KS
   auto src = [&](int step, int operand) -> const T* {
     (void)operand;
     const int qq = step / nch;
@@ -1483,25 +1515,33 @@ __device__ __forceinline__ void syrk_ring_tile(const T* __restrict__ x, int xrow
     for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[mi][ni][r] = (T)0;
-  // The 16-row blocks of each operand at or past nrow hold padding: their MFMAs are skipped.
-  int rbits = 0, cbits = 0;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    rbits |= (mb * kSyrkTile + wm * 64 + b * 16 < nrow) << b;
-    cbits |= (nb * kSyrkTile + wn * 64 + b * 16 < nrow) << b;
+  const int nblk = (nrow + 15) / 16;
+  const int eb = edge / 16;
+  const unsigned mask = block_mask(wm, wn, min(eb, nblk - eb * mb), min(eb, nblk - eb * nb), mb == nb);
+  dma_ring<T, false, CH>(src, off, (qe - qb) * nch, (const T*)nullptr, sign_at, scale_at, acc, mask);
+  store_tile<T>(dst, acc, wm, wn, lane, mask);
+}
+
+// The SYRK of unsigned columns (every sign +1) on the two-workgroups-per-CU
+// ring. (The signed kernel's sign table, shift and per-aux signs cost
+// registers that the FP64 accumulators leave no room for.)
+template <typename T>
+__global__ __launch_bounds__(kThreads, 2) void syrk_ring_kernel(const T* __restrict__ x, int naux, int nao, int xrows,
+                                                                 int ldo, int kcols, int edge, int nsplit, int npairs,
+                                                                 int run, T* __restrict__ partial) {
+  int s, pair;
+  syrk_coords(blockIdx.x, npairs, s, pair);
+  int mb, nb;
+  tile_of(pair, mb, nb);
+  int cb, ce;
+  slot_range(s, nsplit, naux, run, cb, ce);
+  for (int c = cb; c < ce; ++c) {
+    int qb, qe;
+    slot_aux(c, nsplit, naux, run, qb, qe);
+    __syncthreads();  // the previous slot's LDS reads have returned
+    syrk_ring_tile<T, 1>(x, xrows, ldo, kcols, mb, nb, edge, qb, qe,
+                         partial + ((long long)c * npairs + pair) * (kSyrkTile * kSyrkTile), nao);
   }
-  dma_ring<T, false, CH, true>(src, off, (qe - qb) * nch, (const T*)nullptr, sign_at, scale_at, acc, rbits, cbits);
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 4; ++ni) {
-      const int col = wn * 64 + ni * 16 + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = wm * 64 + mi * 16 + Op<T>::row(lane, r);
-        dst[row * kSyrkTile + col] = acc[mi][ni][r];
-      }
-    }
 }
 
 // FP64 / FP32 half-transform on the ring, from a full row-major copy of B
@@ -1512,7 +1552,7 @@ __device__ __forceinline__ void syrk_ring_tile(const T* __restrict__ x, int xrow
 // X rows past npad (xrows may exceed it by up to 32) are written as zeros.
 template <typename T, int CH>
 __global__ __launch_bounds__(kThreads, CH == 1 ? 2 : 1) void xform_dma_kernel(
-    const T* __restrict__ bfull, int npad, const T* __restrict__ ct, int ldo, T* __restrict__ x, int xrows,
+    const T* __restrict__ bfull, int nao, int npad, const T* __restrict__ ct, int ldo, T* __restrict__ x, int xrows,
     int qbase, int nblocks_n, int nblocks_m, int nwg) {
   typedef SyrkDma<T, CH> D;
   constexpr int E = D::E;
@@ -1550,17 +1590,19 @@ __global__ __launch_bounds__(kThreads, CH == 1 ? 2 : 1) void xform_dma_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[mi][ni][r] = (T)0;
 
-  dma_ring<T, false, CH>(src, off, npad / D::KS, (const T*)nullptr, no_sign, no_scale, acc);
+  // Blocks past nao stay zero, blocks past ldo are not written.
+  const unsigned mask = block_mask(wm, wn, (nao + 15) / 16 - 8 * mb, ldo / 16 - 8 * nb, false);
+  dma_ring<T, false, CH>(src, off, npad / D::KS, (const T*)nullptr, no_sign, no_scale, acc, mask);
 
   T* xq = x + (long long)q * xrows * ldo;
 #pragma unroll
   for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) {
-      const int col = nb * kSyrkTile + wn * 64 + ni * 16 + (lane & 15);
+      const int col = nb * kSyrkTile + (wn + 2 * ni) * 16 + (lane & 15);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = mb * kSyrkTile + wm * 64 + mi * 16 + Op<T>::row(lane, r);
+        const int row = mb * kSyrkTile + (wm + 2 * mi) * 16 + Op<T>::row(lane, r);
         if (row < xrows && col < ldo) xq[(long long)row * ldo + col] = row < npad ? acc[mi][ni][r] : (T)0;
       }
     }
@@ -2378,7 +2420,8 @@ __device__ __forceinline__ double2 slot_sum(const T* __restrict__ src, int part,
 // result does not depend on the run. The lower triangle is written to
 // K[bm rows][bn columns] and, through the LDS copy, to its mirror
 // K[bn rows][bm columns]; elements above the diagonal of a diagonal tile are
-// not read (the masked kernels leave them unwritten).
+// not read (the masked kernels leave them unwritten). Tile (bm, bn) holds K
+// from row bm edge and column bn edge on, edge <= 128 rows and columns of it.
 // With ANTI (the non-symmetric exchange), S = sum of `partial`'s slots and
 // A = sum of `anti`'s: K[m][n] (+)= S + A, K[n][m] (+)= S - A.
 //
@@ -2391,7 +2434,8 @@ constexpr int kRedThreads = 512;
 template <typename T, int STRIP, bool ANTI>
 __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __restrict__ partial,
                                                                   const T* __restrict__ anti, int nslot, int npairs,
-                                                                  int nao, int accumulate, double* __restrict__ out) {
+                                                                  int nao, int edge, int accumulate,
+                                                                  double* __restrict__ out) {
   constexpr int PARTS = kRedThreads / (STRIP * (kSyrkTile / 2));
   constexpr int NS = ANTI ? 2 : 1;
   constexpr int LD = kSyrkTile + 2;
@@ -2400,15 +2444,15 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
   const int strip = blockIdx.x % (kSyrkTile / STRIP);
   int bm, bn;
   tile_of(pair, bm, bn);
-  const int row0 = bm * kSyrkTile + strip * STRIP;
-  if (row0 >= nao) return;
+  const int row0 = bm * edge + strip * STRIP;
+  if (strip * STRIP >= edge || row0 >= nao) return;
   const int t = threadIdx.x;
   const int col = (t & (kSyrkTile / 2 - 1)) * 2;
   const int lr = (t / (kSyrkTile / 2)) % STRIP;
   const int part = t / (STRIP * (kSyrkTile / 2));
-  const int row = row0 + lr, gcol = bn * kSyrkTile + col;
+  const int row = row0 + lr, gcol = bn * edge + col;
   const long long stride = (long long)npairs * (kSyrkTile * kSyrkTile);
-  if (row < nao && gcol < nao && gcol <= row) {
+  if (row < nao && col < edge && gcol <= row) {
     const long long at = (long long)pair * (kSyrkTile * kSyrkTile) + (strip * STRIP + lr) * kSyrkTile + col;
     *(double2*)&part_sum[0][part][lr][col] = slot_sum<T, PARTS>(partial + at, part, nslot, stride);
     if constexpr (ANTI)
@@ -2417,8 +2461,8 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
   __syncthreads();
   for (int e = t; e < STRIP * kSyrkTile; e += kRedThreads) {
     const int r = e / kSyrkTile, c = e % kSyrkTile;
-    const int gr = row0 + r, gc = bn * kSyrkTile + c;
-    if (gr >= nao || gc > gr) continue;
+    const int gr = row0 + r, gc = bn * edge + c;
+    if (gr >= nao || c >= edge || gc > gr) continue;
     double ss = 0.0, aa = 0.0;
 #pragma unroll
     for (int q = 0; q < PARTS; ++q) {
@@ -2432,8 +2476,8 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
   __syncthreads();
   for (int e = t; e < STRIP * kSyrkTile; e += kRedThreads) {
     const int c = e / STRIP, r = e % STRIP;
-    const int gr = row0 + r, gc = bn * kSyrkTile + c;
-    if (gr >= nao || gc >= gr) continue;
+    const int gr = row0 + r, gc = bn * edge + c;
+    if (gr >= nao || c >= edge || gc >= gr) continue;
     const long long o = (long long)gc * nao + gr;
     out[o] = (ANTI && accumulate ? out[o] : 0.0) + part_sum[0][0][r][c];
   }
@@ -2550,10 +2594,11 @@ hipError_t launch_half_transform_full(const void* bfull, int precision, int naux
     const int nwg = nbn * nbm * count;
     if (precision == HFJK_FP64) {
       hipLaunchKernelGGL((xform_dma_kernel<double, 1>), dim3((unsigned)nwg), dim3(kThreads), 0, s,
-                         (const double*)bfull, npad, (const double*)ct, ldo, (double*)x, xrows, base, nbn, nbm, nwg);
+                         (const double*)bfull, nao, npad, (const double*)ct, ldo, (double*)x, xrows, base, nbn, nbm,
+                         nwg);
     } else if (precision == HFJK_FP32) {
       hipLaunchKernelGGL((xform_dma_kernel<float, 1>), dim3((unsigned)nwg), dim3(kThreads), 0, s,
-                         (const float*)bfull, npad, (const float*)ct, ldo, (float*)x, xrows, base, nbn, nbm, nwg);
+                         (const float*)bfull, nao, npad, (const float*)ct, ldo, (float*)x, xrows, base, nbn, nbm, nwg);
     } else {
       // BF16x3: B and C^T interleaved (hi and lo per 32-column block), X as hi then lo plane.
       uint16_t* xh = (uint16_t*)x;
@@ -2615,6 +2660,114 @@ hipError_t launch_charges_from_x(const void* x, int precision, int naux, int nao
 int syrk_pairs(int nao) {
   const int nb = (x_rows(nao) + kSyrkTile - 1) / kSyrkTile;
   return nb * (nb + 1) / 2;
+}
+
+// FP64 / FP32 on the direct-LDS ring: 32-bit lane offsets within one aux function's X.
+static bool syrk_dma_ok(int precision, int nao, int ldo, int kind) {
+  return kind != 1 && precision != HFJK_BF16X3 && ldo <= kDmaMaxLdo && (long long)x_rows(nao) * ldo < (1LL << 31);
+}
+
+// The rows are cut into ceil(nao / 128) blocks of equal height rather than
+// into 128-row blocks and a remainder: nao 288 as 3 x 96 instead of 128, 128
+// and 32 gives tiles of 9 and 6 blocks per wave instead of 16, 10, 4 and 1, so
+// that the workgroups end together (210 -> 182 us at naux 1356, nocc 60).
+int syrk_row_block(int nao) {
+  const int nblk = (nao + 15) / 16;
+  const int nb = (nblk + 7) / 8;
+  return (nblk + nb - 1) / nb * 16;
+}
+
+int syrk_edge(int precision, int nao, int ldo, bool is_signed, int kind) {
+  return !is_signed && kind != 3 && syrk_dma_ok(precision, nao, ldo, kind) ? syrk_row_block(nao) : kSyrkTile;
+}
+
+// Blocks of the busiest wave of tile (r, c), of 16.
+static int tile_blocks(int nblk, int eb, int r, int c) {
+  int most = 0;
+  for (int wm = 0; wm < 2; ++wm)
+    for (int wn = 0; wn < 2; ++wn) {
+      int count = 0;
+      for (int br = wm; br < std::min(eb, nblk - eb * r); br += 2)
+        for (int bc = wn; bc < std::min(eb, nblk - eb * c); bc += 2) count += r != c || bc <= br;
+      most = std::max(most, count);
+    }
+  return most;
+}
+
+// The split count with the least modelled time. Workgroups go to two slots
+// per CU, each XCD taking the splits of its residue, in launch order; a k step
+// of a whole tile holds a slot for 1.7 us (32 FP64 or 64 FP32 MFMAs per wave,
+// 2048 cycles, two workgroups sharing the SIMDs), a masked one for its share
+// but no less than the load pipeline's 0.45 us; each workgroup adds 4 us to
+// fill and drain; workgroups drift, so the end is late by a share of the
+// longest one; FP64 writes and reads back a partial per split and tile.
+// (A fixed target of 2048 workgroups wrote 270 MB of partials whatever the
+// size, and at nao 709 / naux 2503 in FP32 left 25 of 104 splits without a
+// slot.) The last answer is kept per thread: a program asks for one shape
+// many times.
+int syrk_split_count(int precision, int naux, int nao, int ldo, int cus) {
+  struct Last {
+    int precision = -1, naux = 0, nao = 0, ldo = 0, cus = 0, splits = 0;
+  };
+  static thread_local Last last;
+  if (last.precision == precision && last.naux == naux && last.nao == nao && last.ldo == ldo && last.cus == cus)
+    return last.splits;
+  const int nblk = (nao + 15) / 16, eb = syrk_row_block(nao) / 16;
+  const int nb = (nblk + 7) / 8, npairs = nb * (nb + 1) / 2;
+  const int run = syrk_run_aux(precision, ldo);
+  const int nslot = run == 0 ? naux : (naux + run - 1) / run;
+  const double chunk_steps = (double)(run == 0 ? 1 : run) * ldo / (precision == HFJK_FP64 ? 8 : 16);
+  const double partial_us = npairs * 2.0 * kSyrkTile * kSyrkTile * 8.0 / 5e6;
+  const int slots = std::max(1, 2 * cus / 8);  // of one XCD
+  std::vector<double> step_us;
+  for (int r = 0; r < nb && npairs <= 1024; ++r)
+    for (int c = 0; c <= r; ++c) step_us.push_back(std::max(0.45, 1.7 * tile_blocks(nblk, eb, r, c) / 16.0));
+  int best = 8;
+  double best_us = 1e300;
+  const int top = std::min((nslot + 7) / 8, npairs <= 1024 ? std::max(1, 24 * slots / npairs) : 1);
+  std::vector<double> busy;
+  for (int n8 = 1; n8 <= top; ++n8) {
+    const int per = (nslot + 8 * n8 - 1) / (8 * n8);  // chunks of the fullest split
+    if (n8 > 1 && per == (nslot + 8 * n8 - 9) / (8 * n8 - 8)) continue;
+    const int used = std::min(n8, (((nslot + per - 1) / per) + 7) / 8);  // splits of one XCD that hold chunks
+    const double alone = used * npairs * 2 <= slots ? 0.58 : 1.0;
+    busy.assign(slots, 0.0);  // a heap: the earliest free slot on top
+    double end = 0.0, longest = 0.0;
+    for (int s = 0; s < used; ++s)
+      for (double step : step_us) {
+        const double job = alone * step * per * chunk_steps + 4.0;
+        std::pop_heap(busy.begin(), busy.end(), std::greater<double>());
+        busy.back() += job;
+        longest = std::max(longest, job);
+        end = std::max(end, busy.back());
+        std::push_heap(busy.begin(), busy.end(), std::greater<double>());
+      }
+    const double us = end + 0.3 * longest + (run == 0 ? 8 * n8 * partial_us : 0.0);
+    if (us < best_us) {
+      best_us = us;
+      best = 8 * n8;
+    }
+  }
+  last = Last{precision, naux, nao, ldo, cus, best};
+  return best;
+}
+
+double syrk_instance_us(int precision, int naux, int nao, int nocc, bool ring, double& whole_us) {
+  const int nblk = (nao + 15) / 16, nb = (nblk + 7) / 8;
+  const bool masked = ring && precision != HFJK_BF16X3;
+  const int eb = masked ? syrk_row_block(nao) / 16 : 8;
+  const double steps = (double)naux * ((nocc + 7) / 8) * (precision == HFJK_FP64 ? 1.0 : 0.5);
+  double sum = 0.0, most = 0.0;
+  for (int r = 0; r < nb; ++r)
+    for (int c = 0; c <= r; ++c) {
+      // BF16x3: about 0.8 us per 32 k of a 128 x 128 tile on its ring, padding included.
+      const double us = masked ? std::max(0.45, 1.7 * tile_blocks(nblk, eb, r, c) / 16.0)
+                               : precision == HFJK_BF16X3 ? 0.4 : 1.7;
+      sum += us;
+      most = std::max(most, us);
+    }
+  whole_us = most * steps;
+  return sum * steps;
 }
 
 int syrk_tile() { return kSyrkTile; }
@@ -2684,8 +2837,10 @@ bool syrk16_tiles256(int nao, int ldo, bool is_signed, int kind, int shift) {
 
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
                        bool is_signed, int nsplit, void* partial, int kind, hipStream_t s, const double* auxsign,
-                       int shift, bool x_ilv) {
+                       int shift, bool x_ilv, int nocc) {
   const int xrows = x_rows(nao);
+  const int edge = syrk_edge(precision, nao, ldo, is_signed, kind);
+  if (nocc <= 0 || nocc > ldo) nocc = ldo;
   const int npairs = syrk_pairs(nao);
   const int run = syrk_run_aux(precision, ldo);
   // Per-aux signs are applied by the signed FP64/FP32 direct-LDS kernels only; a column shift by
@@ -2696,28 +2851,27 @@ hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo,
   const unsigned grid = (unsigned)(npairs * nsplit);
   // The direct-load kernel keeps per-lane element offsets within one aux
   // function's X in 32 bits and the sign table in LDS.
-  const bool dma = kind != 1 && precision != HFJK_BF16X3 && ldo <= kDmaMaxLdo &&
-                   (long long)xrows * ldo < (1LL << 31);
+  const bool dma = syrk_dma_ok(precision, nao, ldo, kind);
   // Signed columns need the LDS sign table: the one-workgroup-per-CU ring.
   const bool two_wg = kind != 3 && !is_signed;
   if (dma && precision == HFJK_FP64 && is_signed)
     hipLaunchKernelGGL((syrk_dma_kernel<double, true, 2>), dim3(grid), dim3(kThreads), 0, s, (const double*)x, naux,
-                       xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (double*)partial);
+                       nao, xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (double*)partial);
   else if (dma && precision == HFJK_FP64 && two_wg)
-    hipLaunchKernelGGL((syrk_dma_kernel<double, false, 1>), dim3(grid), dim3(kThreads), 0, s, (const double*)x, naux,
-                       xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (double*)partial);
+    hipLaunchKernelGGL(syrk_ring_kernel<double>, dim3(grid), dim3(kThreads), 0, s, (const double*)x, naux, nao, xrows,
+                       ldo, nocc, edge, nsplit, npairs, run, (double*)partial);
   else if (dma && precision == HFJK_FP64)
     hipLaunchKernelGGL((syrk_dma_kernel<double, false, 2>), dim3(grid), dim3(kThreads), 0, s, (const double*)x, naux,
-                       xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (double*)partial);
+                       nao, xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (double*)partial);
   else if (dma && is_signed)
     hipLaunchKernelGGL((syrk_dma_kernel<float, true, 2>), dim3(grid), dim3(kThreads), 0, s, (const float*)x, naux,
-                       xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (float*)partial);
+                       nao, xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (float*)partial);
   else if (dma && two_wg)
-    hipLaunchKernelGGL((syrk_dma_kernel<float, false, 1>), dim3(grid), dim3(kThreads), 0, s, (const float*)x, naux,
-                       xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (float*)partial);
+    hipLaunchKernelGGL(syrk_ring_kernel<float>, dim3(grid), dim3(kThreads), 0, s, (const float*)x, naux, nao, xrows,
+                       ldo, nocc, edge, nsplit, npairs, run, (float*)partial);
   else if (dma)
     hipLaunchKernelGGL((syrk_dma_kernel<float, false, 2>), dim3(grid), dim3(kThreads), 0, s, (const float*)x, naux,
-                       xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (float*)partial);
+                       nao, xrows, ldo, signs, auxsign, shift, nsplit, npairs, run, (float*)partial);
   else if (precision == HFJK_FP64)
     hipLaunchKernelGGL(syrk_kernel<double>, dim3(grid), dim3(kThreads), 0, s, (const double*)x, naux, xrows, ldo,
                        signs, nsplit, npairs, run, (double*)partial);
@@ -2760,34 +2914,36 @@ hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo,
 // device four times over, else 2 and 1 rows, whose workgroups split the slots
 // over 4 and 8 thread groups (nao 100: 100 workgroups instead of 13).
 template <typename T, bool ANTI>
-static hipError_t launch_reduce_t(const T* partial, const T* anti, int nslot, int nao, bool accumulate, double* out,
-                                  hipStream_t s) {
+static hipError_t launch_reduce_t(const T* partial, const T* anti, int nslot, int nao, int edge, bool accumulate,
+                                  double* out, hipStream_t s) {
   const int npairs = syrk_pairs(nao);
   const int acc = accumulate ? 1 : 0;
   const dim3 blk(kRedThreads);
   if (npairs * (kSyrkTile / 8) >= 1024)
     hipLaunchKernelGGL((syrk_reduce_kernel<T, 8, ANTI>), dim3((unsigned)(npairs * (kSyrkTile / 8))), blk, 0, s,
-                       partial, anti, nslot, npairs, nao, acc, out);
+                       partial, anti, nslot, npairs, nao, edge, acc, out);
   else if (npairs * (kSyrkTile / 2) >= 512)
     hipLaunchKernelGGL((syrk_reduce_kernel<T, 2, ANTI>), dim3((unsigned)(npairs * (kSyrkTile / 2))), blk, 0, s,
-                       partial, anti, nslot, npairs, nao, acc, out);
+                       partial, anti, nslot, npairs, nao, edge, acc, out);
   else
     hipLaunchKernelGGL((syrk_reduce_kernel<T, 1, ANTI>), dim3((unsigned)(npairs * kSyrkTile)), blk, 0, s, partial,
-                       anti, nslot, npairs, nao, acc, out);
+                       anti, nslot, npairs, nao, edge, acc, out);
   return hipGetLastError();
 }
 
 hipError_t launch_syrk_reduce2(const void* sym, const void* anti, int precision, int nslot, int nao,
                                bool accumulate, double* out, hipStream_t s) {
   if (precision == HFJK_FP64)
-    return launch_reduce_t<double, true>((const double*)sym, (const double*)anti, nslot, nao, accumulate, out, s);
-  return launch_reduce_t<float, true>((const float*)sym, (const float*)anti, nslot, nao, accumulate, out, s);
+    return launch_reduce_t<double, true>((const double*)sym, (const double*)anti, nslot, nao, kSyrkTile, accumulate, out,
+                                         s);
+  return launch_reduce_t<float, true>((const float*)sym, (const float*)anti, nslot, nao, kSyrkTile, accumulate, out, s);
 }
 
-hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, double* out, hipStream_t s) {
+hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, int edge, double* out,
+                              hipStream_t s) {
   if (precision == HFJK_FP64)
-    return launch_reduce_t<double, false>((const double*)partial, nullptr, nslot, nao, false, out, s);
-  return launch_reduce_t<float, false>((const float*)partial, nullptr, nslot, nao, false, out, s);
+    return launch_reduce_t<double, false>((const double*)partial, nullptr, nslot, nao, edge, false, out, s);
+  return launch_reduce_t<float, false>((const float*)partial, nullptr, nslot, nao, edge, false, out, s);
 }
 
 // ------------------------------------------------------------------ batched (persistent)
@@ -2949,7 +3105,7 @@ __global__ __launch_bounds__(kThreads, 2) void batch_syrk_ring_kernel(BatchView 
     tile_of(pair, mb, nb);
     const int qb = (int)((long long)s * in.naux / in.nsplit);
     const int qe = (int)((long long)(s + 1) * in.naux / in.nsplit);
-    syrk_ring_tile<T, 1>(xbase + in.x_off, in.xrows, in.ldo, mb, nb, qb, qe,
+    syrk_ring_tile<T, 1>(xbase + in.x_off, in.xrows, in.ldo, in.nocc, mb, nb, in.se, qb, qe,
                          kbase + in.kp_off + ((long long)s * in.npairs + pair) * (kSyrkTile * kSyrkTile), in.nao);
   }
 }
@@ -3052,11 +3208,12 @@ __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v
     const int pair = (int)(local / strips), strip = (int)(local % strips);
     int bm, bn;
     tile_of(pair, bm, bn);
-    const int row0 = bm * st + strip * rows;
-    if (row0 >= in.nao) continue;
+    const int edge = in.se;
+    const int row0 = bm * edge + strip * rows;
+    if (strip * rows >= edge || row0 >= in.nao) continue;
     const int e = 2 * threadIdx.x;
-    const int row = row0 + e / st, col = bn * st + e % st;
-    if (row < in.nao && col <= row)
+    const int row = row0 + e / st, col = bn * edge + e % st;
+    if (row < in.nao && e % st < edge && col <= row)
       *(double2*)&sum[e] = slot_sum<T, 1>(kbase + in.kp_off + (long long)pair * st * st + (long long)strip * 2 * kThreads + e,
                                           0, in.nsplit, (long long)in.npairs * st * st);
     __syncthreads();
@@ -3064,10 +3221,10 @@ __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int f = threadIdx.x + u * kThreads;
-      const int r = row0 + f / st, c = bn * st + f % st;
-      if (r < in.nao && c <= r) k[(long long)r * in.nao + c] = sum[f];
-      const int mr = row0 + f % rows, mc = bn * st + f / rows;
-      if (mr < in.nao && mc < mr) k[(long long)mc * in.nao + mr] = sum[(f % rows) * st + f / rows];
+      const int r = row0 + f / st, c = bn * edge + f % st;
+      if (r < in.nao && f % st < edge && c <= r) k[(long long)r * in.nao + c] = sum[f];
+      const int mr = row0 + f % rows, mc = bn * edge + f / rows;
+      if (mr < in.nao && f / rows < edge && mc < mr) k[(long long)mc * in.nao + mr] = sum[(f % rows) * st + f / rows];
     }
     // batch_next's barriers keep the next item's sums behind these reads.
   }

@@ -31,14 +31,13 @@ def test_occupied_build_within_the_rounding_bound(nao, naux, nocc):
     c = synthetic.occupied_orbitals(3, nao, nocc)
     jk = MI355XCoulombExchange(b)
     j, k = jk.jk_occupied(c)
-    x = np.einsum("qmn,ni->qmi", b, c)
-    xa = np.einsum("qmn,ni->qmi", np.abs(b), np.abs(c))
+    x, xa = b @ c, np.abs(b) @ np.abs(c)
     gamma, gamma_a = np.einsum("qmi,mi->q", x, c), np.einsum("qmi,mi->q", xa, np.abs(c))
     j_abs = np.einsum("q,qmn->mn", gamma_a, np.abs(b))
-    k_abs = np.einsum("qmi,qni->mn", xa, xa)
+    k_abs = np.tensordot(xa, xa, axes=((0, 2), (0, 2)))
     # The reference sums round too: twice the bound.
     assert np.all(np.abs(j - np.einsum("q,qmn->mn", gamma, b)) <= 2 * _bound(naux + nao * (nocc + 1), j_abs))
-    assert np.all(np.abs(k - np.einsum("qmi,qni->mn", x, x)) <= 2 * _bound(naux * nocc + 2 * nao, k_abs))
+    assert np.all(np.abs(k - np.tensordot(x, x, axes=((0, 2), (0, 2)))) <= 2 * _bound(naux * nocc + 2 * nao, k_abs))
     np.testing.assert_array_equal(k, k.T)
     np.testing.assert_array_equal(j, j.T)
     j2, k2 = jk.jk_occupied(c)
