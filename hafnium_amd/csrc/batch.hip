@@ -294,12 +294,15 @@ __global__ __launch_bounds__(kThreads) void b_orbitals_kernel(BatchView v, const
       hi[idx] = h;
       hi[idx + c_plane] = to_bf16(x - __uint_as_float(((uint32_t)h) << 16));
     } else {
-      const int k = (int)(idx / in.ldo), i = (int)(idx % in.ldo);  // C[k][i]
+      const int k = (int)(idx / in.ldo), i = (int)(idx % in.ldo);  // C[k][i], in the operand order
       const double x = (k < in.nao && i < in.nocc) ? ci[(long long)k * in.nocc + i] : 0.0;
-      if (PREC == HFJK_FP64)
-        ((double*)cbase)[in.cp_off + idx] = x;
-      else
-        ((float*)cbase)[in.cp_off + idx] = (float)x;
+      const ColumnGroups cg = in.cg;
+      if (i / 16 < cg.groups * cg.blocks + cg.tail) {
+        if (PREC == HFJK_FP64)
+          ((double*)cbase)[in.cp_off + fragment_index<double>(cg, npad, k, i)] = x;
+        else
+          ((float*)cbase)[in.cp_off + fragment_index<float>(cg, npad, k, i)] = (float)x;
+      }
     }
   }
   BATCH_END
@@ -425,8 +428,11 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
   if (hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) prop.multiProcessorCount = 256;
   const int cus = std::max(8, prop.multiProcessorCount);
   double batch_us = 0.0;
+  long long x_steps = 0;  // k steps of four units of the FP64 / FP32 half-transform
   for (int i = 0; i < ninst; ++i) {
     double whole_us;
+    const long long nt = hfjk::n_tiles(std::max(1, instances[i].nao));
+    x_steps += (std::max(1, instances[i].naux) * nt + 3) / 4 * nt * ((std::max(1, instances[i].nocc) + 127) / 128);
     if (instances[i].nao > 0 && instances[i].nao <= 46000)
       batch_us += hfjk::syrk_instance_us(precision, instances[i].naux, instances[i].nao, instances[i].nocc, true, whole_us);
   }
@@ -459,15 +465,11 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
       in.npairs = (int)(nb * (nb + 1) / 2);
       in.se = fits_ring && precision != HFJK_BF16X3 ? hfjk::syrk_row_block(src.nao) : in.st;
     }
-    // Half-transform column tile: the smallest of 32 / 64 / 128 that covers the instance's
+    // BF16x3 half-transform column tile: the smallest of 32 / 64 / 128 that covers the instance's
     // columns, at most the batch's tile (whose multiples then cover them); a batch tile of 256
-    // applies to every instance.
-    if (bt->tile == 256) {
-      in.bn = 256;
-    } else {
-      in.bn = in.ldo <= 32 ? 32 : in.ldo <= 64 ? 64 : 128;
-      in.bn = std::min(in.bn, bt->tile);
-    }
+    // applies to every instance. FP64 / FP32: column groups of at most the batch's tile.
+    in.bn = bt->tile == 256 ? 256 : std::min(in.ldo <= 32 ? 32 : in.ldo <= 64 ? 64 : 128, bt->tile);
+    in.cg = hfjk::column_groups(src.nocc, in.ldo, bt->tile);
     // Splits: about 8192 k per item, and where the batch is small enough that the longest such
     // item would outlast the others, as many as bring an instance's slowest tile down to a quarter
     // of the batch's mean load per workgroup slot (12 water clusters: 4 rounds of items instead of
@@ -477,12 +479,20 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     const long long by_k = std::min(64LL, ((long long)src.naux * in.ldo + 8191) / 8192);
     const long long by_load = std::min<long long>(src.naux, (long long)std::ceil(whole_us / item_us));
     in.nsplit = (int)std::max(1LL, std::max(by_k, by_load));
-    in.bm = bt->tile == 256 ? hfjk::batch_tile_rows(precision, 0, 256) : hfjk::batch_tile_rows(precision, in.xrows, in.bn);
-    // Items cover enough aux functions for about 32 pipelined k tiles (small instances have
-    // few k tiles per aux function).
-    in.qg = bt->tile == 256 ? 1 : std::max(1, std::min(src.naux, 32 / in.nt));
-    in.nbm = (in.xrows + in.bm - 1) / in.bm;
-    in.nbn = (in.ldo + in.bn - 1) / in.bn;
+    in.bm = 128;
+    if (precision == HFJK_BF16X3) {
+      // Items cover enough aux functions for about 32 pipelined k tiles (small instances have
+      // few k tiles per aux function).
+      in.qg = bt->tile == 256 ? 1 : std::max(1, std::min(src.naux, 32 / in.nt));
+      in.nbm = (in.xrows + in.bm - 1) / in.bm;
+      in.nbn = (in.ldo + in.bn - 1) / in.bn;
+    } else {
+      // Items of about 32 k steps of four units, fewer where the batch holds too few of them for
+      // four items per workgroup.
+      in.qg = 4 * (int)std::max(1LL, std::min(32LL, x_steps / (8LL * cus)) / in.nt);
+      in.nbm = 1;
+      in.nbn = in.cg.groups + (in.cg.tail > 0 ? 1 : 0);
+    }
     in.p = hfjk::packed_elems(src.nao);
     in.b_off = src.b_offset;
     in.c_off = src.c_offset;
@@ -523,7 +533,10 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     items[hfjk::kPhCoulomb] = ntiles;
     items[hfjk::kPhCoulombUnpack] = (nn + hfjk::kThreads - 1) / hfjk::kThreads;
     items[hfjk::kPhOrbitals] = ((long long)in.nt * hfjk::kTile * in.ldo + hfjk::kThreads - 1) / hfjk::kThreads;
-    items[hfjk::kPhXform] = (long long)((in.naux + in.qg - 1) / in.qg) * in.nbm * in.nbn;
+    const long long x_units = (long long)in.naux * (precision == HFJK_FP64 ? hfjk::xform_units_per_aux<double>(in.nao)
+                                                    : precision == HFJK_FP32 ? hfjk::xform_units_per_aux<float>(in.nao)
+                                                                             : 1);
+    items[hfjk::kPhXform] = (x_units + in.qg - 1) / in.qg * in.nbm * in.nbn;
     // Instances whose X offsets fit the ring's 32-bit lane offsets run on it, in a phase of
     // their own.
     const bool ring = in.ldo <= 2048 && (long long)in.xrows * in.ldo * es < (1LL << 31);

@@ -118,7 +118,8 @@ struct Layout {
   size_t dens_a, dens_w, dens_e, dens_info, dens_stats, dens_c, dens_signs, dens_end;
   // coulomb region (shares the base of the exchange region)
   size_t cw, cgp, cg, cjp, c_end;
-  // exchange region (xct: C^T in FP64 for the half-transform from the full copy)
+  // exchange region (xct: C^T for the half-transform from the full copy, or the
+  // operand fragments of C for the packed one)
   size_t xc, xs, xx, xp, xct, x_end;
   // the Coulomb half of hfjk_jk_occ, after both regions (it runs while the
   // SYRK still reads X): row-group parts of the charges [naux][charge_groups],
@@ -268,9 +269,11 @@ bool x16_interleaved(const hfjk_ctx* ctx, int precision, bool is_signed, int ldo
          hfjk::x16_tiles256(ldo, ctx->x16_bn) && hfjk::syrk16_tiles256(ctx->nao, ldo, is_signed, ctx->syrk_kind, 0);
 }
 
-// Orbitals (and signs) into the workspace and the half-transform X = B C.
-void exchange_front(hfjk_ctx* ctx, const double* orbitals, int nocc, const double* signs, int precision, void* ws,
-                    const Layout& L, hipStream_t s) {
+// Orbitals (and signs) into the workspace and the half-transform X = B C;
+// want_pad also leaves the zero-padded orbitals that the charges of
+// hfjk_jk_occ read (FP64 / FP32 at L.xc, BF16X3 in FP32 at L.qc).
+void exchange_front(hfjk_ctx* ctx, const double* orbitals, int nocc, const double* signs, bool want_pad,
+                    int precision, void* ws, const Layout& L, hipStream_t s) {
   // FP64 and FP32 run the same MFMA kernels on their tensor copy; BF16X3
   // runs the split-product kernels on the bf16 hi/lo planes. The FP32 and
   // BF16X3 buffers have the same sizes (4 bytes per element).
@@ -285,18 +288,22 @@ void exchange_front(hfjk_ctx* ctx, const double* orbitals, int nocc, const doubl
                       : precision == HFJK_FP32 ? (const void*)ctx->b32_full
                                                : (const void*)ctx->b16_full;
   const bool full = bfull != nullptr && ctx->x_full == 0;
-  // BF16X3 takes C^T's bf16 hi/lo (cp; interleaved for the ring from the
-  // full copy) as the second operand.
+  // Second operand: BF16X3 C^T's bf16 hi/lo (cp; interleaved for the ring from the full copy), else
+  // C^T for the ring from the full copy or the operand fragments for the packed tiles.
   void* ct = split ? cp : at<void>(ws, L.xct);
   {
     Stage st(ctx, s, "exchange_prepare");
-    if (split)
+    if (split) {
       check_hip(hfjk::launch_orbitals_bf16x3(orbitals, ctx->nao, nocc, cp, s, full), "orbitals launch");
-    else
-      check_hip(hfjk::launch_orbitals(orbitals, ctx->nao, nocc, precision, cp, s), "orbitals launch");
-    if (full && !split)
-      check_hip(hfjk::launch_orbitals_t(orbitals, ctx->nao, nocc, precision, ct, s), "orbitals launch");
-    check_hip(hfjk::launch_occ_signs(signs, nocc, L.ldo, sg, s), "signs launch");
+      check_hip(hfjk::launch_prepare_orbitals(orbitals, ctx->nao, nocc, HFJK_FP32,
+                                              want_pad ? at<void>(ws, L.qc) : nullptr, nullptr, nullptr, 0, signs, sg,
+                                              s),
+                "orbitals launch");
+    } else {
+      check_hip(hfjk::launch_prepare_orbitals(orbitals, ctx->nao, nocc, precision, want_pad ? cp : nullptr,
+                                              full ? ct : nullptr, full ? nullptr : ct, ctx->x_bn, signs, sg, s),
+                "orbitals launch");
+    }
   }
   {
     Stage st(ctx, s, "exchange_half_transform");
@@ -309,8 +316,8 @@ void exchange_front(hfjk_ctx* ctx, const double* orbitals, int nocc, const doubl
                                                    ctx->x16_bn, s),
                 "half transform launch");
     else
-      check_hip(hfjk::launch_half_transform(b, precision, L.p, ctx->naux, ctx->nao, cp, L.ldo, x, ctx->x_bn,
-                                            ctx->x_bm == 0 ? 64 : ctx->x_bm, s),
+      check_hip(hfjk::launch_half_transform(b, precision, L.p, ctx->naux, ctx->nao, ct, nocc, L.ldo, x, ctx->x_bn,
+                                            ctx->x_bm, s),
                 "half transform launch");
   }
 }
@@ -337,7 +344,7 @@ void exchange_back(hfjk_ctx* ctx, int nocc, bool is_signed, double* out, int pre
 
 void run_exchange(hfjk_ctx* ctx, const double* orbitals, int nocc, const double* signs, double* out, int precision,
                   void* ws, const Layout& L, hipStream_t s) {
-  exchange_front(ctx, orbitals, nocc, signs, precision, ws, L, s);
+  exchange_front(ctx, orbitals, nocc, signs, false, precision, ws, L, s);
   exchange_back(ctx, nocc, signs != nullptr, out, precision, ws, L, s);
 }
 
@@ -505,10 +512,10 @@ void exchange_general(hfjk_ctx* ctx, const double* density, double* out, int pre
                 "general factor launch");
       if (split)
         check_hip(hfjk::launch_orbitals_bf16x3(c, n, ld, cp, s, full), "orbitals launch");
-      else if (full)
-        check_hip(hfjk::launch_orbitals_t(c, n, ld, precision, ct, s), "orbitals launch");
       else
-        check_hip(hfjk::launch_orbitals(c, n, ld, precision, cp, s), "orbitals launch");
+        check_hip(hfjk::launch_prepare_orbitals(c, n, ld, precision, nullptr, full ? ct : nullptr,
+                                                full ? nullptr : cp, ctx->x_bn, nullptr, nullptr, s),
+                  "orbitals launch");
     }
     for (int q0 = 0; q0 < naux; q0 += pc) {
       const int qc = std::min(pc, naux - q0);
@@ -532,7 +539,7 @@ void exchange_general(hfjk_ctx* ctx, const double* density, double* out, int pre
                     "half transform launch");
         } else {
           check_hip(hfjk::launch_half_transform((const char*)b + q0 * p * (long long)es, precision, p, qc, n, cp, ld,
-                                                x, ctx->x_bn, ctx->x_bm == 0 ? 64 : ctx->x_bm, s),
+                                                ld, x, ctx->x_bn, ctx->x_bm, s),
                     "half transform launch");
         }
       }
@@ -891,7 +898,7 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
       check_hip(hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming), "hipEventCreateWithFlags");
     }
     hipStream_t side = serial ? s : ctx->side;
-    exchange_front(ctx, orbitals, nocc, nullptr, precision, workspace, L, s);
+    exchange_front(ctx, orbitals, nocc, nullptr, true, precision, workspace, L, s);
     // The Coulomb half needs only X and the padded orbitals: it runs on the
     // side stream (HBM-bound) while the SYRK (MFMA-bound) runs on s, or with
     // coulomb_serial on s after the SYRK. Its buffers (charges, J partials)
@@ -905,12 +912,7 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
     {
       // gamma_P = sum C o X_P, one pass over X.
       Stage st(ctx, side, "coulomb_gamma");
-      const void* cpad = at<void>(workspace, L.xc);
-      if (precision == HFJK_BF16X3) {
-        check_hip(hfjk::launch_orbitals(orbitals, ctx->nao, nocc, HFJK_FP32, at<void>(workspace, L.qc), side),
-                  "orbitals launch");
-        cpad = at<void>(workspace, L.qc);
-      }
+      const void* cpad = at<void>(workspace, precision == HFJK_BF16X3 ? L.qc : L.xc);
       check_hip(hfjk::launch_charges_from_x(at<void>(workspace, L.xx), precision, ctx->naux, ctx->nao, L.ldo, cpad,
                                             parts, gamma, serial ? 0 : side_groups(ctx, precision), side,
                                             x16_interleaved(ctx, precision, false, L.ldo)),

@@ -78,7 +78,7 @@ struct hfjk_ctx {
   int x_bn = 0;
   int x16_bn = 0;
   int syrk_splits = 0;
-  int x_bm = 0;  // 0 = 64
+  int x_bm = 0;  // 0 = 128
   int syrk_kind = 0;  // 0 = default, 1 = register-staged, 2/3 = direct LDS loads (two / one workgroups per CU)
   // Borrowed full row-major copies of B ([naux][npad][npad], FP64 and FP32) and their use (0 = when
   // bound, 1 = never).
@@ -153,6 +153,39 @@ void hfjk_internal_set_error(const char* message);
 
 namespace hfjk {
 
+// Column groups of the packed FP64 / FP32 half-transform: `groups` groups of
+// `blocks` 16-column blocks and, when tail > 0, one of `tail`. At most
+// kMaxGroupBlocks blocks (what the accumulators of a 32-row unit leave room
+// for), equal groups where ldo holds them (the surplus blocks are zeros).
+constexpr int kMaxGroupBlocks = 8;
+struct ColumnGroups {
+  int groups, blocks, tail;
+};
+inline ColumnGroups column_groups(int nocc, int ldo, int bn) {
+  const int cap = bn == 32 ? 2 : bn == 64 ? 4 : kMaxGroupBlocks;
+  const int n = (nocc + 15) / 16;
+  const int groups = (n + cap - 1) / cap, blocks = (n + groups - 1) / groups;
+  if (groups * blocks * 16 <= ldo) return ColumnGroups{groups, blocks, 0};
+  return ColumnGroups{groups - 1, blocks, n - (groups - 1) * blocks};
+}
+// Its row units per aux function: blocks of 16 rows in FP64, 32 in FP32.
+template <typename T>
+__host__ __device__ inline int xform_units_per_aux(int nao) {
+  return sizeof(T) == 8 ? (nao + 15) / 16 : (nao + 31) / 32;
+}
+// Element (k, i) of C in that kernel's operand order: per group and 32-row k
+// tile, [8 / EV][blocks][64 lanes][EV] with EV elements per 16 bytes.
+template <typename T>
+__host__ __device__ inline long long fragment_index(const ColumnGroups& cg, int npad, int k, int i) {
+  constexpr int EV = 16 / (int)sizeof(T);
+  const int block = i / 16, g = block / cg.blocks;
+  const int nb = g < cg.groups ? cg.blocks : cg.tail;
+  const int kk = k % kTile;
+  const int eg = kk / (4 * EV), lane = kk % (4 * EV) / EV * 16 + i % 16;
+  return (long long)g * cg.blocks * 16 * npad + (long long)(k / kTile) * nb * (kTile * 16) +
+         ((long long)(eg * nb + block - g * cg.blocks) * 64 + lane) * EV + kk % EV;
+}
+
 // Kernel launchers (gen.hip). Each returns a hipError_t.
 hipError_t launch_generate(uint64_t seed, int q0, int naux, int nao, double* out, hipStream_t s);
 hipError_t launch_pack(const double* full, int naux, int nao, double* out,
@@ -173,8 +206,12 @@ hipError_t launch_coulomb_accumulate(const void* b, int precision, long long p, 
 hipError_t launch_coulomb_unpack(const double* partial, int nsplit, long long p, int nao,
                                  double* out, hipStream_t s);
 
-// Exchange (jk.hip).
-hipError_t launch_orbitals(const double* c, int nao, int nocc, int precision, void* out, hipStream_t s);
+// Exchange (jk.hip, xk.hip).
+// C [nao][nocc] as each of: the zero-padded [npad][ldo] matrix (pad), C^T
+// [ldo][npad] (ct), the packed half-transform's operand order for column
+// groups of bn (frag), in the precision's type (FP64 or FP32); signs [ldo].
+hipError_t launch_prepare_orbitals(const double* c, int nao, int nocc, int precision, void* pad, void* ct, void* frag,
+                                   int bn, const double* signs_in, double* signs, hipStream_t s);
 // Pivoted Cholesky of a symmetric PSD density into l (nao * nao doubles:
 // L by columns; diag: nao doubles of scratch), one column per step with its
 // state on the device: init, then steps k = 0..nao (each a no-op once the
@@ -192,10 +229,11 @@ hipError_t launch_pchol_step(const double* density, int nao, int k, double* l, d
 hipError_t launch_factor_residual(const double* density, int nao, const double* l, const PcholState* st,
                                   unsigned long long* residual, hipStream_t s);
 hipError_t launch_compact_factor(const double* l, int nao, int r, double* c, double* signs, hipStream_t s);
-// bn = column tile (32, 64, 128, 256) or 0 for the default for ldo; bm = row
-// tile (64 or 128; 128 applies to column tiles up to 128).
-hipError_t launch_half_transform(const void* b, int precision, long long p, int naux, int nao,
-                                 const void* c, int ldo, void* x, int bn, int bm, hipStream_t s);
+// FP64 / FP32, frag from launch_prepare_orbitals with the same bn: columns of
+// a group at most 32, 64 or 128 (any other bn: 128); bm: rows per workgroup
+// (64: two waves; else 128: four).
+hipError_t launch_half_transform(const void* b, int precision, long long p, int naux, int nao, const void* frag,
+                                 int nocc, int ldo, void* x, int bn, int bm, hipStream_t s);
 // kind: 0 = default, 1 = register-staged FP64/FP32 kernel, 2 = direct LDS
 // loads (FP64/FP32 with ldo <= 2048; otherwise the register-staged kernel
 // runs; two workgroups per CU for unsigned columns), 3 = direct LDS loads with
@@ -241,7 +279,6 @@ hipError_t launch_syrk_reduce2(const void* sym, const void* anti, int precision,
                                bool accumulate, double* out, hipStream_t s);
 hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, int edge, double* out,
                               hipStream_t s);
-hipError_t launch_occ_signs(const double* signs_in, int nocc, int ldo, double* signs_out, hipStream_t s);
 
 // BF16x3 exchange (xk.hip): operands as bf16 hi/lo planes; launch_syrk
 // takes HFJK_BF16X3 for the split-product kernel. launch_orbitals_bf16x3
@@ -255,7 +292,7 @@ hipError_t launch_half_transform_bf16x3(const uint16_t* b, long long p, int naux
                                         void* x, int bn, hipStream_t s, const uint16_t* b_lo = nullptr);
 // Coulomb charges of D = C C^T from the half-transformed X (xk.hip):
 // gamma[q] = sum_{m, i} X_q[m][i] cpad[m][i], cpad = the zero-padded
-// orbitals [npad][ldo] of launch_orbitals (FP64 when X is FP64, FP32 for
+// orbitals [npad][ldo] of launch_prepare_orbitals (FP64 when X is FP64, FP32 for
 // FP32 and BF16x3 X); parts holds naux * charge_groups(nao) doubles.
 int charge_groups(int nao);
 hipError_t launch_charges_from_x(const void* x, int precision, int naux, int nao, int ldo, const void* cpad,
@@ -266,8 +303,7 @@ hipError_t launch_charges_from_x(const void* x, int precision, int naux, int nao
 // bfull[q][npad][npad / 32][64]: each 32-column block of a row as the bf16
 // hi parts of its elements, then their lo parts (the element split of
 // launch_split), so one 128-byte line holds both parts of 32 elements;
-// launch_orbitals_t writes C^T [ldo][npad] in FP64 or FP32 (BF16X3 takes
-// launch_orbitals_bf16x3's interleaved C^T);
+// BF16X3 takes launch_orbitals_bf16x3's interleaved C^T;
 // launch_half_transform_full computes X = B C on the direct-LDS ring (the
 // bf16 ring for BF16X3, X as hi/lo planes; BF16X3 on 256 x 256 tiles when
 // x16_tiles256(ldo, bn16): ldo > 128 and bn16 not asking for a column tile
@@ -276,7 +312,6 @@ hipError_t launch_charges_from_x(const void* x, int precision, int naux, int nao
 // charges).
 hipError_t launch_expand_full(const double* packed, long long p, int naux, int nao, int precision, void* out,
                               hipStream_t s);
-hipError_t launch_orbitals_t(const double* c, int nao, int nocc, int precision, void* ct, hipStream_t s);
 hipError_t launch_half_transform_full(const void* bfull, int precision, int naux, int nao, const void* ct, int ldo,
                                       void* x, hipStream_t s, int bn16 = 0, bool x_ilv = false);
 bool x16_tiles256(int ldo, int bn16);
@@ -324,8 +359,9 @@ struct BatchInst {
   int nao, naux, nocc, ldo;
   int nt, xrows, npairs, nsplit;
   int nbm, nbn;       // half-transform row / column blocks of the instance's tile
-  int bm, qg;         // half-transform tile rows (64 or 128; BF16x3: 128); aux functions per item (FP64 / FP32)
+  int bm, qg;         // BF16x3: half-transform tile rows (128); aux functions per item (FP64 / FP32: units)
   int st, bn;         // SYRK tile storage (64 or 128); half-transform column tile (32, 64, 128 or 256)
+  ColumnGroups cg;    // FP64 / FP32 half-transform
   int se;             // rows and columns of K per SYRK tile (at most st)
   long long p;        // packed elements per aux function
   long long b_off;    // batch tensor (element units of the bound copy)
@@ -384,10 +420,6 @@ hipError_t launch_batch_syrk(BatchView v, int precision, const void* xbase, long
                              void* kbase, int grid, hipStream_t s);
 hipError_t launch_batch_syrk_reduce(BatchView v, int precision, const void* kbase, double* k, int grid,
                                     hipStream_t s);
-// Rows of an instance's half-transform tile: FP64 / FP32 128 when the instance has at least 128
-// X rows and a column tile of 64, else 64; BF16x3 128.
-int batch_tile_rows(int precision, int xrows, int bn);
-
 // Density factorisation helpers (jk.hip).
 hipError_t launch_split_factor(const double* vecs, const double* vals, int nao, int first, int count,
                                double* c, double* signs, hipStream_t s);

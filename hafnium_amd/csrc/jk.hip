@@ -244,27 +244,6 @@ __global__ __launch_bounds__(kThreads* PARTS) void coulomb_unpack_kernel(const d
 
 // ---------------------------------------------------------------- Exchange
 
-// Orbitals [nao][nocc] float64 -> padded [npad][ldo] in T (npad = nt * 32).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void orbitals_kernel(const double* __restrict__ c, int nao, int nocc,
-                                                             int npad, int ldo, T* __restrict__ out) {
-  const long long total = (long long)npad * ldo;
-  for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < total;
-       idx += (long long)gridDim.x * kThreads) {
-    const int k = (int)(idx / ldo);
-    const int i = (int)(idx % ldo);
-    const double v = (k < nao && i < nocc) ? c[(long long)k * nocc + i] : 0.0;
-    out[idx] = (T)v;
-  }
-}
-
-__global__ __launch_bounds__(kThreads) void occ_signs_kernel(const double* __restrict__ in, int nocc, int ldo,
-                                                              double* __restrict__ out) {
-  const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= ldo) return;
-  out[i] = (i < nocc) ? (in != nullptr ? in[i] : 1.0) : 0.0;
-}
-
 // C[k][j'] = V[k][j] sqrt(|l_j|), signs[j'] = sign(l_j), for the retained
 // columns j = j' (j' < first) and j = (nao - count) + j' - first otherwise.
 // V is column-major (rocSOLVER): V[k][j] = vecs[j * nao + k].
@@ -506,26 +485,6 @@ hipError_t launch_coulomb_unpack(const double* partial, int nsplit, long long p,
     hipLaunchKernelGGL(coulomb_unpack_kernel<1>, grid, dim3(kThreads), 0, s, partial, nsplit, p, nao, out);
   else
     hipLaunchKernelGGL(coulomb_unpack_kernel<4>, grid, dim3(kThreads * 4), 0, s, partial, nsplit, p, nao, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_orbitals(const double* c, int nao, int nocc, int precision, void* out, hipStream_t s) {
-  const int npad = n_tiles(nao) * kTile;
-  const int ldo = occ_ld(nocc);
-  const long long n = (long long)npad * ldo;
-  const unsigned blocks = grid_for(n);
-  if (precision == HFJK_FP64)
-    hipLaunchKernelGGL(orbitals_kernel<double>, dim3(blocks), dim3(kThreads), 0, s, c, nao, nocc, npad, ldo,
-                       (double*)out);
-  else
-    hipLaunchKernelGGL(orbitals_kernel<float>, dim3(blocks), dim3(kThreads), 0, s, c, nao, nocc, npad, ldo,
-                       (float*)out);
-  return hipGetLastError();
-}
-
-hipError_t launch_occ_signs(const double* signs_in, int nocc, int ldo, double* signs_out, hipStream_t s) {
-  hipLaunchKernelGGL(occ_signs_kernel, dim3((unsigned)((ldo + kThreads - 1) / kThreads)), dim3(kThreads), 0, s,
-                     signs_in, nocc, ldo, signs_out);
   return hipGetLastError();
 }
 

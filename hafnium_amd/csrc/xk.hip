@@ -3,9 +3,8 @@
 // arithmetics (FP64, FP32, BF16x3).
 //
 // Structure shared by all of them:
-//  * one 256-thread workgroup (4 waves of 64) per output tile;
-//  * global -> register prefetch of the next k step while the MFMAs of the
-//    current one run from LDS (one LDS buffer, two barriers per step);
+//  * workgroups of 4 waves of 64 (8 for the 256 x 256 tiles), each k step's
+//    loads in flight while the MFMAs of the step before run;
 //  * the SYRK grid is XCD-aware: workgroups are dispatched round-robin over
 //    the 8 XCDs, so linear id b runs on XCD b % 8, and every tile of one
 //    aux-slice split s is mapped to the same XCD. The slice of X that those
@@ -18,11 +17,10 @@
 //  * v_mfma_f32_16x16x32_bf16 : A[i][8 (l / 16) + e] in element e of lane l with
 //    i = l % 16, B[8 (l / 16) + e][j] likewise with j = l % 16; D as f32 16x16x4.
 //
-// FP64/FP32 operands are single elements per lane, so the packed B tiles are
-// kept in LDS in their stored (row-major) order and a transposed tile is read
-// with swapped addressing. BF16x3 operands are 8 consecutive k per lane, so
-// tiles stored transposed are transposed in registers (4 x 4 blocks) on their
-// way into a [row][k] LDS tile.
+// FP64/FP32 operands are single elements per lane, so a packed B tile is read
+// directly or transposed by addressing alone. BF16x3 operands are 8
+// consecutive k per lane, so tiles stored transposed are transposed in
+// registers (4 x 4 blocks) on their way into a [row][k] LDS tile.
 #include <algorithm>
 #include <functional>
 #include <type_traits>
@@ -112,369 +110,206 @@ __device__ __forceinline__ f4 mma3(bf8 ah, bf8 al, bf8 bh, bf8 bl, f4 acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc, 0, 0, 0);
 }
 
-// Wave arrangement of a 64 x BN half-transform tile: WN waves across the
-// columns; each wave covers (64 / WM) rows and (BN / WN) columns.
-template <int BN>
-struct XShape {
-  static constexpr int WN = BN >= 256 ? 4 : 2;
-  static constexpr int WM = 4 / WN;
-  static constexpr int MI = 64 / WM / 16;   // 16-row blocks per wave
-  static constexpr int NI = BN / WN / 16;   // 16-column blocks per wave
-};
-
 // ------------------------------------------------------------------ FP64 / FP32 half-transform
-
-// X[q][m][i] = sum_k B[q][m][k] C[k][i]; workgroup tile BM rows (BM / 32
-// layout tile rows r = (BM / 32) mb + h) x BN columns; one layout tile
-// column kt per k step. BM = 128 doubles the MFMAs per LDS read and halves
-// the staged bytes per flop against BM = 64, at two workgroups per CU.
-template <typename T, int BN, int BM = 64>
-struct XformSmem {
-  T At[BM / kTile][kTile][kTile + 1];
-  T Cs[kTile][BN + 1];
+//
+// X[q][m][i] = sum_k B[q][m][k] C[k][i] from the tiled packed B. The rows of
+// every aux function in blocks of 16 MI form one list of units; each wave of a
+// workgroup computes its own unit for the NI 16-column blocks of a column
+// group, so all waves carry the same columns and no wave waits for another's
+// padding. MI is 1 in FP64 (with 2, accumulators, two B tiles and C's operands
+// spill) and 2 in FP32. One layout tile column per k step:
+// * B goes from global memory straight into the MFMA operand registers, the
+//   next step's tile while this one computes. Element e = EV eg + ee of a
+//   lane's 8 per 16 rows is k = 4 EV eg + EV g + ee (g = lane / 16, EV
+//   elements per 16 bytes), so a tile stored as (r, kt) is read as 16-byte
+//   groups along its rows and one stored as (kt, r) as 128-byte runs of its
+//   columns, without a transpose.
+// * C, in the order the MFMA operand reads it (launch_orbital_fragments),
+//   goes by direct-LDS loads into one of two stage buffers shared by the
+//   waves: one barrier per step, 16-byte conflict-free LDS reads.
+//
+// Bound by the MFMAs: 8 MI NI of them per step and wave, 64 cycles each in FP64
+// (32 in FP32), against 4 KB of B and a shared 4 NI KB (2 NI KB) of C.
+// It replaces 64 / 128-row tiles staged through registers into padded LDS
+// (two barriers per step, waves idle on the padding of their quadrant): 128
+// uneven instances 31.6 -> 22.0 ms, nao 288 / naux 1356 / nocc 60 320 -> 248
+// us, nao 501 / naux 1800 / nocc 90 2.15 -> 1.43 ms (FP64), nao 709 / naux
+// 2503 / nocc 117 in FP32 3.38 -> 2.98 ms.
+template <typename T>
+struct XFrag {
+  static constexpr int EV = 16 / (int)sizeof(T);  // elements per 16-byte group
+  static constexpr int NG = 8 / EV;               // groups per lane and 16 rows of a tile
+  static constexpr int KG = 4 * EV;               // k per group over the four lane groups
+  static constexpr int BLOCK = kTile * 16;        // elements of one 16-column block of a k tile
+  static constexpr int LOADS = BLOCK * (int)sizeof(T) / 1024;  // 1 KB loads per block
+  static constexpr int MI = sizeof(T) == 8 ? 1 : 2;   // 16-row blocks per unit
+  typedef T unit __attribute__((ext_vector_type(16 / sizeof(T))));
 };
 
-// One BM x BN tile (row block mb, column block nb) of X_q = B_q C for one
-// aux function: bq = its packed B, xq = its X rows (xrows of them). The
-// whole workgroup calls it; LDS is free again when it returns. With SKIP the
-// MFMAs of 16-row blocks at or past nrow, of 16-column blocks at or past ncol
-// and of k steps at or past kmax are left out (B and C are zero there, so X
-// is the same); each wave decides for its own blocks.
-template <typename T, int BN, int BM = 64, bool SKIP = false>
-__device__ __forceinline__ void xform_tile(const T* __restrict__ bq, int nt, const T* __restrict__ c, int ldo,
-                                           T* __restrict__ xq, int xrows, int mb, int nb,
-                                           XformSmem<T, BN, BM>& sm, int nrow = 0, int ncol = 0, int kmax = 0) {
-  typedef XShape<BN> S;
-  constexpr int NTL = BM / kTile;                  // layout tiles per row block
-  constexpr int MI = BM / S::WM / 16;              // 16-row blocks per wave
-  constexpr int CCH = kTile * BN / 2 / kThreads;  // 2-element chunks of the C tile per thread
-  auto& At = sm.At;
-  auto& Cs = sm.Cs;
-  const int n0 = nb * BN;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int wm = wave % S::WM;
-  const int wn = wave / S::WM;
-
-  typename Op<T>::acc_t acc[MI][S::NI];
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < S::NI; ++ni)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[mi][ni][r] = (T)0;
-
-  // Prefetch registers: 4 consecutive elements of each of the NTL tiles,
-  // and CCH 2-element chunks of the C tile.
-  typename Op<T>::vec2 ra[NTL][2];
-  typename Op<T>::vec2 rc[CCH];
-
-  auto load = [&](int kt) {
-#pragma unroll
-    for (int h = 0; h < NTL; ++h) {
-      const int r = NTL * mb + h;
-      if (r < nt) {
-        const long long off = (r >= kt ? tidx(r, kt) : tidx(kt, r)) * kTileElems + t * 4;
-        const typename Op<T>::vec2* src = (const typename Op<T>::vec2*)(bq + off);
-        ra[h][0] = src[0];
-        ra[h][1] = src[1];
-      } else {
-        ra[h][0].x = ra[h][0].y = ra[h][1].x = ra[h][1].y = (T)0;
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < CCH; ++v) {
-      const int chunk = t + kThreads * v;
-      const int kk = chunk / (BN / 2);
-      const int col = n0 + (chunk % (BN / 2)) * 2;
-      if (col < ldo) {
-        rc[v] = *(const typename Op<T>::vec2*)(c + (long long)(kt * kTile + kk) * ldo + col);
-      } else {
-        rc[v].x = rc[v].y = (T)0;
-      }
-    }
-  };
-  auto store = [&]() {
-    const int a = (t * 4) / kTile;
-    const int bc = (t * 4) % kTile;
-#pragma unroll
-    for (int h = 0; h < NTL; ++h) {
-      At[h][a][bc + 0] = ra[h][0].x;
-      At[h][a][bc + 1] = ra[h][0].y;
-      At[h][a][bc + 2] = ra[h][1].x;
-      At[h][a][bc + 3] = ra[h][1].y;
-    }
-#pragma unroll
-    for (int v = 0; v < CCH; ++v) {
-      const int chunk = t + kThreads * v;
-      const int kk = chunk / (BN / 2);
-      const int jj = (chunk % (BN / 2)) * 2;
-      Cs[kk][jj] = rc[v].x;
-      Cs[kk][jj + 1] = rc[v].y;
-    }
-  };
-
-  // Wave-uniform block masks of SKIP.
-  bool rv[MI], cv[S::NI];
-  if constexpr (SKIP) {
-    const int wu = __builtin_amdgcn_readfirstlane(t >> 6);
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi) rv[mi] = mb * BM + (wu % S::WM) * (BM / S::WM) + mi * 16 < nrow;
-#pragma unroll
-    for (int ni = 0; ni < S::NI; ++ni) cv[ni] = n0 + (wu / S::WM) * (BN / S::WN) + ni * 16 < ncol;
-  }
-
-  load(0);
-  store();
-  __syncthreads();
-  for (int kt = 0; kt < nt; ++kt) {
-    if (kt + 1 < nt) load(kt + 1);
-    // Tile h is stored as (r, kt) when r >= kt (read A[i][k] = At[h][i][k]) and
-    // as (kt, r) otherwise (read A[i][k] = At[h][k][i]).
-    bool direct[NTL];
-#pragma unroll
-    for (int h = 0; h < NTL; ++h) direct[h] = (NTL * mb + h) >= kt;
-#pragma unroll
-    for (int kk = 0; kk < kTile; kk += 4) {
-      if constexpr (SKIP) {
-        if (kt * kTile + kk >= kmax) break;
-      }
-      const int k = kk + (lane >> 4);
-      T af[MI], bf[S::NI];
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi) {
-        const int row = wm * (BM / S::WM) + mi * 16 + (lane & 15);
-        const int h = row >> 5;
-        const int i = row & 31;
-        af[mi] = direct[h] ? At[h][i][k] : At[h][k][i];
-      }
-#pragma unroll
-      for (int ni = 0; ni < S::NI; ++ni) bf[ni] = Cs[k][wn * (BN / S::WN) + ni * 16 + (lane & 15)];
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < S::NI; ++ni) {
-          if constexpr (SKIP) {
-            if (!(rv[mi] && cv[ni])) continue;
-          }
-          acc[mi][ni] = Op<T>::mma(af[mi], bf[ni], acc[mi][ni]);
-        }
-    }
-    __syncthreads();
-    if (kt + 1 < nt) {
-      store();
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < S::NI; ++ni) {
-      const int col = n0 + wn * (BN / S::WN) + ni * 16 + (lane & 15);
-      if (col < ldo) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = mb * BM + wm * (BM / S::WM) + mi * 16 + Op<T>::row(lane, r);
-          if (row < xrows) xq[(long long)row * ldo + col] = acc[mi][ni][r];
-        }
-      }
-    }
+// s_waitcnt vmcnt(VM) lgkmcnt(0) (gfx9 encoding: vmcnt in bits 3:0 and 15:14).
+template <int VM>
+__device__ __forceinline__ void wait_vm_lgkm0() {
+  static_assert(VM >= 0 && VM < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (0x7 << 4));
 }
 
-// The half-transform tile of xform_tile for each aux function q in
-// [q0, q1) (the batched kernels' items): b = the packed B of aux function 0 (q's at
-// stride p), x = X of aux function 0 (q's at stride xrows * ldo). The
-// (q, k tile) steps run as one pipeline: the next step's loads are issued
-// before the current step's MFMAs, across aux functions too, and each q's
-// tile is written out after its last k tile. The whole workgroup calls it;
-// LDS is free again when it returns. With SKIP the MFMAs of 16-row blocks
-// at or past nrow, of 16-column blocks at or past ncol and of k steps at or
-// past kmax are left out (B and C are zero there, so X is the same); each
-// wave decides for its own blocks.
-template <typename T, int BN, int BM = 64, bool SKIP = false>
-__device__ __forceinline__ void xform_tiles(const T* __restrict__ b, long long p, int nt, const T* __restrict__ c,
-                                            int ldo, T* __restrict__ x, int xrows, int mb, int nb, int q0, int q1,
-                                            XformSmem<T, BN, BM>& sm, int nrow = 0, int ncol = 0, int kmax = 0) {
-  typedef XShape<BN> S;
-  constexpr int NTL = BM / kTile;                  // layout tiles per row block
-  constexpr int MI = BM / S::WM / 16;              // 16-row blocks per wave
-  constexpr int CCH = kTile * BN / 2 / kThreads;  // 2-element chunks of the C tile per thread
-  auto& At = sm.At;
-  auto& Cs = sm.Cs;
-  const int n0 = nb * BN;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int wm = wave % S::WM;
-  const int wn = wave / S::WM;
+// Workgroup barrier without a memory fence (a fence would wait for every
+// load in flight, the stages ahead included). The clobber keeps the compiler
+// from moving memory accesses across it.
+__device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" ::: "memory"); }
 
-  typename Op<T>::acc_t acc[MI][S::NI];
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < S::NI; ++ni)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[mi][ni][r] = (T)0;
+typedef __attribute__((address_space(3))) void lds_void_t;
 
-  // Prefetch registers: 4 consecutive elements of each of the NTL tiles,
-  // and CCH 2-element chunks of the C tile.
-  typename Op<T>::vec2 ra[NTL][2];
-  typename Op<T>::vec2 rc[CCH];
+// Units [u0, u1) (unit q nu + r, nu = ceil(nao / 16 MI)) of the column group
+// whose fragments start at cf: b = the packed B of aux function 0, x = X of
+// aux function 0 at the group's first column. zero_block: X's 16 columns
+// after the group are written as zeros (the padding of ldo past an odd number
+// of blocks). Rows past the last unit are not written. The whole workgroup
+// calls it; on return its LDS reads have returned and no load is in flight.
+template <typename T, int NI>
+__device__ __forceinline__ void xform_units(const T* __restrict__ b, long long p, int nt, const T* __restrict__ cf,
+                                            T* __restrict__ x, int xrows, int ldo, int u0, int u1, int nao,
+                                            bool zero_block, T* lds0, T* lds1) {
+  typedef XFrag<T> F;
+  typedef typename F::unit unit;
+  constexpr int MI = F::MI;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = blockDim.x >> 6;
+  const int row16 = lane & 15, grp = lane >> 4;
+  const int nu = xform_units_per_aux<T>(nao);
 
-  auto load = [&](int q, int kt) {
-    const T* bq = b + (long long)q * p;
-#pragma unroll
-    for (int h = 0; h < NTL; ++h) {
-      const int r = NTL * mb + h;
-      if (r < nt) {
-        const long long off = (r >= kt ? tidx(r, kt) : tidx(kt, r)) * kTileElems + t * 4;
-        const typename Op<T>::vec2* src = (const typename Op<T>::vec2*)(bq + off);
-        ra[h][0] = src[0];
-        ra[h][1] = src[1];
-      } else {
-        ra[h][0].x = ra[h][0].y = ra[h][1].x = ra[h][1].y = (T)0;
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < CCH; ++v) {
-      const int chunk = t + kThreads * v;
-      const int kk = chunk / (BN / 2);
-      const int col = n0 + (chunk % (BN / 2)) * 2;
-      if (col < ldo) {
-        rc[v] = *(const typename Op<T>::vec2*)(c + (long long)(kt * kTile + kk) * ldo + col);
-      } else {
-        rc[v].x = rc[v].y = (T)0;
-      }
-    }
-  };
-  auto store = [&]() {
-    const int a = (t * 4) / kTile;
-    const int bc = (t * 4) % kTile;
-#pragma unroll
-    for (int h = 0; h < NTL; ++h) {
-      At[h][a][bc + 0] = ra[h][0].x;
-      At[h][a][bc + 1] = ra[h][0].y;
-      At[h][a][bc + 2] = ra[h][1].x;
-      At[h][a][bc + 3] = ra[h][1].y;
-    }
-#pragma unroll
-    for (int v = 0; v < CCH; ++v) {
-      const int chunk = t + kThreads * v;
-      const int kk = chunk / (BN / 2);
-      const int jj = (chunk % (BN / 2)) * 2;
-      Cs[kk][jj] = rc[v].x;
-      Cs[kk][jj + 1] = rc[v].y;
-    }
-  };
-
-  // Wave-uniform block masks of SKIP.
-  bool rv[MI], cv[S::NI];
-  if constexpr (SKIP) {
-    const int wu = __builtin_amdgcn_readfirstlane(t >> 6);
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi) rv[mi] = mb * BM + (wu % S::WM) * (BM / S::WM) + mi * 16 < nrow;
-#pragma unroll
-    for (int ni = 0; ni < S::NI; ++ni) cv[ni] = n0 + (wu / S::WM) * (BN / S::WN) + ni * 16 < ncol;
+  int steps = ((u1 - u0 + waves - 1) / waves) * nt;
+  int u = u0 + wave;
+  int q = u / nu, r = u - q * nu, kt = 0;
+  int qc = u0 / nu, rc = u0 - qc * nu;  // a unit whose tiles may be read (u0 < u1)
+  if (u < u1) {
+    qc = q;
+    rc = r;
   }
 
-  const int steps = (q1 - q0) * nt;
-  if (steps <= 0) return;
-  load(q0, 0);
-  store();
-  __syncthreads();
-  int q = q0, kt = 0;
-  for (int step = 0; step < steps; ++step) {
-    const int nq = kt + 1 < nt ? q : q + 1;
-    const int nkt = kt + 1 < nt ? kt + 1 : 0;
-    if (step + 1 < steps) load(nq, nkt);
-    // Tile h is stored as (r, kt) when r >= kt (read A[i][k] = At[h][i][k]) and
-    // as (kt, r) otherwise (read A[i][k] = At[h][k][i]).
-    bool direct[NTL];
-#pragma unroll
-    for (int h = 0; h < NTL; ++h) direct[h] = (NTL * mb + h) >= kt;
-#pragma unroll
-    for (int kk = 0; kk < kTile; kk += 4) {
-      if constexpr (SKIP) {
-        if (kt * kTile + kk >= kmax) break;
-      }
-      const int k = kk + (lane >> 4);
-      T af[MI], bf[S::NI];
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi) {
-        const int row = wm * (BM / S::WM) + mi * 16 + (lane & 15);
-        const int h = row >> 5;
-        const int i = row & 31;
-        af[mi] = direct[h] ? At[h][i][k] : At[h][k][i];
-      }
-#pragma unroll
-      for (int ni = 0; ni < S::NI; ++ni) bf[ni] = Cs[k][wn * (BN / S::WN) + ni * 16 + (lane & 15)];
+  auto load_c = [&](int k, T* stage) {
+    const T* src = cf + (long long)k * NI * F::BLOCK + lane * F::EV;
+    for (int c = wave; c < NI * F::LOADS; c += waves)
+      __builtin_amdgcn_global_load_lds((const void*)(src + c * 64 * F::EV), (lds_void_t*)(stage + c * 64 * F::EV), 16,
+                                       0, 0);
+  };
+  auto load_a = [&](int qq, int rr, int k, unit (&a)[MI][F::NG]) {
+    const T* bq = b + (long long)qq * p;
+    const int tr = rr * MI / 2, half = rr * MI % 2;  // layout tile row, its 16-row half
+    if (tr >= k) {
+      const T* src = bq + tidx(tr, k) * kTileElems + (half * 16 + row16) * kTile + grp * F::EV;
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < S::NI; ++ni) {
-          if constexpr (SKIP) {
-            if (!(rv[mi] && cv[ni])) continue;
-          }
-          acc[mi][ni] = Op<T>::mma(af[mi], bf[ni], acc[mi][ni]);
-        }
+        for (int eg = 0; eg < F::NG; ++eg) a[mi][eg] = *(const unit*)(src + mi * 16 * kTile + eg * F::KG);
+    } else {
+      const T* src = bq + tidx(k, tr) * kTileElems + grp * F::EV * kTile + half * 16 + row16;
+#pragma unroll
+      for (int eg = 0; eg < F::NG; ++eg)
+#pragma unroll
+        for (int ee = 0; ee < F::EV; ++ee)
+#pragma unroll
+          for (int mi = 0; mi < MI; ++mi)
+            a[mi][eg][ee] = src[(eg * F::KG + ee) * kTile + mi * 16];
     }
-    __syncthreads();
-    if (kt == nt - 1) {
-      // This aux function's tile is complete: write it and start the next one from zero.
-      const int qw = q;
-      T* xq = x + (long long)qw * xrows * ldo;
+  };
+
+  typename Op<T>::acc_t acc[MI][NI];
+  auto clear = [&]() {
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[mi][ni][e] = (T)0;
+  };
+  auto group = [&](const T* stage, int eg, const unit (&a)[MI][F::NG]) {
+    unit bv[NI];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) bv[ni] = *(const unit*)(stage + ((eg * NI + ni) * 64 + lane) * F::EV);
+#pragma unroll
+    for (int ee = 0; ee < F::EV; ++ee)
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < S::NI; ++ni) {
-          const int col = n0 + wn * (BN / S::WN) + ni * 16 + (lane & 15);
-          if (col < ldo) {
+        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = Op<T>::mma(a[mi][eg][ee], bv[ni][ee], acc[mi][ni]);
+  };
+
+  // Step: this wave's loads for it have landed and its LDS reads of the step
+  // before have returned; after the barrier that holds for every wave, so the
+  // other buffer takes the next step's C while this step computes.
+  auto step = [&](const T* cur, T* next, unit (&a)[MI][F::NG], unit (&an)[MI][F::NG]) {
+    wait_vm_lgkm0<0>();
+    barrier_nofence();
+    const bool last = kt + 1 == nt;
+    int un = u, qn = q, rn = r;
+    if (u < u1) {
+      qc = q;
+      rc = r;
+    }
+    const int kn = last ? 0 : kt + 1;
+    if (last) {
+      un += waves;
+      rn += waves;
+      while (rn >= nu) {
+        rn -= nu;
+        ++qn;
+      }
+    }
+    // (A wave without a next unit reads this one's tile again: a conditional load would end in
+    // register copies, and those in a wait.)
+    if (steps > 1) load_c(kn, next);
+    const bool more = un < u1;
+    load_a(more ? qn : qc, more ? rn : rc, kn, an);
+    if (u < u1) {
+      // k past nao holds zeros.
+      const int kleft = nao - kt * kTile;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int row = mb * BM + wm * (BM / S::WM) + mi * 16 + Op<T>::row(lane, r);
-              if (row < xrows) xq[(long long)row * ldo + col] = acc[mi][ni][r];
-            }
+      for (int eg = 0; eg < F::NG; ++eg)
+        if (eg * F::KG < kleft) group(cur, eg, a);
+      if (last) {
+        T* dst = x + ((long long)q * xrows + r * 16 * MI) * ldo + row16;
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            T* at = dst + (long long)(mi * 16 + Op<T>::row(lane, e)) * ldo;
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) at[ni * 16] = acc[mi][ni][e];
+            if (zero_block) at[NI * 16] = (T)0;
           }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[mi][ni][r] = (T)0;
-        }
+        clear();
+      }
     }
-    if (step + 1 < steps) {
-      store();
-      __syncthreads();
-    }
-    q = nq;
-    kt = nkt;
+    u = un;
+    q = qn;
+    r = rn;
+    kt = kn;
+    return --steps > 0;
+  };
+
+  unit a0[MI][F::NG], a1[MI][F::NG];
+  clear();
+  load_c(0, lds0);
+  load_a(qc, rc, 0, a0);
+  while (step(lds0, lds1, a0, a1) && step(lds1, lds0, a1, a0)) {
   }
 }
 
-template <typename T, int BN, int BM>
-__global__ __launch_bounds__(kThreads) void xform_kernel(const T* __restrict__ b, long long p, int nt,
-                                                          const T* __restrict__ c, int ldo, T* __restrict__ x,
-                                                          int xrows, int qbase, int nblocks_n, int nblocks_m,
-                                                          int nwg) {
-  __shared__ XformSmem<T, BN, BM> sm;
+// Workgroup: `per` units of one column group (wg % ngroups), NI blocks wide
+// except the last group's `tail`, which a launch of its own handles.
+template <typename T, int NI>
+__global__ __launch_bounds__(kThreads, NI <= 4 ? 3 : 2) void xform_units_kernel(
+    const T* __restrict__ b, long long p, int nt, const T* __restrict__ cf, long long group_elems, int ngroups,
+    T* __restrict__ x, int xrows, int ldo, int units, int per, int nao, int zero_block, int nwg) {
+  __shared__ __attribute__((aligned(16))) T lds0[NI * XFrag<T>::BLOCK];
+  __shared__ __attribute__((aligned(16))) T lds1[NI * XFrag<T>::BLOCK];
   const int logical = xcd_remap(blockIdx.x, nwg);
-  const int nb = logical % nblocks_n;
-  const int mb = (logical / nblocks_n) % nblocks_m;
-  const int q = qbase + logical / (nblocks_n * nblocks_m);
-  xform_tile<T, BN, BM>(b + (long long)q * p, nt, c, ldo, x + (long long)q * xrows * ldo, xrows, mb, nb, sm);
-}
-
-// The same kernel held to 256 registers per lane (two waves per SIMD): the
-// 128 x 128 FP64 tile needs 258 otherwise.
-template <typename T, int BN, int BM>
-__global__ __launch_bounds__(kThreads, 2) void xform_kernel_w2(const T* __restrict__ b, long long p, int nt,
-                                                                const T* __restrict__ c, int ldo, T* __restrict__ x,
-                                                                int xrows, int qbase, int nblocks_n, int nblocks_m,
-                                                                int nwg) {
-  __shared__ XformSmem<T, BN, BM> sm;
-  const int logical = xcd_remap(blockIdx.x, nwg);
-  const int nb = logical % nblocks_n;
-  const int mb = (logical / nblocks_n) % nblocks_m;
-  const int q = qbase + logical / (nblocks_n * nblocks_m);
-  xform_tile<T, BN, BM>(b + (long long)q * p, nt, c, ldo, x + (long long)q * xrows * ldo, xrows, mb, nb, sm);
+  const int g = logical % ngroups;
+  const int u0 = logical / ngroups * per;
+  xform_units<T, NI>(b, p, nt, cf + g * group_elems, x + g * NI * 16, xrows, ldo, u0, min(u0 + per, units), nao,
+                     zero_block != 0 && g == ngroups - 1, lds0, lds1);
 }
 
 // ------------------------------------------------------------------ BF16x3 half-transform
@@ -1209,8 +1044,6 @@ __global__ __launch_bounds__(kThreads) void syrk_kernel(const T* __restrict__ x,
 constexpr int kDmaStages = 4;
 constexpr int kDmaMaxLdo = 2048;
 
-typedef __attribute__((address_space(3))) void lds_void_t;
-
 template <typename T, int CH>
 struct SyrkDma {
   static constexpr int E = 16 / (int)sizeof(T);       // elements per 16-byte group
@@ -1221,18 +1054,6 @@ struct SyrkDma {
   static constexpr int LOADS = 4 * CH;                  // load instructions per wave per stage
   typedef T unit __attribute__((ext_vector_type(16 / sizeof(T))));
 };
-
-// s_waitcnt vmcnt(VM) lgkmcnt(0) (gfx9 encoding: vmcnt in bits 3:0 and 15:14).
-template <int VM>
-__device__ __forceinline__ void wait_vm_lgkm0() {
-  static_assert(VM >= 0 && VM < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (0x7 << 4));
-}
-
-// Workgroup barrier without a memory fence (a fence would wait for every
-// load in flight, the stages ahead included). The clobber keeps the compiler
-// from moving memory accesses across it.
-__device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" ::: "memory"); }
 
 // The ring: acc += sum over `steps` k steps of (A rows) x (B rows)^T, the
 // 128 rows of each operand read at step k from src(k, operand) plus this
@@ -1645,17 +1466,25 @@ __global__ __launch_bounds__(kThreads) void expand_full_kernel(const double* __r
   }
 }
 
-// C^T in T: ct[i][k] = C[k][i] for k < nao, i < nocc, zero elsewhere
-// ([ldo][npad]).
+// The orbitals C [nao][nocc] in the forms a build needs, each where its
+// pointer is given, in one pass over the zero-padded [npad][ldo] matrix: the
+// matrix itself (pad), its transpose (ct), the MFMA operand order of the
+// packed half-transform (frag), and the column signs (+1 by default).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void orbitals_t_kernel(const double* __restrict__ c, int nao, int nocc,
-                                                               int npad, int ldo, T* __restrict__ ct) {
+__global__ __launch_bounds__(kThreads) void prepare_orbitals_kernel(const double* __restrict__ c, int nao, int nocc,
+                                                                     int npad, int ldo, T* __restrict__ pad,
+                                                                     T* __restrict__ ct, T* __restrict__ frag,
+                                                                     ColumnGroups cg, const double* __restrict__ signs_in,
+                                                                     double* __restrict__ signs) {
   const long long total = (long long)npad * ldo;
   for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < total;
        idx += (long long)gridDim.x * kThreads) {
-    const int i = (int)(idx / npad);
-    const int k = (int)(idx % npad);
-    ct[idx] = (T)((k < nao && i < nocc) ? c[(long long)k * nocc + i] : 0.0);
+    const int k = (int)(idx / ldo), i = (int)(idx % ldo);
+    const T v = (T)((k < nao && i < nocc) ? c[(long long)k * nocc + i] : 0.0);
+    if (pad != nullptr) pad[idx] = v;
+    if (ct != nullptr) ct[(long long)i * npad + k] = v;
+    if (frag != nullptr && i / 16 < cg.groups * cg.blocks + cg.tail) frag[fragment_index<T>(cg, npad, k, i)] = v;
+    if (signs != nullptr && k == 0) signs[i] = i < nocc ? (signs_in != nullptr ? signs_in[i] : 1.0) : 0.0;
   }
 }
 
@@ -2483,26 +2312,36 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
   }
 }
 
-template <typename T, int BN, int BM, bool W2 = false>
-hipError_t launch_x_t(const T* b, long long p, int naux, int nao, const T* c, int ldo, T* x, hipStream_t s) {
+template <typename T, int NI>
+hipError_t launch_units(const T* b, long long p, int naux, int nao, const T* cf, int ngroups, bool zero_block, T* x,
+                        int ldo, int waves, hipStream_t s) {
   const int nt = n_tiles(nao);
-  const int xrows = x_rows(nao);
-  const int nbn = (ldo + BN - 1) / BN;
-  const int nbm = (xrows + BM - 1) / BM;
-  const int per = std::max(1, (1 << 24) / (nbn * nbm));  // keep a launch below 2^32 work-items
-  for (int base = 0; base < naux; base += per) {
-    const int count = std::min(per, naux - base);
-    const int nwg = nbn * nbm * count;
-    if constexpr (W2)
-      hipLaunchKernelGGL((xform_kernel_w2<T, BN, BM>), dim3((unsigned)nwg), dim3(kThreads), 0, s, b, p, nt, c, ldo,
-                         x, xrows, base, nbn, nbm, nwg);
-    else
-      hipLaunchKernelGGL((xform_kernel<T, BN, BM>), dim3((unsigned)nwg), dim3(kThreads), 0, s, b, p, nt, c, ldo, x,
-                         xrows, base, nbn, nbm, nwg);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
+  const int units = naux * xform_units_per_aux<T>(nao);
+  const long long group_elems = (long long)nt * NI * XFrag<T>::BLOCK;
+  // Units per workgroup: about eight k steps each, so that the first loads of a workgroup are a
+  // small part of its life, unless that leaves fewer than 1024 workgroups.
+  const int most = std::max(1, units / (waves * 1024) * ngroups);
+  const int per = waves * std::max(1, std::min(8 / nt, most));
+  const long long nwg = (long long)((units + per - 1) / per) * ngroups;
+  if (nwg >= (1LL << 24)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((xform_units_kernel<T, NI>), dim3((unsigned)nwg), dim3(64 * waves), 0, s, b, p, nt, cf,
+                     group_elems, ngroups, x, x_rows(nao), ldo, units, per, nao, zero_block ? 1 : 0, (int)nwg);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_units_n(int ni, const T* b, long long p, int naux, int nao, const T* cf, int ngroups,
+                          bool zero_block, T* x, int ldo, int waves, hipStream_t s) {
+  switch (ni) {
+    case 1: return launch_units<T, 1>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    case 2: return launch_units<T, 2>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    case 3: return launch_units<T, 3>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    case 4: return launch_units<T, 4>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    case 5: return launch_units<T, 5>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    case 6: return launch_units<T, 6>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    case 7: return launch_units<T, 7>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
+    default: return launch_units<T, 8>(b, p, naux, nao, cf, ngroups, zero_block, x, ldo, waves, s);
   }
-  return hipSuccess;
 }
 
 template <int BN>
@@ -2542,17 +2381,6 @@ hipError_t launch_expand_full(const double* packed, long long p, int naux, int n
   else
     hipLaunchKernelGGL(expand_full16_kernel, grid, dim3(kThreads), 0, s, packed, p, naux, ntp, npad,
                        (uint16_t*)out);
-  return hipGetLastError();
-}
-
-hipError_t launch_orbitals_t(const double* c, int nao, int nocc, int precision, void* ct, hipStream_t s) {
-  const int npad = n_tiles(nao) * kTile;
-  const int ldo = occ_ld(nocc);
-  const dim3 grid(grid_for((long long)npad * ldo));
-  if (precision == HFJK_FP64)
-    hipLaunchKernelGGL(orbitals_t_kernel<double>, grid, dim3(kThreads), 0, s, c, nao, nocc, npad, ldo, (double*)ct);
-  else
-    hipLaunchKernelGGL(orbitals_t_kernel<float>, grid, dim3(kThreads), 0, s, c, nao, nocc, npad, ldo, (float*)ct);
   return hipGetLastError();
 }
 
@@ -2779,28 +2607,42 @@ static int pick_bn(int bn, int ldo) {
   return ldo <= 32 ? 32 : ldo <= 64 ? 64 : ldo <= 128 ? 128 : 256;
 }
 
+// FP64 / FP32 half-transform from the packed B. bn caps the columns of a
+// group (0 = 128, what the accumulators have room for), bm = 64 runs two
+// waves per workgroup instead of four. A last group narrower than the others
+// runs in a launch of its own.
 template <typename T>
-hipError_t launch_x_typed(const T* b, long long p, int naux, int nao, const T* c, int ldo, T* x, int bn, int bm,
-                          hipStream_t s) {
-  // 128-row tiles for column tiles up to 128 (a 128 x 256 tile would not fit the register file).
-  if (bm == 128 && bn <= 128) {
-    if (bn == 32) return launch_x_t<T, 32, 128>(b, p, naux, nao, c, ldo, x, s);
-    if (bn == 64) return launch_x_t<T, 64, 128>(b, p, naux, nao, c, ldo, x, s);
-    // FP64 128 x 128 is held to two waves per SIMD (see xform_kernel_w2).
-    return launch_x_t<T, 128, 128, sizeof(T) == 8>(b, p, naux, nao, c, ldo, x, s);
-  }
-  if (bn == 32) return launch_x_t<T, 32, 64>(b, p, naux, nao, c, ldo, x, s);
-  if (bn == 64) return launch_x_t<T, 64, 64>(b, p, naux, nao, c, ldo, x, s);
-  if (bn == 128) return launch_x_t<T, 128, 64>(b, p, naux, nao, c, ldo, x, s);
-  return launch_x_t<T, 256, 64>(b, p, naux, nao, c, ldo, x, s);
+hipError_t launch_x_typed(const T* b, long long p, int naux, int nao, const T* cf, int nocc, int ldo, T* x, int bn,
+                          int bm, hipStream_t s) {
+  const ColumnGroups cg = column_groups(nocc, ldo, bn);
+  const int waves = bm == 64 ? 2 : 4;
+  const bool zero = cg.groups * cg.blocks + cg.tail < ldo / 16;
+  hipError_t e = launch_units_n<T>(cg.blocks, b, p, naux, nao, cf, cg.groups, zero && cg.tail == 0, x, ldo, waves, s);
+  if (e != hipSuccess || cg.tail == 0) return e;
+  const long long done = (long long)cg.groups * cg.blocks;
+  return launch_units_n<T>(cg.tail, b, p, naux, nao, cf + done * n_tiles(nao) * XFrag<T>::BLOCK, 1, zero,
+                           x + done * 16, ldo, waves, s);
 }
 
-hipError_t launch_half_transform(const void* b, int precision, long long p, int naux, int nao, const void* c, int ldo,
-                                 void* x, int bn, int bm, hipStream_t s) {
-  bn = pick_bn(bn, ldo);
+hipError_t launch_half_transform(const void* b, int precision, long long p, int naux, int nao, const void* cf,
+                                 int nocc, int ldo, void* x, int bn, int bm, hipStream_t s) {
   if (precision == HFJK_FP64)
-    return launch_x_typed<double>((const double*)b, p, naux, nao, (const double*)c, ldo, (double*)x, bn, bm, s);
-  return launch_x_typed<float>((const float*)b, p, naux, nao, (const float*)c, ldo, (float*)x, bn, bm, s);
+    return launch_x_typed<double>((const double*)b, p, naux, nao, (const double*)cf, nocc, ldo, (double*)x, bn, bm, s);
+  return launch_x_typed<float>((const float*)b, p, naux, nao, (const float*)cf, nocc, ldo, (float*)x, bn, bm, s);
+}
+
+hipError_t launch_prepare_orbitals(const double* c, int nao, int nocc, int precision, void* pad, void* ct, void* frag,
+                                   int bn, const double* signs_in, double* signs, hipStream_t s) {
+  const int npad = n_tiles(nao) * kTile, ldo = occ_ld(nocc);
+  const dim3 grid((unsigned)grid_for((long long)npad * ldo)), blk(kThreads);
+  const ColumnGroups cg = column_groups(nocc, ldo, bn);
+  if (precision == HFJK_FP64)
+    hipLaunchKernelGGL(prepare_orbitals_kernel<double>, grid, blk, 0, s, c, nao, nocc, npad, ldo, (double*)pad,
+                       (double*)ct, (double*)frag, cg, signs_in, signs);
+  else
+    hipLaunchKernelGGL(prepare_orbitals_kernel<float>, grid, blk, 0, s, c, nao, nocc, npad, ldo, (float*)pad,
+                       (float*)ct, (float*)frag, cg, signs_in, signs);
+  return hipGetLastError();
 }
 
 hipError_t launch_half_transform_bf16x3(const uint16_t* b, long long p, int naux, int nao, const void* ct, int ldo,
@@ -2955,26 +2797,6 @@ hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int
 
 namespace {
 
-template <typename T, int BN>
-__global__ __launch_bounds__(kThreads) void batch_xform_kernel(BatchView v, const T* __restrict__ b,
-                                                                const T* __restrict__ cbase, T* __restrict__ xbase) {
-  __shared__ XformSmem<T, BN> sm;
-  const long long* pre = v.prefix + (long long)kPhXform * (v.ninst + 1);
-  for (;;) {
-    long long end;
-    const long long item = batch_next(v.prefix, v.counters, v.ninst, kPhXform, end);
-    if (item >= end) break;
-    const int i = batch_find(pre, v.ninst, item);
-    const BatchInst in = v.insts[i];
-    const long long local = item - pre[i];
-    const int nb = (int)(local % in.nbn);
-    const int mb = (int)((local / in.nbn) % in.nbm);
-    const int q = (int)(local / ((long long)in.nbn * in.nbm));
-    xform_tile<T, BN>(b + in.b_off + (long long)q * in.p, in.nt, cbase + in.cp_off, in.ldo,
-                      xbase + in.x_off + (long long)q * in.xrows * in.ldo, in.xrows, mb, nb, sm);
-  }
-}
-
 template <int BN>
 __global__ __launch_bounds__(kThreads) void batch_xform16_kernel(BatchView v, const uint16_t* __restrict__ b,
                                                                   long long b_plane, const uint16_t* __restrict__ cbase,
@@ -3000,21 +2822,12 @@ __global__ __launch_bounds__(kThreads) void batch_xform16_kernel(BatchView v, co
   }
 }
 
-// The half-transform with each instance's own tile (in.bm x in.bn: 64 x 32,
-// 64 x 64, 64 x 128 or 128 x 64): the tile shapes share one LDS buffer.
+// FP64 / FP32 half-transform items: in.qg units of one column group.
 template <typename T>
-union XformSmemAny {
-  XformSmem<T, 32> s32;
-  XformSmem<T, 64> s64;
-  XformSmem<T, 128> s128;
-  XformSmem<T, 64, 128> t64;
-};
-
-template <typename T>
-__global__ __launch_bounds__(kThreads, 2) void batch_xform_any_kernel(BatchView v, const T* __restrict__ b,
-                                                                    const T* __restrict__ cbase,
-                                                                    T* __restrict__ xbase) {
-  __shared__ XformSmemAny<T> sm;
+__global__ __launch_bounds__(kThreads, 2) void batch_xform_kernel(BatchView v, const T* __restrict__ b,
+                                                                  const T* __restrict__ cbase, T* __restrict__ xbase) {
+  __shared__ __attribute__((aligned(16))) T lds0[kMaxGroupBlocks * XFrag<T>::BLOCK];
+  __shared__ __attribute__((aligned(16))) T lds1[kMaxGroupBlocks * XFrag<T>::BLOCK];
   const long long* pre = v.prefix + (long long)kPhXform * (v.ninst + 1);
   for (;;) {
     long long end;
@@ -3022,26 +2835,25 @@ __global__ __launch_bounds__(kThreads, 2) void batch_xform_any_kernel(BatchView 
     if (item >= end) break;
     const int i = batch_find(pre, v.ninst, item);
     const BatchInst in = v.insts[i];
-    const long long local = item - pre[i];
-    const int nb = (int)(local % in.nbn);
-    const int mb = (int)((local / in.nbn) % in.nbm);
-    const int q0 = (int)(local / ((long long)in.nbn * in.nbm)) * in.qg;
-    const int q1 = min(in.naux, q0 + in.qg);
-    const T* bb = b + in.b_off;
-    const T* cp = cbase + in.cp_off;
-    T* xb = xbase + in.x_off;
-    if (in.bm == 128)
-      xform_tiles<T, 64, 128, true>(bb, in.p, in.nt, cp, in.ldo, xb, in.xrows, mb, nb, q0, q1, sm.t64, in.nao,
-                                    in.nocc, in.nao);
-    else if (in.bn == 32)
-      xform_tiles<T, 32, 64, true>(bb, in.p, in.nt, cp, in.ldo, xb, in.xrows, mb, nb, q0, q1, sm.s32, in.nao,
-                                   in.nocc, in.nao);
-    else if (in.bn == 64)
-      xform_tiles<T, 64, 64, true>(bb, in.p, in.nt, cp, in.ldo, xb, in.xrows, mb, nb, q0, q1, sm.s64, in.nao,
-                                   in.nocc, in.nao);
-    else
-      xform_tiles<T, 128, 64, true>(bb, in.p, in.nt, cp, in.ldo, xb, in.xrows, mb, nb, q0, q1, sm.s128, in.nao,
-                                    in.nocc, in.nao);
+    const int local = (int)(item - pre[i]);
+    const int g = local % in.nbn;
+    const int u0 = local / in.nbn * in.qg;
+    const int u1 = min(u0 + in.qg, in.naux * xform_units_per_aux<T>(in.nao));
+    const ColumnGroups cg = in.cg;
+    const int nb = g < cg.groups ? cg.blocks : cg.tail;
+    const int block0 = g * cg.blocks;
+    const bool zero = g == in.nbn - 1 && block0 + nb < in.ldo / 16;
+    const T* bi = b + in.b_off;
+    const T* cf = cbase + in.cp_off + (long long)block0 * in.nt * XFrag<T>::BLOCK;
+    T* x = xbase + in.x_off + block0 * 16;
+#define HFJK_UNITS(N) \
+  case N: xform_units<T, N>(bi, in.p, in.nt, cf, x, in.xrows, in.ldo, u0, u1, in.nao, zero, lds0, lds1); break;
+    switch (nb) {
+      HFJK_UNITS(1) HFJK_UNITS(2) HFJK_UNITS(3) HFJK_UNITS(4)
+      HFJK_UNITS(5) HFJK_UNITS(6) HFJK_UNITS(7) HFJK_UNITS(8)
+      default: break;
+    }
+#undef HFJK_UNITS
   }
 }
 
@@ -3232,28 +3044,17 @@ __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v
 
 }  // namespace
 
-int batch_tile_rows(int precision, int xrows, int bn) {
-  if (precision == HFJK_BF16X3) return 128;
-  return xrows >= 128 && bn == 64 ? 128 : kBlock;
-}
-
 hipError_t launch_batch_xform(BatchView v, int precision, int bn, const void* b, long long b_plane, const void* cbase,
                               long long c_plane, void* xbase, long long x_plane, int grid, hipStream_t s) {
   const dim3 g((unsigned)grid), blk(kThreads);
-  // bn = 256: one fixed tile for every instance; otherwise each instance's own tile.
   if (precision == HFJK_FP64) {
-    const double* bb = (const double*)b;
-    const double* cb = (const double*)cbase;
-    double* xb = (double*)xbase;
-    if (bn == 256) hipLaunchKernelGGL((batch_xform_kernel<double, 256>), g, blk, 0, s, v, bb, cb, xb);
-    else hipLaunchKernelGGL(batch_xform_any_kernel<double>, g, blk, 0, s, v, bb, cb, xb);
+    hipLaunchKernelGGL(batch_xform_kernel<double>, g, blk, 0, s, v, (const double*)b, (const double*)cbase,
+                       (double*)xbase);
   } else if (precision == HFJK_FP32) {
-    const float* bb = (const float*)b;
-    const float* cb = (const float*)cbase;
-    float* xb = (float*)xbase;
-    if (bn == 256) hipLaunchKernelGGL((batch_xform_kernel<float, 256>), g, blk, 0, s, v, bb, cb, xb);
-    else hipLaunchKernelGGL(batch_xform_any_kernel<float>, g, blk, 0, s, v, bb, cb, xb);
+    hipLaunchKernelGGL(batch_xform_kernel<float>, g, blk, 0, s, v, (const float*)b, (const float*)cbase,
+                       (float*)xbase);
   } else {
+    // bn = 256: one fixed tile for every instance; otherwise each instance's own tile.
     const uint16_t* bb = (const uint16_t*)b;
     const uint16_t* cb = (const uint16_t*)cbase;
     uint16_t* xb = (uint16_t*)xbase;

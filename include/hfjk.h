@@ -333,13 +333,12 @@ HFJK_API int hfjk_ddot(hfjk_ctx *ctx, long long n, const double *x, const double
                        double *out, void *stream);
 
 /* Tuning parameters of the kernels (0 = the library's default choice).
- * HFJK_TUNE_X_BN: column tile of the FP64/FP32 half-transform (32, 64, 128, 256).
+ * HFJK_TUNE_X_BN: most columns a wave of the FP64/FP32 half-transform covers (32, 64, 128; 256 = 128).
  * HFJK_TUNE_X16_BN: column tile of the BF16x3 half-transform (32, 64, 128, 256;
  * from a bound full copy of B: 256 or 0 = 256 x 256 tiles past 128 occupied
  * columns, else the 128 x 128 ring).
  * HFJK_TUNE_SYRK_SPLITS: aux-slice splits of the SYRK (rounded up to a multiple of 8).
- * HFJK_TUNE_X_BM: row tile of the FP64/FP32 half-transform (64, 128; 128 is
- * used with column tiles up to 128).
+ * HFJK_TUNE_X_BM: workgroup of the FP64/FP32 half-transform: 64 = two waves, 128 = four.
  * HFJK_TUNE_SYRK_KIND: SYRK kernel: 1 = operands staged through registers
  * into one LDS buffer (every precision), 2 = operands loaded straight into a
  * ring of LDS stages with 128 x 128 tiles (occupied widths up to 2048;

@@ -84,3 +84,35 @@ def test_batch_equals_single_builds(precision):
             m = batch.matrix(got, i).cpu().numpy()
             assert np.max(np.abs(m - want)) <= tol * np.max(np.abs(want)), (precision, i)
             np.testing.assert_array_equal(m, m.T)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nao,nocc", [(1, 1), (16, 16), (17, 17), (31, 5), (33, 33), (145, 129), (145, 144), (205, 145),
+                                      (420, 390)])
+def test_half_transform_column_groups(precision, nao, nocc):
+    """Every split of the columns into groups (one, several, a narrower last one) and both workgroup sizes."""
+    from hafnium_amd import _lib
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+    from tests.tolerances import FP32_REL_TOL
+
+    naux = 5
+    b = synthetic.tensor_full(8, naux, nao)
+    c = synthetic.occupied_orbitals(8, nao, nocc)
+    x, xa = b @ c, np.abs(b) @ np.abs(c)
+    expect = np.tensordot(x, x, axes=((0, 2), (0, 2)))
+    bound = 2 * _bound(naux * nocc + 2 * nao, np.tensordot(xa, xa, axes=((0, 2), (0, 2))))
+    jk = MI355XCoulombExchange(b, precision=precision)
+    first = None
+    for columns in (0, 32, 64, 128, 256):
+        for rows in (64, 128):
+            jk.set_tuning(_lib.TUNE_X_BN, columns)
+            jk.set_tuning(_lib.TUNE_X_BM, rows)
+            j, k = jk.jk_occupied(c)
+            if precision == "fp64":
+                assert np.all(np.abs(k - expect) <= bound)
+            else:
+                assert np.max(np.abs(k - expect)) <= FP32_REL_TOL * np.max(np.abs(expect))
+            # The grouping changes neither the products nor their order.
+            first = (j, k) if first is None else first
+            np.testing.assert_array_equal(k, first[1])
+            np.testing.assert_array_equal(j, first[0])
