@@ -337,10 +337,19 @@ void to_sph_pair(const Shell& A, const Shell& B, const std::vector<double>& cart
 std::vector<double> norms(const std::vector<Shell>& shells, int nfunc) {
   std::vector<double> out(nfunc, 1.0);
   std::vector<double> cart, sph;
+  std::vector<const Shell*> seen;  // one shell of every kind: the atoms of an element share theirs
   for (const Shell& s : shells) {
+    const int f = s.nfunc();
+    const Shell* same = nullptr;
+    for (const Shell* o : seen)
+      if (o->l == s.l && o->ncontr == s.ncontr && o->exps == s.exps && o->coefs == s.coefs) same = o;
+    if (same != nullptr) {
+      std::copy_n(out.begin() + same->offset, f, out.begin() + s.offset);
+      continue;
+    }
+    seen.push_back(&s);
     pair_1e(s, s, 0, 0, nullptr, nullptr, cart);
     to_sph_pair(s, s, cart, sph);
-    const int f = s.nfunc();
     for (int k = 0; k < f; ++k) out[s.offset + k] = 1.0 / std::sqrt(sph[(size_t)k * f + k]);
   }
   return out;
@@ -789,7 +798,34 @@ int hfjk_int3c2e(const hfjk_basis* aux, const hfjk_basis* orbital, double* out) 
 
 // ------------------------------------------------------------------ on the GPU
 //
-// (P|uv) and (P|Q) on the device: one 64-lane workgroup per shell triple
+// (P|uv) and (P|Q) on the device, two ways:
+// * lane per aux function (pair_kernel + aux_kernel) up to la + lb = 4 and lc =
+//   4, which is every bundled basis;
+// * one 64-lane workgroup per shell triple (triple_kernel) for higher
+//   angular momenta.
+//
+// Lane per aux function. pair_kernel turns each surviving primitive pair of a
+// shell pair into its Gaussian product and the matrix W from Hermite
+// components (t, u, v) of the product to the pair's spherical, contracted and
+// normalised functions. In aux_kernel a wave takes one shell pair and 64 aux
+// primitives of one angular momentum; per primitive pair each lane forms the
+// Hermite Coulomb integrals of its aux centre in registers and contracts them
+// with W, whose elements are wave-uniform scalar operands:
+//   (ab|P) += W[h][ab] * sum_c T_P[c] R_{h + c}.
+// An aux function is a solid harmonic, so S_lm(r) e^{-g r^2} = (1 / 2g)^l
+// S_lm(d/dC) e^{-g r^2} (Hobson's theorem) and only its l-th derivatives c
+// enter, with the coefficients of the harmonic itself.
+//
+// The arithmetic is small (about 4e9 FMA for 12 waters in cc-pVDZ with
+// def2-universal-jkfit, 0.9 GB of results): what bounds it is the chain of
+// primitives in a wave (the latency of each one's table and scalar loads, about
+// 0.5 us), so contracted pairs are shared by four waves and contracted aux
+// functions by neighbouring lanes. 12 waters' (P|uv) and (P|Q) take 3.9 ms, 1
+// water's 1.75; one workgroup per triple took 82 ms on the former (71 in the
+// kernel, one lane building tables while 63 waited, and 5 in a size check over
+// all triples on the host).
+//
+// triple_kernel: one 64-lane workgroup per shell triple
 // (aux shell C, orbital shell pair A >= B; for the metric A is an aux shell
 // and B a unit s function of exponent 0 on A's centre). Per primitive triple
 // the wave forms, in LDS, the Hermite expansion coefficients of the A B pair
@@ -851,22 +887,24 @@ constexpr int kBoysTaylor = 7;
 constexpr int kBoysOrders = kGMaxL + kBoysTaylor + 1;
 constexpr int kBoysPoints = (int)(kBoysTMax / kBoysStep) + 2;
 
-__device__ void boys_d(int nmax, double t, const double* __restrict__ table, double* f) {
+__device__ __forceinline__ void boys_d(int nmax, double t, const double* __restrict__ table, double* f) {
   const double et = exp(-t);
   if (t < kBoysTMax) {
     const int g = (int)(t / kBoysStep + 0.5);
     const double dt = t - g * kBoysStep;
     const double* row = table + (long long)g * kBoysOrders + nmax;
     double term = 1.0, sum = row[0];
+#pragma unroll
     for (int k = 1; k < kBoysTaylor; ++k) {
       term *= -dt / k;
       sum += term * row[k];
     }
     f[nmax] = sum;
-    for (int n = nmax - 1; n >= 0; --n) f[n] = (2.0 * t * f[n + 1] + et) / (2 * n + 1);
+    for (int n = nmax - 1; n >= 0; --n) f[n] = (2.0 * t * f[n + 1] + et) * (1.0 / (2 * n + 1));
   } else {
-    f[0] = 0.5 * sqrt(kPi / t) * erf(sqrt(t));
-    for (int n = 0; n < nmax; ++n) f[n + 1] = ((2 * n + 1) * f[n] - et) / (2.0 * t);
+    f[0] = 0.5 * sqrt(kPi / t);  // erf(sqrt(t)) is 1 to the last bit here
+    const double i2t = 0.5 / t;
+    for (int n = 0; n < nmax; ++n) f[n + 1] = ((2 * n + 1) * f[n] - et) * i2t;
   }
 }
 
@@ -1078,11 +1116,13 @@ __global__ __launch_bounds__(64) void triple_kernel(const DItem* __restrict__ it
     }
     if (metric_mode) {
       const long long i = A.foff + fa, jj = C.foff + fc;
+      if (jj > i) continue;  // within one shell: the mirror of (jj, i)
       const double val = s * norm_x[i] * norm_x[jj];
       out[i * n + jj] = val;
       out[jj * n + i] = val;
     } else {
       const long long ia = A.foff + fa, ib = B.foff + fb, ic = C.foff + fc;
+      if (ib > ia) continue;
       const double val = s * norm_o[ia] * norm_o[ib] * norm_x[ic];
       out[(ic * n + ia) * n + ib] = val;
       out[(ic * n + ib) * n + ia] = val;
@@ -1090,22 +1130,360 @@ __global__ __launch_bounds__(64) void triple_kernel(const DItem* __restrict__ it
   }
 }
 
-// Device copies of the shell tables of one or two bases, the spherical
-// tables, the norms and the item list; freed with the object.
-struct DeviceTables {
-  std::vector<void*> buffers;
-  ~DeviceTables() {
-    for (void* p : buffers) (void)hipFree(p);
+// ---- lane per aux function
+
+constexpr int kLaneMaxAB = 4;      // la + lb
+constexpr int kLaneMaxC = 4;
+constexpr int kLaneMaxL = 8;       // la + lb + lc
+constexpr int kLaneEA = 45;        // Hermite coefficients per dimension: (la + 1)(lb + 1)(la + lb + 1)
+constexpr int kLaneRows = 18;      // pair functions per wave (accumulators of a lane)
+constexpr int kLaneStep = 6;       // rows of W are padded to a multiple of this
+constexpr int kLaneSlots = 16;     // primitive pairs whose Hermite tables pair_kernel holds at once
+constexpr int kLaneWaves = 4;      // most waves sharing a pair's primitives
+constexpr int kPairThreads = 256;
+constexpr int kLaneMaxPrim = 16;   // aux shells with more primitives go to triple_kernel
+
+constexpr __host__ __device__ int n_herm(int l) { return (l + 1) * (l + 2) * (l + 3) / 6; }
+constexpr __host__ __device__ int n_cart(int l) { return (l + 1) * (l + 2) / 2; }
+constexpr __host__ __device__ int r_index(int t, int u, int v) {
+  const int s = t + u + v, m = u + v;
+  return s * (s + 1) * (s + 2) / 6 + m * (m + 1) / 2 + v;
+}
+
+// Exponents (t, u, v) of every Hermite component up to order L, in r_index order.
+template <int L>
+struct HermList {
+  int t[n_herm(L)] = {}, u[n_herm(L)] = {}, v[n_herm(L)] = {};
+  constexpr HermList() {
+    for (int s = 0, k = 0; s <= L; ++s)
+      for (int m = 0; m <= s; ++m)
+        for (int w = 0; w <= m; ++w, ++k) {
+          t[k] = s - m;
+          u[k] = m - w;
+          v[k] = w;
+        }
+  }
+};
+
+// Cartesian components of l: x power descending, then y.
+template <int L>
+struct CartList {
+  int x[n_cart(L)] = {}, y[n_cart(L)] = {}, z[n_cart(L)] = {};
+  constexpr CartList() {
+    for (int i = L, k = 0; i >= 0; --i)
+      for (int j = L - i; j >= 0; --j, ++k) {
+        x[k] = i;
+        y[k] = j;
+        z[k] = L - i - j;
+      }
+  }
+};
+
+struct LanePair {
+  int a, b;        // shells (b < 0: the unit s function on a's centre)
+  int rows, pad;   // pair functions, and padded to kLaneStep
+  int prims, poff; // primitive pairs: capacity, offset of the products
+  long long woff;  // offset of W
+  int fa, fb, nb;  // first functions, functions of b
+};
+
+// One primitive of one aux function: nprim on a function's first primitive,
+// whose lane the others' sums go to (they follow it in the same wave); 0 on
+// the others and on idle lanes, which have f = -1.
+struct LaneAux {
+  double c[3];
+  double g, coef;
+  int nprim, m, f, pad;
+};
+
+struct LanePrim {
+  double p, x, y, z;
+};
+
+__global__ __launch_bounds__(kPairThreads) void pair_kernel(const LanePair* __restrict__ pairs, const DShell* __restrict__ as,
+                                                  const DShell* __restrict__ bs, const double* __restrict__ exps,
+                                                  const double* __restrict__ coefs, const double* __restrict__ norm,
+                                                  const double* __restrict__ sph, const int* __restrict__ sph_off,
+                                                  int* __restrict__ counts, LanePrim* __restrict__ prims,
+                                                  double* __restrict__ w) {
+  __shared__ double e[kLaneSlots][3][kLaneEA];
+  __shared__ double ta[(2 * kLaneMaxAB + 1) * n_cart(kLaneMaxAB)], tb[(2 * kLaneMaxAB + 1) * n_cart(kLaneMaxAB)];
+  __shared__ int list[64];
+  __shared__ int kept_all;
+  const int tid = threadIdx.x;
+  const LanePair pr = pairs[blockIdx.x];
+  const DShell A = as[pr.a];
+  DShell B = A;
+  if (pr.b >= 0) {
+    B = bs[pr.b];
+  } else {
+    B.l = 0;
+    B.nprim = B.ncontr = 1;
+  }
+  const int na = ncart_d(A.l), nb = ncart_d(B.l), nt = A.l + B.l + 1;
+  const int nh = n_herm(A.l + B.l);
+  for (int k = tid; k < (2 * A.l + 1) * na; k += kPairThreads) ta[k] = sph[sph_off[A.l] + k];
+  for (int k = tid; k < (2 * B.l + 1) * nb; k += kPairThreads) tb[k] = sph[sph_off[B.l] + k];
+  const double ab[3] = {A.c[0] - B.c[0], A.c[1] - B.c[1], A.c[2] - B.c[2]};
+  const double ab2 = ab[0] * ab[0] + ab[1] * ab[1] + ab[2] * ab[2];
+  auto exp_b = [&](int j) { return pr.b >= 0 ? exps[B.eoff + j] : 0.0; };
+  int count = 0;
+  for (int base = 0; base < pr.prims; base += 64) {
+    if (tid < 64) {
+      const int ij = base + tid;
+      bool keep = false;
+      double a = 0.0, b = 0.0;
+      if (ij < pr.prims) {
+        a = exps[A.eoff + ij / B.nprim];
+        b = exp_b(ij % B.nprim);
+        keep = !(exp(-a * b / (a + b) * ab2) < kPairCut);
+      }
+      const unsigned long long mask = __ballot(keep);
+      const int at = __popcll(mask & ((1ull << tid) - 1));
+      if (keep) {
+        const double p = a + b;
+        list[at] = ij;
+        prims[pr.poff + count + at] = LanePrim{p, (a * A.c[0] + b * B.c[0]) / p, (a * A.c[1] + b * B.c[1]) / p,
+                                               (a * A.c[2] + b * B.c[2]) / p};
+      }
+      if (tid == 0) kept_all = __popcll(mask);
+    }
+    __syncthreads();
+    const int kept = kept_all;
+    for (int s0 = 0; s0 < kept; s0 += kLaneSlots) {
+      const int ns = min(kLaneSlots, kept - s0);
+      if (tid < 3 * ns) {
+        const int slot = tid / 3, d = tid % 3;
+        const int q = list[s0 + slot];
+        hermite_d(A.l, B.l, exps[A.eoff + q / B.nprim], exp_b(q % B.nprim), ab[d], e[slot][d]);
+      }
+      __syncthreads();
+      for (int idx = tid; idx < ns * nh * pr.pad; idx += kPairThreads) {
+        const int slot = idx / (nh * pr.pad), h = idx / pr.pad % nh, row = idx % pr.pad;
+        double sum = 0.0;
+        if (row < pr.rows) {
+          const int q = list[s0 + slot], i = q / B.nprim, j = q % B.nprim;
+          int s = 0;
+          while ((s + 1) * (s + 2) * (s + 3) / 6 <= h) ++s;
+          const int rem = h - s * (s + 1) * (s + 2) / 6;
+          int m = 0;
+          while ((m + 1) * (m + 2) / 2 <= rem) ++m;
+          const int v = rem - m * (m + 1) / 2, u = m - v, t = s - m;
+          const int fa = row / pr.nb, fb = row % pr.nb;
+          const int ca = fa / (2 * A.l + 1), ma = fa % (2 * A.l + 1), cb = fb / (2 * B.l + 1), mb = fb % (2 * B.l + 1);
+          for (int ia = 0; ia < na; ++ia) {
+            const double wa = ta[ma * na + ia];
+            if (wa == 0.0) continue;
+            int ax, ay, az;
+            cart_of(A.l, ia, ax, ay, az);
+            for (int ib = 0; ib < nb; ++ib) {
+              const double wb = tb[mb * nb + ib];
+              if (wb == 0.0) continue;
+              int bx, by, bz;
+              cart_of(B.l, ib, bx, by, bz);
+              sum += wa * wb * e[slot][0][(ax * (B.l + 1) + bx) * nt + t] * e[slot][1][(ay * (B.l + 1) + by) * nt + u] *
+                     e[slot][2][(az * (B.l + 1) + bz) * nt + v];
+            }
+          }
+          const double p = exps[A.eoff + i] + exp_b(j);
+          sum *= coefs[A.coff + ca * A.nprim + i] * norm[pr.fa + fa] * (2.0 * pow(kPi, 2.5) / p);
+          if (pr.b >= 0) sum *= coefs[B.coff + cb * B.nprim + j] * norm[pr.fb + fb];
+        }
+        w[pr.woff + ((long long)(count + s0 + slot) * nh + h) * pr.pad + row] = sum;
+      }
+      __syncthreads();
+    }
+    count += kept;
+  }
+  if (tid == 0) counts[blockIdx.x] = count;
+}
+
+// Order m of the Hermite Coulomb recursion, then the lower ones, in place: an
+// order's entries from the highest sum t + u + v down, each from entries of
+// lower sums of the order above; f[m] is F_m times (-2 alpha)^m and the
+// prefactors.
+template <int L, int M, typename R>
+__device__ __forceinline__ void hermite_order(R& r, const double (&f)[L + 1], double x, double y, double z) {
+  constexpr HermList<L> herm{};
+#pragma unroll
+  for (int i = n_herm(L - M) - 1; i > 0; --i) {
+    const int t = herm.t[i], u = herm.u[i], v = herm.v[i];
+    double val;
+    if (t > 0) {
+      val = x * r[r_index(t - 1, u, v)];
+      if (t > 1) val += (t - 1) * r[r_index(t > 1 ? t - 2 : 0, u, v)];
+    } else if (u > 0) {
+      val = y * r[r_index(t, u - 1, v)];
+      if (u > 1) val += (u - 1) * r[r_index(t, u > 1 ? u - 2 : 0, v)];
+    } else {
+      val = z * r[r_index(t, u, v > 0 ? v - 1 : 0)];
+      if (v > 1) val += (v - 1) * r[r_index(t, u, v > 1 ? v - 2 : 0)];
+    }
+    r[i] = val;
+  }
+  r[0] = f[M];
+  if constexpr (M > 0) hermite_order<L, M - 1>(r, f, x, y, z);
+}
+
+// The Hermite Coulomb integrals of a lane: in registers up to order
+// kLaneRegL, else in the wave's LDS, one column per lane.
+constexpr int kLaneRegL = 6;
+template <int L, bool REG = (L <= kLaneRegL)>
+struct HermStore {
+  double v[n_herm(L)];
+  __device__ __forceinline__ explicit HermStore(double*) {}
+  __device__ __forceinline__ double& operator[](int i) { return v[i]; }
+};
+template <int L>
+struct HermStore<L, false> {
+  double* v;
+  __device__ __forceinline__ explicit HermStore(double* lds) : v(lds + (threadIdx.x & 63)) {}
+  __device__ __forceinline__ double& operator[](int i) { return v[i * 64]; }
+};
+
+// One workgroup: shell pair blockIdx.x / (nblk nchunk), 64 aux primitives, rows
+// [kLaneRows chunk, + kLaneRows) of the pair's functions. Its waves share the
+// pair's primitives (the chain of primitives is what a wave's time is: the
+// latency of each one's table and scalar loads) and add up in LDS; then a
+// contracted aux function's primitives add up across its lanes.
+template <int LAB, int LC>
+__global__ __launch_bounds__(64 * kLaneWaves) void aux_kernel(
+    const LanePair* __restrict__ pairs, const int* __restrict__ counts, const LanePrim* __restrict__ prims,
+    const double* __restrict__ w, const LaneAux* __restrict__ fns, const double* __restrict__ sph,
+    const double* __restrict__ boys_tab, int nblk, int nchunk, int n, int metric_mode, double* __restrict__ out) {
+  constexpr int L = LAB + LC, NH = n_herm(LAB), NC = n_cart(LC);
+  constexpr HermList<L> herm{};
+  constexpr CartList<LC> cart{};
+  extern __shared__ double lds[];  // waves - 1 sets of sums, or the Hermite integrals of one wave
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = blockDim.x >> 6;
+  const int chunk = blockIdx.x % nchunk;
+  const int blk = blockIdx.x / nchunk % nblk;
+  const int ip = blockIdx.x / nchunk / nblk;
+  const LanePair pr = pairs[ip];
+  const int row0 = chunk * kLaneRows;
+  if (row0 >= pr.pad) return;
+  const int rows = min(kLaneRows, pr.pad - row0);
+  const int count = counts[ip];
+  const LaneAux fn = fns[blk * 64 + lane];
+  // The metric's lower triangle: aux functions past the pair's last one have nothing to do.
+  if (__ballot(fn.f >= 0 && !(metric_mode && fn.f > pr.fa + pr.rows - 1)) == 0) return;
+
+  double tc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) tc[c] = sph[fn.m * NC + c];
+  double acc[kLaneRows];
+#pragma unroll
+  for (int i = 0; i < kLaneRows; ++i) acc[i] = 0.0;
+  const double g = fn.g;
+  double scale = fn.coef / g;
+#pragma unroll
+  for (int c = 0; c < LC; ++c) scale *= -0.5 / g;
+
+  for (int q = wave; q < count; q += waves) {
+    const LanePrim pp = prims[pr.poff + q];
+    const double psum = pp.p + g, alpha = pp.p * g / psum;
+    const double x = pp.x - fn.c[0], y = pp.y - fn.c[1], z = pp.z - fn.c[2];
+    double f[L + 1];
+    boys_d(L, alpha * (x * x + y * y + z * z), boys_tab, f);
+    double fac = scale / sqrt(psum);
+#pragma unroll
+    for (int m = 0; m <= L; ++m) {
+      f[m] *= fac;
+      fac *= -2.0 * alpha;
+    }
+    HermStore<L> r(lds);
+    r[0] = f[L];
+    if constexpr (L > 0) hermite_order<L, L - 1>(r, f, x, y, z);
+    const double* wq = w + pr.woff + (long long)q * NH * pr.pad + row0;
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      double hv = 0.0;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        hv += tc[c] * r[r_index(herm.t[h] + cart.x[c], herm.u[h] + cart.y[c], herm.v[h] + cart.z[c])];
+#pragma unroll
+      for (int s = 0; s < kLaneRows; s += kLaneStep)
+        if (s < rows) {
+#pragma unroll
+          for (int i = 0; i < kLaneStep; ++i) acc[s + i] += wq[h * pr.pad + s + i] * hv;
+        }
+    }
+  }
+  if (waves > 1) {
+    if (wave > 0) {
+#pragma unroll
+      for (int i = 0; i < kLaneRows; ++i) lds[((wave - 1) * kLaneRows + i) * 64 + lane] = acc[i];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    for (int v = 0; v < waves - 1; ++v) {
+#pragma unroll
+      for (int i = 0; i < kLaneRows; ++i) acc[i] += lds[(v * kLaneRows + i) * 64 + lane];
+    }
+  }
+  for (int k = 1; __ballot(k < fn.nprim) != 0; ++k) {
+#pragma unroll
+    for (int i = 0; i < kLaneRows; ++i) {
+      const double other = __shfl_down(acc[i], k);
+      // Adds primitive k of each function; the lanes' own sums change only on first primitives,
+      // which no other function reads.
+      if (k < fn.nprim) acc[i] += other;
+    }
+  }
+  if (fn.nprim == 0) return;
+#pragma unroll
+  for (int i = 0; i < kLaneRows; ++i) {
+    const int row = row0 + i;
+    if (row >= pr.rows) continue;
+    const int ia = pr.fa + row / pr.nb, ib = pr.fb + row % pr.nb;
+    if (metric_mode) {
+      if (fn.f > ia) continue;
+      out[(long long)ia * n + fn.f] = acc[i];
+      out[(long long)fn.f * n + ia] = acc[i];
+    } else {
+      if (ib > ia) continue;  // within one shell: the mirror of (ib, ia)
+      double* plane = out + (long long)fn.f * n * n;
+      plane[(long long)ia * n + ib] = acc[i];
+      plane[(long long)ib * n + ia] = acc[i];
+    }
+  }
+}
+
+// One device allocation of a call: host tables packed end to end and copied
+// at once, then device-only regions; freed with the object.
+struct DeviceArena {
+  std::vector<char> host;
+  size_t bytes = 0;
+  char* base = nullptr;
+  ~DeviceArena() {
+    if (base != nullptr) (void)hipFree(base);
   }
   template <typename T>
-  T* upload(const std::vector<T>& host, hipStream_t s) {
+  size_t put(const std::vector<T>& v) {
+    const size_t at = host.size();
+    host.resize(at + (std::max<size_t>(v.size(), 1) * sizeof(T) + 255) / 256 * 256);
+    if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
+    bytes = host.size();
+    return at;
+  }
+  template <typename T>
+  size_t reserve(size_t count) {  // after the last put
+    const size_t at = bytes;
+    bytes += (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+    return at;
+  }
+  void upload(hipStream_t s) {
     void* p = nullptr;
-    const size_t bytes = std::max<size_t>(host.size(), 1) * sizeof(T);
     if (hipMalloc(&p, bytes) != hipSuccess) throw std::runtime_error("hipMalloc of the integral tables failed");
-    buffers.push_back(p);
-    if (!host.empty() && hipMemcpyAsync(p, host.data(), host.size() * sizeof(T), hipMemcpyHostToDevice, s) != hipSuccess)
+    base = (char*)p;
+    if (hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s) != hipSuccess)
       throw std::runtime_error("hipMemcpyAsync of the integral tables failed");
-    return (T*)p;
+  }
+  template <typename T>
+  T* at(size_t offset) const {
+    return (T*)(base + offset);
   }
 };
 
@@ -1127,23 +1505,71 @@ void device_shells(const std::vector<Shell>& shells, std::vector<DShell>& out, s
   }
 }
 
-// Whether any primitive pair of two shells passes the product cut (the host engine's per-pair test).
+// Whether any primitive pair of two shells passes the product cut (the host
+// engine's per-pair test): the pair of the smallest exponents decays slowest.
 bool pair_survives(const Shell& A, const Shell& B) {
   const double d2 = (A.c[0] - B.c[0]) * (A.c[0] - B.c[0]) + (A.c[1] - B.c[1]) * (A.c[1] - B.c[1]) +
                     (A.c[2] - B.c[2]) * (A.c[2] - B.c[2]);
-  for (double a : A.exps)
-    for (double b : B.exps)
-      if (std::exp(-a * b / (a + b) * d2) >= kPairCut) return true;
-  return false;
+  const double a = *std::min_element(A.exps.begin(), A.exps.end());
+  const double b = *std::min_element(B.exps.begin(), B.exps.end());
+  return std::exp(-a * b / (a + b) * d2) >= kPairCut;
 }
 
-size_t cart_entries(const Shell& A, int bl, int bcontr, const Shell& C) {
-  return (size_t)A.ncontr * ncart(A.l) * bcontr * ncart(bl) * C.ncontr * ncart(C.l);
+// Launch table of aux_kernel over its angular momenta.
+struct LaneArgs {
+  const LanePair* pairs;
+  const int* counts;
+  const LanePrim* prims;
+  const double* w;
+  const LaneAux* fns;
+  const double *sph, *boys_tab;
+  int npairs, nsplit, nblk, nchunk, n, metric_mode;  // the first nsplit pairs have many primitives
+  double* out;
+};
+
+template <int LAB, int LC>
+void launch_aux(const LaneArgs& a, hipStream_t s) {
+  const unsigned per = (unsigned)(a.nblk * a.nchunk);
+  const int most = (int)((1u << 28) / per);  // pairs per launch
+  for (int first = 0; first < a.npairs;) {
+    const bool split = first < a.nsplit && LAB + LC <= kLaneRegL;
+    const size_t lds = LAB + LC > kLaneRegL ? n_herm(LAB + LC) * 512
+                       : split              ? (kLaneWaves - 1) * kLaneRows * 512
+                                            : 0;
+    const int np = std::min(most, (split ? a.nsplit : a.npairs) - first);  // one kind of workgroup per launch
+    hipLaunchKernelGGL((aux_kernel<LAB, LC>), dim3(np * per), dim3(split ? 64 * kLaneWaves : 64), lds, s,
+                       a.pairs + first, a.counts + first, a.prims, a.w, a.fns, a.sph, a.boys_tab, a.nblk, a.nchunk, a.n,
+                       a.metric_mode, a.out);
+    if (hipGetLastError() != hipSuccess) throw std::runtime_error("launch of the integral kernel failed");
+    first += np;
+  }
 }
 
-void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux, const std::vector<DItem>& items,
-                    const std::vector<double>& norm_o, const std::vector<double>& norm_x, int n, bool metric_mode,
-                    double* out, hipStream_t s) {
+template <int LAB, int LC = 0>
+void launch_aux_c(int lc, const LaneArgs& a, hipStream_t s) {
+  if constexpr (LC <= kLaneMaxC && LAB + LC <= kLaneMaxL) {
+    if (lc == LC) return launch_aux<LAB, LC>(a, s);
+    launch_aux_c<LAB, LC + 1>(lc, a, s);
+  }
+}
+
+void launch_aux_any(int lab, int lc, const LaneArgs& a, hipStream_t s) {
+  switch (lab) {
+    case 0: return launch_aux_c<0>(lc, a, s);
+    case 1: return launch_aux_c<1>(lc, a, s);
+    case 2: return launch_aux_c<2>(lc, a, s);
+    case 3: return launch_aux_c<3>(lc, a, s);
+    default: return launch_aux_c<4>(lc, a, s);
+  }
+}
+
+// The integrals of the shell pairs (pair_list: b < 0 for the unit function)
+// with every aux shell (up to the pair's own shell for the metric).
+void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux,
+                    const std::vector<std::pair<int, int>>& pair_list, const std::vector<double>& norm_o,
+                    const std::vector<double>& norm_x, int n, bool metric_mode, double* out, hipStream_t s) {
+  static const std::vector<double> boys_host = boys_table();
+  const std::vector<Shell>& a_shells = metric_mode ? aux : orb;
   std::vector<DShell> dorb, daux;
   std::vector<double> exps, coefs;
   device_shells(orb, dorb, exps, coefs);
@@ -1155,26 +1581,123 @@ void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux
     const auto& t = sph_table(l);
     sph.insert(sph.end(), t.begin(), t.end());
   }
-  DeviceTables dev;
-  const DItem* d_items = dev.upload(items, s);
-  const DShell* d_orb = dev.upload(dorb, s);
-  const DShell* d_aux = dev.upload(daux, s);
-  const double* d_exps = dev.upload(exps, s);
-  const double* d_coefs = dev.upload(coefs, s);
-  const double* d_no = dev.upload(norm_o, s);
-  const double* d_nx = dev.upload(norm_x, s);
-  const double* d_sph = dev.upload(sph, s);
-  const int* d_off = dev.upload(sph_off, s);
-  const std::vector<double> boys_host = boys_table();  // alive until the synchronisation below
-  const double* d_boys = dev.upload(boys_host, s);
+  // Pairs by la + lb (the most primitive pairs first, so that the longest waves start first); the
+  // higher ones go to triple_kernel with every aux shell.
+  std::vector<LanePair> by_l[kLaneMaxAB + 1];
+  std::vector<DItem> items;
+  std::vector<int> aux_by_l[kGL + 1];
+  for (int c = 0; c < (int)aux.size(); ++c) aux_by_l[aux[c].l].push_back(c);
+  auto lane_aux = [&](int c, int lab) {
+    return lab <= kLaneMaxAB && aux[c].l <= kLaneMaxC && lab + aux[c].l <= kLaneMaxL &&
+           (int)aux[c].exps.size() <= kLaneMaxPrim;
+  };
+  bool all_short = true;
+  for (const Shell& x : aux) all_short = all_short && (int)x.exps.size() <= kLaneMaxPrim;
+  for (const auto& [i, j] : pair_list) {
+    const Shell& A = a_shells[i];
+    const int lb = j >= 0 ? orb[j].l : 0, fb = j >= 0 ? orb[j].nfunc() : 1;
+    const bool lanes = A.l + lb <= kLaneMaxAB;
+    for (int l = lanes && all_short ? std::min(kLaneMaxC, kLaneMaxL - A.l - lb) + 1 : 0; l <= kGL; ++l)
+      for (int c : aux_by_l[l])
+        if ((!metric_mode || c <= i) && !lane_aux(c, A.l + lb)) items.push_back(DItem{i, j, c});
+    if (!lanes) continue;
+    LanePair p{};
+    p.a = i;
+    p.b = j;
+    p.rows = A.nfunc() * fb;
+    p.pad = (p.rows + kLaneStep - 1) / kLaneStep * kLaneStep;
+    p.prims = (int)(A.exps.size() * (j >= 0 ? orb[j].exps.size() : 1));
+    p.fa = A.offset;
+    p.fb = j >= 0 ? orb[j].offset : 0;
+    p.nb = fb;
+    by_l[A.l + lb].push_back(p);
+  }
+  std::vector<LanePair> pairs;
+  int first[kLaneMaxAB + 2] = {}, chunks[kLaneMaxAB + 1] = {}, split[kLaneMaxAB + 1] = {};
+  long long wtotal = 0, ptotal = 0;
+  for (int l = 0; l <= kLaneMaxAB; ++l) {
+    std::stable_sort(by_l[l].begin(), by_l[l].end(),
+                     [](const LanePair& x, const LanePair& y) { return x.prims > y.prims; });
+    for (LanePair& p : by_l[l]) {
+      p.poff = (int)ptotal;
+      p.woff = wtotal;
+      ptotal += p.prims;
+      wtotal += (long long)p.prims * n_herm(l) * p.pad;
+      split[l] += p.prims >= 2 * kLaneWaves;
+      chunks[l] = std::max(chunks[l], (p.pad + kLaneRows - 1) / kLaneRows);
+      pairs.push_back(p);
+    }
+    first[l + 1] = (int)pairs.size();
+  }
+  if (ptotal > (1LL << 31) - 1) throw std::invalid_argument("too many primitive pairs for the GPU integrals");
+  // Aux primitives by l, a lane each, in blocks of 64: a function's are neighbours in one block
+  // (idle lanes, whose exponent of 1 keeps their arithmetic finite, fill up).
+  std::vector<LaneAux> fns;
+  int fblock[kLaneMaxC + 2] = {};
+  LaneAux idle{};
+  idle.g = 1.0;
+  idle.f = -1;
+  for (int l = 0; l <= kLaneMaxC; ++l) {
+    std::vector<int> order;
+    for (int c : aux_by_l[l])
+      if ((int)aux[c].exps.size() <= kLaneMaxPrim) order.push_back(c);
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return aux[x].exps.size() > aux[y].exps.size(); });
+    for (int c : order)
+      for (int f = 0; f < aux[c].nfunc(); ++f) {
+        const int np = (int)aux[c].exps.size();
+        if (fns.size() % 64 + np > 64)
+          while (fns.size() % 64) fns.push_back(idle);
+        for (int k = 0; k < np; ++k) {
+          LaneAux x{};
+          for (int d = 0; d < 3; ++d) x.c[d] = aux[c].c[d];
+          x.g = aux[c].exps[k];
+          x.nprim = k == 0 ? np : 0;
+          x.m = f % (2 * l + 1);
+          x.f = aux[c].offset + f;
+          x.coef = aux[c].coefs[(size_t)(f / (2 * l + 1)) * np + k] * norm_x[x.f];
+          fns.push_back(x);
+        }
+      }
+    while (fns.size() % 64) fns.push_back(idle);
+    fblock[l + 1] = (int)(fns.size() / 64);
+  }
+
+  DeviceArena dev;  // its host tables live until the synchronisation below
+  const size_t o_items = dev.put(items), o_orb = dev.put(dorb), o_aux = dev.put(daux), o_exps = dev.put(exps),
+               o_coefs = dev.put(coefs), o_no = dev.put(norm_o), o_nx = dev.put(norm_x), o_sph = dev.put(sph),
+               o_off = dev.put(sph_off), o_boys = dev.put(boys_host), o_pairs = dev.put(pairs), o_fns = dev.put(fns);
+  const size_t o_counts = dev.reserve<int>(pairs.size()), o_prims = dev.reserve<LanePrim>((size_t)ptotal),
+               o_w = dev.reserve<double>((size_t)wtotal);
+  dev.upload(s);
   const size_t total = metric_mode ? (size_t)n * n : (size_t)norm_x.size() * n * n;
-  if (hipMemsetAsync(out, 0, total * sizeof(double), s) != hipSuccess) throw std::runtime_error("hipMemsetAsync failed");
+  // Pairs that do not survive stay zero; the metric has none.
+  if (!metric_mode && hipMemsetAsync(out, 0, total * sizeof(double), s) != hipSuccess)
+    throw std::runtime_error("hipMemsetAsync failed");
+  if (!pairs.empty()) {
+    hipLaunchKernelGGL(pair_kernel, dim3((unsigned)pairs.size()), dim3(kPairThreads), 0, s, dev.at<LanePair>(o_pairs),
+                       dev.at<DShell>(metric_mode ? o_aux : o_orb), dev.at<DShell>(o_orb), dev.at<double>(o_exps),
+                       dev.at<double>(o_coefs), dev.at<double>(metric_mode ? o_nx : o_no), dev.at<double>(o_sph),
+                       dev.at<int>(o_off), dev.at<int>(o_counts), dev.at<LanePrim>(o_prims), dev.at<double>(o_w));
+    if (hipGetLastError() != hipSuccess) throw std::runtime_error("launch of the integral pair kernel failed");
+  }
+  for (int l = kLaneMaxAB; l >= 0; --l)
+    for (int c = kLaneMaxC; c >= 0; --c) {
+      const int np = first[l + 1] - first[l], nblk = fblock[c + 1] - fblock[c];
+      if (np == 0 || nblk == 0 || l + c > kLaneMaxL) continue;
+      LaneArgs a{dev.at<LanePair>(o_pairs) + first[l], dev.at<int>(o_counts) + first[l], dev.at<LanePrim>(o_prims),
+                 dev.at<double>(o_w), dev.at<LaneAux>(o_fns) + (size_t)fblock[c] * 64,
+                 dev.at<double>(o_sph) + sph_off[c], dev.at<double>(o_boys), np, split[l], nblk, chunks[l], n,
+                 metric_mode ? 1 : 0, out};
+      launch_aux_any(l, c, a, s);
+    }
   // At most 2^31 - 1 workgroups per launch.
   const size_t per = (size_t)1 << 30;
   for (size_t base = 0; base < items.size(); base += per) {
     const unsigned count = (unsigned)std::min(per, items.size() - base);
-    hipLaunchKernelGGL(triple_kernel, dim3(count), dim3(64), 0, s, d_items + base, d_orb, d_aux, d_exps, d_coefs,
-                       d_no, d_nx, d_sph, d_off, d_boys, n, metric_mode ? 1 : 0, out);
+    hipLaunchKernelGGL(triple_kernel, dim3(count), dim3(64), 0, s, dev.at<DItem>(o_items) + base,
+                       dev.at<DShell>(o_orb), dev.at<DShell>(o_aux), dev.at<double>(o_exps), dev.at<double>(o_coefs),
+                       dev.at<double>(o_no), dev.at<double>(o_nx), dev.at<double>(o_sph), dev.at<int>(o_off),
+                       dev.at<double>(o_boys), n, metric_mode ? 1 : 0, out);
     if (hipGetLastError() != hipSuccess) throw std::runtime_error("launch of the integral kernel failed");
   }
   // The tables are freed on return: wait for the kernels that read them.
@@ -1192,12 +1715,13 @@ void check_item_sizes(const std::vector<Shell>& a_list, const std::vector<Shell>
   if (la + lb + lc > kGMaxL) throw std::invalid_argument("total angular momentum beyond 12 on the GPU");
   if ((la + 1) * (lb + 1) * (la + lb + 1) > kGEA)
     throw std::invalid_argument("a shell pair's Hermite table exceeds the GPU kernel's LDS table");
-  for (const Shell& A : a_list)
-    for (const Shell& C : c_list) {
-      if (unit_b) worst = std::max(worst, cart_entries(A, 0, 1, C));
-      else
-        for (const Shell& B : *b_list) worst = std::max(worst, cart_entries(A, B.l, B.ncontr, C));
-    }
+  // The largest Cartesian block is the product of the largest of each index.
+  auto largest = [](const std::vector<Shell>& list) {
+    size_t most = 0;
+    for (const Shell& x : list) most = std::max(most, (size_t)x.ncontr * ncart(x.l));
+    return most;
+  };
+  worst = largest(a_list) * largest(c_list) * (unit_b ? 1 : largest(*b_list));
   if (worst > (size_t)kGCart)
     throw std::invalid_argument("a shell triple's Cartesian block exceeds the GPU kernel's LDS block");
 }
@@ -1214,11 +1738,10 @@ int hfjk_int2c2e_device(hfjk_ctx* ctx, const hfjk_basis* aux, double* metric, vo
     const std::vector<Shell> sh = make_shells(aux, n);
     const std::vector<double> nm = norms(sh, n);
     check_item_sizes(sh, sh, true, nullptr);
-    std::vector<DItem> items;
-    for (int i = 0; i < (int)sh.size(); ++i)
-      for (int j = 0; j <= i; ++j) items.push_back(DItem{i, -1, j});
+    std::vector<std::pair<int, int>> pairs;
+    for (int i = 0; i < (int)sh.size(); ++i) pairs.emplace_back(i, -1);
     if (hipSetDevice(ctx->device) != hipSuccess) throw std::runtime_error("hipSetDevice failed");
-    launch_triples(sh, sh, items, nm, nm, n, true, metric, (hipStream_t)stream);
+    launch_triples(sh, sh, pairs, nm, nm, n, true, metric, (hipStream_t)stream);
   });
 }
 
@@ -1232,14 +1755,12 @@ int hfjk_int3c2e_device(hfjk_ctx* ctx, const hfjk_basis* aux, const hfjk_basis* 
     const std::vector<double> nmx = norms(sx, nx);
     const std::vector<double> nmo = norms(so, n);
     check_item_sizes(so, sx, false, &so);
-    std::vector<DItem> items;
+    std::vector<std::pair<int, int>> pairs;
     for (int i = 0; i < (int)so.size(); ++i)
-      for (int j = 0; j <= i; ++j) {
-        if (!pair_survives(so[i], so[j])) continue;
-        for (int c = 0; c < (int)sx.size(); ++c) items.push_back(DItem{i, j, c});
-      }
+      for (int j = 0; j <= i; ++j)
+        if (pair_survives(so[i], so[j])) pairs.emplace_back(i, j);
     if (hipSetDevice(ctx->device) != hipSuccess) throw std::runtime_error("hipSetDevice failed");
-    launch_triples(so, sx, items, nmo, nmx, n, false, out, (hipStream_t)stream);
+    launch_triples(so, sx, pairs, nmo, nmx, n, false, out, (hipStream_t)stream);
   });
 }
 

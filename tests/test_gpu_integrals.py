@@ -59,3 +59,56 @@ def test_twelve_waters_on_the_gpu():
     print(f"12 waters: device integrals {seconds:.4f} s, host {host_seconds:.4f} s", flush=True)
     np.testing.assert_allclose(m.cpu().numpy(), m_host, atol=1e-12 * np.abs(m_host).max())
     np.testing.assert_allclose(tc.cpu().numpy(), tc_host, atol=1e-12 * np.abs(tc_host).max())
+
+
+class _Shells:
+    """A synthetic basis in the C-ABI layout: ``(l, center, exponents, coefficient rows)`` per shell."""
+
+    def __init__(self, shells):
+        self._l = np.asarray([s[0] for s in shells], dtype=np.int32)
+        self._centers = np.asarray([c for s in shells for c in s[1]], dtype=np.float64)
+        self._nprim = np.asarray([len(s[2]) for s in shells], dtype=np.int32)
+        self._ncontr = np.asarray([len(s[3]) for s in shells], dtype=np.int32)
+        self._exps = np.asarray([e for s in shells for e in s[2]], dtype=np.float64)
+        self._coefs = np.asarray([c for s in shells for row in s[3] for c in row], dtype=np.float64)
+        self.n_functions = int(sum((2 * s[0] + 1) * len(s[3]) for s in shells))
+
+    c_struct = molecule.BasisOnAtoms.c_struct
+
+
+def _random_shells(rng, momenta, scale):
+    out = []
+    for l, nprim, ncontr in momenta:
+        rows = rng.standard_normal((ncontr, nprim))
+        if ncontr > 1:
+            rows[0, -1] = 0.0
+        out.append((l, rng.uniform(-1.5, 1.5, 3) * scale, rng.uniform(0.2, 6.0, nprim), rows))
+    return out
+
+
+@pytest.mark.parametrize("orbital,auxiliary", [
+    # Every class of the lane-per-aux kernel, both sides of its limits, contractions on both sides.
+    ([(0, 9, 3), (1, 4, 2), (2, 1, 1), (2, 3, 1)], [(0, 5, 1), (0, 1, 1), (1, 3, 2), (2, 2, 1), (3, 1, 1), (4, 1, 1), (4, 2, 1)]),
+    ([(0, 1, 1), (1, 2, 1), (2, 2, 1)], [(5, 1, 1), (0, 17, 1), (1, 20, 1), (0, 16, 1), (5, 2, 1)]),
+    ([(0, 2, 1), (2, 1, 1), (3, 1, 1), (3, 2, 1)], [(0, 1, 1), (1, 2, 1), (3, 1, 1)]),
+    ([(0, 1, 1)], [(0, 1, 1)]),
+])
+@pytest.mark.parametrize("scale", [1.0, 12.0])
+def test_device_integrals_over_all_classes(orbital, auxiliary, scale):
+    """Both device kernels against the host engine; far centres drop primitive pairs and whole pairs."""
+    rng = np.random.default_rng(7)
+    orb, aux = _Shells(_random_shells(rng, orbital, scale)), _Shells(_random_shells(rng, auxiliary, scale))
+    three = integrals.three_center(aux, orb)
+    got = integrals.three_center_device(aux, orb).cpu().numpy()
+    metric = integrals.metric(aux)
+    # Each result is a sum of terms of either sign (the harmonics' Cartesian terms, the contractions) whose
+    # size the Schwarz bound sqrt((P|P) (uv|uv)) gives, not the result, which far centres cancel to less;
+    # (uv|uv) is below 4 for normalised functions of these exponents.
+    bound = 1e-12 * np.sqrt(4.0 * np.diag(metric))[:, None, None]
+    worst = float(np.max(np.abs(got - three) / bound))
+    assert worst <= 1.0, worst
+    np.testing.assert_array_equal(got, got.transpose(0, 2, 1))
+    dev = integrals.metric_device(aux).cpu().numpy()
+    worst = float(np.max(np.abs(dev - metric) / np.sqrt(np.outer(np.diag(metric), np.diag(metric)))))
+    assert worst <= 1e-12, worst
+    np.testing.assert_array_equal(dev, dev.T)
