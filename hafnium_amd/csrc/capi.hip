@@ -1213,11 +1213,22 @@ struct KpLayout {
   size_t inner, charges;
   // Exchange: the density copy and its eigenpairs, the realified factor and
   // its column signs, the realified block, X, the SYRK partials, the [2n][2n]
-  // real result, a complex [n][n] product for the Madelung term.
-  size_t dz, w, e, info, stats, ct, sg, bh, x, part, kh, tz;
+  // real result.
+  size_t dz, w, e, info, ct, sg, bh, x, part, kh;
+  // Exchange of positive semidefinite densities, over the same bytes: L of
+  // every k (and its diagonals), the states, the operand fragments and column
+  // signs, a complex [nk][n][n] product, the partials of Re K and Im K, X.
+  size_t pl, pst, pfrag, psym, pcross, ptmp, p1, p2, px, px_bytes;
   size_t total;
   int npad2, ldo, xrows, npairs, nsplit;
+  int pairs_n, max_slots;
 };
+
+// X of the batched k-point exchange is kept to this many bytes (blocks of
+// (k1, k2) pairs per pass), or one block.
+constexpr size_t kKpointXBytes = size_t(1) << 30;
+
+int kp_half(int rank) { return (rank + 15) / 16 * 16; }  // columns of Re X, and of Im X
 
 KpLayout kp_layout(const hfjk_ctx* ctx, int nk, int naux, int nao) {
   KpLayout L{};
@@ -1235,16 +1246,106 @@ KpLayout kp_layout(const hfjk_ctx* ctx, int nk, int naux, int nao) {
   L.w = off; off = align_up(off + n * 8);
   L.e = off; off = align_up(off + n * 8);
   L.info = off; off = align_up(off + 8);
-  L.stats = off; off = align_up(off + 16);
   L.ct = off; off = align_up(off + (size_t)L.ldo * L.npad2 * 8);
   L.sg = off; off = align_up(off + (size_t)L.ldo * 8);
   L.bh = off; off = align_up(off + (size_t)naux * L.npad2 * L.npad2 * 8);
   L.x = off; off = align_up(off + (size_t)naux * L.xrows * L.ldo * 8);
   L.part = off; off = align_up(off + (size_t)L.nsplit * L.npairs * tile2 * 8);
   L.kh = off; off = align_up(off + 4 * n * n * 8);
-  L.tz = off; off = align_up(off + n * n * 16);
   L.total = off;
+  off = L.dz;
+  const size_t ldmax = 2 * (size_t)kp_half(nao);
+  L.pairs_n = hfjk::syrk_pairs(nao);
+  L.max_slots = std::max(64, (512 / L.pairs_n + 15) / 8 * 8);
+  L.pl = off; off = align_up(off + (size_t)nk * (n * n * 16 + n * 8));
+  L.pst = off; off = align_up(off + (size_t)nk * sizeof(hfjk::KpState));
+  L.pfrag = off; off = align_up(off + (size_t)nk * L.npad2 * ldmax * 8);
+  L.psym = off; off = align_up(off + ldmax * 8);
+  L.pcross = off; off = align_up(off + ldmax * 8);
+  L.ptmp = off; off = align_up(off + (size_t)nk * n * n * 16);
+  L.p1 = off; off = align_up(off + (size_t)L.max_slots * L.pairs_n * tile2 * 8);
+  L.p2 = off; off = align_up(off + (size_t)L.max_slots * L.pairs_n * tile2 * 8);
+  const size_t block = (size_t)naux * n * ldmax * 8;
+  const size_t blocks = std::max<size_t>(1, std::min<size_t>((size_t)nk * nk, kKpointXBytes / block));
+  L.px = off;
+  L.px_bytes = blocks * block;
+  off = align_up(off + L.px_bytes);
+  L.total = std::max(L.total, off);
   return L;
+}
+
+// The k-point exchange when every density is positive semidefinite (every
+// aufbau or smeared density): D(k) = L L^H by pivoted Cholesky for all k in
+// one launch, the half-transform [Re X, Im X] = B C of whole ranges of
+// (k1, k2) blocks straight from the caller's complex tensor (a complex row is
+// a real row of 2 n), and Re K, Im K as two signed SYRKs on n rows, the second
+// with its columns shifted by half: seven launches per range instead of a
+// zheevd per k and five launches per block. Returns false, with nothing
+// written, where a density does not factorise (the caller's path by
+// eigenpairs then runs); sizes whose offsets the ring's do not hold are left
+// to it too. `states` holds the host copy of every k's statistics.
+bool kpoint_exchange_psd(hfjk_ctx* ctx, int nk, int naux, int n, const double* tensor, const double* signature,
+                         const double* weights, const std::vector<double>& host_weights,
+                         const std::vector<hfjk::KpState>& states, void* out, void* ws, const KpLayout& L,
+                         hipStream_t s) {
+  int rank = 0;
+  for (int k = 0; k < nk; ++k) {
+    double mag, residual;
+    std::memcpy(&mag, &states[k].mag, sizeof(double));
+    std::memcpy(&residual, &states[k].residual, sizeof(double));
+    if (!(residual <= 1e-11 * mag) || states[k].rank < 1 || !(host_weights[k] > 0.0)) return false;
+    rank = std::max(rank, states[k].rank);
+  }
+  const int hb = kp_half(rank), ldo = 2 * hb;
+  if (n < 2 || ldo > 2048 || (long long)n * ldo >= (1LL << 30)) return false;
+  double* frag = at<double>(ws, L.pfrag);
+  double* sym = at<double>(ws, L.psym);
+  double* cross = at<double>(ws, L.pcross);
+  double* x = at<double>(ws, L.px);
+  void* p1 = at<void>(ws, L.p1);
+  void* p2 = at<void>(ws, L.p2);
+  {
+    Stage st(ctx, s, "kpoint_factor");
+    check_hip(hfjk::launch_kp_fragments(at<void>(ws, L.pl), at<hfjk::KpState>(ws, L.pst), weights, nk, n, hb, frag,
+                                        sym, cross, s),
+              "k-point fragments launch");
+  }
+  // Blocks of X per pass: whole k1 rows (at most eight, so that the split counts stay small), or a
+  // range of k2 of one k1.
+  const long long fit = std::max<long long>(1, (long long)(L.px_bytes / ((size_t)naux * n * ldo * 8)));
+  const int kc_max = (int)std::min<long long>(std::min(nk, 8), fit / nk);
+  for (int k1 = 0; k1 < nk;) {
+    const int kc = std::max(1, std::min(kc_max, nk - k1));
+    const int range = kc_max >= 1 ? nk : (int)std::min<long long>(nk, fit);
+    // Splits per k1: a multiple of 8 over all (one XCD per split), about one workgroup per CU.
+    int g = 8;
+    while (kc % g != 0) g /= 2;
+    const int unit = 8 / g;
+    const int c = unit * std::max(1, std::min(256 / L.pairs_n, L.max_slots) / (kc * unit));
+    for (int k2 = 0; k2 < nk; k2 += range) {
+      const int blocks = kc * std::min(range, nk - k2);
+      const int b0 = k1 * nk + k2;
+      {
+        Stage st(ctx, s, "kpoint_half_transform");
+        check_hip(hfjk::launch_rows_transform(tensor, (long long)naux * n, 2 * n, b0, blocks, nk, frag, ldo, x, ldo, s),
+                  "k-point half transform launch");
+      }
+      {
+        Stage st(ctx, s, "kpoint_syrk");
+        const double* sig = signature + (long long)b0 * naux;
+        check_hip(hfjk::launch_syrk(x, HFJK_FP64, blocks * naux, n, ldo, sym, true, kc * c, p1, 0, s, sig, 0, false, 0, n),
+                  "k-point syrk launch");
+        check_hip(hfjk::launch_syrk(x, HFJK_FP64, blocks * naux, n, ldo, cross, true, kc * c, p2, 0, s, sig, hb, false, 0,
+                                    n),
+                  "k-point syrk launch");
+        check_hip(hfjk::launch_syrk_reduce_complex((const double*)p1, (const double*)p2, c, n, kc, k2 > 0,
+                                                   (char*)out + 16 * (long long)k1 * n * n, s),
+                  "k-point reduce launch");
+      }
+    }
+    k1 += kc;
+  }
+  return true;
 }
 
 void kp_check(int nk, int naux, int nao) {
@@ -1311,17 +1412,45 @@ int hfjk_kpoint_exchange(hfjk_ctx* ctx, int nk, int naux, int nao, const void* t
     hipStream_t s = (hipStream_t)stream;
     const int n = nao;
     const long long nn = (long long)n * n;
+    auto madelung_term = [&] {
+      if (madelung == 0.0) return;
+      Stage st(ctx, s, "kpoint_madelung");
+      check_hip(hfjk::launch_kp_madelung(overlap, density, nk, n, madelung, at<void>(workspace, L.ptmp), exchange, s),
+                "k-point zgemm launch");
+    };
     std::vector<double> w(nk);
+    std::vector<hfjk::KpState> states(nk);
+    {
+      Stage st(ctx, s, "kpoint_density_cholesky");
+      check_hip(hfjk::launch_kp_cholesky(density, nk, n, at<void>(workspace, L.pl), at<hfjk::KpState>(workspace, L.pst),
+                                         s),
+                "k-point Cholesky launch");
+    }
     check_hip(hipMemcpyAsync(w.data(), weights, sizeof(double) * nk, hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
+    check_hip(hipMemcpyAsync(states.data(), at<void>(workspace, L.pst), sizeof(hfjk::KpState) * nk,
+                             hipMemcpyDeviceToHost, s),
+              "hipMemcpyAsync");
     check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
     for (int k = 0; k < nk; ++k)
       if (!(w[k] >= 0.0)) fail(HFJK_ERR_INPUT, "k-point weights are non-negative");
+    for (int k = 0; k < nk; ++k) {
+      double asym, mag;
+      std::memcpy(&asym, &states[k].asym, sizeof(double));
+      std::memcpy(&mag, &states[k].mag, sizeof(double));
+      if (!(asym <= 1e-12 * (mag > 0 ? mag : 1.0)))
+        fail(HFJK_ERR_INPUT, "the density of k-point " + std::to_string(k) + " is not Hermitian (max |D - D^H| = " +
+                                 std::to_string(asym) + ")");
+    }
+    if (kpoint_exchange_psd(ctx, nk, naux, n, (const double*)tensor, signature, weights, w, states, exchange, workspace,
+                            L, s)) {
+      madelung_term();
+      return;
+    }
     check_hip(hipMemsetAsync(exchange, 0, sizeof(double) * 2 * nk * nn, s), "hipMemsetAsync");
     auto* dz = at<rocblas_double_complex>(workspace, L.dz);
     double* ev = at<double>(workspace, L.w);
     double* e = at<double>(workspace, L.e);
     rocblas_int* info = at<rocblas_int>(workspace, L.info);
-    unsigned long long* stats = at<unsigned long long>(workspace, L.stats);
     double* ct = at<double>(workspace, L.ct);
     double* sg = at<double>(workspace, L.sg);
     double* bh = at<double>(workspace, L.bh);
@@ -1331,11 +1460,8 @@ int hfjk_kpoint_exchange(hfjk_ctx* ctx, int nk, int naux, int nao, const void* t
     std::vector<double> vals(n);
     for (int k2 = 0; k2 < nk; ++k2) {
       const char* d2 = (const char*)density + 16 * k2 * nn;
-      unsigned long long host_stats[2];
       {
         Stage st(ctx, s, "kpoint_density_eigh");
-        check_hip(hipMemsetAsync(stats, 0, 2 * sizeof(unsigned long long), s), "hipMemsetAsync");
-        check_hip(hfjk::launch_kp_hermitian_stats(d2, n, stats, s), "hermitian stats launch");
         check_hip(hipMemcpyAsync(dz, d2, 16 * nn, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
         rocblas_handle h = blas_handle(ctx);
         if (rocblas_set_stream(h, s) != rocblas_status_success) fail(HFJK_ERR_SOLVER, "rocblas_set_stream failed");
@@ -1346,16 +1472,9 @@ int hfjk_kpoint_exchange(hfjk_ctx* ctx, int nk, int naux, int nao, const void* t
           fail(HFJK_ERR_SOLVER, "rocsolver_zheevd failed to launch");
       }
       rocblas_int host_info = 0;
-      check_hip(hipMemcpyAsync(host_stats, stats, sizeof(host_stats), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
       check_hip(hipMemcpyAsync(vals.data(), ev, sizeof(double) * n, hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
       check_hip(hipMemcpyAsync(&host_info, info, sizeof(host_info), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
       check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-      double asym, mag;
-      std::memcpy(&asym, &host_stats[0], sizeof(double));
-      std::memcpy(&mag, &host_stats[1], sizeof(double));
-      if (!(asym <= 1e-12 * (mag > 0 ? mag : 1.0)))
-        fail(HFJK_ERR_INPUT, "the density of k-point " + std::to_string(k2) + " is not Hermitian (max |D - D^H| = " +
-                                 std::to_string(asym) + ")");
       if (host_info != 0)
         fail(HFJK_ERR_SOLVER, "rocsolver_zheevd did not converge (info " + std::to_string(host_info) + ")");
       double top = 0.0;
@@ -1392,17 +1511,7 @@ int hfjk_kpoint_exchange(hfjk_ctx* ctx, int nk, int naux, int nao, const void* t
         }
       }
     }
-    if (madelung != 0.0) {
-      Stage st(ctx, s, "kpoint_madelung");
-      void* tz = at<void>(workspace, L.tz);
-      for (int k = 0; k < nk; ++k) {
-        const char* sk = (const char*)overlap + 16 * k * nn;
-        const char* dk = (const char*)density + 16 * k * nn;
-        check_hip(hfjk::launch_kp_zgemm(sk, dk, n, 1.0, false, tz, s), "k-point zgemm launch");
-        check_hip(hfjk::launch_kp_zgemm(tz, sk, n, madelung, true, (char*)exchange + 16 * k * nn, s),
-                  "k-point zgemm launch");
-      }
-    }
+    madelung_term();
   });
 }
 

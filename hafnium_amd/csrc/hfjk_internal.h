@@ -259,8 +259,10 @@ int syrk_split_count(int precision, int naux, int nao, int ldo, int cus);
 // (hipErrorInvalidValue for a launch that would not run them).
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
                        bool is_signed, int nsplit, void* partial, int kind, hipStream_t s,
-                       const double* auxsign = nullptr, int shift = 0, bool x_ilv = false, int nocc = 0);
-// nocc (0 = ldo): X's columns past it are zero and may be skipped.
+                       const double* auxsign = nullptr, int shift = 0, bool x_ilv = false, int nocc = 0,
+                       int xrows = 0);
+// nocc (0 = ldo): X's columns past it are zero and may be skipped. xrows
+// (0 = x_rows(nao)): rows of X per aux function.
 // syrk_edge: rows and columns of K that one of launch_syrk's tiles holds for
 // these arguments (tile (r, c) starts at row r edge, column c edge);
 // syrk_row_block: the direct-LDS kernels' equal split of the rows.
@@ -277,6 +279,10 @@ bool syrk16_tiles256(int nao, int ldo, bool is_signed, int kind, int shift);
 // (diagonal tiles: from their lower triangle). accumulate adds to K instead of writing.
 hipError_t launch_syrk_reduce2(const void* sym, const void* anti, int precision, int nslot, int nao,
                                bool accumulate, double* out, hipStream_t s);
+// Complex K [nk][nao][nao] (+)= sym + i anti on the lower triangle and its
+// conjugate above (nslot slots of FP64 tiles per k).
+hipError_t launch_syrk_reduce_complex(const double* sym, const double* anti, int nslot, int nao, int nk,
+                                      bool accumulate, void* out, hipStream_t s);
 hipError_t launch_syrk_reduce(const void* partial, int precision, int nslot, int nao, int edge, double* out,
                               hipStream_t s);
 
@@ -315,6 +321,12 @@ hipError_t launch_expand_full(const double* packed, long long p, int naux, int n
 hipError_t launch_half_transform_full(const void* bfull, int precision, int naux, int nao, const void* ct, int ldo,
                                       void* x, hipStream_t s, int bn16 = 0, bool x_ilv = false);
 bool x16_tiles256(int ldo, int bn16);
+// FP64 rows of `len` doubles times operand fragments (xk.hip): block b0 + i
+// (`rows` rows) uses the fragments of group (b0 + i) % ngroup (fragment_index
+// over column_groups(columns, ldo, 0), k padded to 32; columns a multiple of
+// 16); x[(i rows + row) ldo + column].
+hipError_t launch_rows_transform(const double* b, long long rows, int len, int b0, int nblocks, int ngroup,
+                                 const double* frag, int columns, double* x, int ldo, hipStream_t s);
 // k-point DF-J/K (kpoint.hip): complex values as interleaved double pairs.
 // launch_kp_charges: inner [nk][naux] = w_k <B_k[P], D_k> (conjugated B) and
 // charges [naux] = sum_k inner, for blocks B_k at b + k kstride (elements);
@@ -325,9 +337,8 @@ bool x16_tiles256(int ldo, int bn16);
 // over the nneg lowest and npos highest eigenpairs (U column-major from
 // rocSOLVER zheevd of the column-major view of a row-major Hermitian D), and
 // the column signs; launch_kp_fold: K (+)= (Kh_TL + Kh_BR) + i (Kh_BL - Kh_TR)
-// of a [2 nao][2 nao] real Kh; launch_kp_zgemm: c (+)= alpha a b ([nao][nao]);
-// launch_kp_hermitian_stats: max |D - D^H| and max |D| (atomic max of double
-// bits into stats[0..1]; clear first).
+// of a [2 nao][2 nao] real Kh; launch_kp_madelung: out[k] += alpha S D S of
+// every k (tmp: nk nao^2 complex).
 hipError_t launch_kp_charges(const void* b, long long kstride, int nk, int naux, int nao, const void* density,
                              const double* weights, void* inner, void* charges, hipStream_t s);
 hipError_t launch_kp_coulomb(const void* b, long long kstride, int nk, int naux, int nao, const double* sig,
@@ -336,9 +347,20 @@ hipError_t launch_kp_realify(const void* b, int naux, int nao, double* out, hipS
 hipError_t launch_kp_factor(const void* eigvecs, const double* eigvals, int nao, int nneg, int npos, double weight,
                             int ldo, double* ct, double* signs, hipStream_t s);
 hipError_t launch_kp_fold(const double* kh, int nao, bool accumulate, void* k, hipStream_t s);
-hipError_t launch_kp_zgemm(const void* a, const void* b, int nao, double alpha, bool accumulate, void* c,
-                           hipStream_t s);
-hipError_t launch_kp_hermitian_stats(const void* d, int nao, unsigned long long* stats, hipStream_t s);
+// The factorisation of every k's density at once: max |D - D^H|, max |D| and
+// max |D - L L^H| (KpState, cleared by launch_kp_cholesky) of the pivoted
+// Cholesky D = L L^H, L by columns [nk][nao][nao] (with nk nao doubles of
+// scratch behind it), stopped at 1e-12 of the largest diagonal; launch_kp_fragments: the operand fragments
+// [nk][kpad][2 hb] of sqrt(weight) [Re, Im] of the L of every k.
+struct KpState {
+  unsigned long long asym, mag, residual;  // bits of non-negative doubles
+  int rank, pad;
+};
+hipError_t launch_kp_cholesky(const void* density, int nk, int nao, void* l, KpState* st, hipStream_t s);
+hipError_t launch_kp_fragments(const void* l, const KpState* st, const double* weights, int nk, int nao, int hb,
+                               double* frag, double* sym, double* cross, hipStream_t s);
+hipError_t launch_kp_madelung(const void* overlap, const void* density, int nk, int nao, double alpha, void* tmp,
+                              void* out, hipStream_t s);
 // The non-symmetric exchange (kpoint.hip): H = S + i A of a real D (complex
 // [nao][nao]); the real orbitals [nao][2 hb] = [Re V |l|^1/2, 0, Im V |l|^1/2, 0]
 // of retained eigenpairs j0 .. j0 + rb - 1 of H (the nneg lowest, then the

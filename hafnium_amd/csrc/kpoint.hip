@@ -72,24 +72,45 @@ __global__ __launch_bounds__(kThreads) void kp_charges_kernel(const double2* __r
   charges[p] = acc;
 }
 
-// J_k[xw] = sum_P s_k[P] charges[P] B_k[P][xw]; grid (element blocks, nk).
+// J_k[xw] = sum_P s_k[P] charges[P] B_k[P][xw]; grid (element blocks, nk): 32
+// elements per workgroup, eight thread groups sharing the aux functions
+// (combined in a fixed order; one thread per element walking all of them left
+// most of the device idle: 59 us at nao 28, naux 212, eight k-points).
+constexpr int kCoulombElems = 32;
+
 __global__ __launch_bounds__(kThreads) void kp_coulomb_kernel(const double2* __restrict__ b, long long kstride,
                                                               int naux, long long nn, const double* __restrict__ sig,
                                                               long long sig_kstride, const double2* __restrict__ charges,
                                                               double2* __restrict__ j) {
+  constexpr int kParts = kThreads / kCoulombElems;
+  __shared__ double2 red[kParts][kCoulombElems];
   const int k = blockIdx.y;
   const double2* bk = b + (long long)k * kstride;
   const double* sk = sig + (long long)k * sig_kstride;
-  for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < nn; i += (long long)gridDim.x * kThreads) {
+  const int e = threadIdx.x % kCoulombElems, part = threadIdx.x / kCoulombElems;
+  for (long long i0 = (long long)blockIdx.x * kCoulombElems; i0 < nn; i0 += (long long)gridDim.x * kCoulombElems) {
+    const long long i = i0 + e;
     double2 acc = make_double2(0.0, 0.0);
-    for (int p = 0; p < naux; ++p) {
-      const double2 c = charges[p];
-      const double s = sk[p];
-      const double2 v = cmul(make_double2(s * c.x, s * c.y), bk[(long long)p * nn + i]);
-      acc.x += v.x;
-      acc.y += v.y;
+    if (i < nn) {
+#pragma unroll 4
+      for (int p = part; p < naux; p += kParts) {
+        const double2 c = charges[p];
+        const double s = sk[p];
+        const double2 v = cmul(make_double2(s * c.x, s * c.y), bk[(long long)p * nn + i]);
+        acc.x += v.x;
+        acc.y += v.y;
+      }
     }
-    j[(long long)k * nn + i] = acc;
+    red[part][e] = acc;
+    __syncthreads();
+    if (part == 0 && i < nn) {
+      for (int q = 1; q < kParts; ++q) {
+        acc.x += red[q][e].x;
+        acc.y += red[q][e].y;
+      }
+      j[(long long)k * nn + i] = acc;
+    }
+    __syncthreads();
   }
 }
 
@@ -158,11 +179,14 @@ __global__ __launch_bounds__(kThreads) void kp_fold_kernel(const double* __restr
   }
 }
 
-// c (+)= alpha a b for complex row-major [n][n]; one thread per output element.
+// c (+)= alpha a b for complex row-major [n][n], one triple per blockIdx.y; one thread per output element.
 __global__ __launch_bounds__(kThreads) void kp_zgemm_kernel(const double2* __restrict__ a, const double2* __restrict__ b,
                                                             int n, double alpha, int accumulate,
                                                             double2* __restrict__ c) {
   const long long nn = (long long)n * n;
+  a += blockIdx.y * nn;
+  b += blockIdx.y * nn;
+  c += blockIdx.y * nn;
   for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < nn;
        idx += (long long)gridDim.x * kThreads) {
     const long long r = idx / n, col = idx % n;
@@ -183,29 +207,180 @@ __global__ __launch_bounds__(kThreads) void kp_zgemm_kernel(const double2* __res
   }
 }
 
-// stats[0] = max |D - D^dagger|, stats[1] = max |D| (bits of doubles, atomic max; clear first).
-__global__ __launch_bounds__(kThreads) void kp_hermitian_stats_kernel(const double2* __restrict__ d, int n,
-                                                                      unsigned long long* __restrict__ stats) {
-  double asym = 0.0, mag = 0.0;
+// Pivoted Cholesky of every k's positive semidefinite density, D = L L^H, one
+// workgroup per k (one launch for all columns of all k instead of zheevd's
+// hundreds of small kernels per k, 0.55 ms each): column c takes the largest
+// remaining diagonal p (ties: lowest index), L[:, c] = (D[:, p] - sum_{j<c}
+// L[:, j] conj(L[p][j])) / sqrt(d_p). Bound by the latency of a column.
+constexpr int kCholThreads = 512;
+
+__global__ __launch_bounds__(kCholThreads) void kp_cholesky_kernel(const double2* __restrict__ density, int n,
+                                                                   double2* __restrict__ lmat,
+                                                                   double* __restrict__ diag_all,
+                                                                   KpState* __restrict__ state) {
+  __shared__ double wval[kCholThreads / 64];
+  __shared__ int widx[kCholThreads / 64];
+  __shared__ double s_best;
+  __shared__ int s_at;
+  __shared__ double2 prow[kCholThreads];  // conj(L[p][j0 .. j0 + kCholThreads))
   const long long nn = (long long)n * n;
+  const double2* d = density + blockIdx.x * nn;
+  double2* l = lmat + blockIdx.x * nn;
+  double* diag = diag_all + (long long)blockIdx.x * n;
+  const int t = threadIdx.x;
+  for (int i = t; i < n; i += kCholThreads) diag[i] = d[(long long)i * n + i].x;
+  double cut = 0.0;
+  int rank = n;
+  for (int c = 0; c <= n; ++c) {
+    __syncthreads();  // diag is written
+    double best = -1.0;
+    int at = -1;
+    for (int i = t; i < n; i += kCholThreads)
+      if (diag[i] > best) {
+        best = diag[i];
+        at = i;
+      }
+    for (int off = 32; off > 0; off >>= 1) {
+      const double ov = __shfl_xor(best, off);
+      const int oi = __shfl_xor(at, off);
+      if (ov > best || (ov == best && oi >= 0 && (at < 0 || oi < at))) {
+        best = ov;
+        at = oi;
+      }
+    }
+    if ((t & 63) == 0) {
+      wval[t >> 6] = best;
+      widx[t >> 6] = at;
+    }
+    __syncthreads();
+    if (t == 0) {
+      for (int w = 1; w < kCholThreads / 64; ++w)
+        if (wval[w] > best || (wval[w] == best && widx[w] >= 0 && (at < 0 || widx[w] < at))) {
+          best = wval[w];
+          at = widx[w];
+        }
+      s_best = best;
+      s_at = at;
+    }
+    __syncthreads();
+    const double piv = s_best;
+    const int p = s_at;
+    if (c == 0) cut = 1e-12 * piv;
+    if (c == n || p < 0 || !(piv > cut)) {
+      rank = c;
+      break;
+    }
+    const double inv = 1.0 / sqrt(piv);
+    // Rows in strides of the workgroup; the pivot's row of L through LDS.
+    for (int i0 = 0; i0 < n; i0 += kCholThreads) {
+      const int i = i0 + t;
+      double2 v = make_double2(0.0, 0.0);
+      if (i < n) v = d[(long long)i * n + p];
+      for (int j0 = 0; j0 < c; j0 += kCholThreads) {
+        __syncthreads();
+        if (j0 + t < c) {
+          const double2 q = l[(long long)(j0 + t) * n + p];
+          prow[t] = make_double2(q.x, -q.y);
+        }
+        __syncthreads();
+        const int top = min(kCholThreads, c - j0);
+        if (i < n) {
+#pragma unroll 4
+          for (int j = 0; j < top; ++j) {
+            const double2 m = cmul(l[(long long)(j0 + j) * n + i], prow[j]);
+            v.x -= m.x;
+            v.y -= m.y;
+          }
+        }
+      }
+      if (i < n) {
+        v.x *= inv;
+        v.y *= inv;
+        l[(long long)c * n + i] = v;
+        diag[i] = i == p ? 0.0 : diag[i] - (v.x * v.x + v.y * v.y);
+      }
+    }
+  }
+  if (t == 0) state[blockIdx.x].rank = rank;
+}
+
+// Per k: max |D - D^H|, max |D| and max |D - L L^H| (atomic max of bits).
+__global__ __launch_bounds__(kThreads) void kp_residual_kernel(const double2* __restrict__ density, int n,
+                                                               const double2* __restrict__ lmat,
+                                                               KpState* __restrict__ state) {
+  const long long nn = (long long)n * n;
+  const double2* d = density + blockIdx.y * nn;
+  const double2* l = lmat + blockIdx.y * nn;
+  KpState* st = state + blockIdx.y;
+  const int rank = st->rank;
+  double asym = 0.0, mag = 0.0, worst = 0.0;
   for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < nn;
        idx += (long long)gridDim.x * kThreads) {
-    const long long r = idx / n, c = idx % n;
-    const double2 a = d[idx], t = d[c * n + r];
-    const double a1 = hypot(a.x - t.x, a.y + t.y);
-    const double m = hypot(a.x, a.y);
-    asym = a1 > asym ? a1 : asym;
-    mag = m > mag ? m : mag;
+    const int r = (int)(idx / n), c = (int)(idx % n);
+    double2 a = d[idx];
+    const double2 t = d[(long long)c * n + r];
+    asym = fmax(asym, hypot(a.x - t.x, a.y + t.y));
+    mag = fmax(mag, hypot(a.x, a.y));
+    for (int j = 0; j < rank; ++j) {
+      const double2 u = l[(long long)j * n + r], v = l[(long long)j * n + c];
+      const double2 m = cmul(u, make_double2(v.x, -v.y));
+      a.x -= m.x;
+      a.y -= m.y;
+    }
+    // Not fmax, which would drop a NaN: a NaN must fail the host's test.
+    const double e = fabs(a.x) + fabs(a.y);
+    worst = e > worst || e != e ? e : worst;
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    const double a = __shfl_xor(asym, off);
-    const double m = __shfl_xor(mag, off);
-    asym = a > asym ? a : asym;
-    mag = m > mag ? m : mag;
+  unsigned long long* out[3] = {&st->asym, &st->mag, &st->residual};
+  double v[3] = {asym, mag, worst};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    unsigned long long bits = (unsigned long long)__double_as_longlong(fabs(v[k]));
+    for (int off = 32; off > 0; off >>= 1) {
+      const unsigned long long o = __shfl_xor(bits, off);
+      bits = o > bits ? o : bits;
+    }
+    if ((threadIdx.x & 63) == 0 && bits != 0) atomicMax(out[k], bits);
   }
-  if ((threadIdx.x & 63) == 0) {
-    if (asym > 0.0) atomicMax(&stats[0], (unsigned long long)__double_as_longlong(asym));
-    if (mag > 0.0) atomicMax(&stats[1], (unsigned long long)__double_as_longlong(mag));
+}
+
+__global__ __launch_bounds__(kThreads) void kp_clear_kernel(KpState* __restrict__ st, int nk) {
+  for (int k = threadIdx.x; k < nk; k += kThreads) st[k] = KpState{0, 0, 0, 0, 0};
+}
+
+// Operand fragments of [Re X, Im X] = B [..]: a complex row of B is 2 n reals
+// (re, im, re, im, ..), so the column of Re X_j is (Re C_0j, -Im C_0j, Re C_1j,
+// ..) and that of Im X_j (Im C_0j, Re C_0j, ..), C = sqrt(weight) L. Columns
+// [0, hb) are Re, [hb, 2 hb) Im, zero past the rank; and the column signs of
+// the SYRKs of Re K and (shifted by hb) Im K.
+__global__ __launch_bounds__(kThreads) void kp_fragments_kernel(const double2* __restrict__ lmat,
+                                                                const KpState* __restrict__ state,
+                                                                const double* __restrict__ weights, int n, int hb,
+                                                                int kpad, ColumnGroups cg, double* __restrict__ frag,
+                                                                double* __restrict__ sym, double* __restrict__ cross) {
+  const int kp = blockIdx.y;
+  const int rank = state[kp].rank;
+  const double scale = sqrt(weights[kp]);
+  const double2* l = lmat + (long long)kp * n * n;
+  double* out = frag + (long long)kp * kpad * 2 * hb;
+  const long long total = (long long)kpad * 2 * hb;
+  for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < total;
+       idx += (long long)gridDim.x * kThreads) {
+    const int i = (int)(idx / kpad), k = (int)(idx % kpad);
+    const int j = i < hb ? i : i - hb;
+    double v = 0.0;
+    if (k < 2 * n && j < rank) {
+      const double2 z = l[(long long)j * n + k / 2];
+      if (i < hb)
+        v = k % 2 ? -z.y : z.x;
+      else
+        v = k % 2 ? z.x : z.y;
+    }
+    out[fragment_index<double>(cg, kpad, k, i)] = scale * v;
+    if (kp == 0 && k == 0) {
+      sym[i] = 1.0;
+      cross[i] = i < hb ? -1.0 : 1.0;
+    }
   }
 }
 
@@ -276,7 +451,7 @@ hipError_t launch_kp_charges(const void* b, long long kstride, int nk, int naux,
 hipError_t launch_kp_coulomb(const void* b, long long kstride, int nk, int naux, int nao, const double* sig,
                              long long sig_kstride, const void* charges, void* out, hipStream_t s) {
   const long long nn = (long long)nao * nao;
-  const unsigned gx = (unsigned)std::min<long long>((nn + kThreads - 1) / kThreads, 1 << 16);
+  const unsigned gx = (unsigned)std::min<long long>((nn + kCoulombElems - 1) / kCoulombElems, 1 << 16);
   hipLaunchKernelGGL(kp_coulomb_kernel, dim3(gx, (unsigned)nk), dim3(kThreads), 0, s, (const double2*)b, kstride,
                      naux, nn, sig, sig_kstride, (const double2*)charges, (double2*)out);
   return hipGetLastError();
@@ -303,16 +478,36 @@ hipError_t launch_kp_fold(const double* kh, int nao, bool accumulate, void* k, h
   return hipGetLastError();
 }
 
-hipError_t launch_kp_zgemm(const void* a, const void* b, int nao, double alpha, bool accumulate, void* c,
-                           hipStream_t s) {
-  hipLaunchKernelGGL(kp_zgemm_kernel, dim3(grid_for((long long)nao * nao)), dim3(kThreads), 0, s,
-                     (const double2*)a, (const double2*)b, nao, alpha, accumulate ? 1 : 0, (double2*)c);
+hipError_t launch_kp_madelung(const void* overlap, const void* density, int nk, int nao, double alpha, void* tmp,
+                              void* out, hipStream_t s) {
+  const dim3 grid((unsigned)grid_for((long long)nao * nao), (unsigned)nk);
+  hipLaunchKernelGGL(kp_zgemm_kernel, grid, dim3(kThreads), 0, s, (const double2*)overlap, (const double2*)density,
+                     nao, 1.0, 0, (double2*)tmp);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kp_zgemm_kernel, grid, dim3(kThreads), 0, s, (const double2*)tmp, (const double2*)overlap, nao,
+                     alpha, 1, (double2*)out);
   return hipGetLastError();
 }
 
-hipError_t launch_kp_hermitian_stats(const void* d, int nao, unsigned long long* stats, hipStream_t s) {
-  hipLaunchKernelGGL(kp_hermitian_stats_kernel, dim3(grid_for((long long)nao * nao)), dim3(kThreads), 0, s,
-                     (const double2*)d, nao, stats);
+hipError_t launch_kp_cholesky(const void* density, int nk, int nao, void* l, KpState* st, hipStream_t s) {
+  hipLaunchKernelGGL(kp_clear_kernel, dim3(1), dim3(kThreads), 0, s, st, nk);
+  // The diagonals live behind L.
+  double* diag = (double*)((double2*)l + (long long)nk * nao * nao);
+  hipLaunchKernelGGL(kp_cholesky_kernel, dim3((unsigned)nk), dim3(kCholThreads), 0, s, (const double2*)density, nao,
+                     (double2*)l, diag, st);
+  const unsigned gx = (unsigned)std::min<long long>(((long long)nao * nao + kThreads - 1) / kThreads, 1024);
+  hipLaunchKernelGGL(kp_residual_kernel, dim3(gx, (unsigned)nk), dim3(kThreads), 0, s, (const double2*)density, nao,
+                     (const double2*)l, st);
+  return hipGetLastError();
+}
+
+hipError_t launch_kp_fragments(const void* l, const KpState* st, const double* weights, int nk, int nao, int hb,
+                               double* frag, double* sym, double* cross, hipStream_t s) {
+  const int kpad = n_tiles(2 * nao) * kTile;
+  const dim3 grid((unsigned)grid_for((long long)kpad * 2 * hb), (unsigned)nk);
+  hipLaunchKernelGGL(kp_fragments_kernel, grid, dim3(kThreads), 0, s, (const double2*)l, st, weights, nao, hb, kpad,
+                     column_groups(2 * hb, 2 * hb, 0), frag, sym, cross);
   return hipGetLastError();
 }
 

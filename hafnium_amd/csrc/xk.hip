@@ -312,6 +312,80 @@ __global__ __launch_bounds__(kThreads, NI <= 4 ? 3 : 2) void xform_units_kernel(
                      zero_block != 0 && g == ngroups - 1, lds0, lds1);
 }
 
+// Plain row-major rows times per-group operand fragments (FP64): rows of
+// `len` doubles, `rows` per block, block b0 + i with the fragments of group
+// (b0 + i) % ngroup; x[(i rows + row) ldo + column] for the NI blocks from
+// column 0 of x on. The structure of xform_units with the operand read
+// directly; k past len repeats the row's start against zero fragments.
+template <int NI>
+__global__ __launch_bounds__(kThreads, NI <= 4 ? 3 : 2) void rows_units_kernel(
+    const double* __restrict__ b, long long rows, int len, int b0, int ngroup, const double* __restrict__ cf,
+    long long group_elems, double* __restrict__ x, int ldo, int wgs_per_block) {
+  typedef XFrag<double> F;
+  typedef F::unit unit;
+  __shared__ __attribute__((aligned(16))) double lds0[NI * F::BLOCK];
+  __shared__ __attribute__((aligned(16))) double lds1[NI * F::BLOCK];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row16 = lane & 15, grp = lane >> 4;
+  const int blk = blockIdx.x / wgs_per_block;
+  const long long row0 = ((long long)(blockIdx.x % wgs_per_block) * 4 + wave) * 16;
+  const double* cg = cf + (b0 + blk) % ngroup * group_elems;
+  const double* src = b + ((long long)(b0 + blk) * rows + min(row0 + row16, rows - 1)) * len;
+  const int nt = (len + kTile - 1) / kTile;
+
+  auto load_c = [&](int k, double* stage) {
+    const double* p = cg + (long long)k * NI * F::BLOCK + lane * F::EV;
+    for (int c = wave; c < NI * F::LOADS; c += 4)
+      __builtin_amdgcn_global_load_lds((const void*)(p + c * 64 * F::EV), (lds_void_t*)(stage + c * 64 * F::EV), 16, 0,
+                                       0);
+  };
+  auto load_a = [&](int kt, unit (&a)[F::NG]) {
+#pragma unroll
+    for (int eg = 0; eg < F::NG; ++eg) {
+      const int k = kt * kTile + eg * F::KG + grp * F::EV;
+      a[eg] = *(const unit*)(src + (k < len ? k : 0));
+    }
+  };
+  Op<double>::acc_t acc[NI];
+#pragma unroll
+  for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[ni][e] = 0.0;
+  int kt = 0;
+  auto step = [&](const double* cur, double* next, unit (&a)[F::NG], unit (&an)[F::NG]) {
+    wait_vm_lgkm0<0>();
+    barrier_nofence();
+    if (kt + 1 < nt) load_c(kt + 1, next);
+    load_a(min(kt + 1, nt - 1), an);
+#pragma unroll
+    for (int eg = 0; eg < F::NG; ++eg)
+      if (kt * kTile + eg * F::KG < len) {
+        unit bv[NI];
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) bv[ni] = *(const unit*)(cur + ((eg * NI + ni) * 64 + lane) * F::EV);
+#pragma unroll
+        for (int ee = 0; ee < F::EV; ++ee)
+#pragma unroll
+          for (int ni = 0; ni < NI; ++ni) acc[ni] = Op<double>::mma(a[eg][ee], bv[ni][ee], acc[ni]);
+      }
+    return ++kt < nt;
+  };
+  unit a0[F::NG], a1[F::NG];
+  load_c(0, lds0);
+  load_a(0, a0);
+  while (step(lds0, lds1, a0, a1) && step(lds1, lds0, a1, a0)) {
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const long long row = row0 + Op<double>::row(lane, e);
+    if (row >= rows) continue;
+    double* at = x + ((long long)blk * rows + row) * ldo + row16;
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) at[ni * 16] = acc[ni][e];
+  }
+}
+
 // ------------------------------------------------------------------ BF16x3 half-transform
 
 constexpr int kRowK = 40;  // bf16 LDS row: 32 k + 8 pad (80 bytes, 16-byte aligned rows)
@@ -2260,7 +2334,10 @@ __device__ __forceinline__ double2 slot_sum(const T* __restrict__ src, int part,
 // chain to a few), by HBM otherwise.
 constexpr int kRedThreads = 512;
 
-template <typename T, int STRIP, bool ANTI>
+//
+// With COMPLEX (the k-point exchange, one result per blockIdx.y with nslot
+// slots each): K[m][n] (+)= S + i A, K[n][m] (+)= S - i A, interleaved.
+template <typename T, int STRIP, bool ANTI, bool COMPLEX = false>
 __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __restrict__ partial,
                                                                   const T* __restrict__ anti, int nslot, int npairs,
                                                                   int nao, int edge, int accumulate,
@@ -2281,6 +2358,11 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
   const int part = t / (STRIP * (kSyrkTile / 2));
   const int row = row0 + lr, gcol = bn * edge + col;
   const long long stride = (long long)npairs * (kSyrkTile * kSyrkTile);
+  if constexpr (COMPLEX) {
+    partial += blockIdx.y * nslot * stride;
+    anti += blockIdx.y * nslot * stride;
+    out += 2LL * blockIdx.y * nao * nao;
+  }
   if (row < nao && col < edge && gcol <= row) {
     const long long at = (long long)pair * (kSyrkTile * kSyrkTile) + (strip * STRIP + lr) * kSyrkTile + col;
     *(double2*)&part_sum[0][part][lr][col] = slot_sum<T, PARTS>(partial + at, part, nslot, stride);
@@ -2299,8 +2381,17 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
       if constexpr (ANTI) aa += part_sum[1][q][r][c];
     }
     const long long o = (long long)gr * nao + gc;
-    out[o] = (ANTI && accumulate ? out[o] : 0.0) + ss + aa;
-    part_sum[0][0][r][c] = ss - aa;
+    if constexpr (COMPLEX) {
+      if (gr == gc) aa = 0.0;
+      double2* k = (double2*)out;
+      const double2 old = accumulate ? k[o] : make_double2(0.0, 0.0);
+      k[o] = make_double2(old.x + ss, old.y + aa);
+      part_sum[0][0][r][c] = ss;
+      part_sum[NS - 1][0][r][c] = aa;
+    } else {
+      out[o] = (ANTI && accumulate ? out[o] : 0.0) + ss + aa;
+      part_sum[0][0][r][c] = ss - aa;
+    }
   }
   __syncthreads();
   for (int e = t; e < STRIP * kSyrkTile; e += kRedThreads) {
@@ -2308,7 +2399,13 @@ __global__ __launch_bounds__(kRedThreads) void syrk_reduce_kernel(const T* __res
     const int gr = row0 + r, gc = bn * edge + c;
     if (gr >= nao || c >= edge || gc >= gr) continue;
     const long long o = (long long)gc * nao + gr;
-    out[o] = (ANTI && accumulate ? out[o] : 0.0) + part_sum[0][0][r][c];
+    if constexpr (COMPLEX) {
+      double2* k = (double2*)out;
+      const double2 old = accumulate ? k[o] : make_double2(0.0, 0.0);
+      k[o] = make_double2(old.x + part_sum[0][0][r][c], old.y - part_sum[NS - 1][0][r][c]);
+    } else {
+      out[o] = (ANTI && accumulate ? out[o] : 0.0) + part_sum[0][0][r][c];
+    }
   }
 }
 
@@ -2631,6 +2728,34 @@ hipError_t launch_half_transform(const void* b, int precision, long long p, int 
   return launch_x_typed<float>((const float*)b, p, naux, nao, (const float*)cf, nocc, ldo, (float*)x, bn, bm, s);
 }
 
+template <int NI = 1>
+static hipError_t launch_rows_n(int ni, const double* b, long long rows, int len, int b0, int nblocks, int ngroup,
+                                const double* cf, long long group_elems, double* x, int ldo, hipStream_t s) {
+  if constexpr (NI < kMaxGroupBlocks) {
+    if (ni != NI)
+      return launch_rows_n<NI + 1>(ni, b, rows, len, b0, nblocks, ngroup, cf, group_elems, x, ldo, s);
+  }
+  const long long per = (rows + 63) / 64;
+  if (per * nblocks >= (1LL << 24)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rows_units_kernel<NI>, dim3((unsigned)(per * nblocks)), dim3(kThreads), 0, s, b, rows, len, b0,
+                     ngroup, cf, group_elems, x, ldo, (int)per);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_transform(const double* b, long long rows, int len, int b0, int nblocks, int ngroup,
+                                 const double* frag, int columns, double* x, int ldo, hipStream_t s) {
+  const ColumnGroups cg = column_groups(columns, ldo, 0);
+  const int kpad = (len + kTile - 1) / kTile * kTile;
+  const long long group_elems = (long long)kpad * columns;
+  for (int g = 0; g < cg.groups + (cg.tail > 0 ? 1 : 0); ++g) {
+    const int ni = g < cg.groups ? cg.blocks : cg.tail;
+    const hipError_t e = launch_rows_n(ni, b, rows, len, b0, nblocks, ngroup, frag + (long long)g * cg.blocks * 16 * kpad,
+                                       group_elems, x + g * cg.blocks * 16, ldo, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t launch_prepare_orbitals(const double* c, int nao, int nocc, int precision, void* pad, void* ct, void* frag,
                                    int bn, const double* signs_in, double* signs, hipStream_t s) {
   const int npad = n_tiles(nao) * kTile, ldo = occ_ld(nocc);
@@ -2679,8 +2804,8 @@ bool syrk16_tiles256(int nao, int ldo, bool is_signed, int kind, int shift) {
 
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
                        bool is_signed, int nsplit, void* partial, int kind, hipStream_t s, const double* auxsign,
-                       int shift, bool x_ilv, int nocc) {
-  const int xrows = x_rows(nao);
+                       int shift, bool x_ilv, int nocc, int xrows) {
+  if (xrows <= 0) xrows = x_rows(nao);
   const int edge = syrk_edge(precision, nao, ldo, is_signed, kind);
   if (nocc <= 0 || nocc > ldo) nocc = ldo;
   const int npairs = syrk_pairs(nao);
@@ -2689,7 +2814,8 @@ hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo,
   // the signed direct-LDS kernels of every precision.
   const bool ring_ok = is_signed && kind != 1 && ldo <= kDmaMaxLdo && (long long)xrows * ldo < (1LL << 30);
   if (auxsign != nullptr && (!ring_ok || precision == HFJK_BF16X3)) return hipErrorInvalidValue;
-  if (shift != 0 && (!ring_ok || shift % 32 != 0 || shift < 0 || shift >= ldo)) return hipErrorInvalidValue;
+  const int shift_step = precision == HFJK_FP64 ? 16 : 32;  // columns of a ring step
+  if (shift != 0 && (!ring_ok || shift % shift_step != 0 || shift < 0 || shift >= ldo)) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)(npairs * nsplit);
   // The direct-load kernel keeps per-lane element offsets within one aux
   // function's X in 32 bits and the sign table in LDS.
@@ -2770,6 +2896,15 @@ static hipError_t launch_reduce_t(const T* partial, const T* anti, int nslot, in
   else
     hipLaunchKernelGGL((syrk_reduce_kernel<T, 1, ANTI>), dim3((unsigned)(npairs * kSyrkTile)), blk, 0, s, partial,
                        anti, nslot, npairs, nao, edge, acc, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_syrk_reduce_complex(const double* sym, const double* anti, int nslot, int nao, int nk,
+                                      bool accumulate, void* out, hipStream_t s) {
+  const int npairs = syrk_pairs(nao);
+  hipLaunchKernelGGL((syrk_reduce_kernel<double, 2, true, true>), dim3((unsigned)(npairs * (kSyrkTile / 2)), (unsigned)nk),
+                     dim3(kRedThreads), 0, s, sym, anti, nslot, npairs, nao, kSyrkTile, accumulate ? 1 : 0,
+                     (double*)out);
   return hipGetLastError();
 }
 

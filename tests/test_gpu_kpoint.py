@@ -96,3 +96,64 @@ def test_malformed_inputs_are_rejected():
         jk.exchange(np.ones((2, 4, 4)) + 1j * np.triu(np.ones((2, 4, 4))))
     with pytest.raises(InputError, match="shape"):
         jk.coulomb(np.zeros((2, 3, 3)))
+
+
+@pytest.mark.parametrize("nk,nao,naux,nocc", [(1, 2, 3, 1), (3, 4, 5, 4), (2, 17, 9, 16), (5, 31, 20, 17), (1, 130, 6, 40),
+                                              (9, 12, 7, 3)])
+@pytest.mark.parametrize("positive", [True, False])
+def test_exchange_of_both_factorisations(nk, nao, naux, nocc, positive):
+    """Positive semidefinite densities (Cholesky, whole ranges of blocks) and indefinite ones (eigenpairs, block by
+    block) against the definition, with mixed signatures, uneven weights and ranks, and the Madelung term."""
+    from hafnium_amd.kpoint import KPointMI355XCoulombExchange
+
+    rng = np.random.default_rng(nk * 1000 + nao)
+    z = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)  # noqa: E731
+    b = z(nk, nk, naux, nao, nao)
+    sig = np.where(rng.random((nk, nk, naux)) < 0.3, -1.0, 1.0)
+    w = rng.uniform(0.2, 1.0, nk)
+    s = z(nk, nao, nao)
+    s = s + s.conj().transpose(0, 2, 1)
+    d = np.zeros((nk, nao, nao), dtype=complex)
+    for k in range(nk):
+        c = z(nao, max(1, nocc - k % 3))
+        d[k] = c @ c.conj().T
+        if not positive and k == nk - 1:
+            d[k] -= 3.0 * np.eye(nao)
+        d[k] = 0.5 * (d[k] + d[k].conj().T)
+    expect = np.einsum("k,qkpxy,qkp,kyz,qkpwz->qxw", w, b, sig, d, b.conj(), optimize=True)
+    expect += 0.4 * s @ d @ s
+    got = KPointMI355XCoulombExchange(b, sig, w, s, 0.4).exchange(d)
+    # Sums of nk naux nocc products: their rounding relative to the sum of magnitudes.
+    top = np.einsum("k,qkpxy,kyz,qkpwz->qxw", w, np.abs(b), np.abs(d), np.abs(b), optimize=True).max() + \
+        0.4 * (np.abs(s) @ np.abs(d) @ np.abs(s)).max()
+    assert np.max(np.abs(got - expect)) <= 64 * nao * 2.0 ** -53 * top
+    assert np.max(np.abs(got - got.conj().transpose(0, 2, 1))) <= 16 * nao * 2.0 ** -53 * top
+
+
+def test_exchange_in_several_passes():
+    """More blocks than the workspace holds X of: ranges of k2 accumulate, results equal to one pass."""
+    import ctypes
+
+    import torch
+
+    from hafnium_amd import _lib
+    from hafnium_amd.kpoint import KPointMI355XCoulombExchange
+
+    rng = np.random.default_rng(4)
+    nk, nao, naux = 4, 40, 1500
+    z = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)  # noqa: E731
+    b = torch.from_numpy(z(1, 1, naux, nao, nao)).cuda().expand(nk, nk, naux, nao, nao).contiguous()
+    c = z(nk, nao, nao)
+    d = torch.from_numpy(c @ c.conj().transpose(0, 2, 1)).cuda()
+    jk = KPointMI355XCoulombExchange(b, torch.ones(nk, nk, naux), torch.full((nk,), 1.0 / nk),
+                                     torch.zeros(nk, nao, nao, dtype=torch.complex128), 0.0)
+    size = ctypes.c_size_t()
+    _lib.check(jk._ctx.lib.hfjk_kpoint_workspace_bytes(jk._ctx.handle, nk, naux, nao, ctypes.byref(size)))
+    assert nk * nk * naux * nao * 96 * 8 > 1 << 29  # ranges of whole k1 do not all fit
+    got = jk.exchange(d)
+    flat = b[0, 0]
+    dm = d.mean(0)
+    left = torch.matmul(flat.reshape(-1, nao), dm).view(naux, nao, nao)
+    want = torch.matmul(left.transpose(0, 1).reshape(nao, -1), flat.transpose(0, 1).reshape(nao, -1).conj().T.contiguous())
+    for k in range(nk):
+        assert float((got[k] - want).abs().max()) <= 1e-12 * float(want.abs().max())
