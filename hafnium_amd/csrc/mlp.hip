@@ -11,20 +11,22 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 
 #include "hfjk_internal.h"
 
 namespace {
 
+typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int kT = 256;
-constexpr int kTileM = 64;
-constexpr int kTileN = 64;
-constexpr int kStepK = 32;
-constexpr int kPitch = kStepK + 8;  // LDS row pitch (bf16): 80 bytes keeps 16-byte rows aligned
+constexpr int kTileM = 32;
+constexpr int kTileN = 32;
+constexpr int kWaves = 8;  // per tile
+constexpr int kGemmT = 64 * kWaves;
 
 __device__ __forceinline__ uint16_t to_bf16(float x) {
   uint32_t u = __float_as_uint(x);
@@ -33,15 +35,12 @@ __device__ __forceinline__ uint16_t to_bf16(float x) {
   return (uint16_t)(u >> 16);
 }
 
-__device__ __forceinline__ uint16_t load_bf16(const float* p) { return to_bf16(*p); }
-__device__ __forceinline__ uint16_t load_bf16(const uint16_t* p) { return *p; }
-
-__device__ __forceinline__ bf8 lds_bf8(const uint16_t* p) {
-  const uint4 v = *(const uint4*)p;
-  return __builtin_bit_cast(bf8, v);
-}
-
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + expf(-z)); }
+
+__device__ __forceinline__ float silu_slope(float z) {  // s (1 + z (1 - s)), s = 1 / (1 + e^-z)
+  const float s = 1.0f / (1.0f + expf(-z));
+  return s * (1.0f + z * (1.0f - s));
+}
 
 struct GemmArgs {
   int m, n, k;
@@ -54,102 +53,210 @@ struct GemmArgs {
   float* c;
   int ldc;
   int accumulate;
-  float* h;
+  float* h;            // silu(C)
+  const float* slope;  // C *= silu'(slope[i][j]), leading dimension ldc
+  float* bsum;         // column sums of B over k (FP32, unrounded), TB = float
+  // The weighted squared error of C: grad, and the workgroup's part of the loss.
+  const float* tgt;
+  int ldt;
+  const int* t_rows;
+  const float* w;
+  float scale;
+  float* grad;
+  float* loss_part;
 };
 
-// C[m][n] = op(A) op(B) (+ C) (+ bias); h = silu(C) when h is given.
+// Eight consecutive k of one row (or column) of an operand as a lane holds
+// them, in FP32: element (i, k + e), k + e < kmax, i < imax, zero elsewhere.
+// Stored row i (rows[i] when given) along k, or with trans k along i.
+template <typename T>
+__device__ __forceinline__ void load8(const T* __restrict__ p, int ld, int trans, const int* __restrict__ rows, int i,
+                                      int imax, int k, int kmax, bool vec, float (&v)[8]) {
+  auto f = [](T x) -> float {
+    if constexpr (sizeof(T) == 2)
+      return __uint_as_float((uint32_t)x << 16);
+    else
+      return x;
+  };
+  // Rows and columns past the operand read its last ones and count as zero,
+  // so that every load is unconditional. kmax, imax >= 1 here.
+  const int ic = min(i, imax - 1);
+  const T* src = trans ? p + ic : p + (long long)(rows ? rows[ic] : ic) * ld;
+  if (!trans && vec && k + 8 <= kmax) {
+    if constexpr (sizeof(T) == 2) {
+      const uint4 u = *(const uint4*)(src + k);
+      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(e & 1 ? w[e >> 1] & 0xFFFF0000u : w[e >> 1] << 16);
+    } else {
+      const float4 x = ((const float4*)(src + k))[0], y = ((const float4*)(src + k))[1];
+      v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
+      v[4] = y.x, v[5] = y.y, v[6] = y.z, v[7] = y.w;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = i < imax ? v[e] : 0.0f;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int kc = min(k + e, kmax - 1);
+      const T x = trans ? src[(long long)(rows ? rows[kc] : kc) * ld] : src[kc];
+      v[e] = i < imax && k + e < kmax ? f(x) : 0.0f;
+    }
+  }
+}
+
+__device__ __forceinline__ bf8 round8(const float (&v)[8]) {
+  union {
+    uint16_t u[8];
+    bf8 b;
+  } r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r.u[e] = to_bf16(v[e]);
+  return r.b;
+}
+
+// C[m][n] = op(A) op(B) (+ C) (+ bias) and the epilogues of GemmArgs.
 // op(A) is m x k: A is stored m x k (ta = 0) or k x m (ta = 1), row-major
 // with leading dimension lda; storage row r of A is read from row a_rows[r]
 // when a_rows is given (a gather of minibatch rows). op(B) is k x n: B is
 // stored k x n (tb = 0) or n x k (tb = 1).
-// One 256-thread workgroup per 64 x 64 tile of C; wave w owns the 32 x 32
-// quarter (w / 2, w % 2) as 2 x 2 v_mfma_f32_16x16x32_bf16 tiles
-// (A[i][8 (l / 16) + e] in element e of lane l, i = l % 16; B likewise with
-// j = l % 16; D register r of lane l = D[4 (l / 16) + r][l % 16]).
+// One 512-thread workgroup per 32 x 32 tile of C as 2 x 2
+// v_mfma_f32_16x16x32_bf16 tiles (A[i][8 (l / 16) + e] in element e of lane
+// l, i = l % 16; B likewise with j = l % 16; D register r of lane l =
+// D[4 (l / 16) + r][l % 16]). The waves take every eighth 32-k step each,
+// operands straight from global memory in that order, and add their tiles up
+// in LDS in a fixed order.
+//
+// Bound by latency at the training sizes (256 x 256 x 288): 64 workgroups of
+// one or two steps per wave, 7 us, where 64 x 64 tiles left 16 workgroups
+// walking nine dependent steps of scalar loads and two barriers, 22 us.
 template <typename TA, typename TB>
-__global__ __launch_bounds__(kT) void mlp_gemm_kernel(GemmArgs g) {
-  __shared__ __align__(16) uint16_t as[kTileM][kPitch];
-  __shared__ __align__(16) uint16_t bs[kTileN][kPitch];
-  const TA* __restrict__ a = (const TA*)g.a;
-  const TB* __restrict__ b = (const TB*)g.b;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int row0 = blockIdx.y * kTileM;
-  const int col0 = blockIdx.x * kTileN;
+__device__ void gemm_tile(const GemmArgs& g, int tile_row, int tile_col) {
+  __shared__ float part[kWaves][4][64][4];
+  __shared__ float sums[kWaves][kTileN];
+  __shared__ float losses[kWaves];
+  const TA* a = (const TA*)g.a;
+  const TB* b = (const TB*)g.b;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int row0 = tile_row * kTileM, col0 = tile_col * kTileN;
+  const bool avec = (((uintptr_t)a | (uintptr_t)g.lda * sizeof(TA)) & 15) == 0;
+  const bool bvec = (((uintptr_t)b | (uintptr_t)g.ldb * sizeof(TB)) & 15) == 0;
+  const bool want_sum = g.bsum != nullptr && tile_row == 0;
   f4 acc[2][2];
+#pragma unroll
   for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
     for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = f4{0.f, 0.f, 0.f, 0.f};
-
-  for (int k0 = 0; k0 < g.k; k0 += kStepK) {
-    // A tile -> as[i][kk] (bf16).
-    if (!g.ta) {
-      const int i = t >> 2, kk = (t & 3) * 8;
-      const int gi = row0 + i;
-      const long long sr = gi < g.m ? (g.a_rows ? g.a_rows[gi] : gi) : 0;
-      for (int e = 0; e < 8; ++e) {
-        const int gk = k0 + kk + e;
-        as[i][kk + e] = (gi < g.m && gk < g.k) ? load_bf16(a + sr * g.lda + gk) : (uint16_t)0;
-      }
-    } else {
-      const int kk = t >> 3, i = (t & 7) * 8;
-      const int gk = k0 + kk;
-      const long long sr = gk < g.k ? (g.a_rows ? g.a_rows[gk] : gk) : 0;
-      for (int e = 0; e < 8; ++e) {
-        const int gi = row0 + i + e;
-        as[i + e][kk] = (gi < g.m && gk < g.k) ? load_bf16(a + sr * g.lda + gi) : (uint16_t)0;
-      }
-    }
-    // B tile -> bs[j][kk] (bf16, transposed so that a lane reads 8 consecutive k).
-    if (!g.tb) {
-      const int kk = t >> 3, j = (t & 7) * 8;
-      const int gk = k0 + kk;
-      for (int e = 0; e < 8; ++e) {
-        const int gj = col0 + j + e;
-        bs[j + e][kk] = (gk < g.k && gj < g.n) ? load_bf16(b + (long long)gk * g.ldb + gj) : (uint16_t)0;
-      }
-    } else {
-      const int j = t >> 2, kk = (t & 3) * 8;
-      const int gj = col0 + j;
-      for (int e = 0; e < 8; ++e) {
-        const int gk = k0 + kk + e;
-        bs[j][kk + e] = (gk < g.k && gj < g.n) ? load_bf16(b + (long long)gj * g.ldb + gk) : (uint16_t)0;
-      }
-    }
-    __syncthreads();
+  float bs[2] = {0.f, 0.f};
+  for (int k0 = wave * 32; k0 < g.k; k0 += kWaves * 32) {
+    const int k = k0 + 8 * (lane >> 4);
     bf8 fa[2], fb[2];
-    for (int mi = 0; mi < 2; ++mi) fa[mi] = lds_bf8(&as[wr * 32 + mi * 16 + (lane & 15)][8 * (lane >> 4)]);
-    for (int ni = 0; ni < 2; ++ni) fb[ni] = lds_bf8(&bs[wc * 32 + ni * 16 + (lane & 15)][8 * (lane >> 4)]);
+    float v[8];
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi) {
+      load8(a, g.lda, g.ta, g.a_rows, row0 + mi * 16 + (lane & 15), g.m, k, g.k, avec, v);
+      fa[mi] = round8(v);
+    }
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni) {
+      load8(b, g.ldb, !g.tb, nullptr, col0 + ni * 16 + (lane & 15), g.n, k, g.k, bvec, v);
+      if (want_sum) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bs[ni] += v[e];
+      }
+      fb[ni] = round8(v);
+    }
+#pragma unroll
     for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
       for (int ni = 0; ni < 2; ++ni)
         acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
-    __syncthreads();
   }
-
+#pragma unroll
   for (int mi = 0; mi < 2; ++mi)
-    for (int ni = 0; ni < 2; ++ni)
-      for (int r = 0; r < 4; ++r) {
-        const int i = row0 + wr * 32 + mi * 16 + 4 * (lane >> 4) + r;
-        const int j = col0 + wc * 32 + ni * 16 + (lane & 15);
-        if (i < g.m && j < g.n) {
-          float v = acc[mi][ni][r];
-          const long long at = (long long)i * g.ldc + j;
-          if (g.accumulate) v += g.c[at];
-          if (g.bias) v += g.bias[j];
-          g.c[at] = v;
-          if (g.h) g.h[at] = silu(v);
-        }
-      }
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni) *(f4*)part[wave][2 * mi + ni][lane] = acc[mi][ni];
+  if (want_sum) {
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni) {
+      bs[ni] += __shfl_xor(bs[ni], 16);
+      bs[ni] += __shfl_xor(bs[ni], 32);
+      if (lane < 16) sums[wave][ni * 16 + lane] = bs[ni];
+    }
+  }
+  __syncthreads();
+  if (want_sum && threadIdx.x < kTileN && col0 + (int)threadIdx.x < g.n) {
+    const int j = threadIdx.x;
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) t += sums[w][j];
+    g.bsum[col0 + j] = t;
+  }
+  // Wave w finishes half (w % 2) of the rows of the 16 x 16 block (w / 4, w / 2 % 2).
+  static_assert(kWaves == 8, "two waves per 16 x 16 block");
+  const int half = 2 * (wave & 1);
+  f2 total = f2{0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) total += *(const f2*)&part[w][wave >> 1][lane][half];
+  const int j = col0 + (wave >> 1 & 1) * 16 + (lane & 15);
+  float loss = 0.f;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int i = row0 + (wave >> 2) * 16 + 4 * (lane >> 4) + half + r;
+    if (i >= g.m || j >= g.n) continue;
+    float v = total[r];
+    const long long at = (long long)i * g.ldc + j;
+    if (g.accumulate) v += g.c[at];
+    if (g.bias) v += g.bias[j];
+    if (g.slope) v *= silu_slope(g.slope[at]);
+    g.c[at] = v;
+    if (g.h) g.h[at] = silu(v);
+    if (g.tgt) {
+      const long long tr = g.t_rows ? g.t_rows[i] : i;
+      const float d = v - g.tgt[tr * g.ldt + j];
+      const float wj = g.w ? g.w[j] : 1.0f;
+      loss += wj * d * d;
+      g.grad[at] = 2.0f * g.scale * wj * d;
+    }
+  }
+  if (g.tgt) {
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+    if (lane == 0) losses[wave] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      g.loss_part[tile_row * ((g.n + kTileN - 1) / kTileN) + tile_col] =
+          ((losses[0] + losses[1]) + (losses[2] + losses[3])) + ((losses[4] + losses[5]) + (losses[6] + losses[7]));
+  }
+}
+
+template <typename TA, typename TB>
+__global__ __launch_bounds__(kGemmT) void mlp_gemm_kernel(GemmArgs g) {
+  const int cols = (g.n + kTileN - 1) / kTileN;
+  gemm_tile<TA, TB>(g, blockIdx.x / cols, blockIdx.x % cols);
+}
+
+// One layer of the backward pass: the weight and bias gradients (tiles below
+// split) and the gradient of the layer's input, both of the same dz: 7 us in
+// one launch, where the two products, the column sum and the SiLU backward
+// took 22 + 22 + 7 + 3 us in four.
+__global__ __launch_bounds__(kGemmT) void mlp_backward_kernel(GemmArgs weights, GemmArgs input, int split) {
+  int t = blockIdx.x;
+  if (t < split) {
+    const int cols = (weights.n + kTileN - 1) / kTileN;
+    gemm_tile<float, float>(weights, t / cols, t % cols);
+  } else {
+    t -= split;
+    const int cols = (input.n + kTileN - 1) / kTileN;
+    gemm_tile<float, uint16_t>(input, t / cols, t % cols);
+  }
 }
 
 // grad_z = grad_h * silu'(z), silu'(z) = s (1 + z (1 - s)), s = 1 / (1 + e^-z).
 __global__ __launch_bounds__(kT) void silu_backward_kernel(long long count, const float* __restrict__ grad_h,
                                                            const float* __restrict__ z, float* __restrict__ grad_z) {
   for (long long e = (long long)blockIdx.x * kT + threadIdx.x; e < count; e += (long long)gridDim.x * kT) {
-    const float x = z[e];
-    const float s = 1.0f / (1.0f + expf(-x));
-    grad_z[e] = grad_h[e] * (s * (1.0f + x * (1.0f - s)));
+    grad_z[e] = grad_h[e] * silu_slope(z[e]);
   }
 }
 
@@ -202,7 +309,15 @@ __global__ __launch_bounds__(kT) void adam_kernel(long long count, float* __rest
                                                   float* __restrict__ m1, float* __restrict__ m2,
                                                   uint16_t* __restrict__ p16, float lr_t, float beta1,
                                                   float one_minus_beta1, float beta2, float one_minus_beta2,
-                                                  float eps, float decay) {
+                                                  float eps, float decay, const float* __restrict__ loss_part,
+                                                  int nparts, float scale, float* __restrict__ loss) {
+  // The training step's loss, from the parts of the output tiles in a fixed order.
+  if (loss_part != nullptr && blockIdx.x == 0 && threadIdx.x < 64) {
+    float s = 0.f;
+    for (int i = threadIdx.x; i < nparts; i += 64) s += loss_part[i];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (threadIdx.x == 0) loss[0] = scale * s;
+  }
   for (long long e = (long long)blockIdx.x * kT + threadIdx.x; e < count; e += (long long)gridDim.x * kT) {
     const float gi = g[e];
     const float a = beta1 * m1[e] + one_minus_beta1 * gi;
@@ -249,6 +364,32 @@ int mguard(hfjk_ctx* ctx, F&& body) {
   }
 }
 
+// Float offsets of a training step's workspace: every layer's z and dz, the
+// hidden layers' h, the loss parts of the output tiles.
+constexpr int kMaxLayers = 16;
+struct TrainLayout {
+  long long z[kMaxLayers], h[kMaxLayers], dz[kMaxLayers], loss, total;
+};
+
+TrainLayout train_layout(int layers, const int* sizes, int m) {
+  TrainLayout L{};
+  long long at = 0;
+  auto take = [&](long long n) {
+    const long long here = at;
+    at += (n + 63) / 64 * 64;
+    return here;
+  };
+  for (int l = 0; l < layers && l < kMaxLayers; ++l) {
+    const long long n = (long long)m * sizes[l + 1];
+    L.z[l] = take(n);
+    if (l + 1 < layers) L.h[l] = take(n);
+  }
+  for (int l = 0; l < layers && l < kMaxLayers; ++l) L.dz[l] = take((long long)m * sizes[l + 1]);
+  L.loss = take((long long)((m + kTileM - 1) / kTileM) * ((sizes[layers] + kTileN - 1) / kTileN));
+  L.total = at;
+  return L;
+}
+
 }  // namespace
 
 extern "C" {
@@ -264,19 +405,35 @@ int hfjk_mlp_gemm(hfjk_ctx* ctx, int m, int n, int k, const void* a, int a_bf16,
     if (lda < (trans_a ? m : k) || ldb < (trans_b ? k : n) || ldc < n)
       mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: a leading dimension is smaller than its row");
     if (h_silu == c) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: the activation output must not alias C");
-    GemmArgs g{m, n, k, a, lda, trans_a ? 1 : 0, a_rows, b, ldb, trans_b ? 1 : 0, bias, c, ldc, accumulate ? 1 : 0,
-               h_silu};
-    dim3 grid((n + kTileN - 1) / kTileN, (m + kTileM - 1) / kTileM);
-    if (grid.y > 65535u) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: more than 4194240 rows");
+    if (m > 65535 * 64) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: more than 4194240 rows");
+    GemmArgs g{};
+    g.m = m;
+    g.n = n;
+    g.k = k;
+    g.a = a;
+    g.lda = lda;
+    g.ta = trans_a ? 1 : 0;
+    g.a_rows = a_rows;
+    g.b = b;
+    g.ldb = ldb;
+    g.tb = trans_b ? 1 : 0;
+    g.bias = bias;
+    g.c = c;
+    g.ldc = ldc;
+    g.accumulate = accumulate ? 1 : 0;
+    g.h = h_silu;
+    const long long cols = (n + kTileN - 1) / kTileN, rows = (m + kTileM - 1) / kTileM;
+    if (cols * rows > 0x7FFFFFFFLL) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: too many output tiles");
+    const dim3 grid((unsigned)(cols * rows));
     hipStream_t s = (hipStream_t)stream;
     if (a_bf16 && b_bf16)
-      hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, uint16_t>), grid, dim3(kT), 0, s, g);
+      hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, uint16_t>), grid, dim3(kGemmT), 0, s, g);
     else if (a_bf16)
-      hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, float>), grid, dim3(kT), 0, s, g);
+      hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, float>), grid, dim3(kGemmT), 0, s, g);
     else if (b_bf16)
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), grid, dim3(kT), 0, s, g);
+      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), grid, dim3(kGemmT), 0, s, g);
     else
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, float>), grid, dim3(kT), 0, s, g);
+      hipLaunchKernelGGL((mlp_gemm_kernel<float, float>), grid, dim3(kGemmT), 0, s, g);
     mcheck(hipGetLastError(), "mlp_gemm launch");
   });
 }
@@ -328,7 +485,110 @@ int hfjk_mlp_adam(hfjk_ctx* ctx, long long count, float* params, const float* gr
     if (count == 0) return;
     hipLaunchKernelGGL(adam_kernel, dim3(hfjk::grid_for(count)), dim3(kT), 0, (hipStream_t)stream, count, params,
                        grads, moment1, moment2, params_bf16, (float)lr_t, (float)beta1, (float)(1.0 - beta1),
-                       (float)beta2, (float)(1.0 - beta2), (float)eps, (float)(lr * weight_decay));
+                       (float)beta2, (float)(1.0 - beta2), (float)eps, (float)(lr * weight_decay),
+                       (const float*)nullptr, 0, 0.0f, (float*)nullptr);
+    mcheck(hipGetLastError(), "adam launch");
+  });
+}
+
+long long hfjk_mlp_train_workspace(int layers, const int* sizes, int m) {
+  if (layers < 1 || layers > kMaxLayers || sizes == nullptr || m < 0) return 0;
+  return train_layout(layers, sizes, m).total;
+}
+
+int hfjk_mlp_train_step(hfjk_ctx* ctx, int layers, const int* sizes, int m, const float* x, const int* rows,
+                        const float* target, int ldt, const float* col_weights, double scale, float* params,
+                        uint16_t* params_bf16, float* grads, float* moment1, float* moment2, double lr, double lr_t,
+                        double beta1, double beta2, double eps, double weight_decay, float* workspace, float* loss,
+                        void* stream) {
+  return mguard(ctx, [&] {
+    if (layers < 1 || layers > kMaxLayers || sizes == nullptr || m < 1)
+      mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: 1 to 16 layers and at least one row are required");
+    for (int l = 0; l <= layers; ++l)
+      if (sizes[l] < 1) mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: layer sizes are positive");
+    if (x == nullptr || target == nullptr || params == nullptr || params_bf16 == nullptr || grads == nullptr ||
+        moment1 == nullptr || moment2 == nullptr || workspace == nullptr || loss == nullptr || ldt < sizes[layers])
+      mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: null buffer or a target narrower than the output");
+    if (!(beta1 >= 0.0 && beta1 < 1.0 && beta2 >= 0.0 && beta2 < 1.0 && eps >= 0.0))
+      mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: betas in [0, 1) and eps >= 0 are required");
+    hipStream_t s = (hipStream_t)stream;
+    const TrainLayout L = train_layout(layers, sizes, m);
+    auto tiles = [](int v) { return (v + kTileM - 1) / kTileM; };
+    static_assert(kTileM == kTileN, "square tiles");
+    for (int l = 0; l <= layers; ++l)
+      if ((long long)tiles(m) * tiles(sizes[l]) > (1 << 29) ||
+          (long long)tiles(sizes[l]) * tiles(sizes[std::min(l + 1, layers)]) > (1 << 29))
+        mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: too many output tiles");
+    long long at[kMaxLayers + 1] = {0};  // W [k][n], then b [n], of every layer
+    for (int l = 0; l < layers; ++l) at[l + 1] = at[l] + (long long)sizes[l] * sizes[l + 1] + sizes[l + 1];
+    const int out = layers - 1;
+    for (int l = 0; l < layers; ++l) {
+      const int k = sizes[l], n = sizes[l + 1];
+      GemmArgs g{};
+      g.m = m;
+      g.n = n;
+      g.k = k;
+      g.a = l == 0 ? (const void*)x : (const void*)(workspace + L.h[l - 1]);
+      g.lda = k;
+      g.a_rows = l == 0 ? rows : nullptr;
+      g.b = params_bf16 + at[l];
+      g.ldb = n;
+      g.bias = params + at[l] + (long long)k * n;
+      g.c = workspace + L.z[l];
+      g.ldc = n;
+      if (l < out) {
+        g.h = workspace + L.h[l];
+      } else {
+        g.tgt = target;
+        g.ldt = ldt;
+        g.t_rows = rows;
+        g.w = col_weights;
+        g.scale = (float)scale;
+        g.grad = workspace + L.dz[l];
+        g.loss_part = workspace + L.loss;
+      }
+      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), dim3(tiles(n) * tiles(m)), dim3(kGemmT), 0, s, g);
+      mcheck(hipGetLastError(), "mlp forward launch");
+    }
+    for (int l = out; l >= 0; --l) {
+      const int k = sizes[l], n = sizes[l + 1];
+      GemmArgs w{};
+      w.m = k;
+      w.n = n;
+      w.k = m;
+      w.a = l == 0 ? (const void*)x : (const void*)(workspace + L.h[l - 1]);
+      w.lda = k;
+      w.ta = 1;
+      w.a_rows = l == 0 ? rows : nullptr;
+      w.b = workspace + L.dz[l];
+      w.ldb = n;
+      w.c = grads + at[l];
+      w.ldc = n;
+      w.bsum = grads + at[l] + (long long)k * n;
+      const int split = tiles(k) * tiles(n);
+      GemmArgs d{};
+      if (l > 0) {
+        d.m = m;
+        d.n = k;
+        d.k = n;
+        d.a = workspace + L.dz[l];
+        d.lda = n;
+        d.b = params_bf16 + at[l];
+        d.ldb = n;
+        d.tb = 1;
+        d.c = workspace + L.dz[l - 1];
+        d.ldc = k;
+        d.slope = workspace + L.z[l - 1];
+      }
+      const int grid = split + (l > 0 ? tiles(m) * tiles(k) : 0);
+      hipLaunchKernelGGL(mlp_backward_kernel, dim3(grid), dim3(kGemmT), 0, s, w, d, split);
+      mcheck(hipGetLastError(), "mlp backward launch");
+    }
+    const long long count = at[layers];
+    hipLaunchKernelGGL(adam_kernel, dim3(hfjk::grid_for(count)), dim3(kT), 0, s, count, params, grads, moment1,
+                       moment2, params_bf16, (float)lr_t, (float)beta1, (float)(1.0 - beta1), (float)beta2,
+                       (float)(1.0 - beta2), (float)eps, (float)(lr * weight_decay), workspace + L.loss,
+                       tiles(m) * tiles(sizes[layers]), (float)scale, loss);
     mcheck(hipGetLastError(), "adam launch");
   });
 }

@@ -47,6 +47,7 @@ class Mlp:
             self.offsets.append((at, at + k * n))  # W [k, n], then b [n]
             at += k * n + n
         self.n_params = at
+        self._c_sizes = (ctypes.c_int * len(self.sizes))(*self.sizes)
         self.params = torch.zeros(at, dtype=torch.float32, device=self.device)
         self.params16 = torch.zeros(at, dtype=torch.bfloat16, device=self.device)
         self.grads = torch.zeros(at, dtype=torch.float32, device=self.device)
@@ -149,7 +150,7 @@ class Mlp:
     def backward(self, grad_out) -> None:
         """Parameter gradients (into ``self.grads``) from ``d loss / d outputs`` of the last kept forward."""
         torch = _torch()
-        acts, gather, m = self._acts
+        acts, gather, m = self._kept()
         dz = grad_out
         for index in range(len(self.offsets) - 1, -1, -1):
             k, n = self.sizes[index], self.sizes[index + 1]
@@ -193,12 +194,46 @@ class Mlp:
                                            self._stream()))
 
     def train_step(self, x, target, rows, *, lr: float, col_weights=None, weight_decay: float = 0.0):
-        """One minibatch step (forward, mean weighted squared error, backward, Adam); returns the device loss."""
+        """One minibatch step (forward, mean weighted squared error, backward, Adam); returns the device loss.
+
+        One call into the library: a launch per layer and direction, the loss inside the output
+        layer's, the bias sums and the SiLU slopes inside the gradients' (an empty minibatch and
+        more than 16 layers take the separate calls)."""
         torch = _torch()
-        m, _ = self._rows(x, rows)
-        y = self.forward(x, rows, keep=True)
-        grad = torch.empty_like(y)
-        loss = self.loss(y, target, rows, col_weights, 1.0 / max(m, 1), grad)
-        self.backward(grad)
-        self.adam(lr, weight_decay=weight_decay)
-        return loss
+        m, gather = self._rows(x, rows)
+        layers = len(self.offsets)
+        if m == 0 or layers > 16:
+            y = self.forward(x, rows, keep=True)
+            grad = torch.empty_like(y)
+            loss = self.loss(y, target, rows, col_weights, 1.0 / max(m, 1), grad)
+            self.backward(grad)
+            self.adam(lr, weight_decay=weight_decay)
+            return loss
+        floats = self.lib.hfjk_mlp_train_workspace(layers, self._c_sizes, m)
+        work = torch.empty(floats, dtype=torch.float32, device=self.device)
+        self.step_count += 1
+        beta1, beta2, t = 0.9, 0.999, self.step_count
+        lr_t = lr * math.sqrt(1.0 - beta2 ** t) / (1.0 - beta1 ** t)
+        self._check(self.lib.hfjk_mlp_train_step(
+            self._ctx.handle, layers, self._c_sizes, m, _ptr(x),
+            None if gather is None else self._addr(gather[0], gather[1]), _ptr(target), target.shape[1],
+            None if col_weights is None else _ptr(col_weights), 1.0 / m, _ptr(self.params), _ptr(self.params16),
+            _ptr(self.grads), _ptr(self.moment1), _ptr(self.moment2), float(lr), float(lr_t), beta1, beta2, 1e-8,
+            float(weight_decay), _ptr(work), _ptr(self._loss), self._stream()))
+        self._acts = (None, gather, m)
+        self._work = (work, x)
+        return self._loss
+
+    def _kept(self):
+        """The last kept forward: every layer's input and z, its row indices and their count."""
+        acts, gather, m = self._acts
+        if acts is None:  # in the workspace of a training step: z of every layer, h of the hidden ones after it
+            work, h = self._work
+            acts, at = [], 0
+            for n in self.sizes[1:]:
+                z = work[at:at + m * n].view(m, n)
+                acts.append((h, z))
+                at += -(-m * n // 64) * 64
+                h = work[at:at + m * n].view(m, n) if len(acts) < len(self.offsets) else None
+                at += -(-m * n // 64) * 64
+        return acts, gather, m

@@ -507,6 +507,24 @@ HFJK_API int hfjk_mlp_mse(hfjk_ctx *ctx, int m, int n, const float *y, int ldy, 
 HFJK_API int hfjk_mlp_adam(hfjk_ctx *ctx, long long count, float *params, const float *grads, float *moment1,
                            float *moment2, uint16_t *params_bf16, double lr, double lr_t, double beta1,
                            double beta2, double eps, double weight_decay, void *stream);
+/* One minibatch step over layers (1 to 16) dense layers sizes[0..layers],
+ * hidden ones with SiLU: forward on rows rows[0..m) of x [.][sizes[0]] (NULL:
+ * the first m rows), the loss scale sum w_j (y_ij - t_ij)^2 against the same
+ * rows of target into loss[0], the gradients of every parameter into grads,
+ * and the Adam update of hfjk_mlp_adam. Parameters, their bf16 copy,
+ * gradients and moments hold W [k][n] and then b [n] layer by layer. The
+ * results are those of the separate calls up to the order of the FP32 sums.
+ * workspace: hfjk_mlp_train_workspace floats; afterwards it holds z, h and
+ * dz. */
+HFJK_API int hfjk_mlp_train_step(hfjk_ctx *ctx, int layers, const int *sizes, int m, const float *x, const int *rows,
+                                 const float *target, int ldt, const float *col_weights, double scale, float *params,
+                                 uint16_t *params_bf16, float *grads, float *moment1, float *moment2, double lr,
+                                 double lr_t, double beta1, double beta2, double eps, double weight_decay,
+                                 float *workspace, float *loss, void *stream);
+/* Floats of that workspace: z of every layer, h of the hidden ones (each
+ * rounded up to 64 floats, z and h of one layer next to each other), then dz
+ * and the loss's parts; 0 for an invalid argument. */
+HFJK_API long long hfjk_mlp_train_workspace(int layers, const int *sizes, int m);
 /* dst = bf16(src) (nearest even) over count elements. */
 HFJK_API int hfjk_mlp_to_bf16(hfjk_ctx *ctx, long long count, const float *src, uint16_t *dst, void *stream);
 

@@ -160,3 +160,42 @@ def test_training_fits_a_teacher_network():
             net.train_step(xd, td, (perm, lo, lo + 128), lr=3e-3)
     last = float(net.loss(net.forward(xd, (all_rows, 0, 2048)), td).item()) / 2048
     assert last < 0.05 * first
+
+
+@pytest.mark.parametrize("m", [1, 33, 200])
+@pytest.mark.parametrize("sizes", [[5, 3], [72, 96, 80, 13], [31, 33, 64, 65], [40, 256, 8]])
+def test_training_step_is_the_separate_calls(sizes, m):
+    """Tiles of 32, k split over eight waves of 32: sizes on both sides of each, operands off 16-byte lines."""
+    torch = _torch()
+    from hafnium_amd.mlp import Mlp
+
+    rng = np.random.default_rng(60 + m + len(sizes))
+    fused, split = Mlp(sizes, seed=4), Mlp(sizes, seed=4)
+    dev = fused.device
+    x = torch.from_numpy(rng.standard_normal((m + 7, sizes[0])).astype(np.float32)).to(dev)
+    t = torch.from_numpy(rng.standard_normal((m + 7, sizes[-1])).astype(np.float32)).to(dev)
+    w = torch.from_numpy(rng.uniform(0.5, 2.0, sizes[-1]).astype(np.float32)).to(dev)
+    perm = torch.from_numpy(rng.permutation(m + 7).astype(np.int32)).to(dev)
+    rows = (perm, 3, 3 + m)
+    loss = fused.train_step(x, t, rows, lr=1e-2, col_weights=w, weight_decay=1e-2)
+    y = split.forward(x, rows, keep=True)
+    grad = torch.empty_like(y)
+    loss_ref = split.loss(y, t, rows, w, 1.0 / m, grad)
+    split.backward(grad)
+    split.adam(1e-2, weight_decay=1e-2)
+    torch.cuda.synchronize()
+    # Same operands and products; the slopes multiply before the store instead of
+    # after it. Only sums over at most 256 FP32 terms in another order differ.
+    assert float(loss.item()) == pytest.approx(float(loss_ref.item()), rel=1e-5)
+    for (dw, db), (dw_ref, db_ref) in zip(fused.gradients(), split.gradients()):
+        assert np.abs(dw - dw_ref).max() <= GEMM_REL_TOL * max(np.abs(dw_ref).max(), 1e-30)
+        assert np.abs(db - db_ref).max() <= GEMM_REL_TOL * max(np.abs(db_ref).max(), 1e-30)
+    # A step of Adam is lr_t m1 / (sqrt(m2) + eps): its sensitivity to the gradient is checked on the moments.
+    np.testing.assert_allclose(fused.moment1.cpu().numpy(), 0.1 * fused.grads.cpu().numpy(), rtol=1e-6)
+    np.testing.assert_array_equal(fused.params16.float().cpu().numpy(),
+                                  mlp_ref.bf16_round(fused.params.cpu().numpy()).astype(np.float32))
+    # The kept activations serve a further backward pass, as the separate calls' do.
+    for (h, z), (h_ref, z_ref) in zip(fused._kept()[0], split._kept()[0]):
+        for got, want in ((h, h_ref), (z, z_ref)):
+            assert got.shape == want.shape
+            assert (got - want).abs().max().item() <= GEMM_REL_TOL * max(want.abs().max().item(), 1e-30)
