@@ -1,10 +1,10 @@
-// Batched DF-J/K: many instances of uneven size in one persistent launch
-// per phase (charges, Coulomb, orbitals, half-transform, SYRK, reductions).
+// Batched DF-J/K: many instances of uneven size in one launch per phase
+// (charges, Coulomb, orbitals, half-transform, SYRK, reductions).
 //
 // A plan (hfjk_batch_create) derives every instance's shapes, splits and
 // buffer offsets on the host; hfjk_batch_bind uploads it once into the
 // caller's workspace; hfjk_batch_run only enqueues kernels (a counter reset
-// kernel and one persistent kernel per phase), so a run can be captured in a
+// kernel and one kernel per phase, persistent where the items are uneven), so a run can be captured in a
 // hipGraph and replayed.
 #include <algorithm>
 #include <cmath>
@@ -28,13 +28,17 @@ struct hfjk_batch {
   size_t off_insts = 0, off_prefix = 0, off_counters = 0, off_ws64 = 0, off_cp = 0, off_x = 0, off_kp = 0;
   size_t bytes = 0;
   void* ws = nullptr;
-  int grid_mfma = 0, grid_elem = 0;
+  int grid_mfma = 0;
 };
 
 namespace hfjk {
 namespace {
 
 constexpr int kGammaQb = 64;
+constexpr long long kMaxGrid = 1 << 20;
+
+// Aux functions of one item of b_charges_x_kernel.
+constexpr int charges_per_item(int precision) { return precision == HFJK_BF16X3 ? 8 : 4; }
 
 template <int PREC>
 __device__ __forceinline__ void bload4(const void* b, long long plane, long long off, double out[4]) {
@@ -84,14 +88,15 @@ __global__ __launch_bounds__(kThreads) void reset_kernel(unsigned long long* cou
   for (int i = threadIdx.x; i < n; i += kThreads) counters[i] = 0ull;
 }
 
-#define BATCH_LOOP(PHASE)                                                           \
-  const long long* pre = v.prefix + (long long)(PHASE) * (v.ninst + 1);             \
-  for (;;) {                                                                        \
-    long long end;                                                                  \
-    const long long item = batch_next(v.prefix, v.counters, v.ninst, (PHASE), end); \
-    if (item >= end) break;                                                         \
-    const int inst = batch_find(pre, v.ninst, item);                                \
-    const BatchInst in = v.insts[inst];                                             \
+// Phases whose items are uniform: one item per workgroup, dealt by the
+// hardware (grids are capped at kMaxGrid and stride). Pulling them from the
+// per-XCD counters cost 0.1 ms a phase by itself: every workgroup's last
+// visits to the eight counters are serial atomics.
+#define BATCH_LOOP(PHASE)                                                                          \
+  const long long* pre = v.prefix + (long long)(PHASE) * (v.ninst + 1);                            \
+  for (long long item = blockIdx.x; item < v.items[PHASE]; item += gridDim.x) {                    \
+    const int inst = batch_find(pre, v.ninst, item);                                               \
+    const BatchInst in = v.insts[inst];                                                            \
     const long long local = item - pre[inst];
 
 #define BATCH_END }
@@ -132,12 +137,16 @@ __global__ __launch_bounds__(kThreads) void b_gamma_kernel(BatchView v, const vo
   const double w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
   const int qn = min(kGammaQb, in.naux - q0);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int qi = 0; qi < qn; ++qi) {
-    double bv[4];
-    bload4<PREC>(b, plane, in.b_off + (long long)(q0 + qi) * in.p + e, bv);
-    double s = bv[0] * w0 + bv[1] * w1 + bv[2] * w2 + bv[3] * w3;
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if (lane == 0) red[wave][qi] = s;
+  for (int qi = 0; qi < qn; qi += 8) {
+    double s[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      double bv[4];
+      bload4<PREC>(b, plane, in.b_off + (long long)(q0 + min(qi + x, qn - 1)) * in.p + e, bv);
+      s[x] = bv[0] * w0 + bv[1] * w1 + bv[2] * w2 + bv[3] * w3;
+    }
+    const double total = wave_sums8(s, lane);
+    if ((lane & 7) == 0) red[wave][qi + (lane >> 3)] = total;
   }
   __syncthreads();
   if ((int)threadIdx.x < qn)
@@ -147,44 +156,57 @@ __global__ __launch_bounds__(kThreads) void b_gamma_kernel(BatchView v, const vo
   BATCH_END
 }
 
-// gamma[q] = sum over tiles, 256 aux functions per item.
+// gamma[q] = sum over tiles, 64 aux functions per item: wave g sums every
+// fourth tile.
 __global__ __launch_bounds__(kThreads) void b_gamma_reduce_kernel(BatchView v, double* __restrict__ ws64) {
+  __shared__ double red[kThreads / 64][64];
   BATCH_LOOP(kPhGammaReduce)
-  const int q = (int)local * kThreads + threadIdx.x;
-  if (q < in.naux) {
-    const long long ntiles = in.p / kTileElems;
-    double s = 0.0;
-    for (long long t = 0; t < ntiles; ++t) s += ws64[in.gp_off + t * in.naux + q];
-    ws64[in.g_off + q] = s;
-  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int q = (int)local * 64 + lane;
+  const long long ntiles = in.p / kTileElems;
+  const double* gp = ws64 + in.gp_off + min(q, in.naux - 1);
+  double s = 0.0;
+#pragma unroll 4
+  for (long long t = wave; t < ntiles; t += kThreads / 64) s += gp[t * in.naux];
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && q < in.naux) ws64[in.g_off + q] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+  __syncthreads();
   BATCH_END
 }
 
-// gamma[q] from a caller's flat charge vector (instance i at q_off), 256 per item.
+// gamma[q] from a caller's flat charge vector (instance i at q_off), 64 per item.
 __global__ __launch_bounds__(kThreads) void b_charges_load_kernel(BatchView v, const double* __restrict__ charges,
                                                                   double* __restrict__ ws64) {
   BATCH_LOOP(kPhGammaReduce)
-  const int q = (int)local * kThreads + threadIdx.x;
-  if (q < in.naux) ws64[in.g_off + q] = charges[in.q_off + q];
+  const int q = (int)local * 64 + threadIdx.x;
+  if (threadIdx.x < 64 && q < in.naux) ws64[in.g_off + q] = charges[in.q_off + q];
   BATCH_END
 }
 
 // gamma[q] = <B[q], C C^T> = sum_{mu < nao, i < nocc} C[mu][i] X[q][mu][i] from the
 // half-transformed X of the exchange (mode layout; BF16X3: hi + lo planes)
-// and the caller's FP64 orbitals, one aux function per item. The rows
-// [0, nao) of X[q] are one contiguous range of nao * ldo elements, streamed
-// in 16-byte groups (ldo is a multiple of 32, so no group straddles two
-// rows); columns past nocc are skipped (X is zero there).
+// and the caller's FP64 orbitals, charges_per_item aux functions per item.
+// The rows [0, nao) of X[q] are one contiguous range of nao * ldo elements,
+// streamed in 16-byte groups (ldo is a multiple of 32, so no group straddles
+// two rows); columns past nocc are skipped (X is zero there). Bound by the
+// pass over X: an item's aux functions share the loads of C, which at one
+// aux function per item were 8 bytes from the cache for every 4 (BF16X3) or
+// 8 bytes of X (128 BF16x3 instances to 220 functions: 3.31 -> 1.32 ms).
 template <int PREC>
 __global__ __launch_bounds__(kThreads) void b_charges_x_kernel(BatchView v, const double* __restrict__ c,
                                                                const void* __restrict__ xbase, long long x_plane,
                                                                double* __restrict__ ws64) {
   constexpr int V = PREC == HFJK_FP64 ? 2 : PREC == HFJK_FP32 ? 4 : 8;  // elements per 16-byte group
-  __shared__ double red[kThreads / 64];
+  constexpr int QB = charges_per_item(PREC);
+  __shared__ double red[kThreads / 64][8];
   BATCH_LOOP(kPhCharges)
   const double* ci = c + in.c_off;
-  const long long xq = in.x_off + local * in.xrows * in.ldo;
-  double s = 0.0;
+  const int q0 = (int)local * QB;
+  const long long xstride = (long long)in.xrows * in.ldo;
+  double s[8];
+#pragma unroll
+  for (int x = 0; x < 8; ++x) s[x] = 0.0;
   const int per_row = in.ldo / V;
   const int groups = in.nao * per_row;
   // Group g = mu * per_row + gi, stepped by the block size without a division.
@@ -193,36 +215,43 @@ __global__ __launch_bounds__(kThreads) void b_charges_x_kernel(BatchView v, cons
   for (int g = threadIdx.x; g < groups; g += kThreads) {
     const int i0 = gi * V;
     if (i0 < in.nocc) {
-      const long long at = xq + (long long)mu * in.ldo + i0;
-      float xf[V];
-      double xd[V];
-      if constexpr (PREC == HFJK_FP64) {
-        const double2 w = *(const double2*)((const double*)xbase + at);
-        xd[0] = w.x;
-        xd[1] = w.y;
-      } else if constexpr (PREC == HFJK_FP32) {
-        const float4 w = *(const float4*)((const float*)xbase + at);
-        xf[0] = w.x;
-        xf[1] = w.y;
-        xf[2] = w.z;
-        xf[3] = w.w;
-      } else {
-        const uint16_t* xh = (const uint16_t*)xbase;
-        const uint4 h = *(const uint4*)(xh + at);
-        const uint4 l = *(const uint4*)(xh + at + x_plane);
-        const uint32_t hw[4] = {h.x, h.y, h.z, h.w}, lw[4] = {l.x, l.y, l.z, l.w};
+      const long long at = in.x_off + (long long)mu * in.ldo + i0;
+      uint4 w[QB], wl[PREC == HFJK_BF16X3 ? QB : 1];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t sh = (e & 1) * 16;
-          xf[e] = __uint_as_float(((hw[e >> 1] >> sh) & 0xFFFFu) << 16) +
-                  __uint_as_float(((lw[e >> 1] >> sh) & 0xFFFFu) << 16);
+      for (int x = 0; x < QB; ++x) {
+        const long long here = at + min(q0 + x, in.naux - 1) * xstride;
+        if constexpr (PREC == HFJK_FP64) {
+          w[x] = *(const uint4*)((const double*)xbase + here);
+        } else if constexpr (PREC == HFJK_FP32) {
+          w[x] = *(const uint4*)((const float*)xbase + here);
+        } else {
+          w[x] = *(const uint4*)((const uint16_t*)xbase + here);
+          wl[x] = *(const uint4*)((const uint16_t*)xbase + here + x_plane);
         }
       }
-      const double* crow = ci + (long long)mu * in.nocc;
+      const double* crow = ci + (long long)mu * in.nocc + i0;
+      double cv[V];
 #pragma unroll
-      for (int e = 0; e < V; ++e) {
-        const double x = PREC == HFJK_FP64 ? xd[e] : (double)xf[e];
-        if (i0 + e < in.nocc) s += crow[i0 + e] * x;
+      for (int e = 0; e < V; ++e) cv[e] = crow[min(e, in.nocc - 1 - i0)];
+#pragma unroll
+      for (int x = 0; x < QB; ++x) {
+        const uint32_t hw[4] = {w[x].x, w[x].y, w[x].z, w[x].w};
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          double xe;
+          if constexpr (PREC == HFJK_FP64) {
+            xe = __hiloint2double((int)hw[2 * e + 1], (int)hw[2 * e]);
+          } else if constexpr (PREC == HFJK_FP32) {
+            xe = (double)__uint_as_float(hw[e]);
+          } else {
+            const uint4& l = wl[x];
+            const uint32_t lw[4] = {l.x, l.y, l.z, l.w};
+            const uint32_t sh = (e & 1) * 16;
+            xe = (double)(__uint_as_float(((hw[e >> 1] >> sh) & 0xFFFFu) << 16) +
+                          __uint_as_float(((lw[e >> 1] >> sh) & 0xFFFFu) << 16));
+          }
+          if (i0 + e < in.nocc) s[x] += cv[e] * xe;
+        }
       }
     }
     mu += dm;
@@ -232,45 +261,81 @@ __global__ __launch_bounds__(kThreads) void b_charges_x_kernel(BatchView v, cons
       ++mu;
     }
   }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  const int lane = threadIdx.x & 63;
+  const double total = wave_sums8(s, lane);
+  if ((lane & 7) == 0) red[threadIdx.x >> 6][lane >> 3] = total;
   __syncthreads();
-  if (threadIdx.x == 0) ws64[in.g_off + local] = red[0] + red[1] + red[2] + red[3];
+  const int x = threadIdx.x;
+  if (x < QB && q0 + x < in.naux) ws64[in.g_off + q0 + x] = red[0][x] + red[1][x] + red[2][x] + red[3][x];
   __syncthreads();
   BATCH_END
 }
 
-// Packed J of one tile: sum_q gamma[q] B[q][tile], one tile per item.
+// Part of the packed J of one tile: sum over the jq aux functions of the
+// item's slice of gamma[q] B[q][tile], eight of them in flight. The slices
+// give a batch of few tiles enough workgroups (12 water clusters, 480 tiles:
+// 0.88 ms in one slice, 0.39 ms in slices of 64; 128 BF16x3 instances to 220
+// functions 3.71 -> 3.26 ms, 4.7 TB/s).
 template <int PREC>
 __global__ __launch_bounds__(kThreads) void b_coulomb_kernel(BatchView v, const void* __restrict__ b, long long plane,
                                                              double* __restrict__ ws64) {
   BATCH_LOOP(kPhCoulomb)
-  const long long e = local * kTileElems + threadIdx.x * 4;
+  const long long ntiles = in.p / kTileElems;
+  const int slice = (int)(local / ntiles);
+  const long long e = (local - slice * ntiles) * kTileElems + threadIdx.x * 4;
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   const double* g = ws64 + in.g_off;
-  for (int q = 0; q < in.naux; ++q) {
+  const int q1 = min((slice + 1) * in.jq, in.naux);
+  int q = slice * in.jq;
+  for (; q + 8 <= q1; q += 8) {
+    double bv[8][4];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) bload4<PREC>(b, plane, in.b_off + (long long)(q + x) * in.p + e, bv[x]);
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const double gq = g[q + x];
+      for (int k = 0; k < 4; ++k) acc[k] += gq * bv[x][k];
+    }
+  }
+  for (; q < q1; ++q) {
     double bv[4];
     bload4<PREC>(b, plane, in.b_off + (long long)q * in.p + e, bv);
     const double gq = g[q];
     for (int k = 0; k < 4; ++k) acc[k] += gq * bv[k];
   }
-  double* jp = ws64 + in.jp_off + e;
+  double* jp = ws64 + in.jp_off + (long long)slice * in.p + e;
   for (int k = 0; k < 4; ++k) jp[k] = acc[k];
   BATCH_END
 }
 
-// J [nao][nao] from the packed J, 256 elements per item.
+// J [nao][nao] from the slices of the packed J, one tile per item: the tile
+// and, through LDS, its mirror.
 __global__ __launch_bounds__(kThreads) void b_coulomb_unpack_kernel(BatchView v, const double* __restrict__ ws64,
                                                                     double* __restrict__ j) {
+  __shared__ double tile[kTile][kTile + 1];
   BATCH_LOOP(kPhCoulombUnpack)
-  const long long idx = local * kThreads + threadIdx.x;
-  if (idx < (long long)in.nao * in.nao) {
-    const int row = (int)(idx / in.nao), col = (int)(idx % in.nao);
-    const int r = row / kTile, c = col / kTile;
-    const long long src = r >= c ? tix(r, c) * kTileElems + (row % kTile) * kTile + col % kTile
-                                 : tix(c, r) * kTileElems + (col % kTile) * kTile + row % kTile;
-    j[in.d_off + idx] = ws64[in.jp_off + src];
+  int r, c;
+  rc_of((int)local, r, c);
+  const double* jp = ws64 + in.jp_off + local * kTileElems + threadIdx.x * 4;
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (int slice = 0; slice < in.jsplit; ++slice)
+    for (int k = 0; k < 4; ++k) sum[k] += jp[(long long)slice * in.p + k];
+  double* ji = j + in.d_off;
+  const int tr = threadIdx.x / 8, tc = threadIdx.x % 8 * 4;
+  for (int k = 0; k < 4; ++k) {
+    const int row = r * kTile + tr, col = c * kTile + tc + k;
+    if (row < in.nao && col < in.nao) ji[(long long)row * in.nao + col] = sum[k];
+    tile[tr][tc + k] = sum[k];
   }
+  __syncthreads();
+  if (r != c) {
+    for (int k = 0; k < 4; ++k) {
+      const int row = c * kTile + tr, col = r * kTile + tc + k;
+      if (row < in.nao && col < in.nao) ji[(long long)row * in.nao + col] = tile[tc + k][tr];
+    }
+  }
+  __syncthreads();
   BATCH_END
 }
 
@@ -281,27 +346,30 @@ __global__ __launch_bounds__(kThreads) void b_orbitals_kernel(BatchView v, const
                                                               long long c_plane) {
   BATCH_LOOP(kPhOrbitals)
   const int npad = in.nt * kTile;
-  const long long idx = local * kThreads + threadIdx.x;
   if (local == 0)
     for (int i = threadIdx.x; i < in.ldo; i += kThreads) ws64[in.sg_off + i] = i < in.nocc ? 1.0 : 0.0;
-  if (idx < (long long)npad * in.ldo) {
-    const double* ci = c + in.c_off;
-    if (PREC == HFJK_BF16X3) {
-      const int i = (int)(idx / npad), k = (int)(idx % npad);  // Ct[i][k]
-      const float x = (k < in.nao && i < in.nocc) ? (float)ci[(long long)k * in.nocc + i] : 0.0f;
-      uint16_t* hi = (uint16_t*)cbase + in.cp_off;
-      const uint16_t h = to_bf16(x);
-      hi[idx] = h;
-      hi[idx + c_plane] = to_bf16(x - __uint_as_float(((uint32_t)h) << 16));
-    } else {
-      const int k = (int)(idx / in.ldo), i = (int)(idx % in.ldo);  // C[k][i], in the operand order
-      const double x = (k < in.nao && i < in.nocc) ? ci[(long long)k * in.nocc + i] : 0.0;
-      const ColumnGroups cg = in.cg;
-      if (i / 16 < cg.groups * cg.blocks + cg.tail) {
-        if (PREC == HFJK_FP64)
-          ((double*)cbase)[in.cp_off + fragment_index<double>(cg, npad, k, i)] = x;
-        else
-          ((float*)cbase)[in.cp_off + fragment_index<float>(cg, npad, k, i)] = (float)x;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const long long idx = (local * 4 + u) * kThreads + threadIdx.x;
+    if (idx < (long long)npad * in.ldo) {
+      const double* ci = c + in.c_off;
+      if (PREC == HFJK_BF16X3) {
+        const int i = (int)(idx / npad), k = (int)(idx % npad);  // Ct[i][k]
+        const float x = (k < in.nao && i < in.nocc) ? (float)ci[(long long)k * in.nocc + i] : 0.0f;
+        uint16_t* hi = (uint16_t*)cbase + in.cp_off;
+        const uint16_t h = to_bf16(x);
+        hi[idx] = h;
+        hi[idx + c_plane] = to_bf16(x - __uint_as_float(((uint32_t)h) << 16));
+      } else {
+        const int k = (int)(idx / in.ldo), i = (int)(idx % in.ldo);  // C[k][i], in the operand order
+        const double x = (k < in.nao && i < in.nocc) ? ci[(long long)k * in.nocc + i] : 0.0;
+        const ColumnGroups cg = in.cg;
+        if (i / 16 < cg.groups * cg.blocks + cg.tail) {
+          if (PREC == HFJK_FP64)
+            ((double*)cbase)[in.cp_off + fragment_index<double>(cg, npad, k, i)] = x;
+          else
+            ((float*)cbase)[in.cp_off + fragment_index<float>(cg, npad, k, i)] = (float)x;
+        }
       }
     }
   }
@@ -313,73 +381,79 @@ __global__ __launch_bounds__(kThreads) void b_orbitals_kernel(BatchView v, const
 
 }  // namespace
 
+dim3 batch_grid(long long items) { return dim3((unsigned)std::max(1LL, std::min(items, kMaxGrid))); }
+
+namespace {
+dim3 grid_of(const BatchView& v, int phase) { return batch_grid(v.items[phase]); }
+}  // namespace
+
 hipError_t launch_batch_reset(BatchView v, hipStream_t s) {
   hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(kThreads), 0, s, v.counters, kPhCount * 8);
   return hipGetLastError();
 }
 
 hipError_t launch_batch_coulomb(BatchView v, int precision, const void* b, long long b_plane, const double* d,
-                                double* ws64, double* j, int grid, hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
-  hipLaunchKernelGGL(b_weights_kernel, g, blk, 0, s, v, d, ws64);
+                                double* ws64, double* j, hipStream_t s) {
+  const dim3 blk(kThreads);
+  hipLaunchKernelGGL(b_weights_kernel, grid_of(v, kPhWeights), blk, 0, s, v, d, ws64);
   if (precision == HFJK_FP64) {
-    hipLaunchKernelGGL(b_gamma_kernel<HFJK_FP64>, g, blk, 0, s, v, b, b_plane, ws64);
-    hipLaunchKernelGGL(b_gamma_reduce_kernel, g, blk, 0, s, v, ws64);
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP64>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_gamma_kernel<HFJK_FP64>, grid_of(v, kPhGamma), blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_gamma_reduce_kernel, grid_of(v, kPhGammaReduce), blk, 0, s, v, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP64>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   } else if (precision == HFJK_FP32) {
-    hipLaunchKernelGGL(b_gamma_kernel<HFJK_FP32>, g, blk, 0, s, v, b, b_plane, ws64);
-    hipLaunchKernelGGL(b_gamma_reduce_kernel, g, blk, 0, s, v, ws64);
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP32>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_gamma_kernel<HFJK_FP32>, grid_of(v, kPhGamma), blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_gamma_reduce_kernel, grid_of(v, kPhGammaReduce), blk, 0, s, v, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP32>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   } else {
-    hipLaunchKernelGGL(b_gamma_kernel<HFJK_BF16X3>, g, blk, 0, s, v, b, b_plane, ws64);
-    hipLaunchKernelGGL(b_gamma_reduce_kernel, g, blk, 0, s, v, ws64);
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_BF16X3>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_gamma_kernel<HFJK_BF16X3>, grid_of(v, kPhGamma), blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_gamma_reduce_kernel, grid_of(v, kPhGammaReduce), blk, 0, s, v, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_BF16X3>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   }
-  hipLaunchKernelGGL(b_coulomb_unpack_kernel, g, blk, 0, s, v, ws64, j);
+  hipLaunchKernelGGL(b_coulomb_unpack_kernel, grid_of(v, kPhCoulombUnpack), blk, 0, s, v, ws64, j);
   return hipGetLastError();
 }
 
 hipError_t launch_batch_coulomb_occ(BatchView v, int precision, const void* b, long long b_plane, const double* c,
-                                    const void* xbase, long long x_plane, double* ws64, double* j, int grid,
+                                    const void* xbase, long long x_plane, double* ws64, double* j,
                                     hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
+  const dim3 blk(kThreads);
   if (precision == HFJK_FP64) {
-    hipLaunchKernelGGL(b_charges_x_kernel<HFJK_FP64>, g, blk, 0, s, v, c, xbase, x_plane, ws64);
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP64>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_charges_x_kernel<HFJK_FP64>, grid_of(v, kPhCharges), blk, 0, s, v, c, xbase, x_plane, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP64>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   } else if (precision == HFJK_FP32) {
-    hipLaunchKernelGGL(b_charges_x_kernel<HFJK_FP32>, g, blk, 0, s, v, c, xbase, x_plane, ws64);
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP32>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_charges_x_kernel<HFJK_FP32>, grid_of(v, kPhCharges), blk, 0, s, v, c, xbase, x_plane, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP32>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   } else {
-    hipLaunchKernelGGL(b_charges_x_kernel<HFJK_BF16X3>, g, blk, 0, s, v, c, xbase, x_plane, ws64);
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_BF16X3>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_charges_x_kernel<HFJK_BF16X3>, grid_of(v, kPhCharges), blk, 0, s, v, c, xbase, x_plane, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_BF16X3>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   }
-  hipLaunchKernelGGL(b_coulomb_unpack_kernel, g, blk, 0, s, v, ws64, j);
+  hipLaunchKernelGGL(b_coulomb_unpack_kernel, grid_of(v, kPhCoulombUnpack), blk, 0, s, v, ws64, j);
   return hipGetLastError();
 }
 
 hipError_t launch_batch_coulomb_charges(BatchView v, int precision, const void* b, long long b_plane,
-                                        const double* charges, double* ws64, double* j, int grid, hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
-  hipLaunchKernelGGL(b_charges_load_kernel, g, blk, 0, s, v, charges, ws64);
+                                        const double* charges, double* ws64, double* j, hipStream_t s) {
+  const dim3 blk(kThreads);
+  hipLaunchKernelGGL(b_charges_load_kernel, grid_of(v, kPhGammaReduce), blk, 0, s, v, charges, ws64);
   if (precision == HFJK_FP64)
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP64>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP64>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   else if (precision == HFJK_FP32)
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP32>, g, blk, 0, s, v, b, b_plane, ws64);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_FP32>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
   else
-    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_BF16X3>, g, blk, 0, s, v, b, b_plane, ws64);
-  hipLaunchKernelGGL(b_coulomb_unpack_kernel, g, blk, 0, s, v, ws64, j);
+    hipLaunchKernelGGL(b_coulomb_kernel<HFJK_BF16X3>, grid_of(v, kPhCoulomb), blk, 0, s, v, b, b_plane, ws64);
+  hipLaunchKernelGGL(b_coulomb_unpack_kernel, grid_of(v, kPhCoulombUnpack), blk, 0, s, v, ws64, j);
   return hipGetLastError();
 }
 
 hipError_t launch_batch_orbitals(BatchView v, int precision, const double* c, double* ws64, void* cbase,
-                                 long long c_plane, int grid, hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
+                                 long long c_plane, hipStream_t s) {
+  const dim3 blk(kThreads);
   if (precision == HFJK_FP64)
-    hipLaunchKernelGGL(b_orbitals_kernel<HFJK_FP64>, g, blk, 0, s, v, c, ws64, cbase, c_plane);
+    hipLaunchKernelGGL(b_orbitals_kernel<HFJK_FP64>, grid_of(v, kPhOrbitals), blk, 0, s, v, c, ws64, cbase, c_plane);
   else if (precision == HFJK_FP32)
-    hipLaunchKernelGGL(b_orbitals_kernel<HFJK_FP32>, g, blk, 0, s, v, c, ws64, cbase, c_plane);
+    hipLaunchKernelGGL(b_orbitals_kernel<HFJK_FP32>, grid_of(v, kPhOrbitals), blk, 0, s, v, c, ws64, cbase, c_plane);
   else
-    hipLaunchKernelGGL(b_orbitals_kernel<HFJK_BF16X3>, g, blk, 0, s, v, c, ws64, cbase, c_plane);
+    hipLaunchKernelGGL(b_orbitals_kernel<HFJK_BF16X3>, grid_of(v, kPhOrbitals), blk, 0, s, v, c, ws64, cbase, c_plane);
   return hipGetLastError();
 }
 
@@ -388,6 +462,11 @@ hipError_t launch_batch_orbitals(BatchView v, int precision, const double* c, do
 // ---------------------------------------------------------------- C ABI
 
 namespace {
+
+// The phases' item counts of a plan.
+void fill_items(hfjk::BatchView& v, const std::vector<long long>& prefix) {
+  for (int ph = 0; ph < hfjk::kPhCount; ++ph) v.items[ph] = prefix[(size_t)ph * (v.ninst + 1) + v.ninst];
+}
 
 size_t al256(size_t v) { return (v + 255) & ~size_t(255); }
 
@@ -436,6 +515,13 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     if (instances[i].nao > 0 && instances[i].nao <= 46000)
       batch_us += hfjk::syrk_instance_us(precision, instances[i].naux, instances[i].nao, instances[i].nocc, true, whole_us);
   }
+  // Coulomb slices of at least 64 aux functions, 16 workgroups per CU over the batch.
+  long long tile_aux = 0;
+  for (int i = 0; i < ninst; ++i) {
+    const long long nt = hfjk::n_tiles(std::min(std::max(1, instances[i].nao), 46000));
+    tile_aux += nt * (nt + 1) / 2 * std::max(1, instances[i].naux);
+  }
+  const int jq = (int)std::min(1LL << 30, std::max(64LL, (tile_aux / (16LL * cus) + 7) / 8 * 8));
   const double item_us = std::min(1700.0, std::max(40.0, batch_us / (2.0 * cus) / 4.0));
   for (int i = 0; i < ninst; ++i) {
     const hfjk_batch_instance& src = instances[i];
@@ -505,7 +591,10 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     const long long ntiles = in.p / hfjk::kTileElems;
     auto take64 = [&](long long n) { const long long at = w64; w64 += (n + 31) / 32 * 32; return at; };
     in.w_off = take64(in.p);
-    in.jp_off = take64(in.p);
+    in.jsplit = (src.naux + jq - 1) / jq;
+    in.jq = ((src.naux + in.jsplit - 1) / in.jsplit + 7) / 8 * 8;
+    in.jsplit = (src.naux + in.jq - 1) / in.jq;
+    in.jp_off = take64((long long)in.jsplit * in.p);
     in.gp_off = take64(ntiles * src.naux);
     in.g_off = take64(src.naux);
     in.sg_off = take64(in.ldo);
@@ -525,14 +614,13 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
   for (int i = 0; i < ninst; ++i) {
     const hfjk::BatchInst& in = bt->insts[i];
     const long long ntiles = in.p / hfjk::kTileElems;
-    const long long nn = (long long)in.nao * in.nao;
     long long items[hfjk::kPhCount];
     items[hfjk::kPhWeights] = ntiles;
     items[hfjk::kPhGamma] = ntiles * ((in.naux + 63) / 64);
-    items[hfjk::kPhGammaReduce] = (in.naux + hfjk::kThreads - 1) / hfjk::kThreads;
-    items[hfjk::kPhCoulomb] = ntiles;
-    items[hfjk::kPhCoulombUnpack] = (nn + hfjk::kThreads - 1) / hfjk::kThreads;
-    items[hfjk::kPhOrbitals] = ((long long)in.nt * hfjk::kTile * in.ldo + hfjk::kThreads - 1) / hfjk::kThreads;
+    items[hfjk::kPhGammaReduce] = (in.naux + 63) / 64;
+    items[hfjk::kPhCoulomb] = ntiles * in.jsplit;
+    items[hfjk::kPhCoulombUnpack] = ntiles;
+    items[hfjk::kPhOrbitals] = ((long long)in.nt * hfjk::kTile * in.ldo + 4 * hfjk::kThreads - 1) / (4 * hfjk::kThreads);
     const long long x_units = (long long)in.naux * (precision == HFJK_FP64 ? hfjk::xform_units_per_aux<double>(in.nao)
                                                     : precision == HFJK_FP32 ? hfjk::xform_units_per_aux<float>(in.nao)
                                                                              : 1);
@@ -544,7 +632,8 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     items[hfjk::kPhSyrkRing] = ring ? (long long)in.npairs * in.nsplit : 0;
     // Strips of 512 elements of every lower tile.
     items[hfjk::kPhSyrkReduce] = (long long)in.npairs * (in.st * in.st / (2 * hfjk::kThreads));
-    items[hfjk::kPhCharges] = in.naux;
+    const int per_item = hfjk::charges_per_item(precision);
+    items[hfjk::kPhCharges] = (in.naux + per_item - 1) / per_item;
     for (int ph = 0; ph < hfjk::kPhCount; ++ph) {
       const size_t base = (size_t)ph * (ninst + 1);
       bt->prefix[base + i + 1] = bt->prefix[base + i] + items[ph];
@@ -569,7 +658,6 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
   off = al256(off + (size_t)(precision == HFJK_FP64 ? 8 : 4) * kp);
   bt->bytes = off;
   bt->grid_mfma = ((2 * cus + 7) / 8) * 8;
-  bt->grid_elem = ((4 * cus + 7) / 8) * 8;
   *out = bt;
   return HFJK_OK;
 }
@@ -640,6 +728,7 @@ int hfjk_batch_run(hfjk_batch* batch, const void* tensor, const double* orbitals
   v.prefix = (const long long*)(ws + batch->off_prefix);
   v.counters = (unsigned long long*)(ws + batch->off_counters);
   v.ninst = batch->ninst;
+  fill_items(v, batch->prefix);
   double* ws64 = (double*)(ws + batch->off_ws64);
   void* cbase = ws + batch->off_cp;
   void* xbase = ws + batch->off_x;
@@ -648,19 +737,19 @@ int hfjk_batch_run(hfjk_batch* batch, const void* tensor, const double* orbitals
   hipError_t e = hipSetDevice(batch->ctx->device);
   if (e == hipSuccess) e = hfjk::launch_batch_reset(v, s);
   if (e == hipSuccess && density != nullptr)
-    e = hfjk::launch_batch_coulomb(v, prec, tensor, batch->b_total, density, ws64, coulomb, batch->grid_elem, s);
+    e = hfjk::launch_batch_coulomb(v, prec, tensor, batch->b_total, density, ws64, coulomb, s);
   if (e == hipSuccess)
-    e = hfjk::launch_batch_orbitals(v, prec, orbitals, ws64, cbase, batch->cp_total, batch->grid_elem, s);
+    e = hfjk::launch_batch_orbitals(v, prec, orbitals, ws64, cbase, batch->cp_total, s);
   if (e == hipSuccess)
     e = hfjk::launch_batch_xform(v, prec, batch->tile, tensor, batch->b_total, cbase, batch->cp_total, xbase,
                                  batch->x_total, batch->grid_mfma, s);
   // Without densities D = C C^T: the charges come from X (one pass over X instead of one over B).
   if (e == hipSuccess && density == nullptr)
     e = hfjk::launch_batch_coulomb_occ(v, prec, tensor, batch->b_total, orbitals, xbase, batch->x_total, ws64,
-                                       coulomb, batch->grid_elem, s);
+                                       coulomb, s);
   if (e == hipSuccess)
     e = hfjk::launch_batch_syrk(v, prec, xbase, batch->x_total, ws64, kbase, batch->grid_mfma, s);
-  if (e == hipSuccess) e = hfjk::launch_batch_syrk_reduce(v, prec, kbase, exchange, batch->grid_elem, s);
+  if (e == hipSuccess) e = hfjk::launch_batch_syrk_reduce(v, prec, kbase, exchange, s);
   if (e != hipSuccess) {
     hfjk_internal_set_error((std::string("batched launch: ") + hipGetErrorString(e)).c_str());
     return HFJK_ERR_HIP;
@@ -685,12 +774,12 @@ int hfjk_batch_coulomb_charges(hfjk_batch* batch, const void* tensor, const doub
   v.prefix = (const long long*)(ws + batch->off_prefix);
   v.counters = (unsigned long long*)(ws + batch->off_counters);
   v.ninst = batch->ninst;
+  fill_items(v, batch->prefix);
   double* ws64 = (double*)(ws + batch->off_ws64);
   hipError_t e = hipSetDevice(batch->ctx->device);
   if (e == hipSuccess) e = hfjk::launch_batch_reset(v, s);
   if (e == hipSuccess)
-    e = hfjk::launch_batch_coulomb_charges(v, batch->precision, tensor, batch->b_total, charges, ws64, coulomb,
-                                           batch->grid_elem, s);
+    e = hfjk::launch_batch_coulomb_charges(v, batch->precision, tensor, batch->b_total, charges, ws64, coulomb, s);
   if (e != hipSuccess) {
     hfjk_internal_set_error((std::string("batched launch: ") + hipGetErrorString(e)).c_str());
     return HFJK_ERR_HIP;

@@ -61,41 +61,54 @@ rocblas_handle blas_for(hfjk_ctx* ctx, hipStream_t s) {
   return h;
 }
 
-// out[i] = sum_e x_i[e] y_i[e]; one workgroup per instance.
-__global__ __launch_bounds__(kT) void batched_dot_kernel(long long len, const double* __restrict__ x, long long sx,
-                                                         const double* __restrict__ y, long long sy,
-                                                         double* __restrict__ out) {
-  __shared__ double red[kT];
-  const double* xi = x + (long long)blockIdx.x * sx;
-  const double* yi = y + (long long)blockIdx.x * sy;
-  double s = 0.0;
-  for (long long e = threadIdx.x; e < len; e += kT) s += xi[e] * yi[e];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = kT / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+// sum_e x[e] y[e] over the workgroup, in a fixed order; thread 0 gets it. One
+// workgroup's share is bound by the latency of its loads: 1024 threads with
+// eight pairs in flight (256 threads with one: 105 us for 300 x 300).
+constexpr int kDotT = 1024;
+__device__ double workgroup_dot(long long len, const double* __restrict__ x, const double* __restrict__ y) {
+  __shared__ double red[kDotT / 64];
+  double s[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) s[u] = 0.0;
+  long long e = threadIdx.x;
+  for (; e + 7 * kDotT < len; e += 8 * kDotT) {
+    double a[8], b[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      a[u] = x[e + u * kDotT];
+      b[u] = y[e + u * kDotT];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s[u] += a[u] * b[u];
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = red[0];
+  for (; e < len; e += kDotT) s[0] += x[e] * y[e];
+  double t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+  __syncthreads();
+  t = 0.0;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < kDotT / 64; ++w) t += red[w];
+  return t;
+}
+
+// out[i] = sum_e x_i[e] y_i[e]; one workgroup per instance.
+__global__ __launch_bounds__(kDotT) void batched_dot_kernel(long long len, const double* __restrict__ x, long long sx,
+                                                            const double* __restrict__ y, long long sy,
+                                                            double* __restrict__ out) {
+  const double s = workgroup_dot(len, x + (long long)blockIdx.x * sx, y + (long long)blockIdx.x * sy);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // out[i][a] = <hist[newest][i], hist[a][i]> over len elements, hist [nslots][count][len];
 // one workgroup per (instance, slot), fixed summation order.
-__global__ __launch_bounds__(kT) void history_dots_kernel(long long len, int count, const double* __restrict__ hist,
-                                                          int newest, double* __restrict__ out) {
-  __shared__ double red[kT];
+__global__ __launch_bounds__(kDotT) void history_dots_kernel(long long len, int count, const double* __restrict__ hist,
+                                                             int newest, double* __restrict__ out) {
   const int i = blockIdx.x, a = blockIdx.y;
-  const double* x = hist + ((long long)newest * count + i) * len;
-  const double* y = hist + ((long long)a * count + i) * len;
-  double s = 0.0;
-  for (long long e = threadIdx.x; e < len; e += kT) s += x[e] * y[e];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = kT / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[(long long)i * gridDim.y + a] = red[0];
+  const double s = workgroup_dot(len, hist + ((long long)newest * count + i) * len,
+                                 hist + ((long long)a * count + i) * len);
+  if (threadIdx.x == 0) out[(long long)i * gridDim.y + a] = s;
 }
 
 __global__ __launch_bounds__(kT) void batched_antisym_kernel(int n, const double* __restrict__ m,
@@ -376,7 +389,7 @@ int hfjk_ddot_batched(hfjk_ctx* ctx, int count, long long len, const double* x, 
   return bguard(ctx, [&] {
     check_count(count);
     if (len < 0 || x == nullptr || y == nullptr || out == nullptr) bfail(HFJK_ERR_INPUT, "hfjk_ddot_batched: bad input");
-    hipLaunchKernelGGL(batched_dot_kernel, dim3(count), dim3(kT), 0, (hipStream_t)stream, len, x, stride_x, y,
+    hipLaunchKernelGGL(batched_dot_kernel, dim3(count), dim3(kDotT), 0, (hipStream_t)stream, len, x, stride_x, y,
                        stride_y, out);
     bcheck_hip(hipGetLastError(), "batched_dot launch");
   });
@@ -388,7 +401,7 @@ int hfjk_history_dots_batched(hfjk_ctx* ctx, int count, long long len, int nslot
     check_count(count);
     if (len < 0 || nslots < 1 || nslots > 64 || newest < 0 || newest >= nslots || hist == nullptr || out == nullptr)
       bfail(HFJK_ERR_INPUT, "hfjk_history_dots_batched: bad input");
-    hipLaunchKernelGGL(history_dots_kernel, dim3(count, nslots), dim3(kT), 0, (hipStream_t)stream, len, count, hist,
+    hipLaunchKernelGGL(history_dots_kernel, dim3(count, nslots), dim3(kDotT), 0, (hipStream_t)stream, len, count, hist,
                        newest, out);
     bcheck_hip(hipGetLastError(), "history_dots launch");
   });

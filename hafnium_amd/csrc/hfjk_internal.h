@@ -120,6 +120,11 @@ __device__ inline long long batch_next(const long long* prefix, unsigned long lo
       const int x = (x0 + d) & 7;
       const long long lo = total * x / 8, hi = total * (x + 1) / 8;
       if (lo >= hi) continue;
+      // Counters only grow: a share seen empty stays empty, and a load of it is cheaper than one
+      // more atomic (at the end of a phase every workgroup visits all eight).
+      if (d > 0 && __hip_atomic_load(&counters[ph * 8 + x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >=
+                       (unsigned long long)(hi - lo))
+        continue;
       const long long it = lo + (long long)atomicAdd(&counters[ph * 8 + x], 1ULL);
       if (it < hi) {
         item = it;
@@ -135,6 +140,35 @@ __device__ inline long long batch_next(const long long* prefix, unsigned long lo
   share_end = s_end;
   __syncthreads();
   return item;
+}
+
+// A lane's partner value under a DPP row permutation (ctrl: 0x140 row mirror, 0x141 half-row
+// mirror, quad permutations below 0x100); every lane of the row takes part.
+template <int CTRL>
+__device__ inline double dpp_d(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// Eight sums over the wave at once: on return every lane holds the total of s[lane >> 3].
+// Each halving exchange sends the half of the values the partner keeps (10 exchanges, not 48).
+// The partners differ in lane bit 5, 4, 3, 2, 1, 0 in turn: lane ^ 32 and lane ^ 16 by
+// shuffles, then within a row of 16 by DPP (row mirror 15 - l, half-row mirror 7 - l, quad
+// permutations l ^ 2 and l ^ 1), which pair lanes the same way for these sums.
+__device__ inline double wave_sums8(const double (&s)[8], int lane) {
+  const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8;
+  double t4[4], t2[2];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) t4[x] = (h5 ? s[4 + x] : s[x]) + __shfl_xor(h5 ? s[x] : s[4 + x], 32);
+#pragma unroll
+  for (int x = 0; x < 2; ++x) t2[x] = (h4 ? t4[2 + x] : t4[x]) + __shfl_xor(h4 ? t4[x] : t4[2 + x], 16);
+  double t1 = (h3 ? t2[1] : t2[0]) + dpp_d<0x140>(h3 ? t2[0] : t2[1]);
+  t1 += dpp_d<0x141>(t1);
+  t1 += dpp_d<0x4E>(t1);  // quad permutation [2, 3, 0, 1]
+  t1 += dpp_d<0xB1>(t1);  // quad permutation [1, 0, 3, 2]
+  return t1;
 }
 
 // Instance i with prefix[i] <= item < prefix[i + 1] (prefix non-decreasing).
@@ -385,12 +419,13 @@ struct BatchInst {
   int st, bn;         // SYRK tile storage (64 or 128); half-transform column tile (32, 64, 128 or 256)
   ColumnGroups cg;    // FP64 / FP32 half-transform
   int se;             // rows and columns of K per SYRK tile (at most st)
+  int jq, jsplit;     // aux functions per slice of the Coulomb sum and slices
   long long p;        // packed elements per aux function
   long long b_off;    // batch tensor (element units of the bound copy)
   long long c_off;    // orbitals [nao][nocc] (float64)
   long long d_off;    // density, J and K [nao][nao] (float64)
   long long w_off;    // fp64 workspace: packed weights [p]
-  long long jp_off;   // fp64 workspace: packed J [p]
+  long long jp_off;   // fp64 workspace: packed J [jsplit][p]
   long long gp_off;   // fp64 workspace: charge partials [ntiles][naux]
   long long g_off;    // fp64 workspace: charges [naux]
   long long sg_off;   // fp64 workspace: signs [ldo]
@@ -416,32 +451,34 @@ enum BatchPhase {
 };
 
 // Device view of a batch plan: instances, per-phase item prefix sums
-// ([kPhCount][ninst + 1]) and per-phase, per-XCD work counters ([kPhCount][8]).
+// ([kPhCount][ninst + 1]) and, for the persistent phases, per-XCD work
+// counters ([kPhCount][8]).
 struct BatchView {
   const BatchInst* insts;
   const long long* prefix;
   unsigned long long* counters;
   int ninst;
+  long long items[kPhCount];  // items of every phase (the last entries of its prefix sums)
 };
 
-// Launchers of the batched persistent kernels (batch.hip, xk.hip). `grid`
-// is a multiple of 8 workgroups; mode buffers are typed by `precision`.
+// Launchers of the batched kernels (batch.hip, xk.hip). `grid` is that of a
+// persistent kernel, a multiple of 8 workgroups; mode buffers are typed by `precision`.
+// The grid of a phase whose items are dealt by the hardware.
+dim3 batch_grid(long long items);
 hipError_t launch_batch_reset(BatchView v, hipStream_t s);
 hipError_t launch_batch_coulomb_occ(BatchView v, int precision, const void* b, long long b_plane, const double* c,
-                                    const void* xbase, long long x_plane, double* ws64, double* j, int grid,
-                                    hipStream_t s);
+                                    const void* xbase, long long x_plane, double* ws64, double* j, hipStream_t s);
 hipError_t launch_batch_coulomb_charges(BatchView v, int precision, const void* b, long long b_plane,
-                                        const double* charges, double* ws64, double* j, int grid, hipStream_t s);
+                                        const double* charges, double* ws64, double* j, hipStream_t s);
 hipError_t launch_batch_coulomb(BatchView v, int precision, const void* b, long long b_plane, const double* d,
-                                double* ws64, double* j, int grid, hipStream_t s);
+                                double* ws64, double* j, hipStream_t s);
 hipError_t launch_batch_orbitals(BatchView v, int precision, const double* c, double* ws64, void* cbase,
-                                 long long c_plane, int grid, hipStream_t s);
+                                 long long c_plane, hipStream_t s);
 hipError_t launch_batch_xform(BatchView v, int precision, int bn, const void* b, long long b_plane, const void* cbase,
                               long long c_plane, void* xbase, long long x_plane, int grid, hipStream_t s);
 hipError_t launch_batch_syrk(BatchView v, int precision, const void* xbase, long long x_plane, const double* ws64,
                              void* kbase, int grid, hipStream_t s);
-hipError_t launch_batch_syrk_reduce(BatchView v, int precision, const void* kbase, double* k, int grid,
-                                    hipStream_t s);
+hipError_t launch_batch_syrk_reduce(BatchView v, int precision, const void* kbase, double* k, hipStream_t s);
 // Density factorisation helpers (jk.hip).
 hipError_t launch_split_factor(const double* vecs, const double* vals, int nao, int first, int count,
                                double* c, double* signs, hipStream_t s);

@@ -3142,10 +3142,7 @@ __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v
                                                                       double* __restrict__ kout) {
   __shared__ __attribute__((aligned(16))) double sum[2 * kThreads];
   const long long* pre = v.prefix + (long long)kPhSyrkReduce * (v.ninst + 1);
-  for (;;) {
-    long long end;
-    const long long item = batch_next(v.prefix, v.counters, v.ninst, kPhSyrkReduce, end);
-    if (item >= end) break;
+  for (long long item = blockIdx.x; item < v.items[kPhSyrkReduce]; item += gridDim.x) {
     const int i = batch_find(pre, v.ninst, item);
     const BatchInst in = v.insts[i];
     const int st = in.st;
@@ -3173,15 +3170,22 @@ __global__ __launch_bounds__(kThreads) void batch_syrk_reduce_kernel(BatchView v
       const int mr = row0 + f % rows, mc = bn * edge + f / rows;
       if (mr < in.nao && f / rows < edge && mc < mr) k[(long long)mc * in.nao + mr] = sum[(f % rows) * st + f / rows];
     }
-    // batch_next's barriers keep the next item's sums behind these reads.
+    __syncthreads();
   }
 }
 
 }  // namespace
 
+namespace {
+// A persistent kernel's grid: a workgroup per item up to `grid`, a multiple of 8.
+dim3 persistent_grid(long long items, int grid) {
+  return dim3((unsigned)std::max(8LL, std::min<long long>(grid, (items + 7) / 8 * 8)));
+}
+}  // namespace
+
 hipError_t launch_batch_xform(BatchView v, int precision, int bn, const void* b, long long b_plane, const void* cbase,
                               long long c_plane, void* xbase, long long x_plane, int grid, hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
+  const dim3 g = persistent_grid(v.items[kPhXform], grid), blk(kThreads);
   if (precision == HFJK_FP64) {
     hipLaunchKernelGGL(batch_xform_kernel<double>, g, blk, 0, s, v, (const double*)b, (const double*)cbase,
                        (double*)xbase);
@@ -3203,25 +3207,34 @@ hipError_t launch_batch_xform(BatchView v, int precision, int bn, const void* b,
 
 hipError_t launch_batch_syrk(BatchView v, int precision, const void* xbase, long long x_plane, const double* ws64,
                              void* kbase, int grid, hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
+  const dim3 blk(kThreads);
   // grid = two workgroups per CU, the FP64 / FP32 ring kernel's occupancy; workgroups that find
   // no CU free start late, find their share taken and leave.
+  const dim3 ring = persistent_grid(v.items[kPhSyrkRing], grid), staged = persistent_grid(v.items[kPhSyrk], grid);
+  const bool any_ring = v.items[kPhSyrkRing] > 0, any_staged = v.items[kPhSyrk] > 0;
   if (precision == HFJK_FP64) {
-    hipLaunchKernelGGL(batch_syrk_kernel<double>, g, blk, 0, s, v, (const double*)xbase, ws64, (double*)kbase);
-    hipLaunchKernelGGL(batch_syrk_ring_kernel<double>, g, blk, 0, s, v, (const double*)xbase, (double*)kbase);
+    if (any_staged)
+      hipLaunchKernelGGL(batch_syrk_kernel<double>, staged, blk, 0, s, v, (const double*)xbase, ws64, (double*)kbase);
+    if (any_ring)
+      hipLaunchKernelGGL(batch_syrk_ring_kernel<double>, ring, blk, 0, s, v, (const double*)xbase, (double*)kbase);
   } else if (precision == HFJK_FP32) {
-    hipLaunchKernelGGL(batch_syrk_kernel<float>, g, blk, 0, s, v, (const float*)xbase, ws64, (float*)kbase);
-    hipLaunchKernelGGL(batch_syrk_ring_kernel<float>, g, blk, 0, s, v, (const float*)xbase, (float*)kbase);
+    if (any_staged)
+      hipLaunchKernelGGL(batch_syrk_kernel<float>, staged, blk, 0, s, v, (const float*)xbase, ws64, (float*)kbase);
+    if (any_ring)
+      hipLaunchKernelGGL(batch_syrk_ring_kernel<float>, ring, blk, 0, s, v, (const float*)xbase, (float*)kbase);
   } else {
-    hipLaunchKernelGGL(batch_syrk16_kernel, g, blk, 0, s, v, (const uint16_t*)xbase, x_plane, ws64, (float*)kbase);
-    hipLaunchKernelGGL(batch_syrk16_ring_kernel, g, blk, 0, s, v, (const uint16_t*)xbase, x_plane, (float*)kbase);
+    if (any_staged)
+      hipLaunchKernelGGL(batch_syrk16_kernel, staged, blk, 0, s, v, (const uint16_t*)xbase, x_plane, ws64,
+                         (float*)kbase);
+    if (any_ring)
+      hipLaunchKernelGGL(batch_syrk16_ring_kernel, ring, blk, 0, s, v, (const uint16_t*)xbase, x_plane, (float*)kbase);
   }
   return hipGetLastError();
 }
 
-hipError_t launch_batch_syrk_reduce(BatchView v, int precision, const void* kbase, double* k, int grid,
+hipError_t launch_batch_syrk_reduce(BatchView v, int precision, const void* kbase, double* k,
                                     hipStream_t s) {
-  const dim3 g((unsigned)grid), blk(kThreads);
+  const dim3 g = batch_grid(v.items[kPhSyrkReduce]), blk(kThreads);
   if (precision == HFJK_FP64)
     hipLaunchKernelGGL(batch_syrk_reduce_kernel<double>, g, blk, 0, s, v, (const double*)kbase, k);
   else

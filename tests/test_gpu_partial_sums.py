@@ -116,3 +116,36 @@ def test_half_transform_column_groups(precision, nao, nocc):
             first = (j, k) if first is None else first
             np.testing.assert_array_equal(k, first[1])
             np.testing.assert_array_equal(j, first[0])
+
+
+@pytest.mark.parametrize("length", [0, 1, 63, 1024, 8191, 8192, 8193, 70001])
+def test_batched_dots(length):
+    """1024 threads with eight pairs each: both sides of one round of loads, a remainder, nothing."""
+    import torch
+
+    from hafnium_amd import _lib
+    from hafnium_amd.coulomb_exchange import _Context, _ptr, _stream
+
+    count, slots = 3, 4
+    g = torch.Generator(device="cuda:0").manual_seed(length)
+    hist = torch.randn((slots, count, max(length, 1)), generator=g, dtype=torch.float64, device="cuda:0")
+    stream = _stream(torch, hist.device)
+    context = _Context(0)
+    lib = _lib.load()
+    out = torch.full((count,), 7.0, dtype=torch.float64, device="cuda:0")
+    stride = max(length, 1)
+    _lib.check(lib.hfjk_ddot_batched(context.handle, count, length, _ptr(hist[0]), stride, _ptr(hist[1]), stride,
+                                     _ptr(out), stream))
+    dots = torch.full((count, slots), 7.0, dtype=torch.float64, device="cuda:0")
+    if length:
+        _lib.check(lib.hfjk_history_dots_batched(context.handle, count, length, slots, _ptr(hist), 2, _ptr(dots),
+                                                 stream))
+    torch.cuda.synchronize()
+    h = hist[:, :, :length].cpu().numpy().astype(np.longdouble)
+    # A sum of n products in any order: n eps sum |x y|.
+    for i in range(count):
+        bound = max(length, 1) * 2.3e-16 * float(np.abs(h[0, i] * h[1, i]).sum())
+        assert abs(float(out[i]) - float((h[0, i] * h[1, i]).sum())) <= bound
+        for a in range(slots if length else 0):
+            bound = length * 2.3e-16 * float(np.abs(h[2, i] * h[a, i]).sum())
+            assert abs(float(dots[i, a]) - float((h[2, i] * h[a, i]).sum())) <= bound
