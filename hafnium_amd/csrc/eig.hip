@@ -1,6 +1,6 @@
-// Batched symmetric eigensolver for the lowest eigenpairs, one workgroup
-// per matrix (the Fock diagonalisation of a batched SCF, where rocSOLVER's
-// batched divide and conquer is about 1500 small launches per call):
+// Batched symmetric eigensolver for the lowest eigenpairs in six launches
+// (the Fock diagonalisation of a batched SCF, where rocSOLVER's batched divide
+// and conquer is about 1500 small launches per call):
 //   1. Householder reduction to tridiagonal form, T = Q^T A Q (Golub and
 //      Van Loan, "Matrix Computations", algorithm 8.3.1), the reflector
 //      vectors kept in the rows of A above the diagonal;
@@ -15,6 +15,7 @@
 // A is row-major and symmetric; on return its rows 0 .. nvec - 1 are the
 // eigenvectors of the nvec lowest eigenvalues and w[0 .. nvec) holds those
 // eigenvalues in ascending order (rows nvec .. n - 1 of A hold scratch).
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <string>
@@ -32,9 +33,8 @@ constexpr int kEigMaxCols = kEigMaxN / 64;  // 64-row chunks of a vector
 constexpr int kEigRegVecs = 64;             // nvec up to this: vectors stay in registers, Cholesky QR
 constexpr int kGs = 65;                     // row stride of the Gram matrix and its inverse factor in LDS
 
-// Workspace doubles per matrix: d, e, beta (n each), the nvec eigenvectors [nvec][n], their LU
-// factors (five [n][nvec] arrays) and the inverse-iteration vectors [n][nvec].
-__host__ __device__ inline long long eig_work_per(int n, int nvec) { return 3LL * n + 7LL * nvec * n; }
+// Workspace doubles per matrix: d, e, beta (n each) and the nvec eigenvectors [nvec][n].
+__host__ __device__ inline long long eig_work_per(int n, int nvec) { return 3LL * n + (long long)nvec * n; }
 
 // Sum over the workgroup (every thread passes its part; all get the total).
 __device__ __forceinline__ double wg_sum(double v, double* red) {
@@ -176,6 +176,22 @@ __device__ __forceinline__ void tri_batch_cb(int cb, __amdgpu_buffer_rsrc_t rsrc
   }
 }
 
+// The Householder vector of a column x (ss = |x|^2, x0 its first entry): v = x but v0, beta and the
+// entry that the reflection leaves.
+__device__ __forceinline__ void reflector(double ss, double x0, double& bk, double& ek, double& v0) {
+  const double sigma = ss - x0 * x0;
+  bk = 0.0;
+  ek = x0;
+  v0 = x0;
+  if (sigma > 0.0) {
+    const double norm = sqrt(ss);
+    const double alpha = x0 > 0.0 ? -norm : norm;
+    v0 = x0 - alpha;
+    bk = 2.0 / (sigma + v0 * v0);
+    ek = alpha;
+  }
+}
+
 // One pass over the lower triangle of the m x m trailing block (rows and columns c0 .. n - 1 of
 // A, at byte offset boff of the buffer rsrc, which covers A): applies the previous step's rank-2
 // update A -= v' w'^T + w' v'^T (pv, pw indexed from row c0 - 1) and forms the product of the
@@ -239,47 +255,6 @@ __device__ inline void store_vecs(const double (&y)[8][NC], double* Y, int n, in
         const int r = lane + 64 * c;
         if (r < n) Y[(long long)(j0 + q) * n + r] = y[q][c];
       }
-    }
-  }
-}
-
-// y <- H_0 H_1 ... H_{n-3} y for the wave's eight vectors in registers; reflector k is
-// I - beta_k u u^T with u in row k of A (columns k + 1 .. n - 1). The next reflector's loads are
-// issued before the current one is applied.
-template <int NC>
-__device__ __forceinline__ void back_transform(double (&y)[8][NC], const double* A, const double* lbeta, int n, int lane) {
-  if (n < 3) return;
-  double un[NC];
-  auto load_u = [&](int k) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int r = lane + 64 * c;
-      const double v = A[(long long)k * n + min(max(r, k + 1), n - 1)];
-      un[c] = (r > k && r < n) ? v : 0.0;
-    }
-  };
-  load_u(n - 3);
-  for (int k = n - 3; k >= 0; --k) {
-    double u[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) u[c] = un[c];
-    if (k > 0) load_u(k - 1);
-    const double bk = lbeta[k];
-    if (bk == 0.0) continue;
-    double s[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      double a = 0.0;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) a += u[c] * y[q][c];
-      s[q] = a;
-    }
-    const double tot = wave_sums8(s, lane);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const double f = bk * readlane_d(tot, 8 * q);
-#pragma unroll
-      for (int c = 0; c < NC; ++c) y[q][c] -= f * u[c];
     }
   }
 }
@@ -361,121 +336,226 @@ __device__ __forceinline__ void tri_product(double (&y)[8][NC], const double* Y,
   }
 }
 
-// G = L L^T (G in the lower triangle of gm, nv <= 64) and li = L^{-1}, by wave 0 with every
-// row in registers: lane i holds row i of G, each column of L is broadcast through LDS (the
-// first row of li), and the update of the rows is unrolled over the columns; then L goes to gm
-// and lane c forms column c of L^{-1} by forward substitution, reading L by broadcast. A
-// non-positive pivot is raised to DBL_MIN. Not inlined: one copy serves every vector length.
-__device__ __attribute__((noinline)) void cholesky_inverse(double* gm, double* li, int nv, int lane) {
-  const int i = lane;
-  double g[kEigRegVecs];
+// li = L^{-1} of G = L L^T (G in the lower triangle of gm, nv <= 64) by elimination of [G | 1]: with
+// G = U D U^T, U^{-1} is what the eliminations make of the unit matrix and L^{-1} = D^{-1/2} U^{-1}.
+// Thread (i, c) = (t / 8, t % 8) holds the entries of row i in columns c, c + 8, ... of both; the
+// owners of row k publish it and one barrier a step suffices with two buffers. A non-positive pivot
+// is raised to DBL_MIN.
+__device__ void cholesky_inverse(const double* gm, double* li, double (*rows)[2 * kEigRegVecs], int nv) {
+  const int i = threadIdx.x >> 3, c = threadIdx.x & 7;
+  double g[8], x[8];
 #pragma unroll
-  for (int j = 0; j < kEigRegVecs; ++j) g[j] = (i < nv && j <= i) ? gm[i * kGs + j] : 0.0;
+  for (int m = 0; m < 8; ++m) {
+    const int col = c + 8 * m;
+    g[m] = i < nv && col < nv ? gm[max(i, col) * kGs + min(i, col)] : 0.0;
+    x[m] = i == col ? 1.0 : 0.0;
+  }
+  for (int k = 0; k < nv; ++k) {
+    double* row = rows[k & 1];
+    if (i == k) {
 #pragma unroll
-  for (int k = 0; k < kEigRegVecs; ++k) {
-    if (k < nv) {
-      const double lkk = sqrt(fmax(readlane_d(g[k], k), DBL_MIN));
-      const double lik = i == k ? lkk : g[k] / lkk;  // L[i][k] for i >= k (lanes above: unused)
-      g[k] = lik;
-      li[i] = lik;
-      __builtin_amdgcn_wave_barrier();
+      for (int m = 0; m < 8; ++m) {
+        row[c + 8 * m] = g[m];
+        row[kEigRegVecs + c + 8 * m] = x[m];
+      }
+    }
+    __syncthreads();
+    const double piv = fmax(row[k], DBL_MIN);
+    if (i > k) {
+      const double f = row[i] / piv;
 #pragma unroll
-      for (int j = k + 1; j < kEigRegVecs; ++j) g[j] = fma(-lik, li[j], g[j]);
-      __builtin_amdgcn_wave_barrier();
+      for (int m = 0; m < 8; ++m) {
+        g[m] = fma(-f, row[c + 8 * m], g[m]);
+        x[m] = fma(-f, row[kEigRegVecs + c + 8 * m], x[m]);
+      }
+    } else if (i == k) {
+      const double r = 1.0 / sqrt(piv);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) li[k * kGs + c + 8 * m] = x[m] * r;
     }
   }
-#pragma unroll
-  for (int j = 0; j < kEigRegVecs; ++j) gm[i * kGs + j] = g[j];
-  __builtin_amdgcn_wave_barrier();
-  const int c = lane;
-  double x[kEigRegVecs];  // column c of L^{-1}; x[r] = 0 for r < c falls out of the recurrence
-#pragma unroll
-  for (int r = 0; r < kEigRegVecs; ++r) {
-    if (r < nv) {
-      double sacc = r == c ? 1.0 : 0.0;
-#pragma unroll
-      for (int p = 0; p < r; ++p) sacc = fma(-gm[r * kGs + p], x[p], sacc);
-      x[r] = sacc / gm[r * kGs + r];
-    } else {
-      x[r] = 0.0;
-    }
-  }
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int r = 0; r < kEigRegVecs; ++r)
-    if (r < nv && c < nv) li[r * kGs + c] = x[r];
 }
 
-// Orthonormalisation (Cholesky QR twice) and back-transformation for nvec <= 64, each wave's
-// eight vectors held in registers; the results go to rows 0 .. nvec - 1 of A.
+// Orthonormalisation (Cholesky QR twice) of Y for nvec <= 64, each wave's eight vectors held in
+// registers.
 template <int NC>
-__device__ __forceinline__ void finish_in_registers(double* A, double* Y, const double* lbeta, double* gm, double* li, int n,
-                                    int nvec, int wave, int lane) {
+__device__ __forceinline__ void orthonormalise(double* Y, double* gm, double* li, double (*rows)[2 * kEigRegVecs], int n,
+                                               int nvec, int wave, int lane) {
   const int j0 = 8 * wave;
   double y[8][NC];
   load_vecs<NC>(y, Y, n, nvec, j0, lane);
   for (int pass = 0; pass < 2; ++pass) {
     if (j0 < nvec) gram_rows<NC>(y, Y, n, nvec, j0, lane, gm);
     __syncthreads();
-    if (wave == 0) cholesky_inverse(gm, li, nvec, lane);
+    cholesky_inverse(gm, li, rows, nvec);
     __syncthreads();
     if (j0 < nvec) tri_product<NC>(y, Y, n, nvec, j0, lane, li);
     __syncthreads();  // every wave has read Y
-    if (pass == 0) {
-      store_vecs<NC>(y, Y, n, nvec, j0, lane);
-      __syncthreads();
+    store_vecs<NC>(y, Y, n, nvec, j0, lane);
+    __syncthreads();
+  }
+}
+
+// Y <- H_0 H_1 ... H_{n-3} Y, reflector k = I - beta_k u u^T with u in row k of A (columns k + 1 ..
+// n - 1): one vector per row of 16 lanes, so that a dot product ends in DPP steps alone. A
+// workgroup is one wave with four vectors: the reflectors are a serial chain, and the vectors of
+// all matrices side by side fill the chip (eight vectors in each wave of one workgroup per matrix
+// took 0.2 ms of its 0.6). Reflectors come RB at a time through LDS, the next RB in flight in
+// registers, from the L2 of the XCD that wrote them (one reflector ahead, from any XCD, a step
+// waited 2.9 us).
+template <int NC, int RB>
+__device__ __forceinline__ void back_transform(const double* A, const double* lbeta, double (*lu)[kEigMaxN], double* Y,
+                                               int n, int nvec, int j, int lane) {
+  if (n < 3) return;
+  constexpr int NL = (NC + 3) / 4;
+  const int l16 = lane & 15;
+  double y[NC], un[RB][NL];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int r = 16 * c + l16;
+    const double v = Y[(long long)min(j, nvec - 1) * n + min(r, n - 1)];
+    y[c] = r < n ? v : 0.0;
+  }
+  auto load_block = [&](int k0) {  // reflectors k0, k0 - 1, ...
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+      const int k = max(k0 - q, 0);
+#pragma unroll
+      for (int c = 0; c < NL; ++c) un[q][c] = A[(long long)k * n + min(max(64 * c + lane, k + 1), n - 1)];
+    }
+  };
+  load_block(n - 3);
+  for (int k0 = n - 3; k0 >= 0; k0 -= RB) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RB; ++q)
+#pragma unroll
+      for (int c = 0; c < NL; ++c) {
+        const int r = 64 * c + lane;
+        lu[q][r] = r > k0 - q && r < n ? un[q][c] : 0.0;
+      }
+    __syncthreads();
+    if (k0 >= RB) load_block(k0 - RB);
+#pragma unroll 1
+    for (int q = 0; q < min(RB, k0 + 1); ++q) {
+      double u[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) u[c] = lu[q][16 * c + l16];
+      double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+      for (int c = 0; c < NC; c += 2) {
+        s0 = fma(u[c], y[c], s0);
+        if (c + 1 < NC) s1 = fma(u[c + 1], y[c + 1], s1);
+      }
+      double s = s0 + s1;
+      s += dpp_d<0x140>(s);
+      s += dpp_d<0x141>(s);
+      s += dpp_d<0x4E>(s);
+      s += dpp_d<0xB1>(s);
+      const double f = -lbeta[k0 - q] * s;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) y[c] = fma(f, u[c], y[c]);
     }
   }
-  if (j0 < nvec) back_transform<NC>(y, A, lbeta, n, lane);
-  __syncthreads();  // every wave is done with the reflectors in A
-  store_vecs<NC>(y, A, n, nvec, j0, lane);
-}
-
-// Back-transformation of Y in chunks of 64 vectors (nvec > 64), results in Y.
-template <int NC>
-__device__ __forceinline__ void back_transform_chunks(const double* A, double* Y, const double* lbeta, int n, int nvec, int wave,
-                                      int lane) {
-  for (int cb = 0; cb < nvec; cb += 64) {
-    const int j0 = cb + 8 * wave;
-    if (j0 >= nvec) continue;
-    double y[8][NC];
-    load_vecs<NC>(y, Y, n, nvec, j0, lane);
-    back_transform<NC>(y, A, lbeta, n, lane);
-    store_vecs<NC>(y, Y, n, nvec, j0, lane);
+  if (j < nvec) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int r = 16 * c + l16;
+      if (r < n) Y[(long long)j * n + r] = y[c];
+    }
   }
 }
 
-__global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec, double* __restrict__ a_all,
-                                                                  double* __restrict__ w_all,
-                                                                  double* __restrict__ work_all, int* __restrict__ info) {
+// Workgroup part * (count rounded up to 8) + matrix, so that a matrix stays on the XCD of its
+// tridiagonalisation (workgroup = matrix).
+__global__ __launch_bounds__(64) void eig_back_kernel(int n, int nvec, int count, const double* __restrict__ a_all,
+                                                       double* __restrict__ work_all) {
+  __shared__ double lu[8][kEigMaxN], lbeta[kEigMaxN];
+  const int lane = threadIdx.x;
+  const int stride = (count + 7) & ~7;
+  const int matrix = blockIdx.x % stride, part = blockIdx.x / stride;
+  if (matrix >= count) return;
+  const double* A = a_all + (long long)matrix * n * n;
+  double* work = work_all + (long long)matrix * eig_work_per(n, nvec);
+  double* Y = work + 3 * n;
+  for (int i = lane; i < n; i += 64) lbeta[i] = work[2 * n + i];
+  __syncthreads();
+  const int j = 4 * part + (lane >> 4);
+  switch ((n + 63) >> 6) {
+    case 1: back_transform<4, 8>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    case 2: back_transform<8, 8>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    case 3: back_transform<12, 8>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    case 4: back_transform<16, 8>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    case 5: back_transform<20, 8>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    case 6: back_transform<24, 4>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    case 7: back_transform<28, 4>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+    default: back_transform<32, 4>(A, lbeta, lu, Y, n, nvec, j, lane); break;
+  }
+}
+
+// The vectors to the first rows of A, whose reflectors every wave is done with.
+__global__ __launch_bounds__(kEigThreads) void eig_store_kernel(int n, int nvec, double* __restrict__ a_all,
+                                                                 const double* __restrict__ work_all,
+                                                                 int* __restrict__ info) {
+  double* A = a_all + (long long)blockIdx.x * n * n;
+  const double* Y = work_all + (long long)blockIdx.x * eig_work_per(n, nvec) + 3 * n;
+#pragma unroll 8
+  for (int f = threadIdx.x; f < nvec * n; f += kEigThreads) A[f] = Y[f];
+  if (threadIdx.x == 0) info[blockIdx.x] = 0;
+}
+
+// The trailing block that stays on the chip: its first 256 rows in the
+// workgroup's registers, wave w rows w, w + 8, ... as 64-column chunks of the
+// lower triangle (80 chunks, 160 registers), the last 32 rows in LDS.
+constexpr int kResident = 288;
+constexpr int kResidentBatches = 4;  // of 64 rows, in registers
+constexpr int kResidentTail = kResident - 64 * kResidentBatches;
+constexpr int kResidentCols = (kResident + 63) / 64;
+
+// One chunk of R rows of the pass below: element updates, and the column part
+// of the product; the row part too unless DIAG, the chunk that holds the
+// diagonal, which is kept with both its triangles.
+template <bool DIAG, int R, typename Load, typename Store>
+__device__ __forceinline__ void resident_chunk(const double (&pvj)[R], const double (&pwj)[R], const double (&vj)[R],
+                                               double pv, double pw, double v, double& acc, double (&rs)[8],
+                                               Load load, Store store) {
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const double a = fma(-pwj[r], pv, fma(-pvj[r], pw, load(r)));
+    store(r, a);
+    acc = fma(a, vj[r], acc);
+    if constexpr (!DIAG) rs[r] = fma(a, v, rs[r]);
+  }
+}
+
+// Householder reduction to tridiagonal form on the lower triangle. Step k
+// reflects column k below the diagonal; its rank-2 update of the trailing
+// block is applied in the next step's single pass over the block, which also
+// forms that step's product with the trailing block. nxt holds column k of the
+// matrix as the previous pass left it; lv / lw hold v and w of the current and
+// the previous step. The reflector vectors go to the upper triangle.
+//
+// One workgroup per matrix, so a step is bound by its own chain (two workgroup
+// sums, three barriers) and by the pass. From memory the pass of the 288 x 288
+// block moves 1.2 MB through one CU's L2 port and waits for it in every batch,
+// 8.3 us a step; on the chip it is arithmetic alone, 4.9 us (a 288 x 288 matrix
+// 2.4 -> 1.4 ms). Larger matrices take the pass from memory until the trailing
+// block is that small.
+__global__ __launch_bounds__(kEigThreads) void eig_tridiagonal_kernel(int n, int nvec, double* __restrict__ a_all,
+                                                                       double* __restrict__ work_all) {
   __shared__ double part[kEigWaves][kEigMaxN];
-  __shared__ double lv[2][kEigMaxN], lw[2][kEigMaxN], nxt[kEigMaxN], prow[kEigMaxN], lbeta[kEigMaxN];
-  __shared__ double gm[kEigRegVecs * kGs], li[kEigRegVecs * kGs];
-  __shared__ double red[kEigWaves], red2[2][kEigWaves];
-  __shared__ double bounds[4];
+  __shared__ double lv[2][kEigMaxN], lw[2][kEigMaxN], nxt[kEigMaxN], prow[kEigMaxN];
+  __shared__ double tail[kResidentTail][64 * kResidentCols];
+  __shared__ double red2[2][kEigWaves];
   __shared__ double lsink[64];
+  __shared__ double last;
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  if (nvec == 0) {
-    if (t == 0) info[blockIdx.x] = 0;
-    return;
-  }
   double* A = a_all + (long long)blockIdx.x * n * n;
-  double* w = w_all + (long long)blockIdx.x * n;
-  double* wk = work_all + (long long)blockIdx.x * eig_work_per(n, nvec);
-  double* d = wk;
-  double* e = wk + n;
-  double* beta = wk + 2 * n;
-  double* Y = wk + 3 * n;                // [nvec][n]
-  double* F = Y + (long long)nvec * n;   // [5][n][nvec]: 1 / pivot, U's two superdiagonals, multiplier, swap flag
-  double* Yt = F + 5LL * nvec * n;       // [n][nvec]
-
-  // 1. Householder tridiagonalisation on the lower triangle. Step k reflects column k below the
-  // diagonal; its rank-2 update of the trailing block is applied in the next step's single pass
-  // over the block, which also forms that step's product with the trailing block. nxt holds
-  // column k of the matrix as the previous pass left it; lv / lw hold v and w of the current and
-  // the previous step. The reflector vectors go to the upper triangle.
+  double* d = work_all + (long long)blockIdx.x * eig_work_per(n, nvec);
+  double* e = d + n;
+  double* beta = d + 2 * n;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(A, 0, n * n * 8, 0x00020000);
   for (int i = t; i < n; i += kEigThreads) {
     nxt[i] = A[(long long)i * n];
@@ -483,7 +563,9 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
     lw[1][i] = 0.0;
   }
   __syncthreads();
-  for (int k = 0; k + 2 < n; ++k) {
+  const int M = min(n, kResident);
+  const int s0 = n - M;
+  for (int k = 0; k < s0; ++k) {
     const int m = n - k - 1;
     const int c0 = k + 1;
     const int cur = k & 1;
@@ -501,32 +583,23 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
     const double x0 = nxt[1] - pv[1] * pw0 - pw[1] * pv0;
     const double dk = nxt[0] - 2.0 * pv0 * pw0;
     const double ss = wg_sum1(sq, red2[0]);
-    const double sigma = ss - x0 * x0;
-    double bk = 0.0, ek = x0, v0 = x0;
-    if (sigma > 0.0) {
-      const double norm = sqrt(ss);
-      const double alpha = x0 > 0.0 ? -norm : norm;
-      v0 = x0 - alpha;
-      bk = 2.0 / (sigma + v0 * v0);
-      ek = alpha;
-    }
+    double bk, ek, v0;
+    reflector(ss, x0, bk, ek, v0);
     if (t == 0) {
       d[k] = dk;
       e[k] = ek;
+      beta[k] = bk;
       vv[0] = v0;
     }
-    if (t == k) lbeta[k] = bk;
     const int boff = (c0 * n + c0) * 8;
-    switch ((m + 63) >> 6) {
-      case 1: tri_pass<1>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      case 2: tri_pass<2>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      case 3: tri_pass<3>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      case 4: tri_pass<4>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      case 5: tri_pass<5>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      case 6: tri_pass<6>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      case 7: tri_pass<7>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-      default: tri_pass<8>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink); break;
-    }
+    if (m <= 64 * 5)
+      tri_pass<5>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink);
+    else if (m <= 64 * 6)
+      tri_pass<6>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink);
+    else if (m <= 64 * 7)
+      tri_pass<7>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink);
+    else
+      tri_pass<8>(rsrc, boff, n, m, wave, lane, pv, pw, vv, v0, nxt, part[wave], prow, lsink);
     __syncthreads();
     double p = 0.0, pdv = 0.0, vi = 0.0;
     if (t < m) {
@@ -542,13 +615,170 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
     if (t < m) ww[t] = p - K * vi;
     __syncthreads();
   }
+
+  // The rest on the chip, rows and columns counted from s0 (the pending v and w are too).
+  double val[4 * kResidentBatches * (kResidentBatches + 1)];
+#pragma unroll
+  for (int b = 0; b < kResidentBatches; ++b)
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int c = 0; c <= b; ++c) {
+        const int j = 64 * b + 8 * r + wave, i = 64 * c + lane;
+        const double x = A[(long long)(s0 + min(max(i, j), M - 1)) * n + s0 + min(min(i, j), M - 1)];
+        val[4 * b * (b + 1) + r * (b + 1) + c] = j < M && i < M ? x : 0.0;
+      }
+  for (int r = wave; r < kResidentTail; r += kEigWaves)
+    for (int c = 0; c < kResidentCols; ++c) {
+      const int j = 64 * kResidentBatches + r, i = 64 * c + lane;
+      const double x = A[(long long)(s0 + min(max(i, j), M - 1)) * n + s0 + min(min(i, j), M - 1)];
+      tail[r][i] = j < M && i < M ? x : 0.0;
+    }
+  for (int i = M + t; i < 64 * kResidentCols; i += kEigThreads)  // lanes past the block count as zero
+    lv[0][i] = lv[1][i] = lw[0][i] = lw[1][i] = 0.0;
+  __syncthreads();
+  for (int kk = 0; kk + 2 < M; ++kk) {
+    const int c0 = kk + 1;
+    const int cur = (s0 + kk) & 1;
+    double* vv = lv[cur];
+    double* ww = lw[cur];
+    const double* pv = lv[cur ^ 1];
+    const double* pw = lw[cur ^ 1];
+    const double pv0 = pv[kk], pw0 = pw[kk];
+    double sq = 0.0;
+    if (t < M) {
+      const double x = t > kk ? nxt[t] - pv[t] * pw0 - pw[t] * pv0 : 0.0;
+      vv[t] = x;
+      sq = x * x;
+    }
+    const double x0 = nxt[c0] - pv[c0] * pw0 - pw[c0] * pv0;
+    const double dk = nxt[kk] - 2.0 * pv0 * pw0;
+    const double ss = wg_sum1(sq, red2[0]);
+    double bk, ek, v0;
+    reflector(ss, x0, bk, ek, v0);
+    if (t == c0) {  // readers of vv before the next barrier take v0 at c0
+      d[s0 + kk] = dk;
+      e[s0 + kk] = ek;
+      beta[s0 + kk] = bk;
+      vv[c0] = v0;
+    }
+    const int cc = c0 >> 6, cl = c0 & 63;
+    double acc[kResidentCols];
+#pragma unroll
+    for (int c = 0; c < kResidentCols; ++c) acc[c] = 0.0;
+    double lpv[kResidentCols], lpw[kResidentCols], lvv[kResidentCols];
+#pragma unroll
+    for (int c = 0; c < kResidentCols; ++c) {
+      lpv[c] = pv[64 * c + lane];
+      lpw[c] = pw[64 * c + lane];
+      lvv[c] = vv[64 * c + lane];
+    }
+#pragma unroll
+    for (int c = 0; c < kResidentCols; ++c) {
+      asm volatile("" : "+v"(lvv[c]));  // loads before the selects
+      lvv[c] = 64 * c + lane == c0 ? v0 : lvv[c];
+    }
+    // v, w and the new v of a batch's rows, from the lanes that hold them.
+    auto row_scalars = [&](int b, auto& pvj, auto& pwj, auto& vj) {
+      constexpr int R = sizeof(pvj) / sizeof(double);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        pvj[r] = readlane_d(lpv[b], 8 * r + wave);
+        pwj[r] = readlane_d(lpw[b], 8 * r + wave);
+        vj[r] = readlane_d(lvv[b], 8 * r + wave);
+      }
+    };
+    auto store_sums = [&](const double (&rs)[8], int j0) {
+      const double tot = wave_sums8(rs, lane);
+      const int j = j0 + (lane & 56) + wave;
+      if ((lane & 7) == 0 && j < M) prow[j] = tot;
+    };
+#pragma unroll
+    for (int b = 0; b < kResidentBatches; ++b) {
+      if (64 * b + 63 >= c0 && 64 * b < M) {
+        double pvj[8], pwj[8], vj[8], rs[8];
+        row_scalars(b, pvj, pwj, vj);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) rs[r] = 0.0;
+#pragma unroll
+        for (int c = 0; c <= b; ++c) {
+          if (64 * c + 63 >= c0) {
+            auto load = [&](int r) { return val[4 * b * (b + 1) + r * (b + 1) + c]; };
+            auto store = [&](int r, double a) { val[4 * b * (b + 1) + r * (b + 1) + c] = a; };
+            if (c == b)
+              resident_chunk<true, 8>(pvj, pwj, vj, lpv[c], lpw[c], lvv[c], acc[c], rs, load, store);
+            else
+              resident_chunk<false, 8>(pvj, pwj, vj, lpv[c], lpw[c], lvv[c], acc[c], rs, load, store);
+            if (c == cc && lane == cl) {
+#pragma unroll
+              for (int r = 0; r < 8; ++r) nxt[64 * b + 8 * r + wave] = load(r);
+            }
+          }
+        }
+        if (b > 0 && 64 * b > c0) store_sums(rs, 64 * b);
+      }
+    }
+    if (M > 64 * kResidentBatches) {
+      constexpr int R = kResidentTail / kEigWaves, b = kResidentBatches;
+      double pvj[R], pwj[R], vj[R], rs[8];
+      row_scalars(b, pvj, pwj, vj);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) rs[r] = 0.0;
+#pragma unroll
+      for (int c = 0; c <= b; ++c) {
+        if (64 * c + 63 >= c0) {
+          auto load = [&](int r) { return tail[8 * r + wave][64 * c + lane]; };
+          double* here = &tail[wave][64 * c + lane];
+          double now[R];
+#pragma unroll
+          for (int r = 0; r < R; ++r) now[r] = here[8 * r * 64 * kResidentCols];
+          auto get = [&](int r) { return now[r]; };
+          auto store = [&](int r, double a) { here[8 * r * 64 * kResidentCols] = a; };
+          if (c == b)
+            resident_chunk<true, R>(pvj, pwj, vj, lpv[c], lpw[c], lvv[c], acc[c], rs, get, store);
+          else
+            resident_chunk<false, R>(pvj, pwj, vj, lpv[c], lpw[c], lvv[c], acc[c], rs, get, store);
+          if (c == cc && lane == cl) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) nxt[64 * b + 8 * r + wave] = load(r);
+          }
+        }
+      }
+      if (64 * b > c0) store_sums(rs, 64 * b);
+    }
+#pragma unroll
+    for (int c = 0; c < kResidentCols; ++c)
+      if (64 * c + lane < M) part[wave][64 * c + lane] = acc[c];
+    __syncthreads();
+    double p = 0.0, pdv = 0.0, vi = 0.0;
+    const bool mine = t > kk && t < M;
+    if (mine) {
+      double sacc = 0.0;
+#pragma unroll
+      for (int g = 0; g < kEigWaves; ++g) sacc += part[g][t];
+      p = bk * (t >= 64 && (t & ~63) > c0 ? sacc + prow[t] : sacc);
+      vi = t == c0 ? v0 : vv[t];
+      pdv = p * vi;
+      A[(long long)(s0 + kk) * n + s0 + t] = vi;  // the reflector vector, above the diagonal
+    }
+    const double K = 0.5 * bk * wg_sum1(pdv, red2[1]);
+    if (t < M) ww[t] = mine ? p - K * vi : 0.0;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int b = 0; b < kResidentBatches; ++b)
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (64 * b + 8 * r + wave == M - 1 && lane == ((M - 1) & 63)) last = val[4 * b * (b + 1) + r * (b + 1) + b];
+  if (M > 64 * kResidentBatches && t == 0) last = tail[M - 1 - 64 * kResidentBatches][M - 1];
+  __syncthreads();
   if (t == 0) {
     if (n >= 3) {
       const int cur = (n - 3) & 1;
-      const double v0 = lv[cur][0], v1 = lv[cur][1], w0 = lw[cur][0], w1 = lw[cur][1];
-      d[n - 2] = nxt[0] - 2.0 * v0 * w0;
-      e[n - 2] = nxt[1] - v1 * w0 - w1 * v0;
-      d[n - 1] = A[(long long)(n - 1) * n + n - 1] - 2.0 * v1 * w1;
+      const double v0 = lv[cur][M - 2], v1 = lv[cur][M - 1], w0 = lw[cur][M - 2], w1 = lw[cur][M - 1];
+      d[n - 2] = nxt[M - 2] - 2.0 * v0 * w0;
+      e[n - 2] = nxt[M - 1] - v1 * w0 - w1 * v0;
+      d[n - 1] = last - 2.0 * v1 * w1;
     } else if (n == 2) {
       d[0] = A[0];
       e[0] = A[2];
@@ -556,179 +786,203 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
     } else {
       d[0] = A[0];
     }
-    if (n >= 2) lbeta[n - 2] = 0.0;
+    if (n >= 2) beta[n - 2] = 0.0;
     e[n - 1] = 0.0;
-    lbeta[n - 1] = 0.0;
-    // Gershgorin interval and the pivot guard.
-    double lo = d[0], hi = d[0], emax = 0.0;
-    for (int i = 0; i < n; ++i) {
-      const double r = (i > 0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < n ? fabs(e[i]) : 0.0);
-      lo = fmin(lo, d[i] - r);
-      hi = fmax(hi, d[i] + r);
-      if (i + 1 < n) emax = fmax(emax, e[i] * e[i]);
-    }
-    const double tnorm = fmax(fabs(lo), fabs(hi));
-    bounds[0] = lo - 2.0 * DBL_EPSILON * tnorm - DBL_MIN;
-    bounds[1] = hi + 2.0 * DBL_EPSILON * tnorm + DBL_MIN;
-    bounds[2] = fmax(tnorm, DBL_MIN);
-    bounds[3] = DBL_MIN * fmax(1.0, emax);  // pivmin
+    beta[n - 1] = 0.0;
+  }
+}
+
+__global__ void eig_no_vectors_kernel(int count, int* __restrict__ info) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < count) info[i] = 0;
+}
+
+// Gershgorin interval, |T| and the pivot guard of the tridiagonal matrix, by every wave for itself.
+struct TriBounds {
+  double lo, hi, tnorm, pivmin;
+};
+__device__ TriBounds tri_bounds(const double* d, const double* e, int n, int lane) {
+  double lo = DBL_MAX, hi = -DBL_MAX, emax = 0.0;
+  for (int i = lane; i < n; i += 64) {
+    const double ei = i + 1 < n ? e[i] : 0.0, r = (i > 0 ? fabs(e[i - 1]) : 0.0) + fabs(ei);
+    lo = fmin(lo, d[i] - r);
+    hi = fmax(hi, d[i] + r);
+    emax = fmax(emax, ei * ei);
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o));
+    hi = fmax(hi, __shfl_xor(hi, o));
+    emax = fmax(emax, __shfl_xor(emax, o));
+  }
+  const double tnorm = fmax(fabs(lo), fabs(hi));
+  return TriBounds{lo - 2.0 * DBL_EPSILON * tnorm - DBL_MIN, hi + 2.0 * DBL_EPSILON * tnorm + DBL_MIN,
+                   fmax(tnorm, DBL_MIN), DBL_MIN * fmax(1.0, emax)};
+}
+
+// The nvec lowest eigenvalues by multisection, a wave each: its lanes count at 64 points of the
+// interval, which shrinks 65 times per round (about ten rounds). Bound by the chain of the Sturm
+// recurrence, n steps a round; d and e^2 come from LDS eight steps ahead of it (60 values of a
+// 288 x 288 matrix: 0.13 ms; eight lanes a value need twice the rounds).
+constexpr int kValueWaves = 4;
+__global__ __launch_bounds__(64 * kValueWaves) void eig_values_kernel(int n, int nvec, double* __restrict__ w_all,
+                                                                       const double* __restrict__ work_all) {
+  __shared__ double2 t2[kEigMaxN + 8];  // (d_i, e_{i-1}^2)
+  const int lane = threadIdx.x & 63;
+  const int parts = (nvec + kValueWaves - 1) / kValueWaves;
+  const int matrix = blockIdx.x / parts, part = blockIdx.x % parts;
+  const double* d = work_all + (long long)matrix * eig_work_per(n, nvec);
+  const double* e = d + n;
+  for (int i = threadIdx.x; i < n + 8; i += 64 * kValueWaves) {
+    const double ep = i > 0 && i < n ? e[i - 1] : 0.0;
+    t2[i] = make_double2(i < n ? d[i] : 0.0, ep * ep);
   }
   __syncthreads();
-  const double lo = bounds[0], hi = bounds[1], tnorm = bounds[2], pivmin = bounds[3];
-  for (int i = t; i < n; i += kEigThreads) beta[i] = lbeta[i];
+  const int j = part * kValueWaves + (threadIdx.x >> 6);
+  if (j >= nvec) return;
+  const TriBounds tb = tri_bounds(d, e, n, lane);
+  const double tol = 0.5 * DBL_EPSILON * tb.tnorm;
+  double a = tb.lo, b = tb.hi;
+  for (int it = 0; it < 200; ++it) {
+    if (b - a <= 2.0 * DBL_EPSILON * fmax(fabs(a), fabs(b)) + tol) break;
+    const double x = a + (b - a) * (double)(lane + 1) / 65.0;
+    // count of negative pivots; the first step's e^2 is 0, so its previous pivot does not matter
+    int cnt = 0;
+    double q = 1.0;
+    for (int i0 = 0; i0 < n; i0 += 8) {
+      double2 v[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) v[s] = t2[i0 + s];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        q = (v[s].x - x) - v[s].y * recip(q);
+        if (fabs(q) < tb.pivmin) q = -tb.pivmin;
+        cnt += i0 + s < n && q < 0.0;
+      }
+    }
+    // The first point with count > j bounds the eigenvalue from above.
+    const unsigned long long above = __ballot(cnt > j);
+    const int sf = above ? __builtin_ctzll(above) : 64;
+    const double na = sf == 0 ? a : a + (b - a) * (double)sf / 65.0;
+    const double nb = sf == 64 ? b : a + (b - a) * (double)(sf + 1) / 65.0;
+    a = na;
+    b = nb;
+  }
+  if (lane == 0) w_all[(long long)matrix * n + j] = 0.5 * (a + b);
+}
 
-  // 2. The nvec lowest eigenvalues by multisection: G threads per eigenvalue (consecutive lanes
-  // of one wave) each count at one of G points of the interval, which shrinks G + 1 times per
-  // round; d, e and e^2 from LDS.
-  double* ld = part[0];
-  double* le2 = part[1];
-  double* le = part[2];
-  double* lamv = part[3];
-  for (int i = t; i < n; i += kEigThreads) {
+// Eigenvectors of T, one lane each: the shifts of equal eigenvalues are separated by 10 eps |T|
+// (so that their iterations differ), two inverse iterations from a seeded start with a partially
+// pivoted LU of T - lambda I. A workgroup is one wave with as many vectors as their factors leave
+// room for in LDS, [n][vectors]; every recurrence over n is a serial chain, and from LDS it waits
+// 0.1 us where the same factors in memory cost 0.5 us for each eight steps.
+constexpr int kVectorBytes = 41;  // LDS per vector and row: five doubles and the swap flag
+constexpr int kVectorLds = 48 * 1024;
+__global__ __launch_bounds__(64) void eig_vectors_kernel(int n, int nvec, int per, const double* __restrict__ w_all,
+                                                          double* __restrict__ work_all) {
+  extern __shared__ double vec_lds[];
+  __shared__ double ld[kEigMaxN], le[kEigMaxN], lam_all[kEigMaxN];
+  const int lane = threadIdx.x;
+  const int parts = (nvec + per - 1) / per;
+  const int matrix = blockIdx.x / parts, part = blockIdx.x % parts;
+  const double* d = work_all + (long long)matrix * eig_work_per(n, nvec);
+  const double* e = d + n;
+  double* Y = work_all + (long long)matrix * eig_work_per(n, nvec) + 3 * n;  // [nvec][n]
+  const double* w = w_all + (long long)matrix * n;
+  const int j0 = part * per;
+  const int jn = min(per, nvec - j0);
+  for (int i = lane; i < n; i += 64) {
     ld[i] = d[i];
-    le[i] = e[i];
-    le2[i] = i + 1 < n ? e[i] * e[i] : 0.0;
+    le[i] = i + 1 < n ? e[i] : 0.0;
   }
+  for (int i = lane; i < j0 + jn; i += 64) lam_all[i] = w[i];
+  const double tnorm = tri_bounds(d, e, n, lane).tnorm;
   __syncthreads();
-  {
-    const int G = nvec <= 64 ? 8 : nvec <= 128 ? 4 : nvec <= 256 ? 2 : 1;
-    const int groups = kEigThreads / G;
-    const int s_in = lane % G;      // this thread's point in its group
-    const int gbase = lane - s_in;  // first lane of the group
-    const double tol = 0.5 * DBL_EPSILON * tnorm;
-    for (int jb = 0; jb < nvec; jb += groups) {
-      const int j = jb + t / G;
-      double a = lo, b = hi;
-      for (int it = 0; it < 200; ++it) {
-        const bool done = b - a <= 2.0 * DBL_EPSILON * fmax(fabs(a), fabs(b)) + tol;
-        const double x = a + (b - a) * (double)(s_in + 1) / (double)(G + 1);
-        int cnt = 0;
-        if (j < nvec && !done) {
-          double q = ld[0] - x;
-          if (fabs(q) < pivmin) q = -pivmin;
-          cnt = q < 0.0;
-          for (int i = 1; i < n; ++i) {
-            q = (ld[i] - x) - le2[i - 1] * recip(q);
-            if (fabs(q) < pivmin) q = -pivmin;
-            cnt += q < 0.0;
-          }
-        }
-        // Every lane of the wave takes part in the ballots (a group decides as one).
-        const unsigned long long above = __ballot(cnt > j);
-        const unsigned long long mine = (above >> gbase) & ((1ull << G) - 1);
-        if (__ballot(j < nvec && !done) == 0) break;  // the whole wave is done
-        if (j < nvec && !done) {
-          // The first point with count > j bounds the eigenvalue from above.
-          const int sf = mine ? __builtin_ctzll(mine) : G;
-          const double na = sf == 0 ? a : a + (b - a) * (double)sf / (double)(G + 1);
-          const double nb = sf == G ? b : a + (b - a) * (double)(sf + 1) / (double)(G + 1);
-          a = na;
-          b = nb;
-        }
-      }
-      if (j < nvec && s_in == 0) {
-        w[j] = 0.5 * (a + b);
-        lamv[j] = 0.5 * (a + b);
-      }
-    }
-  }
-  __syncthreads();
-
-  // 3. Eigenvectors of T, one thread each: the shifts of equal eigenvalues are separated by
-  // 10 eps |T| (so that their iterations differ), two inverse iterations from a seeded start
-  // with a partially pivoted LU of T - lambda I. Factors and vectors in [n][nvec] order
-  // (coalesced over the threads), loads in batches of eight.
-  if (t == 0) {
-    double prev = 0.0;
-    for (int j = 0; j < nvec; ++j) {
-      double lam = lamv[j];
-      if (j > 0 && lam - prev < 10.0 * DBL_EPSILON * tnorm) lam = prev + 10.0 * DBL_EPSILON * tnorm;
-      lamv[j] = lam;
+  if (lane == 0) {
+    double prev = lam_all[0];
+    for (int j = 1; j < j0 + jn; ++j) {
+      double lam = lam_all[j];
+      if (lam - prev < 10.0 * DBL_EPSILON * tnorm) lam = prev + 10.0 * DBL_EPSILON * tnorm;
+      lam_all[j] = lam;
       prev = lam;
     }
   }
   __syncthreads();
-  if (t < nvec) {
-    const int j = t;
-    const double lam = lamv[j];
+  double* inv = vec_lds;                 // 1 / pivot
+  double* u1 = inv + (long long)n * per;  // U's two superdiagonals
+  double* u2 = u1 + (long long)n * per;
+  double* mul = u2 + (long long)n * per;
+  double* yv = mul + (long long)n * per;
+  unsigned char* swp = (unsigned char*)(yv + (long long)n * per);
+  if (lane < jn) {
+    const int j = j0 + lane;
+    const double lam = lam_all[j];
     const double tiny = DBL_EPSILON * tnorm;
-    auto fi = [&](int f, int k) { return ((long long)f * n + k) * nvec + j; };
     double p0 = ld[0] - lam, p1 = n > 1 ? le[0] : 0.0;
     for (int k = 0; k + 1 < n; ++k) {
-      const double c = le[k];                                                // below the diagonal
+      const double c = le[k];                                              // below the diagonal
       const double a1 = ld[k + 1] - lam, b1 = k + 2 < n ? le[k + 1] : 0.0;  // the next row
-      if (fabs(c) > fabs(p0)) {
-        const double mult = p0 / c;
-        F[fi(0, k)] = 1.0 / c;
-        F[fi(1, k)] = a1;
-        F[fi(2, k)] = b1;
-        F[fi(3, k)] = mult;
-        F[fi(4, k)] = 1.0;
-        p0 = p1 - mult * a1;
-        p1 = -mult * b1;
-      } else {
-        if (fabs(p0) < tiny) p0 = p0 < 0.0 ? -tiny : tiny;
-        const double mult = c / p0;
-        F[fi(0, k)] = 1.0 / p0;
-        F[fi(1, k)] = p1;
-        F[fi(2, k)] = 0.0;
-        F[fi(3, k)] = mult;
-        F[fi(4, k)] = 0.0;
-        p0 = a1 - mult * p1;
-        p1 = b1;
-      }
+      const bool swap = fabs(c) > fabs(p0);
+      if (!swap && fabs(p0) < tiny) p0 = p0 < 0.0 ? -tiny : tiny;
+      const double piv = swap ? c : p0, rest = swap ? p0 : c;
+      const double mult = rest / piv;
+      const int at = k * per + lane;
+      inv[at] = 1.0 / piv;
+      u1[at] = swap ? a1 : p1;
+      u2[at] = swap ? b1 : 0.0;
+      mul[at] = mult;
+      swp[at] = swap;
+      p0 = swap ? p1 - mult * a1 : a1 - mult * p1;
+      p1 = swap ? -mult * b1 : b1;
     }
     if (fabs(p0) < tiny) p0 = p0 < 0.0 ? -tiny : tiny;
-    F[fi(0, n - 1)] = 1.0 / p0;
-    F[fi(1, n - 1)] = 0.0;
-    F[fi(2, n - 1)] = 0.0;
+    inv[(n - 1) * per + lane] = 1.0 / p0;
+    u1[(n - 1) * per + lane] = 0.0;
+    u2[(n - 1) * per + lane] = 0.0;
     double scale = 1.0;
 #pragma unroll
     for (int iter = 0; iter < 2; ++iter) {
       // Forward elimination of the right-hand side (the seeded start, or the previous iterate
       // times scale), then back substitution; scale makes the result unit length.
-      double carry = iter == 0 ? start_entry(j, 0) : Yt[j] * scale;
+      double carry = iter == 0 ? start_entry(j, 0) : yv[lane] * scale;
       for (int k0 = 0; k0 + 1 < n; k0 += 8) {
-        double lmv[8], pvv[8], yn[8];
+        double lmv[8], yn[8];
+        bool sw[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const int k = min(k0 + s, n - 2);
-          lmv[s] = F[fi(3, k)];
-          pvv[s] = F[fi(4, k)];
-          yn[s] = iter == 0 ? start_entry(j, k + 1) : Yt[(long long)(k + 1) * nvec + j] * scale;
+          lmv[s] = mul[k * per + lane];
+          sw[s] = swp[k * per + lane];
+          yn[s] = iter == 0 ? start_entry(j, k + 1) : yv[(k + 1) * per + lane] * scale;
         }
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const int k = k0 + s;
           if (k + 1 < n) {
-            double yk = carry, yk1 = yn[s];
-            if (pvv[s] != 0.0) {
-              yk = yn[s];
-              yk1 = carry;
-            }
-            Yt[(long long)k * nvec + j] = yk;
+            const double yk = sw[s] ? yn[s] : carry, yk1 = sw[s] ? carry : yn[s];
+            yv[k * per + lane] = yk;
             carry = yk1 - lmv[s] * yk;
           }
         }
       }
-      Yt[(long long)(n - 1) * nvec + j] = carry;
+      yv[(n - 1) * per + lane] = carry;
       double nrm = 0.0, x1 = 0.0, x2 = 0.0;  // x_{i+1}, x_{i+2}
       for (int i0 = n - 1; i0 >= 0; i0 -= 8) {
-        double yv[8], a1[8], a2[8], rr[8];
+        double yy[8], a1[8], a2[8], rr[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-          const int i = max(i0 - s, 0);
-          yv[s] = Yt[(long long)i * nvec + j];
-          rr[s] = F[fi(0, i)];
-          a1[s] = F[fi(1, i)];
-          a2[s] = F[fi(2, i)];
+          const int at = max(i0 - s, 0) * per + lane;
+          yy[s] = yv[at];
+          rr[s] = inv[at];
+          a1[s] = u1[at];
+          a2[s] = u2[at];
         }
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const int i = i0 - s;
           if (i >= 0) {
-            const double xi = (yv[s] - a1[s] * x1 - a2[s] * x2) * rr[s];
-            Yt[(long long)i * nvec + j] = xi;
+            const double xi = (yy[s] - a1[s] * x1 - a2[s] * x2) * rr[s];
+            yv[i * per + lane] = xi;
             nrm += xi * xi;
             x2 = x1;
             x1 = xi;
@@ -737,29 +991,32 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
       }
       scale = nrm > 0.0 ? 1.0 / sqrt(nrm) : 0.0;
     }
-    for (int i0 = 0; i0 < n; i0 += 8) {
-      double yv[8];
-#pragma unroll
-      for (int s = 0; s < 8; ++s) yv[s] = Yt[(long long)min(i0 + s, n - 1) * nvec + j];
-#pragma unroll
-      for (int s = 0; s < 8; ++s)
-        if (i0 + s < n) Y[(long long)j * n + i0 + s] = yv[s] * scale;
-    }
+    lam_all[lane] = scale;  // the eigenvalues are in registers by now
   }
   __syncthreads();
+  for (int q = 0; q < jn; ++q)
+    for (int i = lane; i < n; i += 64) Y[(long long)(j0 + q) * n + i] = yv[i * per + q] * lam_all[q];
+}
 
-  // 4. Orthonormalisation and back-transformation x = Q y = H_0 (H_1 (... H_{n-3} y)).
-  const int nc = (n + 63) >> 6;
+// Orthonormalisation of the vectors, one workgroup per matrix.
+__global__ __launch_bounds__(kEigThreads) void eig_orthonormal_kernel(int n, int nvec, double* __restrict__ work_all) {
+  __shared__ double part[kEigMaxN];
+  __shared__ double gm[kEigRegVecs * kGs], li[kEigRegVecs * kGs], rows[2][2 * kEigRegVecs];
+  __shared__ double red[kEigWaves];
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  double* Y = work_all + (long long)blockIdx.x * eig_work_per(n, nvec) + 3 * n;  // [nvec][n]
   if (nvec <= kEigRegVecs) {
-    switch (nc) {
-      case 1: finish_in_registers<1>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      case 2: finish_in_registers<2>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      case 3: finish_in_registers<3>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      case 4: finish_in_registers<4>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      case 5: finish_in_registers<5>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      case 6: finish_in_registers<6>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      case 7: finish_in_registers<7>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
-      default: finish_in_registers<8>(A, Y, lbeta, gm, li, n, nvec, wave, lane); break;
+    switch ((n + 63) >> 6) {
+      case 1: orthonormalise<1>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      case 2: orthonormalise<2>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      case 3: orthonormalise<3>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      case 4: orthonormalise<4>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      case 5: orthonormalise<5>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      case 6: orthonormalise<6>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      case 7: orthonormalise<7>(Y, gm, li, rows, n, nvec, wave, lane); break;
+      default: orthonormalise<8>(Y, gm, li, rows, n, nvec, wave, lane); break;
     }
   } else {
     // Gram-Schmidt in order: vector j minus its components along vectors 0 .. j - 1 (dots by
@@ -773,12 +1030,12 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
           for (int i = lane; i < n; i += 64) sdot += z[i] * y[i];
 #pragma unroll
           for (int o = 32; o >= 1; o >>= 1) sdot += __shfl_xor(sdot, o);
-          if (lane == 0) part[0][k] = sdot;
+          if (lane == 0) part[k] = sdot;
         }
         __syncthreads();
         for (int i = t; i < n; i += kEigThreads) {
           double v = y[i];
-          for (int k = 0; k < j; ++k) v -= part[0][k] * Y[(long long)k * n + i];
+          for (int k = 0; k < j; ++k) v -= part[k] * Y[(long long)k * n + i];
           y[i] = v;
         }
         __syncthreads();
@@ -790,20 +1047,7 @@ __global__ __launch_bounds__(kEigThreads) void eig_lowest_kernel(int n, int nvec
       for (int i = t; i < n; i += kEigThreads) y[i] *= inv;
       __syncthreads();
     }
-    switch (nc) {
-      case 1: back_transform_chunks<1>(A, Y, lbeta, n, nvec, wave, lane); break;
-      case 2: back_transform_chunks<2>(A, Y, lbeta, n, nvec, wave, lane); break;
-      case 3: back_transform_chunks<3>(A, Y, lbeta, n, nvec, wave, lane); break;
-      case 4: back_transform_chunks<4>(A, Y, lbeta, n, nvec, wave, lane); break;
-      case 5: back_transform_chunks<5>(A, Y, lbeta, n, nvec, wave, lane); break;
-      case 6: back_transform_chunks<6>(A, Y, lbeta, n, nvec, wave, lane); break;
-      case 7: back_transform_chunks<7>(A, Y, lbeta, n, nvec, wave, lane); break;
-      default: back_transform_chunks<8>(A, Y, lbeta, n, nvec, wave, lane); break;
-    }
-    __syncthreads();
-    for (long long f = t; f < (long long)nvec * n; f += kEigThreads) A[f] = Y[f];
   }
-  if (t == 0) info[blockIdx.x] = 0;
 }
 
 }  // namespace
@@ -834,9 +1078,26 @@ int hfjk_eigh_lowest_batched(hfjk_ctx* ctx, int n, int count, int nvec, double* 
   }
   hipError_t err = hipSetDevice(ctx->device);
   if (err == hipSuccess) {
-    hipLaunchKernelGGL(eig_lowest_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n, nvec,
-                       a, w, work, info);
-    err = hipGetLastError();
+    if (nvec == 0) {
+      hipLaunchKernelGGL(eig_no_vectors_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                         count, info);
+      err = hipGetLastError();
+    } else {
+      hipLaunchKernelGGL(eig_tridiagonal_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n,
+                         nvec, a, work);
+      hipLaunchKernelGGL(eig_values_kernel, dim3((unsigned)(count * ((nvec + kValueWaves - 1) / kValueWaves))),
+                         dim3(64 * kValueWaves), 0, (hipStream_t)stream, n, nvec, w, work);
+      const int per = std::max(1, std::min(std::min(nvec, 64), kVectorLds / (kVectorBytes * n)));
+      hipLaunchKernelGGL(eig_vectors_kernel, dim3((unsigned)(count * ((nvec + per - 1) / per))), dim3(64),
+                         (size_t)kVectorBytes * n * per, (hipStream_t)stream, n, nvec, per, w, work);
+      hipLaunchKernelGGL(eig_orthonormal_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n,
+                         nvec, work);
+      hipLaunchKernelGGL(eig_back_kernel, dim3((unsigned)((count + 7) / 8 * 8 * ((nvec + 3) / 4))), dim3(64), 0,
+                         (hipStream_t)stream, n, nvec, count, a, work);
+      hipLaunchKernelGGL(eig_store_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n, nvec, a,
+                         work, info);
+      err = hipGetLastError();
+    }
   }
   if (err != hipSuccess) {
     hfjk_internal_set_error((std::string("eig_lowest_kernel launch: ") + hipGetErrorString(err)).c_str());

@@ -96,3 +96,15 @@ def test_no_vectors_leaves_the_matrices():
     mats = g + g.transpose(0, 2, 1)
     _, a = _solve(mats, 0, full=True)
     np.testing.assert_array_equal(a, mats)
+
+
+@pytest.mark.parametrize("n,nvec,count", [(4, 3, 9), (31, 31, 1), (63, 5, 2), (193, 64, 2), (255, 33, 1), (256, 4, 1),
+                                          (257, 61, 1), (288, 64, 2), (289, 13, 1), (291, 65, 1), (321, 7, 2),
+                                          (449, 30, 1), (96, 96, 17)])
+def test_sizes_around_the_resident_block_and_the_register_chunks(n, nvec, count):
+    """Rows in registers (256), in LDS (288) and in memory, 64-column chunks, part-filled vector groups."""
+    rng = np.random.default_rng(7 * n + nvec)
+    g = rng.standard_normal((count, n, n))
+    mats = g + g.transpose(0, 2, 1)
+    w, x = _solve(mats, nvec)
+    _check(mats, nvec, w, x)
