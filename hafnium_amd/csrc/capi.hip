@@ -981,11 +981,17 @@ int density_factor(hfjk_ctx* ctx, const double* density, void* workspace, const 
   {
     Stage st(ctx, s, "density_cholesky");
     check_hip(hfjk::launch_pchol_init(density, n, 1e-12, e, pst, s), "pivoted Cholesky launch");
-    // Columns in batches of 32 steps; the state is read back after each batch.
-    constexpr int kBatch = 32;
-    for (int k0 = 0; k0 <= n; k0 += kBatch) {
-      for (int k = k0; k < std::min(k0 + kBatch, n + 1); ++k)
-        check_hip(hfjk::launch_pchol_step(density, n, k, a, e, pst, s), "pivoted Cholesky launch");
+    // Columns in batches of 32 steps (64 in panels of one launch, where a step costs less than the
+    // check); the state is read back after each batch.
+    for (int k0 = 0, batch; k0 <= n; k0 += batch) {
+      const bool panel = hfjk::pchol_in_panels(n, std::min(k0 + 64, n + 1));
+      batch = panel ? 64 : 32;
+      const int k1 = std::min(k0 + batch, n + 1);
+      if (panel)
+        check_hip(hfjk::launch_pchol_panel(density, n, k0, k1, a, e, pst, s), "pivoted Cholesky launch");
+      else
+        for (int k = k0; k < k1; ++k)
+          check_hip(hfjk::launch_pchol_step(density, n, k, a, e, pst, s), "pivoted Cholesky launch");
       check_hip(hipMemcpyAsync(&host_st, pst, sizeof(host_st), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
       check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
       if (host_st.stop) break;

@@ -260,6 +260,10 @@ hipError_t launch_pchol_init(const double* density, int nao, double tol, double*
                              hipStream_t s);
 hipError_t launch_pchol_step(const double* density, int nao, int k, double* l, double* diag, PcholState* st,
                              hipStream_t s);
+// Whether steps up to column k1 go in panels of one launch, and one such panel.
+bool pchol_in_panels(int nao, int k1);
+hipError_t launch_pchol_panel(const double* density, int nao, int k0, int k1, double* l, double* diag, PcholState* st,
+                              hipStream_t s);
 hipError_t launch_factor_residual(const double* density, int nao, const double* l, const PcholState* st,
                                   unsigned long long* residual, hipStream_t s);
 hipError_t launch_compact_factor(const double* l, int nao, int r, double* c, double* signs, hipStream_t s);

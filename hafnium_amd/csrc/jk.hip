@@ -268,11 +268,13 @@ __global__ __launch_bounds__(kThreads) void split_factor_kernel(const double* __
 // per step: D = L L^T with L stored by columns (l[k][i] = L[i][k], column
 // stride n), column k pivoted on the largest remaining diagonal r_p,
 // L[i][k] = (D[p][i] - sum_{j<k} L[i][j] L[p][j]) / sqrt(r_p), r -= L[:,k]^2,
-// stopping once that diagonal is <= tol * (largest initial diagonal). Each
-// step is two launches (the pivot in one workgroup, the column across the
-// GPU), and the state lives on the device so the host checks it only
-// every few steps.
+// stopping once that diagonal is <= tol * (largest initial diagonal). The
+// state lives on the device so the host checks it only every few steps. While
+// the columns so far are few (pchol_in_panels) one workgroup takes several
+// steps per launch; past that each step is two launches (the pivot in one
+// workgroup, the column across the GPU).
 constexpr int kPcholThreads = 1024;
+constexpr int kPcholPanelRows = 4096, kPcholPanelColumns = 512;
 
 // diag = diag(D); st: cut = tol * max diag, no stop, rank 0. One workgroup.
 __global__ __launch_bounds__(kPcholThreads) void pchol_init_kernel(const double* __restrict__ d, int n, double tol,
@@ -365,6 +367,111 @@ __global__ __launch_bounds__(kThreads) void pchol_column_kernel(const double* __
   }
 }
 
+// Largest value of the 16 lanes of a row / of the wave, in every lane.
+__device__ __forceinline__ double row_max(double v) {
+  v = fmax(v, dpp_d<0x140>(v));
+  v = fmax(v, dpp_d<0x141>(v));
+  v = fmax(v, dpp_d<0x4E>(v));
+  return fmax(v, dpp_d<0xB1>(v));
+}
+__device__ __forceinline__ double wave_max(double v) {
+  v = fmax(v, __shfl_xor(v, 32));
+  return row_max(fmax(v, __shfl_xor(v, 16)));
+}
+// The lowest `at` among the lanes that hold one (0x7FFFFFFF: none does).
+__device__ __forceinline__ int lowest_index(bool holds, int at) {
+  const unsigned long long who = __ballot(holds);
+  if (who == 0) return 0x7FFFFFFF;
+  if ((who & (who - 1)) == 0) return __builtin_amdgcn_readlane(at, __builtin_ctzll(who));
+  int low = holds ? at : 0x7FFFFFFF;
+  for (int off = 32; off > 0; off >>= 1) low = min(low, __shfl_xor(low, off));
+  return low;
+}
+
+// Columns k0 .. k1 - 1 by one workgroup, the remaining diagonal in LDS. Groups
+// of threads (as many as rows of 64 threads leave room for) split the sum over
+// the earlier columns. A step is bound by its chain (pivot, the pivot row of
+// L, the columns, the column's store): 4.3 us in the first 64 of a 501 x 501
+// density, where two launches with their gaps take 10 (90 columns: 1.0 -> 0.55
+// ms).
+__global__ __launch_bounds__(kPcholThreads) void pchol_panel_kernel(const double* __restrict__ d, int n, int k0, int k1,
+                                                                   double* l, double* __restrict__ diag,
+                                                                   PcholState* __restrict__ st) {
+  __shared__ double ldiag[kPcholPanelRows], lp[kPcholPanelColumns], red[kPcholThreads];
+  __shared__ double wval[kPcholThreads / 64];
+  __shared__ int widx[kPcholThreads / 64];
+  if (st->stop) return;
+  const double cut = st->cut;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int width = min(kPcholThreads, (n + 63) & ~63);
+  const int groups = kPcholThreads / width;
+  const int group = t / width, first = t % width;
+  for (int i = t; i < n; i += kPcholThreads) ldiag[i] = diag[i];
+  __syncthreads();
+  for (int k = k0; k < k1; ++k) {
+    double best = -1.0;
+    int at = n;
+    for (int i = t; i < n; i += kPcholThreads) {
+      const double v = ldiag[i];
+      if (v > best) {
+        best = v;
+        at = i;
+      }
+    }
+    // The largest, then the lowest index among its holders: of the wave, then of the waves.
+    const double wbest = wave_max(best);
+    const int wat = lowest_index(best == wbest, at);
+    if (lane == 0) {
+      wval[wave] = wbest;
+      widx[wave] = wat;
+    }
+    __syncthreads();
+    best = row_max(wval[lane & 15]);
+    at = lowest_index(lane < 16 && wval[lane & 15] == best, widx[lane & 15]);
+    if (k >= n || at >= n || !(best > cut)) {  // the same in every thread
+      if (t == 0) {
+        st->stop = 1;
+        st->rank = k;
+      }
+      break;
+    }
+    const double inv = 1.0 / sqrt(best);
+    for (int j = t; j < k; j += kPcholThreads) lp[j] = l[(long long)j * n + at];
+    __syncthreads();
+    for (int r0 = 0; r0 < n; r0 += width) {  // one round unless n > 1024, and then one group
+      const int row = r0 + first;
+      const double dv = group == 0 && row < n ? d[(long long)at * n + row] : 0.0;
+      double s = 0.0;
+      if (group < groups && row < n) {
+        double p[4] = {0.0, 0.0, 0.0, 0.0};
+        // Sixteen columns in flight; those past k are the last one with a zero factor.
+        for (int j = group; j < k; j += 16 * groups) {
+          double x[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) x[u] = l[(long long)min(j + u * groups, k - 1) * n + row];
+#pragma unroll
+          for (int u = 0; u < 16; ++u)
+            p[u & 3] = fma(x[u], j + u * groups < k ? lp[min(j + u * groups, k - 1)] : 0.0, p[u & 3]);
+        }
+        s = (p[0] + p[1]) + (p[2] + p[3]);
+      }
+      if (groups > 1) {
+        red[t] = s;
+        __syncthreads();
+        if (group == 0)
+          for (int g = 1; g < groups; ++g) s += red[g * width + first];
+      }
+      if (group == 0 && row < n) {
+        const double v = (dv - s) * inv;
+        l[(long long)k * n + row] = v;
+        ldiag[row] -= v * v;
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = t; i < n; i += kPcholThreads) diag[i] = ldiag[i];
+}
+
 // max |D[i][j] - sum_{k < rank} L[i][k] L[j][k]| into *out (bits of a
 // non-negative double, atomic max; L by columns as above); rank read from
 // the device.
@@ -418,6 +525,19 @@ hipError_t launch_pchol_step(const double* density, int nao, int k, double* l, d
   const long long threads = 4LL * nao;
   hipLaunchKernelGGL(pchol_column_kernel, dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0,
                      s, density, nao, k, l, diag, st);
+  return hipGetLastError();
+}
+
+// One workgroup reads the k earlier columns of a step (8 n k bytes) through
+// its own cache port: up to 120000 elements in less than the 10 us of a step
+// of two launches.
+bool pchol_in_panels(int nao, int k1) {
+  return nao <= kPcholPanelRows && k1 <= kPcholPanelColumns && (long long)nao * k1 <= 120000;
+}
+
+hipError_t launch_pchol_panel(const double* density, int nao, int k0, int k1, double* l, double* diag, PcholState* st,
+                              hipStream_t s) {
+  hipLaunchKernelGGL(pchol_panel_kernel, dim3(1), dim3(kPcholThreads), 0, s, density, nao, k0, k1, l, diag, st);
   return hipGetLastError();
 }
 

@@ -149,3 +149,25 @@ def test_batched_dots(length):
         for a in range(slots if length else 0):
             bound = length * 2.3e-16 * float(np.abs(h[2, i] * h[a, i]).sum())
             assert abs(float(dots[i, a]) - float((h[2, i] * h[a, i]).sum())) <= bound
+
+
+@pytest.mark.parametrize("nao,rank", [(1, 1), (2, 2), (63, 1), (64, 63), (65, 64), (192, 65), (193, 128), (512, 130),
+                                      (513, 40), (700, 200), (1025, 150)])
+def test_density_factor_in_panels_and_in_steps(nao, rank):
+    """Every number of thread groups, panels that end at, before and after the rank, and the change to steps."""
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+
+    naux = 3
+    b = synthetic.tensor_full(5, naux, nao)
+    rng = np.random.default_rng(nao + rank)
+    c = rng.standard_normal((nao, rank)) * np.geomspace(1.0, 0.1, rank)
+    d = c @ c.T
+    jk = MI355XCoulombExchange(b)
+    k = jk.exchange(d)
+    x = b @ c
+    expect = np.tensordot(x, x, axes=((0, 2), (0, 2)))
+    # The factor's residual, checked by the library, is at most 1e-11 max |D|, and
+    # each element of D enters K through products of two rows of B.
+    rows = np.abs(b).sum(axis=2)
+    assert np.all(np.abs(k - expect) <= 2e-11 * np.abs(d).max() * np.einsum("qm,qn->mn", rows, rows))
+    np.testing.assert_array_equal(k, k.T)
