@@ -127,7 +127,7 @@ struct Layout {
   // only the bf16 planes of C^T), and the J partials
   size_t qt, qg, qc, qj, q_end;
   size_t total;
-  int nsplit_j, nsplit_k, nslot_k, ldo, xrows, npairs;
+  int nsplit_j, nsplit_k, nslot_k, run_k, ldo, xrows, npairs;
   long long p, ntiles;
 };
 
@@ -143,10 +143,12 @@ Layout make_layout(const hfjk_ctx* ctx, int nocc, int precision, int nsplit_k = 
   (void)nb;
   L.npairs = hfjk::syrk_pairs(n);
   L.nsplit_j = coulomb_splits(L.ntiles, naux);
+  L.run_k = nsplit_k > 0 ? hfjk::syrk_run_aux(precision, L.ldo)
+                         : hfjk::syrk_run_for(precision, naux, n, L.ldo, ctx->cus);
   L.nsplit_k = nsplit_k > 0 ? nsplit_k
                : ctx->syrk_splits > 0 ? ((ctx->syrk_splits + 7) / 8) * 8
-                                       : hfjk::syrk_split_count(precision, naux, n, L.ldo, ctx->cus);
-  L.nslot_k = hfjk::syrk_slots(precision, naux, L.ldo, L.nsplit_k);
+                                       : hfjk::syrk_split_count(precision, naux, n, L.ldo, L.run_k, ctx->cus);
+  L.nslot_k = hfjk::syrk_slots(naux, L.run_k, L.nsplit_k);
   size_t off = 0;
   const size_t nn = (size_t)n * n;
   L.dens_a = off; off = align_up(off + nn * 8);
@@ -330,7 +332,7 @@ void exchange_back(hfjk_ctx* ctx, int nocc, bool is_signed, double* out, int pre
   void* part = at<void>(ws, L.xp);
   {
     Stage st(ctx, s, "exchange_syrk");
-    check_hip(hfjk::launch_syrk(x, precision, ctx->naux, ctx->nao, L.ldo, sg, is_signed, L.nsplit_k, part,
+    check_hip(hfjk::launch_syrk(x, precision, ctx->naux, ctx->nao, L.ldo, sg, is_signed, L.nsplit_k, L.run_k, part,
                                 ctx->syrk_kind, s, nullptr, 0, x16_interleaved(ctx, precision, is_signed, L.ldo), nocc),
               "syrk launch");
   }
@@ -389,7 +391,7 @@ GeneralLayout general_layout(const hfjk_ctx* ctx, int precision, int rank, int p
   G.npairs = hfjk::syrk_pairs(ctx->nao);
   // Split counts capped so the two partial sets stay small for small matrices.
   G.nsplit = std::min(syrk_splits(G.npairs, pc), std::max(8, ((512 / G.npairs + 7) / 8) * 8));
-  G.nslot = hfjk::syrk_slots(precision, pc, G.ld, G.nsplit);
+  G.nslot = hfjk::syrk_slots(pc, hfjk::syrk_run_aux(precision, G.ld), G.nsplit);
   const size_t tile2 = (size_t)hfjk::syrk_tile() * hfjk::syrk_tile();
   size_t off = base;
   G.hz = off; off = align_up(off + n * n * 16);
@@ -520,7 +522,8 @@ void exchange_general(hfjk_ctx* ctx, const double* density, double* out, int pre
     for (int q0 = 0; q0 < naux; q0 += pc) {
       const int qc = std::min(pc, naux - q0);
       const int nsplit = std::min(syrk_splits(G.npairs, qc), G.nsplit);
-      const int nslot = hfjk::syrk_slots(precision, qc, ld, nsplit);
+      const int run = hfjk::syrk_run_aux(precision, ld);
+      const int nslot = hfjk::syrk_slots(qc, run, nsplit);
       {
         Stage st(ctx, s, "general_half_transform");
         if (full && split) {
@@ -545,8 +548,8 @@ void exchange_general(hfjk_ctx* ctx, const double* density, double* out, int pre
       }
       {
         Stage st(ctx, s, "general_syrk");
-        check_hip(hfjk::launch_syrk(x, precision, qc, n, ld, sym, true, nsplit, p1, 0, s), "syrk launch");
-        check_hip(hfjk::launch_syrk(x, precision, qc, n, ld, cross, true, nsplit, p2, 0, s, nullptr, hb),
+        check_hip(hfjk::launch_syrk(x, precision, qc, n, ld, sym, true, nsplit, run, p1, 0, s), "syrk launch");
+        check_hip(hfjk::launch_syrk(x, precision, qc, n, ld, cross, true, nsplit, run, p2, 0, s, nullptr, hb),
                   "syrk launch");
       }
       {
@@ -891,7 +894,15 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
     double* parts = at<double>(workspace, L.qt);
     double* gamma = at<double>(workspace, L.qg);
     double* jp = at<double>(workspace, L.qj);
-    const bool serial = ctx->coulomb_serial != 0;
+    // Fork and join of the side stream cost 40 us, and the Coulomb kernels beside the SYRK have a
+    // capped grid. FP64: the whole GPU serves either half nearly as well alone; on the launch
+    // stream nao 24 takes 32 us for 75, 264 / nocc 55 363 us for 375, 600 / nocc 30 2.1 ms for 2.6,
+    // 1500 / nocc 100 27.3 ms for 27.7, and only where the SYRK is long is beside it better: 1000 /
+    // nocc 200 (0.7e12 products) equal, 1500 / nocc 250 58.5 ms for 59.7. The FP32 and BF16x3 SYRK
+    // leave more of the memory's time unused: 144 / nocc 30 (3e8 products) 65 us for 74 on the
+    // launch stream, 192 / nocc 40 (1e9) 104 for 95, 336 / nocc 70 601 for 524.
+    const double products = (double)ctx->naux * ctx->nao * ctx->nao * nocc;
+    const bool serial = ctx->coulomb_serial != 0 || products < (precision == HFJK_FP64 ? 7e11 : 4e8);
     if (ctx->side == nullptr && !serial) {
       check_hip(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking), "hipStreamCreateWithFlags");
       check_hip(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming), "hipEventCreateWithFlags");
@@ -900,8 +911,8 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
     hipStream_t side = serial ? s : ctx->side;
     exchange_front(ctx, orbitals, nocc, nullptr, true, precision, workspace, L, s);
     // The Coulomb half needs only X and the padded orbitals: it runs on the
-    // side stream (HBM-bound) while the SYRK (MFMA-bound) runs on s, or with
-    // coulomb_serial on s after the SYRK. Its buffers (charges, J partials)
+    // side stream (HBM-bound) while the SYRK (MFMA-bound) runs on s, or serially
+    // on s after the SYRK. Its buffers (charges, J partials)
     // lie outside the regions the SYRK uses.
     if (serial) {
       exchange_back(ctx, nocc, false, exchange, precision, workspace, L, s);
@@ -1339,9 +1350,9 @@ bool kpoint_exchange_psd(hfjk_ctx* ctx, int nk, int naux, int n, const double* t
       {
         Stage st(ctx, s, "kpoint_syrk");
         const double* sig = signature + (long long)b0 * naux;
-        check_hip(hfjk::launch_syrk(x, HFJK_FP64, blocks * naux, n, ldo, sym, true, kc * c, p1, 0, s, sig, 0, false, 0, n),
+        check_hip(hfjk::launch_syrk(x, HFJK_FP64, blocks * naux, n, ldo, sym, true, kc * c, 0, p1, 0, s, sig, 0, false, 0, n),
                   "k-point syrk launch");
-        check_hip(hfjk::launch_syrk(x, HFJK_FP64, blocks * naux, n, ldo, cross, true, kc * c, p2, 0, s, sig, hb, false, 0,
+        check_hip(hfjk::launch_syrk(x, HFJK_FP64, blocks * naux, n, ldo, cross, true, kc * c, 0, p2, 0, s, sig, hb, false, 0,
                                     n),
                   "k-point syrk launch");
         check_hip(hfjk::launch_syrk_reduce_complex((const double*)p1, (const double*)p2, c, n, kc, k2 > 0,
@@ -1510,7 +1521,7 @@ int hfjk_kpoint_exchange(hfjk_ctx* ctx, int nk, int naux, int nao, const void* t
         }
         {
           Stage st(ctx, s, "kpoint_syrk");
-          check_hip(hfjk::launch_syrk(x, HFJK_FP64, naux, 2 * n, ldo, sg, true, L.nsplit, part, 0, s, sig),
+          check_hip(hfjk::launch_syrk(x, HFJK_FP64, naux, 2 * n, ldo, sg, true, L.nsplit, 0, part, 0, s, sig),
                     "k-point syrk launch");
           check_hip(hfjk::launch_syrk_reduce(part, HFJK_FP64, L.nsplit, 2 * n, hfjk::syrk_tile(), kh, s), "k-point reduce launch");
           check_hip(hfjk::launch_kp_fold(kh, n, true, (char*)exchange + 16 * k1 * nn, s), "k-point fold launch");

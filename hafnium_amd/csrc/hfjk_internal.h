@@ -88,7 +88,7 @@ struct hfjk_ctx {
   int x_full = 0;
   int general_chunk = 0;  // aux functions per chunk of the non-symmetric exchange (0 = fit)
   int side_groups = 0;    // grid cap of the Coulomb kernels beside the SYRK in hfjk_jk_occ (0 = default)
-  int coulomb_serial = 0; // hfjk_jk_occ: 1 = the Coulomb half after the SYRK on the launch stream
+  int coulomb_serial = 0; // hfjk_jk_occ: 1 = always the Coulomb half after the SYRK on the launch stream
   int cus = 256;          // compute units of the device
   // Second stream of hfjk_jk_occ (default priority, created on first use):
   // the Coulomb half runs there beside the SYRK, fenced by fork/join events.
@@ -280,23 +280,25 @@ hipError_t launch_half_transform(const void* b, int precision, long long p, int 
 // lets the direct-LDS kernel skip them.
 // Partials: FP64 keeps one 128 x 128 tile per split and lower tile pair
 // (blocks above the diagonal or past nao may be left unwritten);
-// the FP32-accumulating modes (FP32, BF16x3) one per run of
-// syrk_run_aux(precision, ldo) aux functions (at most kSyrkRunProducts
-// products per FP32 accumulator, whatever the split count).
+// the FP32-accumulating modes (FP32, BF16x3) one per run of `run` aux
+// functions (at most syrk_run_aux(precision, ldo), kSyrkRunProducts products
+// per FP32 accumulator, whatever the split count; 0 in FP64).
+// syrk_run_for = the run of a build of that size on `cus` compute units.
 // syrk_slots = the number of partial tiles per pair; launch_syrk_reduce sums
 // them in FP64 in a fixed order.
 constexpr int kSyrkRunProducts = 4096;
 int syrk_run_aux(int precision, int ldo);
-int syrk_slots(int precision, int naux, int ldo, int nsplit);
+int syrk_run_for(int precision, int naux, int nao, int ldo, int cus);
+int syrk_slots(int naux, int run, int nsplit);
 // Default split count of the unsigned SYRK (a multiple of 8) on a device of `cus` compute units.
-int syrk_split_count(int precision, int naux, int nao, int ldo, int cus);
+int syrk_split_count(int precision, int naux, int nao, int ldo, int run, int cus);
 // auxsign (optional, [naux]): one more factor per aux function on the signed
 // FP64/FP32 direct-LDS kernels; shift (a multiple of 32 below ldo): the
 // second operand's columns rotated, sum_k X[m][k] S_k X[n][(k + shift) mod
 // ldo], on the signed direct-LDS kernels of every precision
 // (hipErrorInvalidValue for a launch that would not run them).
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
-                       bool is_signed, int nsplit, void* partial, int kind, hipStream_t s,
+                       bool is_signed, int nsplit, int run, void* partial, int kind, hipStream_t s,
                        const double* auxsign = nullptr, int shift = 0, bool x_ilv = false, int nocc = 0,
                        int xrows = 0);
 // nocc (0 = ldo): X's columns past it are zero and may be skipped. xrows

@@ -2630,16 +2630,16 @@ static int tile_blocks(int nblk, int eb, int r, int c) {
 // size, and at nao 709 / naux 2503 in FP32 left 25 of 104 splits without a
 // slot.) The last answer is kept per thread: a program asks for one shape
 // many times.
-int syrk_split_count(int precision, int naux, int nao, int ldo, int cus) {
+int syrk_split_count(int precision, int naux, int nao, int ldo, int run, int cus) {
   struct Last {
-    int precision = -1, naux = 0, nao = 0, ldo = 0, cus = 0, splits = 0;
+    int precision = -1, naux = 0, nao = 0, ldo = 0, run = 0, cus = 0, splits = 0;
   };
   static thread_local Last last;
-  if (last.precision == precision && last.naux == naux && last.nao == nao && last.ldo == ldo && last.cus == cus)
+  if (last.precision == precision && last.naux == naux && last.nao == nao && last.ldo == ldo && last.run == run &&
+      last.cus == cus)
     return last.splits;
   const int nblk = (nao + 15) / 16, eb = syrk_row_block(nao) / 16;
   const int nb = (nblk + 7) / 8, npairs = nb * (nb + 1) / 2;
-  const int run = syrk_run_aux(precision, ldo);
   const int nslot = run == 0 ? naux : (naux + run - 1) / run;
   const double chunk_steps = (double)(run == 0 ? 1 : run) * ldo / (precision == HFJK_FP64 ? 8 : 16);
   const double partial_us = npairs * 2.0 * kSyrkTile * kSyrkTile * 8.0 / 5e6;
@@ -2673,7 +2673,7 @@ int syrk_split_count(int precision, int naux, int nao, int ldo, int cus) {
       best = 8 * n8;
     }
   }
-  last = Last{precision, naux, nao, ldo, cus, best};
+  last = Last{precision, naux, nao, ldo, run, cus, best};
   return best;
 }
 
@@ -2792,24 +2792,32 @@ int syrk_run_aux(int precision, int ldo) {
   return std::max(1, kSyrkRunProducts / std::max(ldo, 1));
 }
 
-int syrk_slots(int precision, int naux, int ldo, int nsplit) {
-  const int run = syrk_run_aux(precision, ldo);
-  return run == 0 ? nsplit : (naux + run - 1) / run;
+// A run is one workgroup's least work, and runs of 4096 products leave a small
+// build a handful of workgroups (nao 96 / naux 336 / nocc 20: 3 runs of 128
+// aux functions, 225 us). Shorter runs only add FP64 sums of partial tiles, so
+// they go down to a workgroup per CU, and no further than 128 columns of X,
+// eight ring steps, where filling the ring costs as much as the products.
+int syrk_run_for(int precision, int naux, int nao, int ldo, int cus) {
+  const int most = syrk_run_aux(precision, ldo);
+  if (most == 0) return 0;
+  const long long even = ((long long)naux * syrk_pairs(nao) + cus - 1) / cus;
+  return (int)std::max(1LL, std::min<long long>(most, std::max<long long>(even, (128 + ldo - 1) / ldo)));
 }
+
+int syrk_slots(int naux, int run, int nsplit) { return run == 0 ? nsplit : (naux + run - 1) / run; }
 
 bool syrk16_tiles256(int nao, int ldo, bool is_signed, int kind, int shift) {
   return !is_signed && shift == 0 && kind != 1 && kind != 2 && ldo <= kDmaMaxLdo &&
-         (long long)x_rows(nao) * ldo * 2 < (1LL << 31) && syrk_run_aux(HFJK_BF16X3, ldo) > 0;
+         (long long)x_rows(nao) * ldo * 2 < (1LL << 31);
 }
 
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
-                       bool is_signed, int nsplit, void* partial, int kind, hipStream_t s, const double* auxsign,
-                       int shift, bool x_ilv, int nocc, int xrows) {
+                       bool is_signed, int nsplit, int run, void* partial, int kind, hipStream_t s,
+                       const double* auxsign, int shift, bool x_ilv, int nocc, int xrows) {
   if (xrows <= 0) xrows = x_rows(nao);
   const int edge = syrk_edge(precision, nao, ldo, is_signed, kind);
   if (nocc <= 0 || nocc > ldo) nocc = ldo;
   const int npairs = syrk_pairs(nao);
-  const int run = syrk_run_aux(precision, ldo);
   // Per-aux signs are applied by the signed FP64/FP32 direct-LDS kernels only; a column shift by
   // the signed direct-LDS kernels of every precision.
   const bool ring_ok = is_signed && kind != 1 && ldo <= kDmaMaxLdo && (long long)xrows * ldo < (1LL << 30);

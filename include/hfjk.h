@@ -355,7 +355,8 @@ HFJK_API int hfjk_ddot(hfjk_ctx *ctx, long long n, const double *x, const double
  * compute unit in FP64, no cap in FP32 and BF16X3, whose shorter SYRK would
  * not hide the capped kernels).
  * HFJK_TUNE_COULOMB_SERIAL: hfjk_jk_occ runs its Coulomb half 0 = on a
- * second stream beside the SYRK, 1 = on the launch stream after the SYRK.
+ * second stream beside the SYRK where the build is large enough, 1 = always on
+ * the launch stream after the SYRK.
  * Set by the project's autotuner (hafnium_amd/autotune.py); the workspace size
  * depends on HFJK_TUNE_SYRK_SPLITS, so query it after tuning. No counterpart
  * in the reference. */

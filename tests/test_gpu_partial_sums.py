@@ -171,3 +171,27 @@ def test_density_factor_in_panels_and_in_steps(nao, rank):
     rows = np.abs(b).sum(axis=2)
     assert np.all(np.abs(k - expect) <= 2e-11 * np.abs(d).max() * np.einsum("qm,qn->mn", rows, rows))
     np.testing.assert_array_equal(k, k.T)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16x3"])
+@pytest.mark.parametrize("nao,naux,nocc", [(9, 1, 1), (24, 84, 5), (96, 336, 20), (130, 257, 33), (192, 512, 64),
+                                           (192, 672, 40), (300, 700, 130)])
+def test_short_runs_of_the_single_precision_syrk(precision, nao, naux, nocc):
+    """Runs from four aux functions to 4096 products, one workgroup per run or several runs, both stream orders."""
+    from hafnium_amd import _lib
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+    from tests.tolerances import BF16X3_REL_TOL, FP32_REL_TOL
+
+    b = synthetic.tensor_full(11, naux, nao)
+    c = synthetic.occupied_orbitals(11, nao, nocc)
+    x = b @ c
+    k_ref = np.tensordot(x, x, axes=((0, 2), (0, 2)))
+    j_ref = np.tensordot(np.einsum("qmi,mi->q", x, c), b, axes=(0, 0))
+    tol = FP32_REL_TOL if precision == "fp32" else BF16X3_REL_TOL
+    jk = MI355XCoulombExchange(b, precision=precision)
+    for splits, serial in ((0, 0), (0, 1), (8, 0), (200, 0)):
+        jk.set_tuning(_lib.TUNE_SYRK_SPLITS, splits)
+        jk.set_tuning(_lib.TUNE_COULOMB_SERIAL, serial)
+        j, k = jk.jk_occupied(c)
+        assert np.max(np.abs(k - k_ref)) <= tol * np.max(np.abs(k_ref))
+        assert np.max(np.abs(j - j_ref)) <= tol * np.max(np.abs(j_ref))
