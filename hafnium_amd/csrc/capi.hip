@@ -903,11 +903,7 @@ int hfjk_jk_occ(hfjk_ctx* ctx, const double* orbitals, int nocc, double* coulomb
     // launch stream, 192 / nocc 40 (1e9) 104 for 95, 336 / nocc 70 601 for 524.
     const double products = (double)ctx->naux * ctx->nao * ctx->nao * nocc;
     const bool serial = ctx->coulomb_serial != 0 || products < (precision == HFJK_FP64 ? 7e11 : 4e8);
-    if (ctx->side == nullptr && !serial) {
-      check_hip(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking), "hipStreamCreateWithFlags");
-      check_hip(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming), "hipEventCreateWithFlags");
-      check_hip(hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming), "hipEventCreateWithFlags");
-    }
+    if (!serial) check_hip(hfjk::side_stream(ctx), "side stream");
     hipStream_t side = serial ? s : ctx->side;
     exchange_front(ctx, orbitals, nocc, nullptr, true, precision, workspace, L, s);
     // The Coulomb half needs only X and the padded orbitals: it runs on the

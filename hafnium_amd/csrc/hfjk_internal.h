@@ -15,6 +15,7 @@
 #include <stddef.h>
 
 #include <string>
+#include <mutex>
 #include <vector>
 
 #include "../../include/hfjk.h"
@@ -90,7 +91,7 @@ struct hfjk_ctx {
   int side_groups = 0;    // grid cap of the Coulomb kernels beside the SYRK in hfjk_jk_occ (0 = default)
   int coulomb_serial = 0; // hfjk_jk_occ: 1 = always the Coulomb half after the SYRK on the launch stream
   int cus = 256;          // compute units of the device
-  // Second stream of hfjk_jk_occ (default priority, created on first use):
+  // Second stream of hfjk_jk_occ and of the integrals (default priority, created on first use):
   // the Coulomb half runs there beside the SYRK, fenced by fork/join events.
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr;
@@ -101,6 +102,18 @@ struct hfjk_ctx {
 };
 
 namespace hfjk {
+// Creates the context's side stream and its events on first use.
+inline hipError_t side_stream(hfjk_ctx* ctx) {
+  static std::mutex guard;
+  std::lock_guard<std::mutex> hold(guard);
+  if (ctx->side != nullptr) return hipSuccess;
+  hipError_t e = hipSuccess;
+  if (ctx->fork == nullptr) e = hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming);
+  if (e == hipSuccess && ctx->join == nullptr) e = hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking);
+  return e;
+}
+
 // Persistent work fetch: the workgroup's next item of phase `ph`. Items are
 // dealt in eight shares [total x / 8, total (x + 1) / 8), one per XCD (x =
 // blockIdx.x % 8, so an instance's items stay in one XCD's L2); once its own

@@ -1487,6 +1487,14 @@ struct DeviceArena {
   }
 };
 
+struct CallEvent {
+  hipEvent_t event = nullptr;
+  hipError_t create() { return hipEventCreateWithFlags(&event, hipEventDisableTiming); }
+  ~CallEvent() {
+    if (event != nullptr) (void)hipEventDestroy(event);
+  }
+};
+
 void device_shells(const std::vector<Shell>& shells, std::vector<DShell>& out, std::vector<double>& exps,
                    std::vector<double>& coefs) {
   for (const Shell& s : shells) {
@@ -1527,8 +1535,17 @@ struct LaneArgs {
   double* out;
 };
 
+// The launch stream and the context's side stream, which takes the launches
+// that do not fill the chip (kFillWaves waves, 16 per CU): the classes of high
+// angular momentum have long lanes and few of them, 120 waves of 130 us for
+// (4, 4) of 12 water molecules, 0.9 ms of 3.1 in all.
+constexpr long long kFillWaves = 4096;
+struct Streams {
+  hipStream_t main, side;
+};
+
 template <int LAB, int LC>
-void launch_aux(const LaneArgs& a, hipStream_t s) {
+void launch_aux(const LaneArgs& a, Streams st) {
   const unsigned per = (unsigned)(a.nblk * a.nchunk);
   const int most = (int)((1u << 28) / per);  // pairs per launch
   for (int first = 0; first < a.npairs;) {
@@ -1537,6 +1554,7 @@ void launch_aux(const LaneArgs& a, hipStream_t s) {
                        : split              ? (kLaneWaves - 1) * kLaneRows * 512
                                             : 0;
     const int np = std::min(most, (split ? a.nsplit : a.npairs) - first);  // one kind of workgroup per launch
+    hipStream_t s = (long long)np * per * (split ? kLaneWaves : 1) < kFillWaves ? st.side : st.main;
     hipLaunchKernelGGL((aux_kernel<LAB, LC>), dim3(np * per), dim3(split ? 64 * kLaneWaves : 64), lds, s,
                        a.pairs + first, a.counts + first, a.prims, a.w, a.fns, a.sph, a.boys_tab, a.nblk, a.nchunk, a.n,
                        a.metric_mode, a.out);
@@ -1546,14 +1564,14 @@ void launch_aux(const LaneArgs& a, hipStream_t s) {
 }
 
 template <int LAB, int LC = 0>
-void launch_aux_c(int lc, const LaneArgs& a, hipStream_t s) {
+void launch_aux_c(int lc, const LaneArgs& a, Streams s) {
   if constexpr (LC <= kLaneMaxC && LAB + LC <= kLaneMaxL) {
     if (lc == LC) return launch_aux<LAB, LC>(a, s);
     launch_aux_c<LAB, LC + 1>(lc, a, s);
   }
 }
 
-void launch_aux_any(int lab, int lc, const LaneArgs& a, hipStream_t s) {
+void launch_aux_any(int lab, int lc, const LaneArgs& a, Streams s) {
   switch (lab) {
     case 0: return launch_aux_c<0>(lc, a, s);
     case 1: return launch_aux_c<1>(lc, a, s);
@@ -1565,7 +1583,7 @@ void launch_aux_any(int lab, int lc, const LaneArgs& a, hipStream_t s) {
 
 // The integrals of the shell pairs (pair_list: b < 0 for the unit function)
 // with every aux shell (up to the pair's own shell for the metric).
-void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux,
+void launch_triples(hfjk_ctx* ctx, const std::vector<Shell>& orb, const std::vector<Shell>& aux,
                     const std::vector<std::pair<int, int>>& pair_list, const std::vector<double>& norm_o,
                     const std::vector<double>& norm_x, int n, bool metric_mode, double* out, hipStream_t s) {
   static const std::vector<double> boys_host = boys_table();
@@ -1668,18 +1686,39 @@ void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux
                o_off = dev.put(sph_off), o_boys = dev.put(boys_host), o_pairs = dev.put(pairs), o_fns = dev.put(fns);
   const size_t o_counts = dev.reserve<int>(pairs.size()), o_prims = dev.reserve<LanePrim>((size_t)ptotal),
                o_w = dev.reserve<double>((size_t)wtotal);
+  auto check = [](hipError_t e) {
+    if (e != hipSuccess) throw std::runtime_error("streams of the integral kernels failed");
+  };
+  check(hfjk::side_stream(ctx));
+  hipStream_t side = ctx->side;
+  // The side stream after everything on s so far, and s after the side stream; events of this
+  // call's own, so that calls of several threads on one context do not wait for each other's.
+  CallEvent forked, joined;
+  check(forked.create());
+  check(joined.create());
+  auto fork = [&] {
+    check(hipEventRecord(forked.event, s));
+    check(hipStreamWaitEvent(side, forked.event, 0));
+  };
+  auto join = [&] {
+    check(hipEventRecord(joined.event, side));
+    check(hipStreamWaitEvent(s, joined.event, 0));
+  };
   dev.upload(s);
+  fork();
   const size_t total = metric_mode ? (size_t)n * n : (size_t)norm_x.size() * n * n;
   // Pairs that do not survive stay zero; the metric has none.
   if (!metric_mode && hipMemsetAsync(out, 0, total * sizeof(double), s) != hipSuccess)
     throw std::runtime_error("hipMemsetAsync failed");
   if (!pairs.empty()) {
-    hipLaunchKernelGGL(pair_kernel, dim3((unsigned)pairs.size()), dim3(kPairThreads), 0, s, dev.at<LanePair>(o_pairs),
+    hipLaunchKernelGGL(pair_kernel, dim3((unsigned)pairs.size()), dim3(kPairThreads), 0, side, dev.at<LanePair>(o_pairs),
                        dev.at<DShell>(metric_mode ? o_aux : o_orb), dev.at<DShell>(o_orb), dev.at<double>(o_exps),
                        dev.at<double>(o_coefs), dev.at<double>(metric_mode ? o_nx : o_no), dev.at<double>(o_sph),
                        dev.at<int>(o_off), dev.at<int>(o_counts), dev.at<LanePrim>(o_prims), dev.at<double>(o_w));
     if (hipGetLastError() != hipSuccess) throw std::runtime_error("launch of the integral pair kernel failed");
   }
+  join();
+  fork();
   for (int l = kLaneMaxAB; l >= 0; --l)
     for (int c = kLaneMaxC; c >= 0; --c) {
       const int np = first[l + 1] - first[l], nblk = fblock[c + 1] - fblock[c];
@@ -1688,7 +1727,7 @@ void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux
                  dev.at<double>(o_w), dev.at<LaneAux>(o_fns) + (size_t)fblock[c] * 64,
                  dev.at<double>(o_sph) + sph_off[c], dev.at<double>(o_boys), np, split[l], nblk, chunks[l], n,
                  metric_mode ? 1 : 0, out};
-      launch_aux_any(l, c, a, s);
+      launch_aux_any(l, c, a, Streams{s, side});
     }
   // At most 2^31 - 1 workgroups per launch.
   const size_t per = (size_t)1 << 30;
@@ -1700,6 +1739,7 @@ void launch_triples(const std::vector<Shell>& orb, const std::vector<Shell>& aux
                        dev.at<double>(o_boys), n, metric_mode ? 1 : 0, out);
     if (hipGetLastError() != hipSuccess) throw std::runtime_error("launch of the integral kernel failed");
   }
+  join();
   // The tables are freed on return: wait for the kernels that read them.
   if (hipStreamSynchronize(s) != hipSuccess) throw std::runtime_error("the integral kernel failed");
 }
@@ -1741,7 +1781,7 @@ int hfjk_int2c2e_device(hfjk_ctx* ctx, const hfjk_basis* aux, double* metric, vo
     std::vector<std::pair<int, int>> pairs;
     for (int i = 0; i < (int)sh.size(); ++i) pairs.emplace_back(i, -1);
     if (hipSetDevice(ctx->device) != hipSuccess) throw std::runtime_error("hipSetDevice failed");
-    launch_triples(sh, sh, pairs, nm, nm, n, true, metric, (hipStream_t)stream);
+    launch_triples(ctx, sh, sh, pairs, nm, nm, n, true, metric, (hipStream_t)stream);
   });
 }
 
@@ -1760,7 +1800,7 @@ int hfjk_int3c2e_device(hfjk_ctx* ctx, const hfjk_basis* aux, const hfjk_basis* 
       for (int j = 0; j <= i; ++j)
         if (pair_survives(so[i], so[j])) pairs.emplace_back(i, j);
     if (hipSetDevice(ctx->device) != hipSuccess) throw std::runtime_error("hipSetDevice failed");
-    launch_triples(so, sx, pairs, nmo, nmx, n, false, out, (hipStream_t)stream);
+    launch_triples(ctx, so, sx, pairs, nmo, nmx, n, false, out, (hipStream_t)stream);
   });
 }
 
