@@ -29,6 +29,16 @@ struct hfjk_batch {
   size_t bytes = 0;
   void* ws = nullptr;
   int grid_mfma = 0;
+  // Second stream of builds with densities (bind creates it where the plan uses it): the Coulomb
+  // half beside the half-transform.
+  bool beside = false;
+  hipStream_t side = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
+  ~hfjk_batch() {
+    if (fork != nullptr) (void)hipEventDestroy(fork);
+    if (join != nullptr) (void)hipEventDestroy(join);
+    if (side != nullptr) (void)hipStreamDestroy(side);
+  }
 };
 
 namespace hfjk {
@@ -468,6 +478,10 @@ void fill_items(hfjk::BatchView& v, const std::vector<long long>& prefix) {
   for (int ph = 0; ph < hfjk::kPhCount; ++ph) v.items[ph] = prefix[(size_t)ph * (v.ninst + 1) + v.ninst];
 }
 
+// Bytes of B from which the Coulomb half runs beside the half-transform (its two passes over B then
+// take ten times the 40 us of fork and join).
+constexpr double kBesideBytes = 1e9;
+
 size_t al256(size_t v) { return (v + 255) & ~size_t(255); }
 
 }  // namespace
@@ -658,6 +672,7 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
   off = al256(off + (size_t)(precision == HFJK_FP64 ? 8 : 4) * kp);
   bt->bytes = off;
   bt->grid_mfma = ((2 * cus + 7) / 8) * 8;
+  bt->beside = (double)bt->b_total * (precision == HFJK_FP64 ? 8 : 4) > kBesideBytes;
   *out = bt;
   return HFJK_OK;
 }
@@ -703,6 +718,11 @@ int hfjk_batch_bind(hfjk_batch* batch, void* workspace, size_t bytes, void* stre
     e = hipMemcpyAsync(ws + batch->off_prefix, batch->prefix.data(), sizeof(long long) * batch->prefix.size(),
                        hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess && batch->beside && batch->side == nullptr) {
+    if (batch->fork == nullptr) e = hipEventCreateWithFlags(&batch->fork, hipEventDisableTiming);
+    if (e == hipSuccess && batch->join == nullptr) e = hipEventCreateWithFlags(&batch->join, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&batch->side, hipStreamNonBlocking);
+  }
   if (e != hipSuccess) {
     hfjk_internal_set_error((std::string("uploading the batch plan: ") + hipGetErrorString(e)).c_str());
     return HFJK_ERR_HIP;
@@ -736,8 +756,16 @@ int hfjk_batch_run(hfjk_batch* batch, const void* tensor, const double* orbitals
   const int prec = batch->precision;
   hipError_t e = hipSetDevice(batch->ctx->device);
   if (e == hipSuccess) e = hfjk::launch_batch_reset(v, s);
+  // With densities the Coulomb half needs nothing of the exchange: it streams B beside the
+  // matrix-core-bound half-transform, whose waves leave register room for its own (128 FP64
+  // instances to 220 functions 45.9 -> 42.2 ms; 96 to 220, FP32 3.66 -> 3.44, BF16x3 3.85 -> 3.59).
+  const bool beside = density != nullptr && batch->side != nullptr;
+  hipStream_t cs = beside ? batch->side : s;
+  if (e == hipSuccess && beside) e = hipEventRecord(batch->fork, s);
+  if (e == hipSuccess && beside) e = hipStreamWaitEvent(cs, batch->fork, 0);
   if (e == hipSuccess && density != nullptr)
-    e = hfjk::launch_batch_coulomb(v, prec, tensor, batch->b_total, density, ws64, coulomb, s);
+    e = hfjk::launch_batch_coulomb(v, prec, tensor, batch->b_total, density, ws64, coulomb, cs);
+  if (e == hipSuccess && beside) e = hipEventRecord(batch->join, cs);
   if (e == hipSuccess)
     e = hfjk::launch_batch_orbitals(v, prec, orbitals, ws64, cbase, batch->cp_total, s);
   if (e == hipSuccess)
@@ -750,6 +778,7 @@ int hfjk_batch_run(hfjk_batch* batch, const void* tensor, const double* orbitals
   if (e == hipSuccess)
     e = hfjk::launch_batch_syrk(v, prec, xbase, batch->x_total, ws64, kbase, batch->grid_mfma, s);
   if (e == hipSuccess) e = hfjk::launch_batch_syrk_reduce(v, prec, kbase, exchange, s);
+  if (e == hipSuccess && beside) e = hipStreamWaitEvent(s, batch->join, 0);
   if (e != hipSuccess) {
     hfjk_internal_set_error((std::string("batched launch: ") + hipGetErrorString(e)).c_str());
     return HFJK_ERR_HIP;

@@ -93,3 +93,35 @@ def test_graph_replays_match_eager_runs(torch):
         # Eager work between replays must not disturb the next replay.
         bt.run(c, d, precision="fp64")
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "bf16x3"])
+def test_coulomb_half_beside_the_half_transform(torch, precision):
+    """A tensor past 1e9 bytes: the Coulomb half on the batch's side stream, eagerly, back to back and in replays."""
+    from hafnium_amd.batch import BatchedCoulombExchange
+
+    shapes = [(300, 1000 if precision == "fp64" else 2000, 20)] * 2 + [(290, 1000, 33), (40, 140, 8)]
+    seeds = [3000, 3001, 3002, 3003]
+    bt = BatchedCoulombExchange(shapes)
+    bt.generate(seeds)
+    cs = [synthetic.occupied_orbitals(s, n, o) for s, (n, q, o) in zip(seeds, shapes)]
+    c, d = bt.pack_orbitals(cs), bt.pack_matrices([x @ x.T for x in cs])
+    j_x, k_x = bt.run(c, precision=precision)  # occupied form: one stream
+    j_x, k_x = j_x.clone(), k_x.clone()
+    for _ in range(3):  # each build's fork waits for the one before
+        j0, k0 = bt.run(c, d, precision=precision)
+    j0, k0 = j0.clone(), k0.clone()
+    assert torch.equal(k0, k_x)
+    for i in range(len(shapes)):
+        a, b = bt.matrix(j0, i), bt.matrix(j_x, i)
+        assert float((a - b).abs().max()) <= TOL[precision] * float(b.abs().max())
+    graph, (j, k) = bt.capture(c, d, precision=precision)
+    for _ in range(3):
+        j.zero_()
+        k.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(j, j0) and torch.equal(k, k0)
+        bt.run(c, d, precision=precision)
+        torch.cuda.synchronize()
