@@ -614,11 +614,11 @@ def main(argv=None):
         achieved = x_flops / (x_ms * 1e-3) / 1e12
         peak = PEAK_TFLOPS[head]
         tile = (main_entry.get("tuning") or {}).get("x_bn") or (256 if o > 128 else 128)
-        rows = (main_entry.get("tuning") or {}).get("x_bm") or 64
-        if tile > 128:
-            rows = 64
-        w2 = "_w2" if (tile, rows) == (128, 128) else ""  # the FP64 128 x 128 tile's two-wave variant
-        kernel = {"fp64": f"xform_kernel{w2}<double, {tile}, {rows}>", "fp32": f"xform_kernel<float, {tile}, {rows}>",
+        # The packed FP64 / FP32 kernel is named by its 16-column blocks per group.
+        blocks16 = (o + 15) // 16
+        groups = -(-blocks16 // {32: 2, 64: 4}.get(tile, 8))
+        per_group = -(-blocks16 // groups)
+        kernel = {"fp64": f"xform_units_kernel<double, {per_group}>", "fp32": f"xform_units_kernel<float, {per_group}>",
                   "bf16x3": f"xform_bf16x3_kernel<{tile}>"}[head]
         # B bytes per launch: the packed lower triangle, or with the full copy both triangles.
         b_bytes = q * n * (n + 1) / 2 * (8 if head == "fp64" else 4)

@@ -1,8 +1,8 @@
 """Autotuner of the exchange kernels' tile schedule.
 
 For a bound tensor, an occupied width and a precision it times every
-candidate tile of the half-transform (column tile, and for FP64/FP32 the
-64- or 128-row tile) and every candidate SYRK split count with the
+candidate tile of the half-transform (column tile, and for FP64/FP32 two
+or four waves per workgroup) and every candidate SYRK split count with the
 library's HIP-event stage timers, keeps the fastest of each
 (the two kernels are independent: the split count only moves the SYRK, the
 tile only the half-transform) and leaves them set on the context. Results are
@@ -137,7 +137,7 @@ def autotune(jk, orbitals, precision: str = "fp64", *, repeats: int = 2, cache_p
         jk.set_tuning(_lib.TUNE_SYRK_SPLITS, best_split)
     finally:
         jk.profile(False)
-    # Tile labels: "BN" for 64-row tiles, "BNx128" for 128-row tiles.
+    # Tile labels: "BN" for two waves per workgroup, "BNx128" for four.
     label = lambda t: str(t[0]) if t[1] == 64 else f"{t[0]}x{t[1]}"  # noqa: E731
     result = TuningResult(key, best_tile[0], best_split, {label(k): v for k, v in x_ms.items()},
                           {str(k): v for k, v in syrk_ms.items()}, time.perf_counter() - start, False, best_tile[1])

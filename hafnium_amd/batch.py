@@ -4,7 +4,7 @@ Each instance i has its fitted tensor ``B_i [naux_i, nao_i, nao_i]`` (tiled
 packed, laid end to end in one batch tensor), its occupied orbitals
 ``C_i [nao_i, nocc_i]`` and density ``D_i``; one run computes every
 ``J_i = sum_P B_i[P] <B_i[P], D_i>`` and ``K_i = sum_P (B_i[P] C_i)(B_i[P] C_i)^T``
-with one persistent kernel launch per phase (``hfjk_batch_run``), which a
+with one kernel launch per phase (``hfjk_batch_run``), which a
 hipGraph can capture (:meth:`BatchedCoulombExchange.capture`).
 
 The single-instance counterpart is ``MI355XCoulombExchange``; the reference
@@ -241,7 +241,7 @@ class BatchedCoulombExchange:
         """A hipGraph (``torch.cuda.CUDAGraph``) of one batched build and its output buffers.
 
         The plan and tensor copy are prepared before capture; the captured work
-        is the counter reset and the persistent phase kernels only. The graph
+        is the counter reset and the phase kernels only. The graph
         addresses the plan's workspace, the tensor copy and the input buffers
         by pointer, so it holds references to all of them: a later ``plan`` with
         another tile or ``release`` drops the batch's own references, and the

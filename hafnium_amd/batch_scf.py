@@ -1,7 +1,7 @@
 """Batched restricted Hartree-Fock: many molecules converged together on one GPU.
 
 Every iteration advances all molecules at once: one batched DF-J/K build
-(``BatchedCoulombExchange``: one persistent launch per phase for every
+(``BatchedCoulombExchange``: one launch per phase for every
 molecule), strided-batched GEMMs and a batched eigensolver on matrices
 zero-padded to the largest basis (for the Fock matrices the library's
 one-launch solver of the occupied eigenpairs, ``hfjk_eigh_lowest_batched``;

@@ -16,8 +16,9 @@ Drop-ins for the reference's periodic builders (hafnium/scf/coulomb_exchange.py:
 The tensors live in HBM as complex128; the contractions run in the HIP
 kernels of ``libhfjk.so`` (``hfjk_kpoint_coulomb`` / ``hfjk_kpoint_exchange``):
 the Coulomb charges and J as streaming complex reductions, the exchange of
-each (k, k') block through its real form on the FP64 direct-LDS
-half-transform and the signed SYRK. FP64 only.
+ranges of (k, k') blocks on an FP64 half-transform of the complex rows and
+the signed SYRK (of one block through its real form where a density is not
+positive semidefinite). FP64 only.
 """
 
 from __future__ import annotations

@@ -216,7 +216,7 @@ HFJK_API int hfjk_general_workspace_bytes(hfjk_ctx *ctx, int precision, int aux_
 HFJK_API int hfjk_exchange_general(hfjk_ctx *ctx, const double *density, double *exchange, int precision,
                                    void *workspace, size_t workspace_bytes, void *stream);
 
-/* ---- Batched J/K: many instances of uneven size, one persistent launch per phase ----
+/* ---- Batched J/K: many instances of uneven size, one launch per phase ----
  * No counterpart in the reference (it builds one molecule's J/K at a time:
  * coulomb_exchange.py:176-190 per call). For instance i:
  *   J_i = sum_P B_i[P] <B_i[P], D_i>,   K_i = sum_P (B_i[P] C_i)(B_i[P] C_i)^T.
@@ -402,12 +402,12 @@ HFJK_API long long hfjk_dsyev_batched_work(int n, int count);
 HFJK_API int hfjk_dsyev_batched(hfjk_ctx *ctx, int n, int count, double *a, double *w, double *work, int *info,
                                 int method, void *stream);
 /* The lowest eigenpairs of count symmetric [n][n] matrices at stride n*n
- * (row-major, n <= 512), one workgroup per matrix: Householder
- * tridiagonalisation, multisection on the Sturm count for the nvec lowest
+ * (row-major, n <= 512): Householder tridiagonalisation (one workgroup per
+ * matrix), multisection on the Sturm count for the nvec lowest
  * eigenvalues (w[i][0 .. nvec), ascending; w is [count][n], its other
  * entries untouched), inverse iteration and orthonormalisation for their
  * eigenvectors, which become rows 0 .. nvec - 1 of each matrix (its other
- * rows are left as scratch). One launch, no allocation: work is device
+ * rows are left as scratch). Six launches, no allocation: work is device
  * scratch of hfjk_eigh_lowest_batched_work(n, count, nvec) doubles; info[i]
  * is set to 0. Replaces the rocSOLVER call of hfjk_dsyev_batched where only
  * the occupied orbitals are needed (the batched SCF); no counterpart in the
@@ -541,7 +541,10 @@ HFJK_API int hfjk_mlp_to_bf16(hfjk_ctx *ctx, long long count, const float *src, 
  *   J(k) = sum_P s[k,k,P] c_P B[k,k,P].
  * hfjk_kpoint_exchange: K(k) = sum_k' w_k' sum_P s[k,k',P] B[k,k',P] D(k')
  *   B[k,k',P]^H + madelung S(k) D(k) S(k) for Hermitian D(k') (1e-12
- *   relative, else HFJK_ERR_INPUT): D(k') = V diag(l) V^H by rocSOLVER zheevd
+ *   relative, else HFJK_ERR_INPUT). Positive semidefinite D(k') with weights
+ *   > 0 factorise by pivoted Cholesky and go through the half-transform of the
+ *   complex rows and the signed SYRK over ranges of blocks, at most 1 GiB of X
+ *   at a time. Otherwise D(k') = V diag(l) V^H by rocSOLVER zheevd
  *   (|l| <= 1e-12 max |l| dropped), and per (k, k') block the real form
  *   [[Re B, -Im B], [Im B, Re B]] against [Re C; Im C], C = V |l|^1/2
  *   sqrt(w_k'), through the FP64 direct-LDS half-transform and the signed
