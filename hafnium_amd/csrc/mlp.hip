@@ -364,6 +364,8 @@ int mguard(hfjk_ctx* ctx, F&& body) {
   }
 }
 
+constexpr int kMaxRows = 65535 * 64;  // of a product
+
 // Float offsets of a training step's workspace: every layer's z and dz, the
 // hidden layers' h, the loss parts of the output tiles.
 constexpr int kMaxLayers = 16;
@@ -405,7 +407,7 @@ int hfjk_mlp_gemm(hfjk_ctx* ctx, int m, int n, int k, const void* a, int a_bf16,
     if (lda < (trans_a ? m : k) || ldb < (trans_b ? k : n) || ldc < n)
       mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: a leading dimension is smaller than its row");
     if (h_silu == c) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: the activation output must not alias C");
-    if (m > 65535 * 64) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: more than 4194240 rows");
+    if (m > kMaxRows) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: more than 4194240 rows");
     GemmArgs g{};
     g.m = m;
     g.n = n;
@@ -505,7 +507,8 @@ int hfjk_mlp_train_step(hfjk_ctx* ctx, int layers, const int* sizes, int m, cons
     if (layers < 1 || layers > kMaxLayers || sizes == nullptr || m < 1)
       mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: 1 to 16 layers and at least one row are required");
     for (int l = 0; l <= layers; ++l)
-      if (sizes[l] < 1) mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: layer sizes are positive");
+      if (sizes[l] < 1 || (l < layers && sizes[l] > kMaxRows) || m > kMaxRows)
+        mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: layer sizes are positive, rows and inputs at most 4194240");
     if (x == nullptr || target == nullptr || params == nullptr || params_bf16 == nullptr || grads == nullptr ||
         moment1 == nullptr || moment2 == nullptr || workspace == nullptr || loss == nullptr || ldt < sizes[layers])
       mfail(HFJK_ERR_INPUT, "hfjk_mlp_train_step: null buffer or a target narrower than the output");
