@@ -18,8 +18,8 @@
 
 namespace {
 
-typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int kT = 256;
@@ -55,7 +55,6 @@ struct GemmArgs {
   int accumulate;
   float* h;            // silu(C)
   const float* slope;  // C *= silu'(slope[i][j]), leading dimension ldc
-  float* bsum;         // column sums of B over k (FP32, unrounded), TB = float
   // The weighted squared error of C: grad, and the workgroup's part of the loss.
   const float* tgt;
   int ldt;
@@ -67,53 +66,66 @@ struct GemmArgs {
 };
 
 // Eight consecutive k of one row (or column) of an operand as a lane holds
-// them, in FP32: element (i, k + e), k + e < kmax, i < imax, zero elsewhere.
-// Stored row i (rows[i] when given) along k, or with trans k along i.
+// them: element (i, k + e), k + e < kmax, i < imax, zero elsewhere. Stored row
+// i (rows[i] when given) along k, or with trans k along i. load8 only loads
+// (bf16 in pairs where `vec` and the row's end let it); operand8 rounds and
+// masks once the values are needed.
+template <typename T>
+struct Raw8 {
+  T x[8];
+  u4 pair;  // bf16: elements 2 w and 2 w + 1 in word w, when `pairs`
+  bool pairs;
+};
+
 template <typename T>
 __device__ __forceinline__ void load8(const T* __restrict__ p, int ld, int trans, const int* __restrict__ rows, int i,
-                                      int imax, int k, int kmax, bool vec, float (&v)[8]) {
-  auto f = [](T x) -> float {
-    if constexpr (sizeof(T) == 2)
-      return __uint_as_float((uint32_t)x << 16);
-    else
-      return x;
-  };
+                                      int imax, int k, int kmax, bool vec, Raw8<T>& r) {
   // Rows and columns past the operand read its last ones and count as zero,
   // so that every load is unconditional. kmax, imax >= 1 here.
   const int ic = min(i, imax - 1);
   const T* src = trans ? p + ic : p + (long long)(rows ? rows[ic] : ic) * ld;
-  if (!trans && vec && k + 8 <= kmax) {
+  r.pairs = !trans && vec && k + 8 <= kmax;
+  if (r.pairs) {
     if constexpr (sizeof(T) == 2) {
-      const uint4 u = *(const uint4*)(src + k);
-      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(e & 1 ? w[e >> 1] & 0xFFFF0000u : w[e >> 1] << 16);
+      r.pair = *(const u4*)(src + k);
     } else {
-      const float4 x = ((const float4*)(src + k))[0], y = ((const float4*)(src + k))[1];
-      v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
-      v[4] = y.x, v[5] = y.y, v[6] = y.z, v[7] = y.w;
-    }
+      const f4 u = ((const f4*)(src + k))[0], v = ((const f4*)(src + k))[1];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = i < imax ? v[e] : 0.0f;
+      for (int e = 0; e < 4; ++e) r.x[e] = u[e], r.x[4 + e] = v[e];
+    }
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int kc = min(k + e, kmax - 1);
-      const T x = trans ? src[(long long)(rows ? rows[kc] : kc) * ld] : src[kc];
-      v[e] = i < imax && k + e < kmax ? f(x) : 0.0f;
+      r.x[e] = trans ? src[(long long)(rows ? rows[kc] : kc) * ld] : src[kc];
     }
   }
 }
 
-__device__ __forceinline__ bf8 round8(const float (&v)[8]) {
+template <typename T>
+__device__ __forceinline__ bf8 operand8(const Raw8<T>& r, int i, int imax, int k, int kmax) {
   union {
     uint16_t u[8];
     bf8 b;
-  } r;
+  } o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) r.u[e] = to_bf16(v[e]);
-  return r.b;
+  for (int e = 0; e < 8; ++e) {
+    uint16_t v;
+    if constexpr (sizeof(T) == 2)
+      v = r.pairs ? (uint16_t)(r.pair[e >> 1] >> (e & 1) * 16) : r.x[e];
+    else
+      v = to_bf16(r.x[e]);
+    o.u[e] = i < imax && k + e < kmax ? v : (uint16_t)0;
+  }
+  return o.b;
 }
+
+// The operands of a k step of a tile as the MFMA reads them (16 rows of A, 16
+// more, 16 columns of B, 16 more), a step per wave, two rounds of them.
+struct GemmSmem {
+  bf8 step[2][kWaves][4][64];
+  float losses[4];
+};
 
 // C[m][n] = op(A) op(B) (+ C) (+ bias) and the epilogues of GemmArgs.
 // op(A) is m x k: A is stored m x k (ta = 0) or k x m (ta = 1), row-major
@@ -123,18 +135,22 @@ __device__ __forceinline__ bf8 round8(const float (&v)[8]) {
 // One 512-thread workgroup per 32 x 32 tile of C as 2 x 2
 // v_mfma_f32_16x16x32_bf16 tiles (A[i][8 (l / 16) + e] in element e of lane
 // l, i = l % 16; B likewise with j = l % 16; D register r of lane l =
-// D[4 (l / 16) + r][l % 16]). The waves take every eighth 32-k step each,
-// operands straight from global memory in that order, and add their tiles up
-// in LDS in a fixed order.
+// D[4 (l / 16) + r][l % 16]). The waves fetch every eighth 32-k step each,
+// straight from global memory, and leave its operands in LDS; wave w < 4 then
+// runs the chain of products of block (w / 2, w % 2), one step after another,
+// while the next eight steps are on their way: an element's sum runs along k
+// in order, whatever the tile or the number of waves.
 //
 // Bound by latency at the training sizes (256 x 256 x 288): 64 workgroups of
-// one or two steps per wave, 7 us, where 64 x 64 tiles left 16 workgroups
-// walking nine dependent steps of scalar loads and two barriers, 22 us.
+// one or two steps per wave, 8 to 9 us, where 64 x 64 tiles left 16 workgroups
+// walking nine dependent steps of scalar loads and two barriers, 22 us. Larger
+// products are bound by the loads of their operands, which the 64 x 64 tiles
+// share twice as widely, in a serial order: 2048 x 384 x 384 28 -> 14 us,
+// 4096^3 3.4 -> 1.7 ms, 288 x 256 x 65536 4.8 -> 0.70 ms; only gradients of
+// very wide layers with few rows lose (65536 x 256 x 288, A transposed: 263 ->
+// 302 us, nine steps in two rounds of eight).
 template <typename TA, typename TB>
-__device__ void gemm_tile(const GemmArgs& g, int tile_row, int tile_col) {
-  __shared__ float part[kWaves][4][64][4];
-  __shared__ float sums[kWaves][kTileN];
-  __shared__ float losses[kWaves];
+__device__ void gemm_tile(const GemmArgs& g, int tile_row, int tile_col, GemmSmem& sm) {
   const TA* a = (const TA*)g.a;
   const TB* b = (const TB*)g.b;
   const int lane = threadIdx.x & 63;
@@ -142,113 +158,117 @@ __device__ void gemm_tile(const GemmArgs& g, int tile_row, int tile_col) {
   const int row0 = tile_row * kTileM, col0 = tile_col * kTileN;
   const bool avec = (((uintptr_t)a | (uintptr_t)g.lda * sizeof(TA)) & 15) == 0;
   const bool bvec = (((uintptr_t)b | (uintptr_t)g.ldb * sizeof(TB)) & 15) == 0;
-  const bool want_sum = g.bsum != nullptr && tile_row == 0;
-  f4 acc[2][2];
+  const int mi = wave >> 1 & 1, ni = wave & 1;
+  const int steps = (g.k + 31) / 32;
+  Raw8<TA> ra[2];
+  Raw8<TB> rb[2];
+  auto fetch = [&](int step) {
+    const int k = 32 * step + 8 * (lane >> 4);
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = f4{0.f, 0.f, 0.f, 0.f};
-  float bs[2] = {0.f, 0.f};
-  for (int k0 = wave * 32; k0 < g.k; k0 += kWaves * 32) {
-    const int k = k0 + 8 * (lane >> 4);
-    bf8 fa[2], fb[2];
-    float v[8];
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi) {
-      load8(a, g.lda, g.ta, g.a_rows, row0 + mi * 16 + (lane & 15), g.m, k, g.k, avec, v);
-      fa[mi] = round8(v);
+    for (int f = 0; f < 2; ++f) {
+      load8(a, g.lda, g.ta, g.a_rows, row0 + f * 16 + (lane & 15), g.m, k, g.k, avec, ra[f]);
+      load8(b, g.ldb, !g.tb, nullptr, col0 + f * 16 + (lane & 15), g.n, k, g.k, bvec, rb[f]);
     }
+  };
+  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+  if (wave < steps) fetch(wave);
+  for (int s0 = 0, round = 0; s0 < steps; s0 += kWaves, round ^= 1) {
+    if (s0 + wave < steps) {
+      const int k = 32 * (s0 + wave) + 8 * (lane >> 4);
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-      load8(b, g.ldb, !g.tb, nullptr, col0 + ni * 16 + (lane & 15), g.n, k, g.k, bvec, v);
-      if (want_sum) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) bs[ni] += v[e];
+      for (int f = 0; f < 2; ++f) {
+        sm.step[round][wave][f][lane] = operand8(ra[f], row0 + f * 16 + (lane & 15), g.m, k, g.k);
+        sm.step[round][wave][2 + f][lane] = operand8(rb[f], col0 + f * 16 + (lane & 15), g.n, k, g.k);
       }
-      fb[ni] = round8(v);
     }
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni)
-        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
-  }
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni) *(f4*)part[wave][2 * mi + ni][lane] = acc[mi][ni];
-  if (want_sum) {
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-      bs[ni] += __shfl_xor(bs[ni], 16);
-      bs[ni] += __shfl_xor(bs[ni], 32);
-      if (lane < 16) sums[wave][ni * 16 + lane] = bs[ni];
+    // This round's operands are in LDS, and the round before is read: the next one may replace it.
+    __syncthreads();
+    if (s0 + kWaves + wave < steps) fetch(s0 + kWaves + wave);
+    if (wave < 4) {
+      const int count = min(kWaves, steps - s0);
+#pragma unroll 4
+      for (int s = 0; s < count; ++s)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm.step[round][s][mi][lane], sm.step[round][s][2 + ni][lane], acc,
+                                                      0, 0, 0);
     }
   }
-  __syncthreads();
-  if (want_sum && threadIdx.x < kTileN && col0 + (int)threadIdx.x < g.n) {
-    const int j = threadIdx.x;
-    float t = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) t += sums[w][j];
-    g.bsum[col0 + j] = t;
-  }
-  // Wave w finishes half (w % 2) of the rows of the 16 x 16 block (w / 4, w / 2 % 2).
-  static_assert(kWaves == 8, "two waves per 16 x 16 block");
-  const int half = 2 * (wave & 1);
-  f2 total = f2{0.f, 0.f};
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) total += *(const f2*)&part[w][wave >> 1][lane][half];
-  const int j = col0 + (wave >> 1 & 1) * 16 + (lane & 15);
   float loss = 0.f;
+  if (wave < 4) {
+    const int j = col0 + ni * 16 + (lane & 15);
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int i = row0 + (wave >> 2) * 16 + 4 * (lane >> 4) + half + r;
-    if (i >= g.m || j >= g.n) continue;
-    float v = total[r];
-    const long long at = (long long)i * g.ldc + j;
-    if (g.accumulate) v += g.c[at];
-    if (g.bias) v += g.bias[j];
-    if (g.slope) v *= silu_slope(g.slope[at]);
-    g.c[at] = v;
-    if (g.h) g.h[at] = silu(v);
-    if (g.tgt) {
-      const long long tr = g.t_rows ? g.t_rows[i] : i;
-      const float d = v - g.tgt[tr * g.ldt + j];
-      const float wj = g.w ? g.w[j] : 1.0f;
-      loss += wj * d * d;
-      g.grad[at] = 2.0f * g.scale * wj * d;
+    for (int r = 0; r < 4; ++r) {
+      const int i = row0 + mi * 16 + 4 * (lane >> 4) + r;
+      if (i >= g.m || j >= g.n) continue;
+      float v = acc[r];
+      const long long at = (long long)i * g.ldc + j;
+      if (g.accumulate) v += g.c[at];
+      if (g.bias) v += g.bias[j];
+      if (g.slope) v *= silu_slope(g.slope[at]);
+      g.c[at] = v;
+      if (g.h) g.h[at] = silu(v);
+      if (g.tgt) {
+        const long long tr = g.t_rows ? g.t_rows[i] : i;
+        const float d = v - g.tgt[tr * g.ldt + j];
+        const float wj = g.w ? g.w[j] : 1.0f;
+        loss += wj * d * d;
+        g.grad[at] = 2.0f * g.scale * wj * d;
+      }
     }
   }
   if (g.tgt) {
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-    if (lane == 0) losses[wave] = loss;
+    if (lane == 0 && wave < 4) sm.losses[wave] = loss;
     __syncthreads();
     if (threadIdx.x == 0)
       g.loss_part[tile_row * ((g.n + kTileN - 1) / kTileN) + tile_col] =
-          ((losses[0] + losses[1]) + (losses[2] + losses[3])) + ((losses[4] + losses[5]) + (losses[6] + losses[7]));
+          (sm.losses[0] + sm.losses[1]) + (sm.losses[2] + sm.losses[3]);
   }
 }
 
 template <typename TA, typename TB>
 __global__ __launch_bounds__(kGemmT) void mlp_gemm_kernel(GemmArgs g) {
+  __shared__ GemmSmem sm;
   const int cols = (g.n + kTileN - 1) / kTileN;
-  gemm_tile<TA, TB>(g, blockIdx.x / cols, blockIdx.x % cols);
+  gemm_tile<TA, TB>(g, blockIdx.x / cols, blockIdx.x % cols, sm);
 }
 
-// One layer of the backward pass: the weight and bias gradients (tiles below
-// split) and the gradient of the layer's input, both of the same dz: 7 us in
-// one launch, where the two products, the column sum and the SiLU backward
-// took 22 + 22 + 7 + 3 us in four.
-__global__ __launch_bounds__(kGemmT) void mlp_backward_kernel(GemmArgs weights, GemmArgs input, int split) {
+// out[j] = sum_i x[i][j] of 64 columns by 256 threads: 4 row phases, fixed order.
+__device__ __forceinline__ void column_sums(int m, int n, const float* __restrict__ x, int ldx,
+                                            float* __restrict__ out, int block, float (*part)[64]) {
+  const int c = threadIdx.x & 63;
+  const int phase = threadIdx.x >> 6;
+  const int j = block * 64 + c;
+  float s = 0.f;
+  if (j < n && phase < 4) {
+#pragma unroll 16
+    for (int i = phase; i < m; i += 4) s += x[(long long)i * ldx + j];
+  }
+  if (phase < 4) part[phase][c] = s;
+  __syncthreads();
+  if (phase == 0 && j < n) out[j] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+}
+
+// One layer of the backward pass: the bias gradients (the first `sums`
+// workgroups), the weight gradients (tiles below split) and the gradient of
+// the layer's input, all of the same dz: 7 us in one launch, where the two
+// products, the column sum and the SiLU backward took 22 + 22 + 7 + 3 us in
+// four. Every sum has the order of the separate calls'.
+__global__ __launch_bounds__(kGemmT) void mlp_backward_kernel(GemmArgs weights, GemmArgs input, int sums, int split,
+                                                              float* __restrict__ bias) {
+  __shared__ GemmSmem sm;
   int t = blockIdx.x;
+  if (t < sums) {
+    column_sums(weights.k, weights.n, (const float*)weights.b, weights.ldb, bias, t, (float(*)[64]) & sm);
+    return;
+  }
+  t -= sums;
   if (t < split) {
     const int cols = (weights.n + kTileN - 1) / kTileN;
-    gemm_tile<float, float>(weights, t / cols, t % cols);
+    gemm_tile<float, float>(weights, t / cols, t % cols, sm);
   } else {
     t -= split;
     const int cols = (input.n + kTileN - 1) / kTileN;
-    gemm_tile<float, uint16_t>(input, t / cols, t % cols);
+    gemm_tile<float, uint16_t>(input, t / cols, t % cols, sm);
   }
 }
 
@@ -260,19 +280,10 @@ __global__ __launch_bounds__(kT) void silu_backward_kernel(long long count, cons
   }
 }
 
-// out[j] = sum_i x[i][j]: 64 columns per workgroup, 4 row phases, fixed order.
 __global__ __launch_bounds__(kT) void column_sum_kernel(int m, int n, const float* __restrict__ x, int ldx,
                                                         float* __restrict__ out) {
   __shared__ float part[4][64];
-  const int c = threadIdx.x & 63;
-  const int phase = threadIdx.x >> 6;
-  const int j = blockIdx.x * 64 + c;
-  float s = 0.f;
-  if (j < n)
-    for (int i = phase; i < m; i += 4) s += x[(long long)i * ldx + j];
-  part[phase][c] = s;
-  __syncthreads();
-  if (phase == 0 && j < n) out[j] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+  column_sums(m, n, x, ldx, out, blockIdx.x, part);
 }
 
 // Weighted squared error over y [m][n]: loss[0] = scale sum_ij w_j (y_ij - t_ij)^2,
@@ -567,7 +578,6 @@ int hfjk_mlp_train_step(hfjk_ctx* ctx, int layers, const int* sizes, int m, cons
       w.ldb = n;
       w.c = grads + at[l];
       w.ldc = n;
-      w.bsum = grads + at[l] + (long long)k * n;
       const int split = tiles(k) * tiles(n);
       GemmArgs d{};
       if (l > 0) {
@@ -583,8 +593,10 @@ int hfjk_mlp_train_step(hfjk_ctx* ctx, int layers, const int* sizes, int m, cons
         d.ldc = k;
         d.slope = workspace + L.z[l - 1];
       }
-      const int grid = split + (l > 0 ? tiles(m) * tiles(k) : 0);
-      hipLaunchKernelGGL(mlp_backward_kernel, dim3(grid), dim3(kGemmT), 0, s, w, d, split);
+      const int sums = (n + 63) / 64;
+      const int grid = sums + split + (l > 0 ? tiles(m) * tiles(k) : 0);
+      hipLaunchKernelGGL(mlp_backward_kernel, dim3(grid), dim3(kGemmT), 0, s, w, d, sums, split,
+                         grads + at[l] + (long long)k * n);
       mcheck(hipGetLastError(), "mlp backward launch");
     }
     const long long count = at[layers];

@@ -199,3 +199,43 @@ def test_training_step_is_the_separate_calls(sizes, m):
         for got, want in ((h, h_ref), (z, z_ref)):
             assert got.shape == want.shape
             assert (got - want).abs().max().item() <= GEMM_REL_TOL * max(want.abs().max().item(), 1e-30)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("k", [32, 9 * 32, 16 * 32, 17 * 32 + 5, 1300])
+def test_products_sum_along_k_in_order(net, k, ta, tb):
+    """One product per 32 k, so the FP32 sum of an element depends on the order of the steps alone: large terms
+    that swallow small ones and cancel later leave what the chain from k = 0 leaves, exactly."""
+    m, n = 37, 35
+    a = np.zeros((m, k))
+    want = np.float32(0.0)
+    for s, at in enumerate(range(0, k, 32)):
+        value = (2.0 ** 30, float(s % 100 + 1), -(2.0 ** 30))[s % 3]
+        a[:, at] = value
+        want = np.float32(want + np.float32(value))
+    c, _ = _gemm(net, a.T if ta else a, np.ones((n, k) if tb else (k, n)), ta, tb)
+    np.testing.assert_array_equal(c, np.full((m, n), want, dtype=np.float64))
+
+
+@pytest.mark.parametrize("m", [1, 33, 700])
+@pytest.mark.parametrize("sizes", [[5, 3], [72, 96, 80, 13], [31, 33, 64, 65], [288, 256, 256, 77]])
+def test_training_step_has_the_gradients_of_the_separate_calls(sizes, m):
+    """The same products and sums in the same order: the same gradients and parameters, bit for bit."""
+    torch = _torch()
+    from hafnium_amd.mlp import Mlp
+
+    rng = np.random.default_rng(80 + m + len(sizes))
+    fused, split = Mlp(sizes, seed=6), Mlp(sizes, seed=6)
+    dev = fused.device
+    x = torch.from_numpy(rng.standard_normal((m + 7, sizes[0])).astype(np.float32)).to(dev)
+    t = torch.from_numpy(rng.standard_normal((m + 7, sizes[-1])).astype(np.float32)).to(dev)
+    rows = (torch.from_numpy(rng.permutation(m + 7).astype(np.int32)).to(dev), 3, 3 + m)
+    for _ in range(2):
+        fused.train_step(x, t, rows, lr=1e-3, weight_decay=1e-2)
+        y = split.forward(x, rows, keep=True)
+        grad = torch.empty_like(y)
+        split.loss(y, t, rows, None, 1.0 / m, grad)
+        split.backward(grad)
+        split.adam(1e-3, weight_decay=1e-2)
+        assert torch.equal(fused.grads, split.grads)
+        assert torch.equal(fused.params, split.params)
