@@ -1250,6 +1250,7 @@ __global__ __launch_bounds__(kPairThreads) void pair_kernel(const LanePair* __re
     }
     __syncthreads();
     const int kept = kept_all;
+    __syncthreads();  // every wave has read kept_all: without a survivor the next batch is next
     for (int s0 = 0; s0 < kept; s0 += kLaneSlots) {
       const int ns = min(kLaneSlots, kept - s0);
       if (tid < 3 * ns) {

@@ -112,3 +112,25 @@ def test_device_integrals_over_all_classes(orbital, auxiliary, scale):
     worst = float(np.max(np.abs(dev - metric) / np.sqrt(np.outer(np.diag(metric), np.diag(metric)))))
     assert worst <= 1e-12, worst
     np.testing.assert_array_equal(dev, dev.T)
+
+
+@pytest.mark.parametrize("distance", [13.8, 15.0, 16.5, 18.0])
+def test_first_batch_of_primitive_pairs_without_a_survivor(distance):
+    """Oxygens in cc-pVDZ whose first 64 of 81 s-s primitive pairs the product cut drops, and later ones not."""
+    basis = molecule.load_basis("cc-pvdz")["8"]
+    e = np.asarray(next(s["exponents"] for s in basis if s["l"] == 0))
+    assert len(e) == 9
+    kept = np.exp(-np.outer(e, e) / np.add.outer(e, e) * distance ** 2).reshape(-1) >= 1e-22
+    assert not kept[:64].any() and kept[64:].any()
+    positions = np.zeros((6, 3))
+    positions[:, 0] = distance * np.arange(6)  # the neighbours only: the next pair has no survivor, or its own
+    mol = molecule.Molecule((8,) * 6, positions)
+    orb, aux = molecule.BasisOnAtoms("cc-pvdz", mol), molecule.BasisOnAtoms("def2-universal-jkfit", mol)
+    host = integrals.three_center(aux, orb)
+    got = integrals.three_center_device(aux, orb).cpu().numpy()
+    n = orb.n_functions // 6
+    for i in range(6):
+        for j in range(i + 1):
+            a, b = slice(i * n, (i + 1) * n), slice(j * n, (j + 1) * n)
+            # Against the block's own size: the far blocks are 1e-13 of the others.
+            assert np.abs(got[:, a, b] - host[:, a, b]).max() <= 1e-10 * np.abs(host[:, a, b]).max(), (i, j)
