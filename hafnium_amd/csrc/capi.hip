@@ -1306,7 +1306,7 @@ bool kpoint_exchange_psd(hfjk_ctx* ctx, int nk, int naux, int n, const double* t
     double mag, residual;
     std::memcpy(&mag, &states[k].mag, sizeof(double));
     std::memcpy(&residual, &states[k].residual, sizeof(double));
-    if (!(residual <= 1e-11 * mag) || states[k].rank < 1 || !(host_weights[k] > 0.0)) return false;
+    if (!(residual <= 1e-12 * mag) || states[k].rank < 1 || !(host_weights[k] > 0.0)) return false;
     rank = std::max(rank, states[k].rank);
   }
   const int hb = kp_half(rank), ldo = 2 * hb;

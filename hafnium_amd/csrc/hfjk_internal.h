@@ -401,10 +401,11 @@ hipError_t launch_kp_factor(const void* eigvecs, const double* eigvals, int nao,
                             int ldo, double* ct, double* signs, hipStream_t s);
 hipError_t launch_kp_fold(const double* kh, int nao, bool accumulate, void* k, hipStream_t s);
 // The factorisation of every k's density at once: max |D - D^H|, max |D| and
-// max |D - L L^H| (KpState, cleared by launch_kp_cholesky) of the pivoted
-// Cholesky D = L L^H, L by columns [nk][nao][nao] (with nk nao doubles of
-// scratch behind it), stopped at 1e-12 of the largest diagonal; launch_kp_fragments: the operand fragments
-// [nk][kpad][2 hb] of sqrt(weight) [Re, Im] of the L of every k.
+// the largest row sum of |D - L L^H| (KpState, cleared by launch_kp_cholesky)
+// of the pivoted Cholesky D = L L^H, L by columns [nk][nao][nao] (with nk nao
+// doubles of scratch behind it), stopped at 1e-14 of the largest diagonal;
+// launch_kp_fragments: the operand fragments [nk][kpad][2 hb] of sqrt(weight)
+// [Re, Im] of the L of every k.
 struct KpState {
   unsigned long long asym, mag, residual;  // bits of non-negative doubles
   int rank, pad;

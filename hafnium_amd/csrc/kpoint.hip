@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kCholThreads) void kp_cholesky_kernel(const double2
     __syncthreads();
     const double piv = s_best;
     const int p = s_at;
-    if (c == 0) cut = 1e-12 * piv;
+    if (c == 0) cut = 1e-14 * piv;
     if (c == n || p < 0 || !(piv > cut)) {
       rank = c;
       break;
@@ -304,7 +304,8 @@ __global__ __launch_bounds__(kCholThreads) void kp_cholesky_kernel(const double2
   if (t == 0) state[blockIdx.x].rank = rank;
 }
 
-// Per k: max |D - D^H|, max |D| and max |D - L L^H| (atomic max of bits).
+// Per k: max |D - D^H|, max |D| and the largest row sum of |D - L L^H|, which
+// bounds its largest eigenvalue (atomic max of bits). A wave per row.
 __global__ __launch_bounds__(kThreads) void kp_residual_kernel(const double2* __restrict__ density, int n,
                                                                const double2* __restrict__ lmat,
                                                                KpState* __restrict__ state) {
@@ -313,23 +314,26 @@ __global__ __launch_bounds__(kThreads) void kp_residual_kernel(const double2* __
   const double2* l = lmat + blockIdx.y * nn;
   KpState* st = state + blockIdx.y;
   const int rank = st->rank;
+  const int lane = threadIdx.x & 63;
   double asym = 0.0, mag = 0.0, worst = 0.0;
-  for (long long idx = (long long)blockIdx.x * kThreads + threadIdx.x; idx < nn;
-       idx += (long long)gridDim.x * kThreads) {
-    const int r = (int)(idx / n), c = (int)(idx % n);
-    double2 a = d[idx];
-    const double2 t = d[(long long)c * n + r];
-    asym = fmax(asym, hypot(a.x - t.x, a.y + t.y));
-    mag = fmax(mag, hypot(a.x, a.y));
-    for (int j = 0; j < rank; ++j) {
-      const double2 u = l[(long long)j * n + r], v = l[(long long)j * n + c];
-      const double2 m = cmul(u, make_double2(v.x, -v.y));
-      a.x -= m.x;
-      a.y -= m.y;
+  for (int r = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); r < n; r += gridDim.x * (kThreads / 64)) {
+    double sum = 0.0;
+    for (int c = lane; c < n; c += 64) {
+      double2 a = d[(long long)r * n + c];
+      const double2 t = d[(long long)c * n + r];
+      asym = fmax(asym, hypot(a.x - t.x, a.y + t.y));
+      mag = fmax(mag, hypot(a.x, a.y));
+      for (int j = 0; j < rank; ++j) {
+        const double2 u = l[(long long)j * n + r], v = l[(long long)j * n + c];
+        const double2 m = cmul(u, make_double2(v.x, -v.y));
+        a.x -= m.x;
+        a.y -= m.y;
+      }
+      sum += fabs(a.x) + fabs(a.y);
     }
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     // Not fmax, which would drop a NaN: a NaN must fail the host's test.
-    const double e = fabs(a.x) + fabs(a.y);
-    worst = e > worst || e != e ? e : worst;
+    worst = sum > worst || sum != sum ? sum : worst;
   }
   unsigned long long* out[3] = {&st->asym, &st->mag, &st->residual};
   double v[3] = {asym, mag, worst};
@@ -496,7 +500,7 @@ hipError_t launch_kp_cholesky(const void* density, int nk, int nao, void* l, KpS
   double* diag = (double*)((double2*)l + (long long)nk * nao * nao);
   hipLaunchKernelGGL(kp_cholesky_kernel, dim3((unsigned)nk), dim3(kCholThreads), 0, s, (const double2*)density, nao,
                      (double2*)l, diag, st);
-  const unsigned gx = (unsigned)std::min<long long>(((long long)nao * nao + kThreads - 1) / kThreads, 1024);
+  const unsigned gx = (unsigned)std::min((nao + kThreads / 64 - 1) / (kThreads / 64), 1024);
   hipLaunchKernelGGL(kp_residual_kernel, dim3(gx, (unsigned)nk), dim3(kThreads), 0, s, (const double2*)density, nao,
                      (const double2*)l, st);
   return hipGetLastError();

@@ -542,7 +542,8 @@ HFJK_API int hfjk_mlp_to_bf16(hfjk_ctx *ctx, long long count, const float *src, 
  * hfjk_kpoint_exchange: K(k) = sum_k' w_k' sum_P s[k,k',P] B[k,k',P] D(k')
  *   B[k,k',P]^H + madelung S(k) D(k) S(k) for Hermitian D(k') (1e-12
  *   relative, else HFJK_ERR_INPUT). Positive semidefinite D(k') with weights
- *   > 0 factorise by pivoted Cholesky and go through the half-transform of the
+ *   > 0 (no row of |D - L L^H| sums to more than 1e-12 max |D|) factorise by
+ *   pivoted Cholesky and go through the half-transform of the
  *   complex rows and the signed SYRK over ranges of blocks, at most 1 GiB of X
  *   at a time. Otherwise D(k') = V diag(l) V^H by rocSOLVER zheevd
  *   (|l| <= 1e-12 max |l| dropped), and per (k, k') block the real form

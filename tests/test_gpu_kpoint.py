@@ -157,3 +157,35 @@ def test_exchange_in_several_passes():
     want = torch.matmul(left.transpose(0, 1).reshape(nao, -1), flat.transpose(0, 1).reshape(nao, -1).conj().T.contiguous())
     for k in range(nk):
         assert float((got[k] - want).abs().max()) <= 1e-12 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("extra", [-8e-12, -2e-12, 2e-12, 8e-12, 3e-11])
+@pytest.mark.parametrize("spread", [False, True])
+def test_exchange_keeps_small_eigenvalues_above_the_cut(extra, spread):
+    """Four unit eigenvalues and a small one of either sign above 1e-12 of them, on one function or spread over
+    all: it enters K in full, where the factor of a nearly semidefinite density would have dropped it."""
+    from hafnium_amd.kpoint import KPointMI355XCoulombExchange
+
+    rng = np.random.default_rng(11)
+    nk, naux, nao = 2, 40, 28
+    z = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)  # noqa: E731
+    b = z(nk, nk, naux, nao, nao)
+    # The small eigenvector's products are 1e6 times the others', so that its part of K shows.
+    b[..., 0] *= 1e6
+    d = np.zeros((nk, nao, nao), dtype=complex)
+    for k in range(nk):
+        u = np.zeros((nao, 5), dtype=complex)
+        u[1:, :4] = np.linalg.qr(z(nao - 1, 4))[0]
+        if spread:
+            u[1:, 4] = np.linalg.qr(np.concatenate([u[1:, :4], z(nao - 1, 1)], 1))[0][:, 4]
+            u[:, 4] = (u[:, 4] + np.eye(nao)[0]) / np.sqrt(2.0)
+        else:
+            u[0, 4] = 1.0
+        d[k] = (u * np.array([1.0, 1.0, 1.0, 1.0, extra])) @ u.conj().T
+        d[k] = 0.5 * (d[k] + d[k].conj().T)
+    w = np.full(nk, 1.0 / nk)
+    got = KPointMI355XCoulombExchange(b, np.ones((nk, nk, naux)), w, np.zeros((nk, nao, nao)), 0.0).exchange(d)
+    want = np.einsum("k,qkpxy,kyz,qkpwz->qxw", w, b, d, b.conj(), optimize=True)
+    # D's own rounding reaches K 1e12-fold through the scaled function (1e-4 and less, from NumPy's eigenpairs);
+    # without the extra eigenvalue K would be off by 0.22 and more.
+    assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
