@@ -130,33 +130,36 @@ def test_exchange_of_both_factorisations(nk, nao, naux, nocc, positive):
     assert np.max(np.abs(got - got.conj().transpose(0, 2, 1))) <= 16 * nao * 2.0 ** -53 * top
 
 
-def test_exchange_in_several_passes():
-    """More blocks than the workspace holds X of: ranges of k2 accumulate, results equal to one pass."""
-    import ctypes
-
+@pytest.mark.parametrize("nk,naux", [(4, 9000), (6, 2300)])
+def test_exchange_in_several_passes(nk, naux):
+    """More blocks than the workspace holds X of (1 GiB): ranges of k2 within one k1, which accumulate, and whole
+    k1 a few at a time. Every block, signature and weight differs."""
     import torch
 
-    from hafnium_amd import _lib
     from hafnium_amd.kpoint import KPointMI355XCoulombExchange
 
-    rng = np.random.default_rng(4)
-    nk, nao, naux = 4, 40, 1500
-    z = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)  # noqa: E731
-    b = torch.from_numpy(z(1, 1, naux, nao, nao)).cuda().expand(nk, nk, naux, nao, nao).contiguous()
-    c = z(nk, nao, nao)
-    d = torch.from_numpy(c @ c.conj().transpose(0, 2, 1)).cuda()
-    jk = KPointMI355XCoulombExchange(b, torch.ones(nk, nk, naux), torch.full((nk,), 1.0 / nk),
-                                     torch.zeros(nk, nao, nao, dtype=torch.complex128), 0.0)
-    size = ctypes.c_size_t()
-    _lib.check(jk._ctx.lib.hfjk_kpoint_workspace_bytes(jk._ctx.handle, nk, naux, nao, ctypes.byref(size)))
-    assert nk * nk * naux * nao * 96 * 8 > 1 << 29  # ranges of whole k1 do not all fit
-    got = jk.exchange(d)
-    flat = b[0, 0]
-    dm = d.mean(0)
-    left = torch.matmul(flat.reshape(-1, nao), dm).view(naux, nao, nao)
-    want = torch.matmul(left.transpose(0, 1).reshape(nao, -1), flat.transpose(0, 1).reshape(nao, -1).conj().T.contiguous())
-    for k in range(nk):
-        assert float((got[k] - want).abs().max()) <= 1e-12 * float(want.abs().max())
+    nao = 40
+    columns = 96  # of X for full rank: Re and Im, 40 rounded up to 16 each
+    fit = (1 << 30) // (naux * nao * columns * 8)
+    assert 1 < fit < nk if nk == 4 else nk <= fit < nk * nk  # ranges of k2; whole k1, not all of them
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(4)
+    c128 = torch.complex128
+    b = torch.randn((nk, nk, naux, nao, nao), generator=g, dtype=c128, device="cuda:0")
+    sig = torch.where(torch.rand((nk, nk, naux), generator=g, device="cuda:0") < 0.3, -1.0, 1.0).double()
+    w = torch.linspace(0.3, 1.0, nk, dtype=torch.float64, device="cuda:0")
+    c = torch.randn((nk, nao, nao), generator=g, dtype=c128, device="cuda:0")
+    d = torch.matmul(c, c.conj().transpose(1, 2).contiguous())
+    d = 0.5 * (d + d.conj().transpose(1, 2)).contiguous()
+    got = KPointMI355XCoulombExchange(b, sig, w, torch.zeros((nk, nao, nao), dtype=c128, device="cuda:0"),
+                                      0.0).exchange(d)
+    for k1 in range(nk):
+        want = torch.zeros((nao, nao), dtype=c128, device="cuda:0")
+        for k2 in range(nk):
+            left = torch.matmul(b[k1, k2].reshape(-1, nao), d[k2]).view(naux, nao, nao) * sig[k1, k2][:, None, None]
+            left = left.transpose(0, 1).reshape(nao, -1).contiguous()
+            want += w[k2] * torch.matmul(left, b[k1, k2].transpose(0, 1).reshape(nao, -1).conj().T.contiguous())
+        assert float((got[k1] - want).abs().max()) <= 1e-12 * float(want.abs().max()), k1
 
 
 @pytest.mark.parametrize("extra", [-8e-12, -2e-12, 2e-12, 8e-12, 3e-11])
