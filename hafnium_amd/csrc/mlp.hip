@@ -225,11 +225,12 @@ __device__ void gemm_tile(const GemmArgs& g, int tile_row, int tile_col, GemmSme
   }
 }
 
+// Tiles from `first` on.
 template <typename TA, typename TB>
-__global__ __launch_bounds__(kGemmT) void mlp_gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(kGemmT) void mlp_gemm_kernel(GemmArgs g, int first) {
   __shared__ GemmSmem sm;
-  const int cols = (g.n + kTileN - 1) / kTileN;
-  gemm_tile<TA, TB>(g, blockIdx.x / cols, blockIdx.x % cols, sm);
+  const int cols = (g.n + kTileN - 1) / kTileN, t = first + blockIdx.x;
+  gemm_tile<TA, TB>(g, t / cols, t % cols, sm);
 }
 
 // out[j] = sum_i x[i][j] of 64 columns by 256 threads: 4 row phases, fixed order.
@@ -254,9 +255,9 @@ __device__ __forceinline__ void column_sums(int m, int n, const float* __restric
 // products, the column sum and the SiLU backward took 22 + 22 + 7 + 3 us in
 // four. Every sum has the order of the separate calls'.
 __global__ __launch_bounds__(kGemmT) void mlp_backward_kernel(GemmArgs weights, GemmArgs input, int sums, int split,
-                                                              float* __restrict__ bias) {
+                                                              float* __restrict__ bias, int first) {
   __shared__ GemmSmem sm;
-  int t = blockIdx.x;
+  int t = first + blockIdx.x;
   if (t < sums) {
     column_sums(weights.k, weights.n, (const float*)weights.b, weights.ldb, bias, t, (float(*)[64]) & sm);
     return;
@@ -375,7 +376,20 @@ int mguard(hfjk_ctx* ctx, F&& body) {
   }
 }
 
-constexpr int kMaxRows = 65535 * 64;  // of a product
+constexpr int kMaxRows = 65535 * 64;  // of a product: the entry points' limit
+
+// launch(first, count) for all of `tiles` workgroups of kGemmT threads, at
+// most 2^31 work-items at a time (a grid holds less than 2^32).
+template <typename F>
+void in_launches(int tiles, const char* what, F&& launch) {
+  constexpr int kMost = (1 << 30) / (kGemmT / 2);
+  for (int first = 0; first < tiles;) {
+    const int count = std::min(kMost, tiles - first);
+    launch(first, dim3((unsigned)count));
+    mcheck(hipGetLastError(), what);
+    first += count;
+  }
+}
 
 // Float offsets of a training step's workspace: every layer's z and dz, the
 // hidden layers' h, the loss parts of the output tiles.
@@ -437,17 +451,17 @@ int hfjk_mlp_gemm(hfjk_ctx* ctx, int m, int n, int k, const void* a, int a_bf16,
     g.h = h_silu;
     const long long cols = (n + kTileN - 1) / kTileN, rows = (m + kTileM - 1) / kTileM;
     if (cols * rows > 0x7FFFFFFFLL) mfail(HFJK_ERR_INPUT, "hfjk_mlp_gemm: too many output tiles");
-    const dim3 grid((unsigned)(cols * rows));
     hipStream_t s = (hipStream_t)stream;
-    if (a_bf16 && b_bf16)
-      hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, uint16_t>), grid, dim3(kGemmT), 0, s, g);
-    else if (a_bf16)
-      hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, float>), grid, dim3(kGemmT), 0, s, g);
-    else if (b_bf16)
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), grid, dim3(kGemmT), 0, s, g);
-    else
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, float>), grid, dim3(kGemmT), 0, s, g);
-    mcheck(hipGetLastError(), "mlp_gemm launch");
+    in_launches((int)(cols * rows), "mlp_gemm launch", [&](int first, dim3 grid) {
+      if (a_bf16 && b_bf16)
+        hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, uint16_t>), grid, dim3(kGemmT), 0, s, g, first);
+      else if (a_bf16)
+        hipLaunchKernelGGL((mlp_gemm_kernel<uint16_t, float>), grid, dim3(kGemmT), 0, s, g, first);
+      else if (b_bf16)
+        hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), grid, dim3(kGemmT), 0, s, g, first);
+      else
+        hipLaunchKernelGGL((mlp_gemm_kernel<float, float>), grid, dim3(kGemmT), 0, s, g, first);
+    });
   });
 }
 
@@ -561,8 +575,9 @@ int hfjk_mlp_train_step(hfjk_ctx* ctx, int layers, const int* sizes, int m, cons
         g.grad = workspace + L.dz[l];
         g.loss_part = workspace + L.loss;
       }
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), dim3(tiles(n) * tiles(m)), dim3(kGemmT), 0, s, g);
-      mcheck(hipGetLastError(), "mlp forward launch");
+      in_launches(tiles(n) * tiles(m), "mlp forward launch", [&](int first, dim3 grid) {
+        hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t>), grid, dim3(kGemmT), 0, s, g, first);
+      });
     }
     for (int l = out; l >= 0; --l) {
       const int k = sizes[l], n = sizes[l + 1];
@@ -594,10 +609,10 @@ int hfjk_mlp_train_step(hfjk_ctx* ctx, int layers, const int* sizes, int m, cons
         d.slope = workspace + L.z[l - 1];
       }
       const int sums = (n + 63) / 64;
-      const int grid = sums + split + (l > 0 ? tiles(m) * tiles(k) : 0);
-      hipLaunchKernelGGL(mlp_backward_kernel, dim3(grid), dim3(kGemmT), 0, s, w, d, sums, split,
-                         grads + at[l] + (long long)k * n);
-      mcheck(hipGetLastError(), "mlp backward launch");
+      in_launches(sums + split + (l > 0 ? tiles(m) * tiles(k) : 0), "mlp backward launch", [&](int first, dim3 grid) {
+        hipLaunchKernelGGL(mlp_backward_kernel, grid, dim3(kGemmT), 0, s, w, d, sums, split,
+                           grads + at[l] + (long long)k * n, first);
+      });
     }
     const long long count = at[layers];
     hipLaunchKernelGGL(adam_kernel, dim3(hfjk::grid_for(count)), dim3(kT), 0, s, count, params, grads, moment1,

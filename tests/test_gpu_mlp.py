@@ -239,3 +239,49 @@ def test_training_step_has_the_gradients_of_the_separate_calls(sizes, m):
         split.adam(1e-3, weight_decay=1e-2)
         assert torch.equal(fused.grads, split.grads)
         assert torch.equal(fused.params, split.params)
+
+
+def _free_memory(need):
+    torch = _torch()
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < need:
+        pytest.skip(f"needs {need >> 30} GiB of free GPU memory")
+
+
+def test_product_of_more_tiles_than_one_grid(net):
+    """8.5 million output tiles (2^32 work-items and more): an outer product of small whole numbers, exact."""
+    torch = _torch()
+    m, n = 4194240, 2080
+    _free_memory(40 << 30)
+    a = (torch.arange(m, device=net.device) % 97).float().view(m, 1)
+    b = (torch.arange(n, device=net.device) % 89).float().view(1, n)
+    c = torch.full((m, n), -1.0, device=net.device)
+    net._gemm(m, n, 1, a, 0, False, 1, False, None, b, 0, False, n, False, None, c)
+    for lo in range(0, m, m // 15):
+        assert torch.equal(c[lo:lo + m // 15], a[lo:lo + m // 15] * b)
+
+
+def test_training_step_of_more_tiles_than_one_grid():
+    """The forward and the backward launches of 8.5 million tiles: 65535 times the same 64 rows are those rows."""
+    torch = _torch()
+    from hafnium_amd.mlp import Mlp
+
+    times = 65535
+    _free_memory(140 << 30)
+    big, small = Mlp([1, 2080, 1], seed=9), Mlp([1, 2080, 1], seed=9)
+    dev = big.device
+    g = torch.Generator(device=dev)
+    g.manual_seed(2)
+    x = torch.randn((64, 1), generator=g, device=dev)
+    t = torch.randn((64, 1), generator=g, device=dev)
+    rows = torch.arange(64, dtype=torch.int32, device=dev)
+    loss = big.train_step(x, t, (rows.repeat(times), 0, 64 * times), lr=1e-3)
+    want = small.train_step(x, t, (rows, 0, 64), lr=1e-3)
+    # Sums of 4.2 million FP32 terms in a row (the bias gradients: four chains of a million) lose up to 2^-24 of
+    # the running sum each, a few 1e-3 in all; a launch's tiles left out would take half of them.
+    assert float(loss.item()) == pytest.approx(float(want.item()), rel=1e-2)
+    for (dw, db), (dw_ref, db_ref) in zip(big.gradients(), small.gradients()):
+        assert np.linalg.norm(dw - dw_ref) <= 2e-2 * np.linalg.norm(dw_ref)
+        assert np.linalg.norm(db - db_ref) <= 2e-2 * np.linalg.norm(db_ref)
+    del big
+    torch.cuda.empty_cache()
