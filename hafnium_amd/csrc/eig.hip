@@ -1082,25 +1082,31 @@ int hfjk_eigh_lowest_batched(hfjk_ctx* ctx, int n, int count, int nvec, double* 
       hipLaunchKernelGGL(eig_no_vectors_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                          count, info);
       err = hipGetLastError();
-    } else {
-      hipLaunchKernelGGL(eig_tridiagonal_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n,
-                         nvec, a, work);
-      hipLaunchKernelGGL(eig_values_kernel, dim3((unsigned)(count * ((nvec + kValueWaves - 1) / kValueWaves))),
-                         dim3(64 * kValueWaves), 0, (hipStream_t)stream, n, nvec, w, work);
-      const int per = std::max(1, std::min(std::min(nvec, 64), kVectorLds / (kVectorBytes * n)));
-      hipLaunchKernelGGL(eig_vectors_kernel, dim3((unsigned)(count * ((nvec + per - 1) / per))), dim3(64),
-                         (size_t)kVectorBytes * n * per, (hipStream_t)stream, n, nvec, per, w, work);
-      hipLaunchKernelGGL(eig_orthonormal_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n,
-                         nvec, work);
-      hipLaunchKernelGGL(eig_back_kernel, dim3((unsigned)((count + 7) / 8 * 8 * ((nvec + 3) / 4))), dim3(64), 0,
-                         (hipStream_t)stream, n, nvec, count, a, work);
-      hipLaunchKernelGGL(eig_store_kernel, dim3((unsigned)count), dim3(kEigThreads), 0, (hipStream_t)stream, n, nvec, a,
-                         work, info);
+    }
+    const int per = nvec > 0 ? std::max(1, std::min(std::min(nvec, 64), kVectorLds / (kVectorBytes * n))) : 1;
+    // A grid holds less than 2^32 work-items and the values take a wave per vector: 2^31 / 64 vectors at a
+    // time (a multiple of 8 matrices, the XCDs' turn).
+    const int most = std::max(8, (1 << 25) / std::max(nvec, 8) & ~7);
+    for (int first = 0; nvec > 0 && first < count && err == hipSuccess; first += most) {
+      const int now = std::min(most, count - first);
+      double* ai = a + (long long)first * n * n;
+      double* wi = w + (long long)first * n;
+      double* ti = work + first * eig_work_per(n, nvec);
+      const hipStream_t s = (hipStream_t)stream;
+      hipLaunchKernelGGL(eig_tridiagonal_kernel, dim3((unsigned)now), dim3(kEigThreads), 0, s, n, nvec, ai, ti);
+      hipLaunchKernelGGL(eig_values_kernel, dim3((unsigned)(now * ((nvec + kValueWaves - 1) / kValueWaves))),
+                         dim3(64 * kValueWaves), 0, s, n, nvec, wi, ti);
+      hipLaunchKernelGGL(eig_vectors_kernel, dim3((unsigned)(now * ((nvec + per - 1) / per))), dim3(64),
+                         (size_t)kVectorBytes * n * per, s, n, nvec, per, wi, ti);
+      hipLaunchKernelGGL(eig_orthonormal_kernel, dim3((unsigned)now), dim3(kEigThreads), 0, s, n, nvec, ti);
+      hipLaunchKernelGGL(eig_back_kernel, dim3((unsigned)((now + 7) / 8 * 8 * ((nvec + 3) / 4))), dim3(64), 0, s, n,
+                         nvec, now, ai, ti);
+      hipLaunchKernelGGL(eig_store_kernel, dim3((unsigned)now), dim3(kEigThreads), 0, s, n, nvec, ai, ti, info + first);
       err = hipGetLastError();
     }
   }
   if (err != hipSuccess) {
-    hfjk_internal_set_error((std::string("eig_lowest_kernel launch: ") + hipGetErrorString(err)).c_str());
+    hfjk_internal_set_error((std::string("eigensolver launch: ") + hipGetErrorString(err)).c_str());
     return HFJK_ERR_HIP;
   }
   return HFJK_OK;

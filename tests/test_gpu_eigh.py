@@ -108,3 +108,36 @@ def test_sizes_around_the_resident_block_and_the_register_chunks(n, nvec, count)
     mats = g + g.transpose(0, 2, 1)
     w, x = _solve(mats, nvec)
     _check(mats, nvec, w, x)
+
+
+def test_more_matrices_than_one_grid():
+    """4.2 million 16 x 16 matrices (2^32 work-items and more of the eigenvalues' grid): traces of all, the
+    eigenvalues of those around the launches' ends."""
+    import torch
+
+    from hafnium_amd import _lib
+    from hafnium_amd.coulomb_exchange import _Context
+
+    ctx = _Context(0)
+    n, count = 16, (1 << 22) + 13
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GiB of free GPU memory")
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(3)
+    a = torch.randn((count, n, n), generator=g, dtype=torch.float64, device="cuda:0")
+    a += a.transpose(1, 2).clone()
+    trace = a.diagonal(dim1=1, dim2=2).sum(1)
+    at = [i for start in range(0, count, 1 << 19) for i in (start - 1, start, start + 1) if i >= 0] + [count - 1]
+    want = np.linalg.eigvalsh(a[at].cpu().numpy())
+    w = torch.empty((count, n), dtype=torch.float64, device="cuda:0")
+    work = torch.empty(int(ctx.lib.hfjk_eigh_lowest_batched_work(n, count, n)), dtype=torch.float64, device="cuda:0")
+    info = torch.full((count,), 7, dtype=torch.int32, device="cuda:0")
+    p = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
+    _lib.check(ctx.lib.hfjk_eigh_lowest_batched(ctx.handle, n, count, n, p(a), p(w), p(work), p(info),
+                                                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert int(info.abs().max()) == 0
+    assert float((w.sum(1) - trace).abs().max()) <= 1e-10
+    assert np.abs(w[at].cpu().numpy() - want).max() <= 1e-11
+    # Rows of A are the eigenvectors: unit length, all of them.
+    assert float((a.square().sum(2) - 1.0).abs().max()) <= 1e-12
