@@ -1548,7 +1548,8 @@ struct Streams {
 template <int LAB, int LC>
 void launch_aux(const LaneArgs& a, Streams st) {
   const unsigned per = (unsigned)(a.nblk * a.nchunk);
-  const int most = (int)((1u << 28) / per);  // pairs per launch
+  // Pairs per launch: a grid holds less than 2^32 work-items.
+  const int most = std::max(1, (int)((1u << 31) / (64 * kLaneWaves) / per));
   for (int first = 0; first < a.npairs;) {
     const bool split = first < a.nsplit && LAB + LC <= kLaneRegL;
     const size_t lds = LAB + LC > kLaneRegL ? n_herm(LAB + LC) * 512
@@ -1730,8 +1731,8 @@ void launch_triples(hfjk_ctx* ctx, const std::vector<Shell>& orb, const std::vec
                  metric_mode ? 1 : 0, out};
       launch_aux_any(l, c, a, Streams{s, side});
     }
-  // At most 2^31 - 1 workgroups per launch.
-  const size_t per = (size_t)1 << 30;
+  // A grid holds less than 2^32 work-items.
+  const size_t per = ((size_t)1 << 31) / 64;
   for (size_t base = 0; base < items.size(); base += per) {
     const unsigned count = (unsigned)std::min(per, items.size() - base);
     hipLaunchKernelGGL(triple_kernel, dim3(count), dim3(64), 0, s, dev.at<DItem>(o_items) + base,
