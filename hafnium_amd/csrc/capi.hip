@@ -109,10 +109,6 @@ int syrk_splits(long long npairs, int naux) {
   return (int)(((std::max(1LL, s) + 7) / 8) * 8);
 }
 
-// Exchange operands in BF16X3 are not implemented by a dedicated kernel yet;
-// the exchange in that precision runs on the FP32 tensor copy through the
-// FP32 MFMA path only when that copy is bound (see exchange_precision).
-
 struct Layout {
   // density factorisation region
   size_t dens_a, dens_w, dens_e, dens_info, dens_stats, dens_c, dens_signs, dens_end;
@@ -131,6 +127,7 @@ struct Layout {
   long long p, ntiles;
 };
 
+// nsplit_k: SYRK splits (0: the tuned or modelled count, with shortened runs).
 Layout make_layout(const hfjk_ctx* ctx, int nocc, int precision, int nsplit_k = 0) {
   Layout L{};
   const int n = ctx->nao, naux = ctx->naux;
@@ -772,7 +769,8 @@ int hfjk_coulomb_charges(hfjk_ctx* ctx, const double* charges, double* coulomb, 
     check_precision(precision);
     check_bound(ctx, precision);
     if (charges == nullptr || coulomb == nullptr) fail(HFJK_ERR_INPUT, "null pointer");
-    const Layout L = make_layout(ctx, 1, precision == HFJK_FP64 ? HFJK_FP64 : HFJK_FP32);
+    // The Coulomb region alone, which no SYRK split count moves.
+    const Layout L = make_layout(ctx, 1, precision == HFJK_FP64 ? HFJK_FP64 : HFJK_FP32, 8);
     if (workspace_bytes < L.c_end || workspace == nullptr)
       fail(HFJK_ERR_WORKSPACE, "workspace smaller than the coulomb needs (" + std::to_string(L.c_end) + " bytes)");
     if (((uintptr_t)workspace & 255) != 0) fail(HFJK_ERR_WORKSPACE, "workspace must be 256-byte aligned");
@@ -800,7 +798,8 @@ int hfjk_coulomb(hfjk_ctx* ctx, const double* density, double* coulomb, int prec
     check_precision(precision);
     check_bound(ctx, precision);
     if (density == nullptr || coulomb == nullptr) fail(HFJK_ERR_INPUT, "null matrix pointer");
-    const Layout L = make_layout(ctx, 1, precision == HFJK_FP64 ? HFJK_FP64 : HFJK_FP32);
+    // The Coulomb region alone, which no SYRK split count moves.
+    const Layout L = make_layout(ctx, 1, precision == HFJK_FP64 ? HFJK_FP64 : HFJK_FP32, 8);
     if (workspace_bytes < L.c_end || workspace == nullptr)
       fail(HFJK_ERR_WORKSPACE, "workspace smaller than the coulomb needs (" + std::to_string(L.c_end) + " bytes)");
     if (((uintptr_t)workspace & 255) != 0) fail(HFJK_ERR_WORKSPACE, "workspace must be 256-byte aligned");

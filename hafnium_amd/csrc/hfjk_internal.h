@@ -303,7 +303,7 @@ constexpr int kSyrkRunProducts = 4096;
 int syrk_run_aux(int precision, int ldo);
 int syrk_run_for(int precision, int naux, int nao, int ldo, int cus);
 int syrk_slots(int naux, int run, int nsplit);
-// Default split count of the unsigned SYRK (a multiple of 8) on a device of `cus` compute units.
+// Default split count of the SYRK (a multiple of 8) on a device of `cus` compute units.
 int syrk_split_count(int precision, int naux, int nao, int ldo, int run, int cus);
 // auxsign (optional, [naux]): one more factor per aux function on the signed
 // FP64/FP32 direct-LDS kernels; shift (a multiple of 32 below ldo): the

@@ -2628,53 +2628,117 @@ static int tile_blocks(int nblk, int eb, int r, int c) {
 // longest one; FP64 writes and reads back a partial per split and tile.
 // (A fixed target of 2048 workgroups wrote 270 MB of partials whatever the
 // size, and at nao 709 / naux 2503 in FP32 left 25 of 104 splits without a
-// slot.) The last answer is kept per thread: a program asks for one shape
-// many times.
-int syrk_split_count(int precision, int naux, int nao, int ldo, int run, int cus) {
-  struct Last {
-    int precision = -1, naux = 0, nao = 0, ldo = 0, run = 0, cus = 0, splits = 0;
-  };
-  static thread_local Last last;
-  if (last.precision == precision && last.naux == naux && last.nao == nao && last.ldo == ldo && last.run == run &&
-      last.cus == cus)
-    return last.splits;
+// slot.) Signed columns run one workgroup per CU on 128-row tiles and take the
+// same count: within 9 % of the best of 2048, 1024, 512 and 256 workgroups
+// from nao 50 to 1500 (FP64 288 / 1356 / 60 569 us for 523, the largest
+// distance), where the fixed target took 1180 us there and 355 for 32 at 100.
+struct SplitModel {
+  int npairs, slots;
+  bool partials;
+  double chunk_steps;
+  std::vector<double> step_us;  // of every tile, in launch order
+  double step_sum = 0.0, step_max = 0.0;
+};
+
+struct SplitCandidate {
+  int n8, per, used;
+  double alone, least;  // least: no schedule of its jobs ends before
+};
+
+// The schedule's end; past `limit` some time that is past it too.
+static double split_model_us(const SplitModel& m, const SplitCandidate& c, double limit, std::vector<double>& busy) {
+  busy.assign(m.slots, 0.0);  // a heap: the earliest free slot on top
+  const double work = c.alone * c.per * m.chunk_steps;
+  double end = 0.0;
+  for (int s = 0; s < c.used && end <= limit; ++s)
+    for (double step : m.step_us) {
+      const double t = busy[0] + (work * step + 4.0);
+      end = std::max(end, t);
+      int at = 0;
+      for (int child = 1; child < m.slots; child = 2 * at + 1) {
+        child += child + 1 < m.slots && busy[child + 1] < busy[child];
+        if (busy[child] >= t) break;
+        busy[at] = busy[child];
+        at = child;
+      }
+      busy[at] = t;
+    }
+  return end;
+}
+
+static int modelled_split_count(int precision, int naux, int nao, int ldo, int run, int cus) {
   const int nblk = (nao + 15) / 16, eb = syrk_row_block(nao) / 16;
-  const int nb = (nblk + 7) / 8, npairs = nb * (nb + 1) / 2;
+  const int nb = (nblk + 7) / 8;
+  SplitModel m;
+  m.npairs = nb * (nb + 1) / 2;
+  m.slots = std::max(1, 2 * cus / 8);  // of one XCD
+  m.partials = run == 0;
+  m.chunk_steps = (double)(run == 0 ? 1 : run) * ldo / (precision == HFJK_FP64 ? 8 : 16);
   const int nslot = run == 0 ? naux : (naux + run - 1) / run;
-  const double chunk_steps = (double)(run == 0 ? 1 : run) * ldo / (precision == HFJK_FP64 ? 8 : 16);
-  const double partial_us = npairs * 2.0 * kSyrkTile * kSyrkTile * 8.0 / 5e6;
-  const int slots = std::max(1, 2 * cus / 8);  // of one XCD
-  std::vector<double> step_us;
-  for (int r = 0; r < nb && npairs <= 1024; ++r)
-    for (int c = 0; c <= r; ++c) step_us.push_back(std::max(0.45, 1.7 * tile_blocks(nblk, eb, r, c) / 16.0));
+  const double partial_us = m.npairs * 2.0 * kSyrkTile * kSyrkTile * 8.0 / 5e6;
+  for (int r = 0; r < nb && m.npairs <= 1024; ++r)
+    for (int c = 0; c <= r; ++c) {
+      m.step_us.push_back(std::max(0.45, 1.7 * tile_blocks(nblk, eb, r, c) / 16.0));
+      m.step_sum += m.step_us.back();
+      m.step_max = std::max(m.step_max, m.step_us.back());
+    }
+  // The candidates' costs with the schedule's end bounded from below by the mean load of a slot and
+  // by the longest job; schedules are formed from the least bound on, until no bound left is below
+  // the best of them.
+  const int top = std::min((nslot + 7) / 8, m.npairs <= 1024 ? std::max(1, 24 * m.slots / m.npairs) : 1);
+  std::vector<SplitCandidate> list;
+  for (int n8 = 1; n8 <= top; ++n8) {
+    SplitCandidate c;
+    c.n8 = n8;
+    c.per = (nslot + 8 * n8 - 1) / (8 * n8);  // chunks of the fullest split
+    if (n8 > 1 && c.per == (nslot + 8 * n8 - 9) / (8 * n8 - 8)) continue;
+    c.used = std::min(n8, (((nslot + c.per - 1) / c.per) + 7) / 8);  // splits of one XCD that hold chunks
+    c.alone = c.used * m.npairs * 2 <= m.slots ? 0.58 : 1.0;
+    const double work = c.alone * c.per * m.chunk_steps;
+    const double longest = work * m.step_max + 4.0;
+    const double load = c.used * (work * m.step_sum + 4.0 * m.npairs) / m.slots;
+    c.least = std::max(load, longest) + 0.3 * longest + (m.partials ? 8 * n8 * partial_us : 0.0);
+    list.push_back(c);
+  }
+  std::sort(list.begin(), list.end(), [](const SplitCandidate& x, const SplitCandidate& y) { return x.least < y.least; });
   int best = 8;
   double best_us = 1e300;
-  const int top = std::min((nslot + 7) / 8, npairs <= 1024 ? std::max(1, 24 * slots / npairs) : 1);
   std::vector<double> busy;
-  for (int n8 = 1; n8 <= top; ++n8) {
-    const int per = (nslot + 8 * n8 - 1) / (8 * n8);  // chunks of the fullest split
-    if (n8 > 1 && per == (nslot + 8 * n8 - 9) / (8 * n8 - 8)) continue;
-    const int used = std::min(n8, (((nslot + per - 1) / per) + 7) / 8);  // splits of one XCD that hold chunks
-    const double alone = used * npairs * 2 <= slots ? 0.58 : 1.0;
-    busy.assign(slots, 0.0);  // a heap: the earliest free slot on top
-    double end = 0.0, longest = 0.0;
-    for (int s = 0; s < used; ++s)
-      for (double step : step_us) {
-        const double job = alone * step * per * chunk_steps + 4.0;
-        std::pop_heap(busy.begin(), busy.end(), std::greater<double>());
-        busy.back() += job;
-        longest = std::max(longest, job);
-        end = std::max(end, busy.back());
-        std::push_heap(busy.begin(), busy.end(), std::greater<double>());
-      }
-    const double us = end + 0.3 * longest + (run == 0 ? 8 * n8 * partial_us : 0.0);
-    if (us < best_us) {
+  for (const SplitCandidate& c : list) {
+    if (c.least * (1.0 - 1e-9) > best_us || m.step_us.empty()) break;
+    const double longest = c.alone * m.step_max * c.per * m.chunk_steps + 4.0;
+    const double rest = 0.3 * longest + (m.partials ? 8 * c.n8 * partial_us : 0.0);
+    const double us = split_model_us(m, c, best_us - rest, busy) + rest;
+    if (us < best_us || (us == best_us && 8 * c.n8 < best)) {
       best_us = us;
-      best = 8 * n8;
+      best = 8 * c.n8;
     }
   }
-  last = Last{precision, naux, nao, ldo, run, cus, best};
   return best;
+}
+
+// The model takes 1 us at nao 100 and 0.3 ms at 1500, on the host, and every
+// call and workspace query of a build asks it: the last answers are kept per
+// thread, for as many shapes as a loop over molecules and both spins meets.
+int syrk_split_count(int precision, int naux, int nao, int ldo, int run, int cus) {
+  struct Shape {
+    int precision, naux, nao, ldo, run, cus;
+    bool operator==(const Shape& o) const {
+      return precision == o.precision && naux == o.naux && nao == o.nao && ldo == o.ldo && run == o.run && cus == o.cus;
+    }
+  };
+  constexpr int kKept = 64;
+  static thread_local Shape shapes[kKept];
+  static thread_local int splits[kKept], kept = 0, next = 0;
+  const Shape shape{precision, naux, nao, ldo, run, cus};
+  for (int i = 0; i < kept; ++i)
+    if (shapes[i] == shape) return splits[i];
+  const int count = modelled_split_count(precision, naux, nao, ldo, run, cus);
+  shapes[next] = shape;
+  splits[next] = count;
+  kept = std::max(kept, next + 1);
+  next = (next + 1) % kKept;
+  return count;
 }
 
 double syrk_instance_us(int precision, int naux, int nao, int nocc, bool ring, double& whole_us) {

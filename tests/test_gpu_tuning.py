@@ -148,3 +148,28 @@ def test_capped_coulomb_grids_give_the_same_build(precision):
     jk.set_tuning(_lib.TUNE_COULOMB_SERIAL, 0)
     with pytest.raises(ValueError):
         jk.set_tuning(_lib.TUNE_COULOMB_SERIAL, 2)
+
+
+def test_split_counts_of_alternating_shapes_are_found_once():
+    """The modelled split count of the SYRK: a program that alternates shapes (both calls of a density, spins,
+    molecules) pays for the model once per shape, not in every call and query."""
+    import ctypes
+    import time
+
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+
+    jk = MI355XCoulombExchange.synthetic(3, 2500, 400)
+    lib, size = jk._ctx.lib, ctypes.c_size_t()
+
+    def queries():
+        start = time.perf_counter()
+        sizes = []
+        for nocc in range(16, 400, 32):
+            _lib.check(lib.hfjk_workspace_bytes(jk._ctx.handle, nocc, _lib.FP64, ctypes.byref(size)))
+            sizes.append(size.value)
+        return time.perf_counter() - start, sizes
+
+    first, sizes = queries()
+    again = [queries() for _ in range(5)]
+    assert all(s == sizes for _, s in again)
+    assert min(t for t, _ in again) < 0.2 * first, (first, again)
