@@ -1080,8 +1080,12 @@ int hfjk_exchange_density(hfjk_ctx* ctx, const double* density, double* exchange
       check_hip(hipMemsetAsync(exchange, 0, sizeof(double) * n * n, s), "hipMemsetAsync");
       return;
     }
+    // The workspace is that of full rank. A modelled split count need not fall with the rank: with 8
+    // splits (the least) and full runs the layout does.
+    Layout R = make_layout(ctx, r, kprec);
+    if (R.x_end > workspace_bytes) R = make_layout(ctx, r, kprec, 8);
     // All signs +1 (a positive semidefinite density): the unsigned SYRK.
-    run_exchange(ctx, cf, r, nneg > 0 ? sg : nullptr, exchange, precision, workspace, make_layout(ctx, r, kprec), s);
+    run_exchange(ctx, cf, r, nneg > 0 ? sg : nullptr, exchange, precision, workspace, R, s);
   });
 }
 
