@@ -211,8 +211,7 @@ class Mlp:
             return loss
         floats = self.lib.hfjk_mlp_train_workspace(layers, self._c_sizes, m)
         work = torch.empty(floats, dtype=torch.float32, device=self.device)
-        self.step_count += 1
-        beta1, beta2, t = 0.9, 0.999, self.step_count
+        beta1, beta2, t = 0.9, 0.999, self.step_count + 1
         lr_t = lr * math.sqrt(1.0 - beta2 ** t) / (1.0 - beta1 ** t)
         self._check(self.lib.hfjk_mlp_train_step(
             self._ctx.handle, layers, self._c_sizes, m, _ptr(x),
@@ -220,6 +219,7 @@ class Mlp:
             None if col_weights is None else _ptr(col_weights), 1.0 / m, _ptr(self.params), _ptr(self.params16),
             _ptr(self.grads), _ptr(self.moment1), _ptr(self.moment2), float(lr), float(lr_t), beta1, beta2, 1e-8,
             float(weight_decay), _ptr(work), _ptr(self._loss), self._stream()))
+        self.step_count = t
         self._acts = (None, gather, m)
         self._work = (work, x)
         return self._loss

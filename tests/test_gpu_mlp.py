@@ -285,3 +285,21 @@ def test_training_step_of_more_tiles_than_one_grid():
         assert np.linalg.norm(db - db_ref) <= 2e-2 * np.linalg.norm(db_ref)
     del big
     torch.cuda.empty_cache()
+
+
+def test_refused_training_step_leaves_the_state():
+    """A target narrower than the output is refused; the next step is then the first, as if it had not been asked."""
+    torch = _torch()
+    from hafnium_amd.mlp import Mlp
+
+    net, fresh = Mlp([6, 10, 4], seed=12), Mlp([6, 10, 4], seed=12)
+    g = torch.Generator(device=net.device)
+    g.manual_seed(7)
+    x = torch.randn((20, 6), generator=g, device=net.device)
+    t = torch.randn((20, 4), generator=g, device=net.device)
+    with pytest.raises(ValueError):
+        net.train_step(x, t[:, :3].contiguous(), None, lr=1e-2)
+    assert net.step_count == 0
+    for n in (net, fresh):
+        n.train_step(x, t, None, lr=1e-2)
+    assert net.step_count == 1 and torch.equal(net.params, fresh.params)
