@@ -763,9 +763,13 @@ int hfjk_batch_run(hfjk_batch* batch, const void* tensor, const double* orbitals
   hipStream_t cs = beside ? batch->side : s;
   if (e == hipSuccess && beside) e = hipEventRecord(batch->fork, s);
   if (e == hipSuccess && beside) e = hipStreamWaitEvent(cs, batch->fork, 0);
+  const bool forked = e == hipSuccess && beside;
   if (e == hipSuccess && density != nullptr)
     e = hfjk::launch_batch_coulomb(v, prec, tensor, batch->b_total, density, ws64, coulomb, cs);
-  if (e == hipSuccess && beside) e = hipEventRecord(batch->join, cs);
+  // Once forked, s waits for the side stream whatever fails: the caller may free J and the
+  // workspace on return, and a capture must not end with a stream of its own.
+  const hipError_t recorded = forked ? hipEventRecord(batch->join, cs) : hipSuccess;
+  if (e == hipSuccess) e = recorded;
   if (e == hipSuccess)
     e = hfjk::launch_batch_orbitals(v, prec, orbitals, ws64, cbase, batch->cp_total, s);
   if (e == hipSuccess)
@@ -778,7 +782,10 @@ int hfjk_batch_run(hfjk_batch* batch, const void* tensor, const double* orbitals
   if (e == hipSuccess)
     e = hfjk::launch_batch_syrk(v, prec, xbase, batch->x_total, ws64, kbase, batch->grid_mfma, s);
   if (e == hipSuccess) e = hfjk::launch_batch_syrk_reduce(v, prec, kbase, exchange, s);
-  if (e == hipSuccess && beside) e = hipStreamWaitEvent(s, batch->join, 0);
+  if (forked && recorded == hipSuccess) {
+    const hipError_t joined = hipStreamWaitEvent(s, batch->join, 0);
+    if (e == hipSuccess) e = joined;
+  }
   if (e != hipSuccess) {
     hfjk_internal_set_error((std::string("batched launch: ") + hipGetErrorString(e)).c_str());
     return HFJK_ERR_HIP;
