@@ -573,11 +573,14 @@ int hfjk_batch_create(hfjk_ctx* ctx, const hfjk_batch_instance* instances, int n
     // Splits: about 8192 k per item, and where the batch is small enough that the longest such
     // item would outlast the others, as many as bring an instance's slowest tile down to a quarter
     // of the batch's mean load per workgroup slot (12 water clusters: 4 rounds of items instead of
-    // a first round that holds 1.7 ms items, 2.07 -> 0.8 ms).
+    // a first round that holds 1.7 ms items, 2.07 -> 0.8 ms). Eight rounds of one instance's items
+    // are enough: its partials stay below 0.6 GB, where items of 1.7 ms would take 7.5 GB at nao
+    // 3000 / naux 5000 / nocc 300.
     double whole_us;
     hfjk::syrk_instance_us(precision, src.naux, src.nao, src.nocc, in.se != 64, whole_us);
     const long long by_k = std::min(64LL, ((long long)src.naux * in.ldo + 8191) / 8192);
-    const long long by_load = std::min<long long>(src.naux, (long long)std::ceil(whole_us / item_us));
+    const long long by_load = std::min<long long>(std::min<long long>(src.naux, 16LL * cus / in.npairs),
+                                                  (long long)std::ceil(whole_us / item_us));
     in.nsplit = (int)std::max(1LL, std::max(by_k, by_load));
     in.bm = 128;
     if (precision == HFJK_BF16X3) {

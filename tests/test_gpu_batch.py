@@ -125,3 +125,26 @@ def test_coulomb_half_beside_the_half_transform(torch, precision):
         assert torch.equal(j, j0) and torch.equal(k, k0)
         bt.run(c, d, precision=precision)
         torch.cuda.synchronize()
+
+
+def test_partials_of_large_instances_stay_bounded(torch):
+    """The workspace of one large instance: X, the Coulomb half and at most 64 splits' partials (a plan, not run)."""
+    import ctypes
+
+    from hafnium_amd import _lib
+    from hafnium_amd.batch import _Instance
+    from hafnium_amd.coulomb_exchange import _Context
+
+    ctx, inst, plan, size = _Context(0), (_Instance * 1)(), ctypes.c_void_p(), ctypes.c_size_t()
+    for nao, naux, nocc in ((3000, 5000, 300), (1500, 5000, 250), (288, 1356, 60)):
+        inst[0] = _Instance(nao, naux, nocc, 0, 0, 0)
+        _lib.check(ctx.lib.hfjk_batch_create(ctx.handle, inst, 1, _lib.FP64, 0, ctypes.byref(plan)))
+        _lib.check(ctx.lib.hfjk_batch_workspace_bytes(plan, ctypes.byref(size)))
+        _lib.check(ctx.lib.hfjk_batch_destroy(plan))
+        rows, ldo = -(-nao // 64) * 64, -(-nocc // 32) * 32
+        tiles = -(-nao // 32) * (-(-nao // 32) + 1) // 2
+        blocks = -(-rows // 128)
+        x = naux * rows * ldo * 8
+        coulomb = tiles * (naux + 1024 * (1 + naux / 64)) * 8  # charge partials, weights and slices of J
+        partials = 64 * blocks * (blocks + 1) / 2 * 128 * 128 * 8
+        assert size.value <= x + coulomb + max(partials, 0.6e9) + 1e8, (nao, size.value)
