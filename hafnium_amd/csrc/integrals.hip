@@ -887,6 +887,14 @@ constexpr int kBoysTaylor = 7;
 constexpr int kBoysOrders = kGMaxL + kBoysTaylor + 1;
 constexpr int kBoysPoints = (int)(kBoysTMax / kBoysStep) + 2;
 
+// a / b from r, the rounded reciprocal of b: the product's remainder corrects it to the rounded
+// quotient (the last step of Markstein's division). The products alone took the upward recursion
+// from 6.6 to 11.2 half units in the last place at order 8, the downward one from 5.6 to 6.3.
+__device__ __forceinline__ double quotient(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
+}
+
 __device__ __forceinline__ void boys_d(int nmax, double t, const double* __restrict__ table, double* f) {
   const double et = exp(-t);
   if (t < kBoysTMax) {
@@ -900,11 +908,11 @@ __device__ __forceinline__ void boys_d(int nmax, double t, const double* __restr
       sum += term * row[k];
     }
     f[nmax] = sum;
-    for (int n = nmax - 1; n >= 0; --n) f[n] = (2.0 * t * f[n + 1] + et) * (1.0 / (2 * n + 1));
+    for (int n = nmax - 1; n >= 0; --n) f[n] = quotient(2.0 * t * f[n + 1] + et, 2 * n + 1, 1.0 / (2 * n + 1));
   } else {
     f[0] = 0.5 * sqrt(kPi / t);  // erf(sqrt(t)) is 1 to the last bit here
     const double i2t = 0.5 / t;
-    for (int n = 0; n < nmax; ++n) f[n + 1] = ((2 * n + 1) * f[n] - et) * i2t;
+    for (int n = 0; n < nmax; ++n) f[n + 1] = quotient((2 * n + 1) * f[n] - et, 2.0 * t, i2t);
   }
 }
 
