@@ -23,6 +23,8 @@ from hafnium_amd import _lib
 
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "hafnium_amd", "tuning.json")
 TILE_CANDIDATES = (32, 64, 128, 256)
+# Of the kernels that a cached schedule was timed on: an entry of other kernels is timed anew.
+KERNELS = 2
 
 
 @dataclass
@@ -34,7 +36,7 @@ class TuningResult:
     syrk_ms: dict = field(default_factory=dict)
     seconds: float = 0.0
     from_cache: bool = False
-    x_bm: int = 64
+    x_bm: int = 0
 
 
 def _device_name(jk) -> str:
@@ -57,7 +59,7 @@ def tuning_key(jk, nocc: int, precision: str) -> str:
 def _split_candidates(jk) -> list[int]:
     nb = (-(-jk.n_ao // 64) * 64 + 127) // 128
     pairs = nb * (nb + 1) // 2
-    out = set()
+    out = {0}  # the library's own count
     for target in (512, 1024, 2048, 4096):
         s = max(1, min(-(-target // pairs), jk.n_aux))
         out.add(-(-s // 8) * 8)
@@ -75,9 +77,10 @@ def autotune(jk, orbitals, precision: str = "fp64", *, repeats: int = 2, cache_p
 
     ``orbitals`` is a representative ``[nao, nocc]`` matrix (values do not
     affect the timing). Both are timed inside the combined J + K build
-    (``jk_occupied``), where the Coulomb half runs beside the SYRK; among
-    split counts within 1 % of the fastest the smallest is kept (fewer
-    partials to reduce). The chosen parameters stay set on ``jk``.
+    (``jk_occupied``), where the Coulomb half may run beside the SYRK; among
+    split counts within 1 % of the fastest the library's own (0) is kept, else
+    the smallest (fewer partials to reduce), and among FP64 / FP32 tiles
+    within 1 % the library's default. The chosen parameters stay set on ``jk``.
     """
     import torch
 
@@ -87,10 +90,10 @@ def autotune(jk, orbitals, precision: str = "fp64", *, repeats: int = 2, cache_p
     if use_cache and cache_path and os.path.exists(cache_path):
         with open(cache_path) as fh:
             cached = json.load(fh).get(key)
-        if cached:
+        if cached and cached.get("kernels") == KERNELS:
             jk.set_tuning(tile_param, cached["x_bn"])
             jk.set_tuning(_lib.TUNE_SYRK_SPLITS, cached["syrk_splits"])
-            bm = int(cached.get("x_bm", 64))
+            bm = int(cached.get("x_bm", 0))
             if precision != "bf16x3":
                 jk.set_tuning(_lib.TUNE_X_BM, bm)
             return TuningResult(key, cached["x_bn"], cached["syrk_splits"], cached.get("x_ms", {}),
@@ -99,8 +102,8 @@ def autotune(jk, orbitals, precision: str = "fp64", *, repeats: int = 2, cache_p
     start = time.perf_counter()
     ldo = -(-nocc // 32) * 32
     tiles = [(t, 64) for t in TILE_CANDIDATES if t // 2 < ldo or t == 32]
-    if precision != "bf16x3":
-        tiles += [(t, 128) for t, _ in tiles if t <= 128]
+    if precision != "bf16x3":  # 128 columns is the widest group, four waves the default
+        tiles = [(t, 128) for t, _ in reversed(tiles) if t <= 128] + [t for t in tiles if t[0] <= 128]
     splits = _split_candidates(jk)
     x_ms: dict = {}
     syrk_ms: dict[int, float] = {}
@@ -120,6 +123,8 @@ def autotune(jk, orbitals, precision: str = "fp64", *, repeats: int = 2, cache_p
                 jk.jk_occupied(orbitals, precision=precision)
             x_ms[tile] = _stage_ms(jk.stage_times(), "exchange_half_transform")
         best_tile = min(x_ms, key=x_ms.get)
+        if precision != "bf16x3" and x_ms[tiles[0]] <= 1.01 * x_ms[best_tile]:
+            best_tile = tiles[0]
         jk.set_tuning(tile_param, best_tile[0])
         if precision != "bf16x3":
             jk.set_tuning(_lib.TUNE_X_BM, best_tile[1])
@@ -156,7 +161,7 @@ def _store(path: str, key: str, result: TuningResult) -> None:
         except (OSError, ValueError):
             data = {}
     data[key] = {"x_bn": result.x_bn, "x_bm": result.x_bm, "syrk_splits": result.syrk_splits,
-                 "x_ms": result.x_ms, "syrk_ms": result.syrk_ms}
+                 "x_ms": result.x_ms, "syrk_ms": result.syrk_ms, "kernels": KERNELS}
     tmp = path + ".tmp"
     with open(tmp, "w") as fh:
         json.dump(data, fh, indent=1)

@@ -68,6 +68,29 @@ def test_autotune_sets_a_valid_schedule(tmp_path):
     assert jk_ref.max_relative_error(k, jk_ref.exchange_occupied(b, c)) < BF16X3_REL_TOL
 
 
+@pytest.mark.parametrize("stale", [{}, {"kernels": 1}])
+def test_autotune_candidates_and_stale_entries(tmp_path, stale):
+    """The library's own split count and default tile are among the candidates, no kernel is timed twice, and a
+    cached schedule of other kernels is not applied."""
+    import json
+
+    from hafnium_amd.autotune import autotune, tuning_key
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+
+    b, c, _ = synthetic.jk_inputs(5, 40, 200, 60)
+    jk = MI355XCoulombExchange(b)
+    cache = tmp_path / "tuning.json"
+    cache.write_text(json.dumps({tuning_key(jk, 60, "fp64"): {"x_bn": 32, "syrk_splits": 8, **stale}}))
+    result = autotune(jk, c, "fp64", cache_path=str(cache))
+    assert not result.from_cache
+    assert set(result.x_ms) == {"32", "64", "32x128", "64x128"} and "0" in result.syrk_ms
+    assert (jk.get_tuning(_lib.TUNE_X_BN), jk.get_tuning(_lib.TUNE_X_BM)) == (result.x_bn, result.x_bm)
+    assert result.syrk_ms[str(result.syrk_splits)] <= 1.01 * min(result.syrk_ms.values())
+    if result.syrk_ms["0"] <= 1.01 * min(result.syrk_ms.values()):
+        assert result.syrk_splits == 0
+    assert autotune(MI355XCoulombExchange(b), c, "fp64", cache_path=str(cache)).from_cache
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
 @pytest.mark.parametrize("naux,nao,nocc,splits", [
     (9, 150, 70, 8),     # last 128-row block holds 64 rows of X
