@@ -134,3 +134,78 @@ def test_first_batch_of_primitive_pairs_without_a_survivor(distance):
             a, b = slice(i * n, (i + 1) * n), slice(j * n, (j + 1) * n)
             # Against the block's own size: the far blocks are 1e-13 of the others.
             assert np.abs(got[:, a, b] - host[:, a, b]).max() <= 1e-10 * np.abs(host[:, a, b]).max(), (i, j)
+
+
+def _three_center_into(ctx, aux, orb, out, stream):
+    import ctypes
+
+    from hafnium_amd import _lib
+
+    a, o = aux.c_struct(), orb.c_struct()
+    _lib.check(ctx.lib.hfjk_int3c2e_device(ctx.handle, ctypes.byref(a), ctypes.byref(o),
+                                           ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(stream.cuda_stream)))
+
+
+@pytest.mark.parametrize("threads", [1, 2])
+def test_integrals_beside_builds_of_the_same_context(threads):
+    """The integrals and a J/K build share the context's side stream: on streams of their own, behind work that
+    writes the output first, from one thread and from two, each gives what it gives alone."""
+    import threading
+
+    import torch
+
+    from hafnium_amd import synthetic
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+
+    mol = molecule.water_cluster(3, 9)
+    orb, aux = molecule.BasisOnAtoms("cc-pvdz", mol), molecule.BasisOnAtoms("def2-universal-jkfit", mol)
+    nao, naux, nocc = 200, 600, 30  # 7e8 products: in FP32 the Coulomb half runs on the side stream
+    jk = MI355XCoulombExchange.synthetic(4, naux, nao, precision="fp32")
+    c = torch.from_numpy(synthetic.occupied_orbitals(4, nao, nocc)).cuda()
+    want_j, want_k = (x.clone() for x in jk.jk_occupied(c))
+    want = integrals.three_center_device(aux, orb)
+    load = torch.randn((2048, 2048), device="cuda:0")
+    torch.cuda.synchronize()
+    failures = []
+
+    def build(times):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(times):
+                j, k = jk.jk_occupied(c)
+                if not (torch.equal(j, want_j) and torch.equal(k, want_k)):
+                    failures.append("build")
+        stream.synchronize()
+
+    def integrate(times):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(times):
+                out = torch.empty_like(want)
+                for _ in range(4):
+                    torch.matmul(load, load)
+                out.fill_(float("nan"))  # behind the products: the integrals wait for it on every stream
+                _three_center_into(jk._ctx, aux, orb, out, stream)
+                if not torch.equal(out, want):
+                    failures.append("integrals")
+        stream.synchronize()
+
+    if threads == 1:
+        for _ in range(6):
+            build(1)
+            integrate(1)
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        with torch.cuda.stream(streams[0]):  # a build in flight while the integrals run
+            j, k = jk.jk_occupied(c)
+        out = torch.empty_like(want)
+        streams[1].wait_stream(torch.cuda.current_stream())
+        _three_center_into(jk._ctx, aux, orb, out, streams[1])
+        torch.cuda.synchronize()
+        assert torch.equal(j, want_j) and torch.equal(k, want_k) and torch.equal(out, want)
+    else:
+        workers = [threading.Thread(target=build, args=(20,)), threading.Thread(target=integrate, args=(20,))]
+        for w in workers:
+            w.start()
+        for w in workers:
+            w.join()
+    assert not failures
