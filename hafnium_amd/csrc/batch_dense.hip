@@ -61,27 +61,30 @@ rocblas_handle blas_for(hfjk_ctx* ctx, hipStream_t s) {
   return h;
 }
 
-// sum_e x[e] y[e] over the workgroup, in a fixed order; thread 0 gets it. One
-// workgroup's share is bound by the latency of its loads: 1024 threads with
-// eight pairs in flight (256 threads with one: 105 us for 300 x 300).
+// sum_e x[e] y[e] over the workgroup of T threads, in a fixed order; thread 0
+// gets it. One workgroup's share is bound by the latency of its loads: 1024
+// threads with eight pairs in flight (256 threads with one: 105 us for 300 x
+// 300). Sums of less than a round of those take 256 threads (5000 of 400
+// elements: 15 us by 1024).
 constexpr int kDotT = 1024;
+template <int T>
 __device__ double workgroup_dot(long long len, const double* __restrict__ x, const double* __restrict__ y) {
-  __shared__ double red[kDotT / 64];
+  __shared__ double red[T / 64];
   double s[8];
 #pragma unroll
   for (int u = 0; u < 8; ++u) s[u] = 0.0;
   long long e = threadIdx.x;
-  for (; e + 7 * kDotT < len; e += 8 * kDotT) {
+  for (; e + 7 * T < len; e += 8 * T) {
     double a[8], b[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      a[u] = x[e + u * kDotT];
-      b[u] = y[e + u * kDotT];
+      a[u] = x[e + u * T];
+      b[u] = y[e + u * T];
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) s[u] += a[u] * b[u];
   }
-  for (; e < len; e += kDotT) s[0] += x[e] * y[e];
+  for (; e < len; e += T) s[0] += x[e] * y[e];
   double t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o);
@@ -89,25 +92,27 @@ __device__ double workgroup_dot(long long len, const double* __restrict__ x, con
   __syncthreads();
   t = 0.0;
   if (threadIdx.x == 0)
-    for (int w = 0; w < kDotT / 64; ++w) t += red[w];
+    for (int w = 0; w < T / 64; ++w) t += red[w];
   return t;
 }
 
 // out[i] = sum_e x_i[e] y_i[e]; one workgroup per instance.
-__global__ __launch_bounds__(kDotT) void batched_dot_kernel(long long len, const double* __restrict__ x, long long sx,
-                                                            const double* __restrict__ y, long long sy,
-                                                            double* __restrict__ out) {
-  const double s = workgroup_dot(len, x + (long long)blockIdx.x * sx, y + (long long)blockIdx.x * sy);
+template <int T>
+__global__ __launch_bounds__(T) void batched_dot_kernel(long long len, const double* __restrict__ x, long long sx,
+                                                        const double* __restrict__ y, long long sy,
+                                                        double* __restrict__ out) {
+  const double s = workgroup_dot<T>(len, x + (long long)blockIdx.x * sx, y + (long long)blockIdx.x * sy);
   if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // out[i][a] = <hist[newest][i], hist[a][i]> over len elements, hist [nslots][count][len];
 // one workgroup per (instance, slot), fixed summation order.
-__global__ __launch_bounds__(kDotT) void history_dots_kernel(long long len, int count, const double* __restrict__ hist,
-                                                             int newest, double* __restrict__ out) {
+template <int T>
+__global__ __launch_bounds__(T) void history_dots_kernel(long long len, int count, const double* __restrict__ hist,
+                                                         int newest, double* __restrict__ out) {
   const int i = blockIdx.x, a = blockIdx.y;
-  const double s = workgroup_dot(len, hist + ((long long)newest * count + i) * len,
-                                 hist + ((long long)a * count + i) * len);
+  const double s = workgroup_dot<T>(len, hist + ((long long)newest * count + i) * len,
+                                    hist + ((long long)a * count + i) * len);
   if (threadIdx.x == 0) out[(long long)i * gridDim.y + a] = s;
 }
 
@@ -389,8 +394,12 @@ int hfjk_ddot_batched(hfjk_ctx* ctx, int count, long long len, const double* x, 
   return bguard(ctx, [&] {
     check_count(count);
     if (len < 0 || x == nullptr || y == nullptr || out == nullptr) bfail(HFJK_ERR_INPUT, "hfjk_ddot_batched: bad input");
-    hipLaunchKernelGGL(batched_dot_kernel, dim3(count), dim3(kDotT), 0, (hipStream_t)stream, len, x, stride_x, y,
-                       stride_y, out);
+    if (len < 8 * kDotT)
+      hipLaunchKernelGGL(batched_dot_kernel<kT>, dim3(count), dim3(kT), 0, (hipStream_t)stream, len, x, stride_x, y,
+                         stride_y, out);
+    else
+      hipLaunchKernelGGL(batched_dot_kernel<kDotT>, dim3(count), dim3(kDotT), 0, (hipStream_t)stream, len, x, stride_x,
+                         y, stride_y, out);
     bcheck_hip(hipGetLastError(), "batched_dot launch");
   });
 }
@@ -401,8 +410,12 @@ int hfjk_history_dots_batched(hfjk_ctx* ctx, int count, long long len, int nslot
     check_count(count);
     if (len < 0 || nslots < 1 || nslots > 64 || newest < 0 || newest >= nslots || hist == nullptr || out == nullptr)
       bfail(HFJK_ERR_INPUT, "hfjk_history_dots_batched: bad input");
-    hipLaunchKernelGGL(history_dots_kernel, dim3(count, nslots), dim3(kDotT), 0, (hipStream_t)stream, len, count, hist,
-                       newest, out);
+    if (len < 8 * kDotT)
+      hipLaunchKernelGGL(history_dots_kernel<kT>, dim3(count, nslots), dim3(kT), 0, (hipStream_t)stream, len, count,
+                         hist, newest, out);
+    else
+      hipLaunchKernelGGL(history_dots_kernel<kDotT>, dim3(count, nslots), dim3(kDotT), 0, (hipStream_t)stream, len,
+                         count, hist, newest, out);
     bcheck_hip(hipGetLastError(), "history_dots launch");
   });
 }
