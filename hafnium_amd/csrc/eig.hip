@@ -820,16 +820,22 @@ __device__ TriBounds tri_bounds(const double* d, const double* e, int n, int lan
                    fmax(tnorm, DBL_MIN), DBL_MIN * fmax(1.0, emax)};
 }
 
-// The nvec lowest eigenvalues by multisection, a wave each: its lanes count at 64 points of the
-// interval, which shrinks 65 times per round (about ten rounds). Bound by the chain of the Sturm
-// recurrence, n steps a round; d and e^2 come from LDS eight steps ahead of it (60 values of a
-// 288 x 288 matrix: 0.13 ms; eight lanes a value need twice the rounds).
+// The nvec lowest eigenvalues by multisection, LANES lanes each, which count at
+// LANES points of the interval: it shrinks LANES + 1 times per round. Bound by
+// the chain of the Sturm recurrence, n steps a round, while the waves find
+// SIMDs of their own: a wave per value then takes the fewest rounds (about ten;
+// 60 values of a 288 x 288 matrix: 0.13 ms). Past that by the operations, of
+// which eight lanes and 17 rounds take a quarter (256 matrices of 400 x 400, 80
+// values: 1.95 ms by whole waves). d and e^2 come from LDS eight steps ahead.
 constexpr int kValueWaves = 4;
+constexpr long long kValueFill = 4096;  // values from which eight lanes take one
+template <int LANES>
 __global__ __launch_bounds__(64 * kValueWaves) void eig_values_kernel(int n, int nvec, double* __restrict__ w_all,
                                                                        const double* __restrict__ work_all) {
+  constexpr int VALUES = 64 / LANES;  // of a wave
   __shared__ double2 t2[kEigMaxN + 8];  // (d_i, e_{i-1}^2)
   const int lane = threadIdx.x & 63;
-  const int parts = (nvec + kValueWaves - 1) / kValueWaves;
+  const int parts = (nvec + kValueWaves * VALUES - 1) / (kValueWaves * VALUES);
   const int matrix = blockIdx.x / parts, part = blockIdx.x % parts;
   const double* d = work_all + (long long)matrix * eig_work_per(n, nvec);
   const double* e = d + n;
@@ -838,14 +844,16 @@ __global__ __launch_bounds__(64 * kValueWaves) void eig_values_kernel(int n, int
     t2[i] = make_double2(i < n ? d[i] : 0.0, ep * ep);
   }
   __syncthreads();
-  const int j = part * kValueWaves + (threadIdx.x >> 6);
-  if (j >= nvec) return;
   const TriBounds tb = tri_bounds(d, e, n, lane);
+  const int j = (part * kValueWaves + (threadIdx.x >> 6)) * VALUES + lane / LANES;
+  if (j >= nvec) return;
+  const int point = lane % LANES, group = lane - point;
+  constexpr double sections = LANES + 1;
   const double tol = 0.5 * DBL_EPSILON * tb.tnorm;
   double a = tb.lo, b = tb.hi;
   for (int it = 0; it < 200; ++it) {
     if (b - a <= 2.0 * DBL_EPSILON * fmax(fabs(a), fabs(b)) + tol) break;
-    const double x = a + (b - a) * (double)(lane + 1) / 65.0;
+    const double x = a + (b - a) * (double)(point + 1) / sections;
     // count of negative pivots; the first step's e^2 is 0, so its previous pivot does not matter
     int cnt = 0;
     double q = 1.0;
@@ -860,24 +868,31 @@ __global__ __launch_bounds__(64 * kValueWaves) void eig_values_kernel(int n, int
         cnt += i0 + s < n && q < 0.0;
       }
     }
-    // The first point with count > j bounds the eigenvalue from above.
-    const unsigned long long above = __ballot(cnt > j);
-    const int sf = above ? __builtin_ctzll(above) : 64;
-    const double na = sf == 0 ? a : a + (b - a) * (double)sf / 65.0;
-    const double nb = sf == 64 ? b : a + (b - a) * (double)(sf + 1) / 65.0;
+    // The first point with count > j bounds the eigenvalue from above. (The lanes of a value are in
+    // the loop together; others may have left it.)
+    const unsigned long long above = __ballot(cnt > j) >> group & (~0ull >> (64 - LANES));
+    const int sf = above ? __builtin_ctzll(above) : LANES;
+    const double na = sf == 0 ? a : a + (b - a) * (double)sf / sections;
+    const double nb = sf == LANES ? b : a + (b - a) * (double)(sf + 1) / sections;
     a = na;
     b = nb;
   }
-  if (lane == 0) w_all[(long long)matrix * n + j] = 0.5 * (a + b);
+  if (point == 0) w_all[(long long)matrix * n + j] = 0.5 * (a + b);
 }
 
 // Eigenvectors of T, one lane each: the shifts of equal eigenvalues are separated by 10 eps |T|
 // (so that their iterations differ), two inverse iterations from a seeded start with a partially
 // pivoted LU of T - lambda I. A workgroup is one wave with as many vectors as their factors leave
 // room for in LDS, [n][vectors]; every recurrence over n is a serial chain, and from LDS it waits
-// 0.1 us where the same factors in memory cost 0.5 us for each eight steps.
-constexpr int kVectorBytes = 41;  // LDS per vector and row: five doubles and the swap flag
+// 0.1 us where the same factors in memory cost 0.5 us for each eight steps. U's superdiagonals
+// are stored too unless COMPACT, which forms them again from T, the swaps and the multipliers: that
+// adds to the chain (12 matrices of 288 x 288, 60 vectors: 0.08 ms of 1.92 in the whole solver), but
+// two fifths of the vectors in flight were the time of a batch that fills the chip (256 matrices of
+// 400 x 400, 80 vectors: 3.4 ms of 16.4).
+template <bool COMPACT>
+constexpr int kVectorBytes = COMPACT ? 25 : 41;  // LDS per vector and row: doubles and the swap flag
 constexpr int kVectorLds = 48 * 1024;
+template <bool COMPACT>
 __global__ __launch_bounds__(64) void eig_vectors_kernel(int n, int nvec, int per, const double* __restrict__ w_all,
                                                           double* __restrict__ work_all) {
   extern __shared__ double vec_lds[];
@@ -908,12 +923,12 @@ __global__ __launch_bounds__(64) void eig_vectors_kernel(int n, int nvec, int pe
     }
   }
   __syncthreads();
-  double* inv = vec_lds;                 // 1 / pivot
-  double* u1 = inv + (long long)n * per;  // U's two superdiagonals
-  double* u2 = u1 + (long long)n * per;
-  double* mul = u2 + (long long)n * per;
+  double* inv = vec_lds;  // 1 / pivot
+  double* mul = inv + (long long)n * per;
   double* yv = mul + (long long)n * per;
-  unsigned char* swp = (unsigned char*)(yv + (long long)n * per);
+  double* u1 = yv + (long long)n * per;  // U's two superdiagonals
+  double* u2 = u1 + (long long)n * per;
+  unsigned char* swp = (unsigned char*)(COMPACT ? u1 : u2 + (long long)n * per);
   if (lane < jn) {
     const int j = j0 + lane;
     const double lam = lam_all[j];
@@ -928,8 +943,10 @@ __global__ __launch_bounds__(64) void eig_vectors_kernel(int n, int nvec, int pe
       const double mult = rest / piv;
       const int at = k * per + lane;
       inv[at] = 1.0 / piv;
-      u1[at] = swap ? a1 : p1;
-      u2[at] = swap ? b1 : 0.0;
+      if constexpr (!COMPACT) {
+        u1[at] = swap ? a1 : p1;
+        u2[at] = swap ? b1 : 0.0;
+      }
       mul[at] = mult;
       swp[at] = swap;
       p0 = swap ? p1 - mult * a1 : a1 - mult * p1;
@@ -937,8 +954,11 @@ __global__ __launch_bounds__(64) void eig_vectors_kernel(int n, int nvec, int pe
     }
     if (fabs(p0) < tiny) p0 = p0 < 0.0 ? -tiny : tiny;
     inv[(n - 1) * per + lane] = 1.0 / p0;
-    u1[(n - 1) * per + lane] = 0.0;
-    u2[(n - 1) * per + lane] = 0.0;
+    swp[(n - 1) * per + lane] = false;  // no row below to swap with
+    if constexpr (!COMPACT) {
+      u1[(n - 1) * per + lane] = 0.0;
+      u2[(n - 1) * per + lane] = 0.0;
+    }
     double scale = 1.0;
 #pragma unroll
     for (int iter = 0; iter < 2; ++iter) {
@@ -969,13 +989,25 @@ __global__ __launch_bounds__(64) void eig_vectors_kernel(int n, int nvec, int pe
       double nrm = 0.0, x1 = 0.0, x2 = 0.0;  // x_{i+1}, x_{i+2}
       for (int i0 = n - 1; i0 >= 0; i0 -= 8) {
         double yy[8], a1[8], a2[8], rr[8];
+        bool sw = COMPACT && swp[i0 * per + lane];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-          const int at = max(i0 - s, 0) * per + lane;
+          const int i = max(i0 - s, 0), at = i * per + lane, before = max(i - 1, 0) * per + lane;
           yy[s] = yv[at];
           rr[s] = inv[at];
-          a1[s] = u1[at];
-          a2[s] = u2[at];
+          if constexpr (!COMPACT) {
+            a1[s] = u1[at];
+            a2[s] = u2[at];
+            continue;
+          }
+          // Row i of U: the row below where they were swapped, else row i of T less its elimination
+          // (which touches its superdiagonal only if the row it came from had been swapped). le[n - 1]
+          // is 0.
+          const bool swb = i > 0 && swp[before];
+          const double kept = swb ? -mul[before] * le[i] : le[i];
+          a1[s] = sw ? ld[min(i + 1, n - 1)] - lam : kept;
+          a2[s] = sw ? le[min(i + 1, n - 1)] : 0.0;
+          sw = swb;
         }
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
@@ -1083,7 +1115,8 @@ int hfjk_eigh_lowest_batched(hfjk_ctx* ctx, int n, int count, int nvec, double* 
                          count, info);
       err = hipGetLastError();
     }
-    const int per = nvec > 0 ? std::max(1, std::min(std::min(nvec, 64), kVectorLds / (kVectorBytes * n))) : 1;
+    const auto per_wave = [&](int bytes) { return std::max(1, std::min(std::min(nvec, 64), kVectorLds / (bytes * n))); };
+    const int per = nvec > 0 ? per_wave(kVectorBytes<false>) : 1, compact = nvec > 0 ? per_wave(kVectorBytes<true>) : 1;
     // A grid holds less than 2^32 work-items and the values take a wave per vector: 2^31 / 64 vectors at a
     // time (a multiple of 8 matrices, the XCDs' turn).
     const int most = std::max(8, (1 << 25) / std::max(nvec, 8) & ~7);
@@ -1094,10 +1127,20 @@ int hfjk_eigh_lowest_batched(hfjk_ctx* ctx, int n, int count, int nvec, double* 
       double* ti = work + first * eig_work_per(n, nvec);
       const hipStream_t s = (hipStream_t)stream;
       hipLaunchKernelGGL(eig_tridiagonal_kernel, dim3((unsigned)now), dim3(kEigThreads), 0, s, n, nvec, ai, ti);
-      hipLaunchKernelGGL(eig_values_kernel, dim3((unsigned)(now * ((nvec + kValueWaves - 1) / kValueWaves))),
-                         dim3(64 * kValueWaves), 0, s, n, nvec, wi, ti);
-      hipLaunchKernelGGL(eig_vectors_kernel, dim3((unsigned)(now * ((nvec + per - 1) / per))), dim3(64),
-                         (size_t)kVectorBytes * n * per, s, n, nvec, per, wi, ti);
+      if ((long long)now * nvec < kValueFill)
+        hipLaunchKernelGGL(eig_values_kernel<64>, dim3((unsigned)(now * ((nvec + kValueWaves - 1) / kValueWaves))),
+                           dim3(64 * kValueWaves), 0, s, n, nvec, wi, ti);
+      else
+        hipLaunchKernelGGL(eig_values_kernel<8>, dim3((unsigned)(now * ((nvec + 8 * kValueWaves - 1) / (8 * kValueWaves)))),
+                           dim3(64 * kValueWaves), 0, s, n, nvec, wi, ti);
+      // Two rounds of the three workgroups that a CU holds: past that a batch is bound by the vectors
+      // in flight (64 matrices of 288 x 288 with 60 vectors lose 0.1 ms to COMPACT, 300 gain 0.4).
+      if ((long long)now * nvec < 6LL * ctx->cus * per)
+        hipLaunchKernelGGL(eig_vectors_kernel<false>, dim3((unsigned)(now * ((nvec + per - 1) / per))), dim3(64),
+                           (size_t)kVectorBytes<false> * n * per, s, n, nvec, per, wi, ti);
+      else
+        hipLaunchKernelGGL(eig_vectors_kernel<true>, dim3((unsigned)(now * ((nvec + compact - 1) / compact))), dim3(64),
+                           (size_t)kVectorBytes<true> * n * compact, s, n, nvec, compact, wi, ti);
       hipLaunchKernelGGL(eig_orthonormal_kernel, dim3((unsigned)now), dim3(kEigThreads), 0, s, n, nvec, ti);
       hipLaunchKernelGGL(eig_back_kernel, dim3((unsigned)((now + 7) / 8 * 8 * ((nvec + 3) / 4))), dim3(64), 0, s, n,
                          nvec, now, ai, ti);

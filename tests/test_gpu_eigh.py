@@ -110,6 +110,27 @@ def test_sizes_around_the_resident_block_and_the_register_chunks(n, nvec, count)
     _check(mats, nvec, w, x)
 
 
+@pytest.mark.parametrize("n,nvec,count", [(1, 1, 30000), (2, 2, 20000), (3, 1, 9000), (33, 33, 1700), (65, 7, 1300),
+                                          (130, 64, 300), (257, 61, 170), (288, 33, 300), (300, 100, 90)])
+def test_batches_that_fill_the_chip(n, nvec, count):
+    """Eight lanes per eigenvalue and the vectors whose factors are formed again: every matrix's residuals and
+    orthonormality, and the eigenvalues of a few matrices alone, where a wave takes each."""
+    rng = np.random.default_rng(n + count)
+    g = rng.standard_normal((count, n, n))
+    mats = g + g.transpose(0, 2, 1)
+    mats[0] = np.diag(rng.standard_normal(n))  # every reflector empty
+    mats[1] = np.eye(n)
+    w, x = _solve(mats, nvec)
+    few = [0, 1, 2, count // 2, count - 1]
+    _check(mats[few], nvec, w[few], x[few])
+    alone, _ = _solve(mats[few], nvec)
+    scale = np.abs(mats).sum(2).max(1)
+    assert (np.abs(w[few, :nvec] - alone[:, :nvec]) <= 1e-13 * scale[few, None]).all()
+    resid = np.matmul(x, mats) - x * w[:, :nvec, None]
+    assert (np.abs(resid).max((1, 2)) <= 1e-11 * scale).all()
+    assert np.abs(np.matmul(x, x.transpose(0, 2, 1)) - np.eye(nvec)).max() <= 1e-11
+
+
 def test_more_matrices_than_one_grid():
     """4.2 million 16 x 16 matrices (2^32 work-items and more of the eigenvalues' grid): traces of all, the
     eigenvalues of those around the launches' ends."""
