@@ -802,7 +802,7 @@ int hfjk_int3c2e(const hfjk_basis* aux, const hfjk_basis* orbital, double* out) 
 // * lane per aux function (pair_kernel + aux_kernel) up to la + lb = 4 and lc =
 //   4, which is every bundled basis;
 // * one 64-lane workgroup per shell triple (triple_kernel) for higher
-//   angular momenta.
+//   angular momenta, and for the metric of few shells.
 //
 // Lane per aux function. pair_kernel turns each surviving primitive pair of a
 // shell pair into its Gaussian product and the matrix W from Hermite
@@ -1150,6 +1150,7 @@ constexpr int kLaneSlots = 16;     // primitive pairs whose Hermite tables pair_
 constexpr int kLaneWaves = 4;      // most waves sharing a pair's primitives
 constexpr int kPairThreads = 256;
 constexpr int kLaneMaxPrim = 16;   // aux shells with more primitives go to triple_kernel
+constexpr int kFewShells = 224;    // metrics of at most as many shells go to triple_kernel
 
 constexpr __host__ __device__ int n_herm(int l) { return (l + 1) * (l + 2) * (l + 3) / 6; }
 constexpr __host__ __device__ int n_cart(int l) { return (l + 1) * (l + 2) / 2; }
@@ -1615,8 +1616,12 @@ void launch_triples(hfjk_ctx* ctx, const std::vector<Shell>& orb, const std::vec
   std::vector<DItem> items;
   std::vector<int> aux_by_l[kGL + 1];
   for (int c = 0; c < (int)aux.size(); ++c) aux_by_l[aux[c].l].push_back(c);
+  // A small metric is bound by the 26 launches of the lane kernels and takes triple_kernel's one: (P|Q)
+  // of 1 water 0.41 ms for 0.69, 4 waters (148 shells) 0.52 / 0.77, 6 (222) 0.74 / 0.83, 8 (296) 1.04 /
+  // 0.84, 12 (444) 1.95 / 0.88.
+  const bool few = metric_mode && (int)aux.size() <= kFewShells;
   auto lane_aux = [&](int c, int lab) {
-    return lab <= kLaneMaxAB && aux[c].l <= kLaneMaxC && lab + aux[c].l <= kLaneMaxL &&
+    return !few && lab <= kLaneMaxAB && aux[c].l <= kLaneMaxC && lab + aux[c].l <= kLaneMaxL &&
            (int)aux[c].exps.size() <= kLaneMaxPrim;
   };
   bool all_short = true;
@@ -1624,7 +1629,7 @@ void launch_triples(hfjk_ctx* ctx, const std::vector<Shell>& orb, const std::vec
   for (const auto& [i, j] : pair_list) {
     const Shell& A = a_shells[i];
     const int lb = j >= 0 ? orb[j].l : 0, fb = j >= 0 ? orb[j].nfunc() : 1;
-    const bool lanes = A.l + lb <= kLaneMaxAB;
+    const bool lanes = !few && A.l + lb <= kLaneMaxAB;
     for (int l = lanes && all_short ? std::min(kLaneMaxC, kLaneMaxL - A.l - lb) + 1 : 0; l <= kGL; ++l)
       for (int c : aux_by_l[l])
         if ((!metric_mode || c <= i) && !lane_aux(c, A.l + lb)) items.push_back(DItem{i, j, c});
@@ -1699,18 +1704,21 @@ void launch_triples(hfjk_ctx* ctx, const std::vector<Shell>& orb, const std::vec
   auto check = [](hipError_t e) {
     if (e != hipSuccess) throw std::runtime_error("streams of the integral kernels failed");
   };
-  check(hfjk::side_stream(ctx));
+  const bool lanes = !pairs.empty();  // else triple_kernel alone, on s
+  if (lanes) check(hfjk::side_stream(ctx));
   hipStream_t side = ctx->side;
   // The side stream after everything on s so far, and s after the side stream; events of this
   // call's own, so that calls of several threads on one context do not wait for each other's.
   CallEvent forked, joined;
-  check(forked.create());
-  check(joined.create());
+  if (lanes) check(forked.create());
+  if (lanes) check(joined.create());
   auto fork = [&] {
+    if (!lanes) return;
     check(hipEventRecord(forked.event, s));
     check(hipStreamWaitEvent(side, forked.event, 0));
   };
   auto join = [&] {
+    if (!lanes) return;
     check(hipEventRecord(joined.event, side));
     check(hipStreamWaitEvent(s, joined.event, 0));
   };
@@ -1720,7 +1728,7 @@ void launch_triples(hfjk_ctx* ctx, const std::vector<Shell>& orb, const std::vec
   // Pairs that do not survive stay zero; the metric has none.
   if (!metric_mode && hipMemsetAsync(out, 0, total * sizeof(double), s) != hipSuccess)
     throw std::runtime_error("hipMemsetAsync failed");
-  if (!pairs.empty()) {
+  if (lanes) {
     hipLaunchKernelGGL(pair_kernel, dim3((unsigned)pairs.size()), dim3(kPairThreads), 0, side, dev.at<LanePair>(o_pairs),
                        dev.at<DShell>(metric_mode ? o_aux : o_orb), dev.at<DShell>(o_orb), dev.at<double>(o_exps),
                        dev.at<double>(o_coefs), dev.at<double>(metric_mode ? o_nx : o_no), dev.at<double>(o_sph),

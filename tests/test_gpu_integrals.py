@@ -114,6 +114,21 @@ def test_device_integrals_over_all_classes(orbital, auxiliary, scale):
     np.testing.assert_array_equal(dev, dev.T)
 
 
+@pytest.mark.parametrize("momenta", [
+    [(0, 5, 1), (0, 1, 1), (1, 3, 2), (2, 2, 1), (3, 1, 1), (4, 1, 1), (4, 2, 1)],
+    [(0, 17, 1), (1, 16, 1), (5, 1, 1), (2, 3, 2)],
+])
+@pytest.mark.parametrize("shells", [224, 225])
+def test_metric_of_few_and_many_shells(momenta, shells):
+    """Both sides of the number of shells from which the metric goes by lanes, over all classes."""
+    rng = np.random.default_rng(21)
+    aux = _Shells(_random_shells(rng, [momenta[i % len(momenta)] for i in range(shells)], 4.0))
+    host = integrals.metric(aux)
+    dev = integrals.metric_device(aux).cpu().numpy()
+    assert float(np.max(np.abs(dev - host) / np.sqrt(np.outer(np.diag(host), np.diag(host))))) <= 1e-12
+    np.testing.assert_array_equal(dev, dev.T)
+
+
 @pytest.mark.parametrize("distance", [13.8, 15.0, 16.5, 18.0])
 def test_first_batch_of_primitive_pairs_without_a_survivor(distance):
     """Oxygens in cc-pVDZ whose first 64 of 81 s-s primitive pairs the product cut drops, and later ones not."""
