@@ -109,6 +109,12 @@ int syrk_splits(long long npairs, int naux) {
   return (int)(((std::max(1LL, s) + 7) / 8) * 8);
 }
 
+// Aux functions of a run, splits and partial slots of a SYRK.
+struct SyrkPlan {
+  int run, nsplit, nslot;
+};
+enum SyrkColumns { kUnsignedColumns, kSignedColumns, kBf16Columns };  // the last: unsigned in BF16X3
+
 struct Layout {
   // density factorisation region
   size_t dens_a, dens_w, dens_e, dens_info, dens_stats, dens_c, dens_signs, dens_end;
@@ -123,7 +129,8 @@ struct Layout {
   // only the bf16 planes of C^T), and the J partials
   size_t qt, qg, qc, qj, q_end;
   size_t total;
-  int nsplit_j, nsplit_k, nslot_k, run_k, ldo, xrows, npairs;
+  int nsplit_j, slots_k, ldo, xrows, npairs;
+  SyrkPlan syrk[3];  // by SyrkColumns
   long long p, ntiles;
 };
 
@@ -140,12 +147,25 @@ Layout make_layout(const hfjk_ctx* ctx, int nocc, int precision, int nsplit_k = 
   (void)nb;
   L.npairs = hfjk::syrk_pairs(n);
   L.nsplit_j = coulomb_splits(L.ntiles, naux);
-  L.run_k = nsplit_k > 0 ? hfjk::syrk_run_aux(precision, L.ldo)
-                         : hfjk::syrk_run_for(precision, naux, n, L.ldo, ctx->cus);
-  L.nsplit_k = nsplit_k > 0 ? nsplit_k
+  // The three kinds of SYRK columns; BF16X3 asks for its layout as FP32. The split count is modelled
+  // for the unsigned ones; signed columns whose runs differ take a split per run, and the 256 x 256
+  // tiles have a count of their own.
+  L.slots_k = 0;
+  for (int kind = 0; kind < 3; ++kind) {
+    SyrkPlan& p = L.syrk[kind];
+    const int prec = kind == kBf16Columns && precision != HFJK_FP64 ? HFJK_BF16X3 : precision;
+    p.run = nsplit_k > 0 ? hfjk::syrk_run_aux(prec, L.ldo)
+                         : hfjk::syrk_run_for(prec, naux, n, L.ldo, ctx->cus, kind == kSignedColumns);
+    p.nsplit = nsplit_k > 0           ? nsplit_k
                : ctx->syrk_splits > 0 ? ((ctx->syrk_splits + 7) / 8) * 8
-                                       : hfjk::syrk_split_count(precision, naux, n, L.ldo, L.run_k, ctx->cus);
-  L.nslot_k = hfjk::syrk_slots(naux, L.run_k, L.nsplit_k);
+               : kind == kUnsignedColumns
+                   ? hfjk::syrk_split_count(precision, naux, n, L.ldo, p.run, ctx->cus)
+               : kind == kSignedColumns && p.run != L.syrk[kUnsignedColumns].run
+                   ? (hfjk::syrk_slots(naux, p.run, 8) + 7) / 8 * 8
+                   : L.syrk[kUnsignedColumns].nsplit;
+    p.nslot = hfjk::syrk_slots(naux, p.run, p.nsplit);
+    L.slots_k = std::max(L.slots_k, p.nslot);
+  }
   size_t off = 0;
   const size_t nn = (size_t)n * n;
   L.dens_a = off; off = align_up(off + nn * 8);
@@ -171,7 +191,7 @@ Layout make_layout(const hfjk_ctx* ctx, int nocc, int precision, int nsplit_k = 
   L.xs = off; off = align_up(off + (size_t)L.ldo * 8);
   L.xx = off; off = align_up(off + (size_t)naux * L.xrows * L.ldo * es);
   const size_t tile2 = (size_t)hfjk::syrk_tile() * hfjk::syrk_tile();
-  L.xp = off; off = align_up(off + (size_t)L.nslot_k * L.npairs * tile2 * es);
+  L.xp = off; off = align_up(off + (size_t)L.slots_k * L.npairs * tile2 * es);
   L.xct = off; off = align_up(off + npad * L.ldo * 8);
   L.x_end = off;
   off = std::max(L.c_end, L.x_end);
@@ -327,9 +347,11 @@ void exchange_back(hfjk_ctx* ctx, int nocc, bool is_signed, double* out, int pre
   double* sg = at<double>(ws, L.xs);
   void* x = at<void>(ws, L.xx);
   void* part = at<void>(ws, L.xp);
+  const SyrkPlan& plan =
+      L.syrk[is_signed ? kSignedColumns : precision == HFJK_BF16X3 ? kBf16Columns : kUnsignedColumns];
   {
     Stage st(ctx, s, "exchange_syrk");
-    check_hip(hfjk::launch_syrk(x, precision, ctx->naux, ctx->nao, L.ldo, sg, is_signed, L.nsplit_k, L.run_k, part,
+    check_hip(hfjk::launch_syrk(x, precision, ctx->naux, ctx->nao, L.ldo, sg, is_signed, plan.nsplit, plan.run, part,
                                 ctx->syrk_kind, s, nullptr, 0, x16_interleaved(ctx, precision, is_signed, L.ldo), nocc),
               "syrk launch");
   }
@@ -337,7 +359,7 @@ void exchange_back(hfjk_ctx* ctx, int nocc, bool is_signed, double* out, int pre
     Stage st(ctx, s, "exchange_reduce");
     const int rprec = precision == HFJK_FP64 ? HFJK_FP64 : HFJK_FP32;  // BF16X3 partials are FP32
     const int edge = hfjk::syrk_edge(precision, ctx->nao, L.ldo, is_signed, ctx->syrk_kind);
-    check_hip(hfjk::launch_syrk_reduce(part, rprec, L.nslot_k, ctx->nao, edge, out, s), "syrk reduce launch");
+    check_hip(hfjk::launch_syrk_reduce(part, rprec, plan.nslot, ctx->nao, edge, out, s), "syrk reduce launch");
   }
 }
 

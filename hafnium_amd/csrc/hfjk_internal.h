@@ -296,20 +296,22 @@ hipError_t launch_half_transform(const void* b, int precision, long long p, int 
 // the FP32-accumulating modes (FP32, BF16x3) one per run of `run` aux
 // functions (at most syrk_run_aux(precision, ldo), kSyrkRunProducts products
 // per FP32 accumulator, whatever the split count; 0 in FP64).
-// syrk_run_for = the run of a build of that size on `cus` compute units.
+// syrk_run_for = the run of a build of that size on `cus` compute units, for
+// unsigned or signed columns (BF16X3: of the 256 x 256 tiles when unsigned).
 // syrk_slots = the number of partial tiles per pair; launch_syrk_reduce sums
 // them in FP64 in a fixed order.
 constexpr int kSyrkRunProducts = 4096;
 int syrk_run_aux(int precision, int ldo);
-int syrk_run_for(int precision, int naux, int nao, int ldo, int cus);
+int syrk_run_for(int precision, int naux, int nao, int ldo, int cus, bool is_signed);
 int syrk_slots(int naux, int run, int nsplit);
 // Default split count of the SYRK (a multiple of 8) on a device of `cus` compute units.
 int syrk_split_count(int precision, int naux, int nao, int ldo, int run, int cus);
 // auxsign (optional, [naux]): one more factor per aux function on the signed
-// FP64/FP32 direct-LDS kernels; shift (a multiple of 32 below ldo): the
-// second operand's columns rotated, sum_k X[m][k] S_k X[n][(k + shift) mod
-// ldo], on the signed direct-LDS kernels of every precision
-// (hipErrorInvalidValue for a launch that would not run them).
+// FP64/FP32 direct-LDS kernels; shift (below ldo, a multiple of a ring step's
+// columns, 16 in FP64 and 32 else): the second operand's columns rotated,
+// sum_k X[m][k] S_k X[n][(k + shift) mod ldo], on the signed direct-LDS kernels
+// of every precision (hipErrorInvalidValue for a launch that would not run
+// them).
 hipError_t launch_syrk(const void* x, int precision, int naux, int nao, int ldo, const double* signs,
                        bool is_signed, int nsplit, int run, void* partial, int kind, hipStream_t s,
                        const double* auxsign = nullptr, int shift = 0, bool x_ilv = false, int nocc = 0,

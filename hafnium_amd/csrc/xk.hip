@@ -2629,9 +2629,10 @@ static int tile_blocks(int nblk, int eb, int r, int c) {
 // (A fixed target of 2048 workgroups wrote 270 MB of partials whatever the
 // size, and at nao 709 / naux 2503 in FP32 left 25 of 104 splits without a
 // slot.) Signed columns run one workgroup per CU on 128-row tiles and take the
-// same count: within 9 % of the best of 2048, 1024, 512 and 256 workgroups
-// from nao 50 to 1500 (FP64 288 / 1356 / 60 569 us for 523, the largest
-// distance), where the fixed target took 1180 us there and 355 for 32 at 100.
+// same count where their runs are the same: within 9 % of the best of 2048,
+// 1024, 512 and 256 workgroups from nao 50 to 1500 (FP64 288 / 1356 / 60 569
+// us for 523, the largest distance), where the fixed target took 1180 us there
+// and 355 for 32 at 100.
 struct SplitModel {
   int npairs, slots;
   bool partials;
@@ -2861,11 +2862,38 @@ int syrk_run_aux(int precision, int ldo) {
 // aux functions, 225 us). Shorter runs only add FP64 sums of partial tiles, so
 // they go down to a workgroup per CU, and no further than 128 columns of X,
 // eight ring steps, where filling the ring costs as much as the products.
-int syrk_run_for(int precision, int naux, int nao, int ldo, int cus) {
+// The XCDs take the runs of 128-row tiles in turn, so their number is a
+// multiple of eight: 18 runs of 15 tiles gave some XCDs 45 workgroups for
+// their 32 CUs where 16 give each 30 (FP32 600 / 2000 / nocc 30: J and K 1.07
+// -> 0.95 ms, signed 1.05 -> 0.83). BF16x3's unsigned 256 x 256 tiles, fewer
+// and larger, take as many runs as there are CUs per 128-row tile (a multiple
+// of eight below it cost 2 to 3 % from nao 250 to 450).
+// Signed columns run one workgroup per CU, so where 4096 products end the runs
+// before they fit a round, runs that fill two to four rounds evenly are shorter
+// in all (500 / 1750 / 60: 28 runs of 64 in two rounds, 48 of 37 too, 1.22 ->
+// 0.99 ms); unsigned ones, two to a CU, fill the gaps themselves and only pay
+// for the partials (288 / 1356 / 200: 0.85 -> 0.91).
+int syrk_run_for(int precision, int naux, int nao, int ldo, int cus, bool is_signed) {
   const int most = syrk_run_aux(precision, ldo);
   if (most == 0) return 0;
-  const long long even = ((long long)naux * syrk_pairs(nao) + cus - 1) / cus;
-  return (int)std::max(1LL, std::min<long long>(most, std::max<long long>(even, (128 + ldo - 1) / ldo)));
+  const int pairs = syrk_pairs(nao), xcd = std::max(1, cus / 8);
+  const int least = std::min(most, (128 + ldo - 1) / ldo);
+  const bool tiles256 = precision == HFJK_BF16X3 && !is_signed;
+  const long long slots = 8 * std::max(1, xcd / pairs);
+  const long long even = tiles256 ? ((long long)naux * pairs + cus - 1) / cus : (naux + slots - 1) / slots;
+  const int run = (int)std::max<long long>(least, std::min<long long>(most, even));
+  if (!is_signed || run < most) return run;
+  int best = most;
+  double best_us = 1e300;  // rounds of 0.85 us per 16 columns and 4 us to fill and drain, and the partials
+  for (long long k = (naux + 8LL * most - 1) / (8LL * most); k * pairs <= 4 * xcd; ++k) {
+    const int cut = (int)std::max<long long>(least, (naux + 8 * k - 1) / (8 * k));
+    const double us = (k * pairs + xcd - 1) / xcd * (0.85 * cut * ldo / 16 + 4.0) + 8.0 * k * pairs * 0.026;
+    if (us < best_us) {
+      best_us = us;
+      best = cut;
+    }
+  }
+  return best;
 }
 
 int syrk_slots(int naux, int run, int nsplit) { return run == 0 ? nsplit : (naux + run - 1) / run; }

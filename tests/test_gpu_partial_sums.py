@@ -195,3 +195,26 @@ def test_short_runs_of_the_single_precision_syrk(precision, nao, naux, nocc):
         j, k = jk.jk_occupied(c)
         assert np.max(np.abs(k - k_ref)) <= tol * np.max(np.abs(k_ref))
         assert np.max(np.abs(j - j_ref)) <= tol * np.max(np.abs(j_ref))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("nao,naux,nocc", [(9, 1, 1), (24, 84, 5), (96, 336, 20), (130, 257, 33), (192, 672, 40),
+                                           (260, 640, 250), (260, 700, 250)])
+def test_runs_of_signed_columns(precision, nao, naux, nocc):
+    """Signed columns: runs of a round, of two rounds (the last shape) and at the limit of products, split counts of
+    their own and given ones."""
+    from hafnium_amd import _lib
+    from hafnium_amd.coulomb_exchange import MI355XCoulombExchange
+    from tests.tolerances import BF16X3_REL_TOL, FP32_REL_TOL, FP64_REL_TOL
+
+    b = synthetic.tensor_full(13, naux, nao)
+    c = synthetic.occupied_orbitals(13, nao, nocc)
+    signs = np.where(np.arange(nocc) % 3 == 1, -1.0, 1.0)
+    x = b @ c
+    k_ref = np.tensordot(x * signs, x, axes=((0, 2), (0, 2)))
+    scale = np.max(np.abs(np.tensordot(x, x, axes=((0, 2), (0, 2)))))  # the sum of magnitudes' size
+    tol = {"fp64": FP64_REL_TOL, "fp32": FP32_REL_TOL, "bf16x3": BF16X3_REL_TOL}[precision]
+    jk = MI355XCoulombExchange(b, precision=precision)
+    for splits in (0, 8, 200):
+        jk.set_tuning(_lib.TUNE_SYRK_SPLITS, splits)
+        assert np.max(np.abs(jk.exchange_occupied(c, signs) - k_ref)) <= tol * scale, splits
