@@ -85,8 +85,6 @@ __device__ __forceinline__ void rc_of(int tile, int& r, int& c) {
   c = tile - rr * (rr + 1) / 2;
 }
 
-__device__ __forceinline__ long long tix(int r, int c) { return (long long)r * (r + 1) / 2 + c; }
-
 __device__ __forceinline__ uint16_t to_bf16(float x) {
   uint32_t u = __float_as_uint(x);
   if ((u & 0x7F800000u) == 0x7F800000u) return (uint16_t)((u >> 16) | ((u & 0xFFFFu) ? 0x40u : 0u));

@@ -29,7 +29,6 @@ typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 constexpr int kEigThreads = 512;
 constexpr int kEigWaves = kEigThreads / 64;
 constexpr int kEigMaxN = 512;
-constexpr int kEigMaxCols = kEigMaxN / 64;  // 64-row chunks of a vector
 constexpr int kEigRegVecs = 64;             // nvec up to this: vectors stay in registers, Cholesky QR
 constexpr int kGs = 65;                     // row stride of the Gram matrix and its inverse factor in LDS
 

@@ -820,8 +820,8 @@ int hfjk_int3c2e(const hfjk_basis* aux, const hfjk_basis* orbital, double* out) 
 // def2-universal-jkfit, 0.9 GB of results): what bounds it is the chain of
 // primitives in a wave (the latency of each one's table and scalar loads, about
 // 0.5 us), so contracted pairs are shared by four waves and contracted aux
-// functions by neighbouring lanes. 12 waters' (P|uv) and (P|Q) take 3.9 ms, 1
-// water's 1.75; one workgroup per triple took 82 ms on the former (71 in the
+// functions by neighbouring lanes. 12 waters' (P|uv) and (P|Q) take 3.5 ms, 1
+// water's 1.8; one workgroup per triple took 82 ms on the former (71 in the
 // kernel, one lane building tables while 63 waited, and 5 in a size check over
 // all triples on the host).
 //

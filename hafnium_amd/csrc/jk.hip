@@ -274,7 +274,9 @@ __global__ __launch_bounds__(kThreads) void split_factor_kernel(const double* __
 // steps per launch; past that each step is two launches (the pivot in one
 // workgroup, the column across the GPU).
 constexpr int kPcholThreads = 1024;
-constexpr int kPcholPanelRows = 4096, kPcholPanelColumns = 512;
+// pchol_in_panels ends the panels at 120000 elements: 1875 rows of the first 64 columns, 346 columns
+// of as many rows.
+constexpr int kPcholPanelRows = 1920, kPcholPanelColumns = 352;
 
 // diag = diag(D); st: cut = tol * max diag, no stop, rank 0. One workgroup.
 __global__ __launch_bounds__(kPcholThreads) void pchol_init_kernel(const double* __restrict__ d, int n, double tol,

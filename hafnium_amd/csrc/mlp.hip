@@ -185,11 +185,16 @@ __device__ void gemm_tile(const GemmArgs& g, int tile_row, int tile_col, GemmSme
     __syncthreads();
     if (s0 + kWaves + wave < steps) fetch(s0 + kWaves + wave);
     if (wave < 4) {
-      const int count = min(kWaves, steps - s0);
-#pragma unroll 4
-      for (int s = 0; s < count; ++s)
+      auto product = [&](int s) {
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm.step[round][s][mi][lane], sm.step[round][s][2 + ni][lane], acc,
                                                       0, 0, 0);
+      };
+      if (steps - s0 >= kWaves) {
+#pragma unroll
+        for (int s = 0; s < kWaves; ++s) product(s);
+      } else {
+        for (int s = 0; s < steps - s0; ++s) product(s);
+      }
     }
   }
   float loss = 0.f;
@@ -376,7 +381,7 @@ int mguard(hfjk_ctx* ctx, F&& body) {
   }
 }
 
-constexpr int kMaxRows = 65535 * 64;  // of a product: the entry points' limit
+constexpr int kMaxRows = 65535 * 64;  // of a product: part of the entry points' contract
 
 // launch(first, count) for all of `tiles` workgroups of kGemmT threads, at
 // most 2^31 work-items at a time (a grid holds less than 2^32).

@@ -124,7 +124,7 @@ __device__ __forceinline__ f4 mma3(bf8 ah, bf8 al, bf8 bh, bf8 bl, f4 acc) {
 //   elements per 16 bytes), so a tile stored as (r, kt) is read as 16-byte
 //   groups along its rows and one stored as (kt, r) as 128-byte runs of its
 //   columns, without a transpose.
-// * C, in the order the MFMA operand reads it (launch_orbital_fragments),
+// * C, in the order the MFMA operand reads it (launch_prepare_orbitals),
 //   goes by direct-LDS loads into one of two stage buffers shared by the
 //   waves: one barrier per step, 16-byte conflict-free LDS reads.
 //
