@@ -113,7 +113,7 @@ int syrk_splits(long long npairs, int naux) {
 struct SyrkPlan {
   int run, nsplit, nslot;
 };
-enum SyrkColumns { kUnsignedColumns, kSignedColumns, kBf16Columns };  // the last: unsigned in BF16X3
+enum SyrkColumns { kUnsignedColumns, kSignedColumns, kTiles256 };  // the last: unsigned, 256 x 256 tiles of BF16X3
 
 struct Layout {
   // density factorisation region
@@ -153,7 +153,7 @@ Layout make_layout(const hfjk_ctx* ctx, int nocc, int precision, int nsplit_k = 
   L.slots_k = 0;
   for (int kind = 0; kind < 3; ++kind) {
     SyrkPlan& p = L.syrk[kind];
-    const int prec = kind == kBf16Columns && precision != HFJK_FP64 ? HFJK_BF16X3 : precision;
+    const int prec = kind == kTiles256 && precision != HFJK_FP64 ? HFJK_BF16X3 : precision;
     p.run = nsplit_k > 0 ? hfjk::syrk_run_aux(prec, L.ldo)
                          : hfjk::syrk_run_for(prec, naux, n, L.ldo, ctx->cus, kind == kSignedColumns);
     p.nsplit = nsplit_k > 0           ? nsplit_k
@@ -347,8 +347,9 @@ void exchange_back(hfjk_ctx* ctx, int nocc, bool is_signed, double* out, int pre
   double* sg = at<double>(ws, L.xs);
   void* x = at<void>(ws, L.xx);
   void* part = at<void>(ws, L.xp);
-  const SyrkPlan& plan =
-      L.syrk[is_signed ? kSignedColumns : precision == HFJK_BF16X3 ? kBf16Columns : kUnsignedColumns];
+  const bool tiles256 =
+      precision == HFJK_BF16X3 && hfjk::syrk16_tiles256(ctx->nao, L.ldo, is_signed, ctx->syrk_kind, 0);
+  const SyrkPlan& plan = L.syrk[is_signed ? kSignedColumns : tiles256 ? kTiles256 : kUnsignedColumns];
   {
     Stage st(ctx, s, "exchange_syrk");
     check_hip(hfjk::launch_syrk(x, precision, ctx->naux, ctx->nao, L.ldo, sg, is_signed, plan.nsplit, plan.run, part,
