@@ -305,24 +305,26 @@ __global__ __launch_bounds__(kCholThreads) void kp_cholesky_kernel(const double2
 }
 
 // Per k: max |D - D^H|, max |D| and the largest row sum of |D - L L^H|, which
-// bounds its largest eigenvalue (atomic max of bits). A wave per row.
+// bounds its largest eigenvalue (atomic max of bits). A workgroup per row, so
+// that a thread's chain is one pass over the rank.
 __global__ __launch_bounds__(kThreads) void kp_residual_kernel(const double2* __restrict__ density, int n,
                                                                const double2* __restrict__ lmat,
                                                                KpState* __restrict__ state) {
+  __shared__ double part[kThreads / 64];
   const long long nn = (long long)n * n;
   const double2* d = density + blockIdx.y * nn;
   const double2* l = lmat + blockIdx.y * nn;
   KpState* st = state + blockIdx.y;
   const int rank = st->rank;
-  const int lane = threadIdx.x & 63;
   double asym = 0.0, mag = 0.0, worst = 0.0;
-  for (int r = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); r < n; r += gridDim.x * (kThreads / 64)) {
+  for (int r = blockIdx.x; r < n; r += gridDim.x) {
     double sum = 0.0;
-    for (int c = lane; c < n; c += 64) {
+    for (int c = threadIdx.x; c < n; c += kThreads) {
       double2 a = d[(long long)r * n + c];
       const double2 t = d[(long long)c * n + r];
       asym = fmax(asym, hypot(a.x - t.x, a.y + t.y));
       mag = fmax(mag, hypot(a.x, a.y));
+#pragma unroll 4
       for (int j = 0; j < rank; ++j) {
         const double2 u = l[(long long)j * n + r], v = l[(long long)j * n + c];
         const double2 m = cmul(u, make_double2(v.x, -v.y));
@@ -332,9 +334,14 @@ __global__ __launch_bounds__(kThreads) void kp_residual_kernel(const double2* __
       sum += fabs(a.x) + fabs(a.y);
     }
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    sum = (part[0] + part[1]) + (part[2] + part[3]);
     // Not fmax, which would drop a NaN: a NaN must fail the host's test.
     worst = sum > worst || sum != sum ? sum : worst;
+    __syncthreads();
   }
+  if (threadIdx.x >= 64) worst = 0.0;  // every thread has it
   unsigned long long* out[3] = {&st->asym, &st->mag, &st->residual};
   double v[3] = {asym, mag, worst};
 #pragma unroll
@@ -500,7 +507,7 @@ hipError_t launch_kp_cholesky(const void* density, int nk, int nao, void* l, KpS
   double* diag = (double*)((double2*)l + (long long)nk * nao * nao);
   hipLaunchKernelGGL(kp_cholesky_kernel, dim3((unsigned)nk), dim3(kCholThreads), 0, s, (const double2*)density, nao,
                      (double2*)l, diag, st);
-  const unsigned gx = (unsigned)std::min((nao + kThreads / 64 - 1) / (kThreads / 64), 1024);
+  const unsigned gx = (unsigned)std::min(nao, 1024);
   hipLaunchKernelGGL(kp_residual_kernel, dim3(gx, (unsigned)nk), dim3(kThreads), 0, s, (const double2*)density, nao,
                      (const double2*)l, st);
   return hipGetLastError();
